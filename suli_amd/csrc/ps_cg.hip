@@ -1549,9 +1549,14 @@ void launch_refresh(const ProbDev *P, const TileRef *t1, int nt1, const TileRef 
                     int nprobs, int grid, StepRef step, hipStream_t s)
 {
     hipLaunchKernelGGL(k_refresh_e, dim3(std::min(grid, nt1)), dim3(kThreads), 0, s, P, t1, nt1, step);
+    launch_true_residual(P, t3, nt3, grid, step, s);
+    hipLaunchKernelGGL(k_refresh_decide, dim3(nprobs), dim3(kThreads), 0, s, P, probs, step);
+}
+
+void launch_true_residual(const ProbDev *P, const TileRef *t3, int nt3, int grid, StepRef step, hipStream_t s)
+{
     hipLaunchKernelGGL((k_true_residual<true, false>), dim3(std::min(grid, nt3)), dim3(kThreads), 0, s, P, t3, nt3,
                        step);
-    hipLaunchKernelGGL(k_refresh_decide, dim3(nprobs), dim3(kThreads), 0, s, P, probs, step);
 }
 
 void launch_finish(const ProbDev *P, const TileRef *t3, int nt3, const int *probs, int nprobs, int grid,

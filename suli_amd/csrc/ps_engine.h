@@ -55,6 +55,9 @@ struct Slot {
     bool own_block = true;     // taken from the engine's pool (else the caller's)
     double *prd1_out = nullptr;  // device prd1 (halo box) written at the end
     const uint8_t *solid = nullptr;  // solid-cell mask (device), if any
+    bool mg = false;           // multigrid-preconditioned: n0 counts multigrid steps
+    suli_ps_grid grid{};       // what it was admitted with, for a second set-up
+    SetupIn in{};
     int n0 = 0;
     int user = -1;             // caller's index for this problem
     CgScalars status{};        // last status read on the host
@@ -63,6 +66,13 @@ struct Slot {
 // Bytes of device memory a problem of this size and precision needs (for
 // any tile depth kz >= kMinKz).
 size_t problem_bytes(int nx, int ny, int nz, bool mixed);
+
+// Whether the multigrid iteration serves solves with these options.
+bool mg_applies(const SolveOpts &o);
+// Launch-table entries its kernels need for a mixed problem on this grid
+// beside the replacement's (3-D and 1-D tiles of make_geo's default shape);
+// 0: it does not apply to the grid.
+long long mg_entries(const Geo &g);
 
 constexpr int kMinKz = 2;
 
@@ -158,6 +168,9 @@ public:
 private:
     int fail(int code, const std::string &msg);
     int rebuild_tables();
+    // Descriptor and set-up kernels of a slot whose geometry and block stand;
+    // multi: by the multigrid iteration where it applies.
+    int setup_slot(int si, bool multi, hipEvent_t wait_ev);
     int enqueue_chunk(int K, bool timing);
     int enqueue_steps_direct(int nsteps, bool timing);
     int enqueue_group_graph();
@@ -166,6 +179,7 @@ private:
     void reap_graphs(bool wait);
     int finish(const std::vector<int> &done);
     int next_chunk_len() const;
+    int plain_count() const;
     bool refresh_may_be_due(int step) const;
 
     hipStream_t s_ = nullptr;
@@ -178,10 +192,12 @@ private:
     CgScalars *h_final_ = nullptr;     // pinned [max_slots]
     hipEvent_t ev_status_[2] = {nullptr, nullptr};
     int status_step_[2] = {0, 0};      // global step when each status copy was queued
+    int status_mstep_[2] = {0, 0};     // and multigrid step
     int pend_[2] = {0, 0};             // status slots of chunks not yet read (FIFO)
     int pend_head_ = 0, npend_ = 0;
     int max_slots_ = 0;
     int step_ = 0;                     // global step of the last enqueued iteration
+    int mstep_ = 0;                    // multigrid problems' own step count
     int chunk_idx_ = 0;
     bool tables_dirty_ = true;
     void *d_fin_ = nullptr;            // tables of the problems being finished
@@ -190,7 +206,13 @@ private:
     struct Tables {
         std::vector<TileRef> t3_64, t1_64, t3_32, t1_32;
         std::vector<int> mixed_probs;
+        // multigrid problems: fine tiles, 3-D and 1-D tiles of the
+        // replacement, coarse levels
+        std::vector<TileRef> mg_fine, mg_t3, mg_t1, mg_lev;
+        std::vector<int> mg_probs;
     } tab_;
+    MgTables mgt_;                     // the same on the device
+    int off_mg_t3_ = 0, off_mg_t1_ = 0;
     TileRef *d_tab_ = nullptr;
     int *d_probs_list_ = nullptr;
     size_t tab_cap_ = 0, probs_cap_ = 0;

@@ -272,6 +272,11 @@ int Engine::reserve(int entries)
     tab_.t3_32.reserve(ntab);
     tab_.t1_32.reserve(ntab);
     tab_.mixed_probs.reserve(max_slots_);
+    tab_.mg_fine.reserve(ntab);
+    tab_.mg_t3.reserve(ntab);
+    tab_.mg_t1.reserve(ntab);
+    tab_.mg_lev.reserve(ntab);
+    tab_.mg_probs.reserve(max_slots_);
     pool_.reserve(max_slots_);
     fin_t3_.reserve(ntab);
     run_slots_.reserve(max_slots_);
@@ -290,10 +295,38 @@ void Engine::cached_shape(int nx, int ny, int nz, bool mixed, int *kz, int *vx) 
     *vx = hit != tuned_.end() ? hit->second.vx : 0;
 }
 
+// Active problems that iterate by plain CG.
+int Engine::plain_count() const
+{
+    int n = 0;
+    for (const auto &s : slots_) n += s.active && !s.finished && !s.mg;
+    return n;
+}
+
 int Engine::active_count() const
 {
     int n = 0;
     for (const auto &s : slots_) n += s.active && !s.finished;
+    return n;
+}
+
+// The multigrid iteration serves mixed solves that any cap leaves room to
+// converge; keep_null and stored_residual name properties of the plain CG
+// iteration.
+bool mg_applies(const SolveOpts &o)
+{
+    return o.mixed && !o.keep_null && !o.store_r && o.max_iter >= kMgMinCap;
+}
+
+long long mg_entries(const Geo &g)
+{
+    Carver cv{nullptr};
+    ProbDev pd{};
+    const int nt3 = spmv_tiles(g);
+    carve(cv, g, true, nt3, vec_tiles(g.n), pd);
+    if (!mg_plan(g, true, nullptr, nullptr, 2 * (size_t)g.n, pd) || 3 * pd.ntm > 8 * nt3) return 0;
+    long long n = pd.ntm;
+    for (int l = 1; l < pd.lbot; ++l) n += mg_down_tiles(pd, l) + mg_up_tiles(pd, l);
     return n;
 }
 
@@ -312,7 +345,15 @@ int Engine::admit(const suli_ps_grid &gr, const SetupIn &in, double *prd1_out, c
     sl = Slot{};
     int kz = o.kz > 0 ? std::max(o.kz, kMinKz) : 0;
     int vx = o.vx > 0 ? o.vx : 0;
-    if ((kz == 0 || vx == 0) && autotune_ && no_alloc_active()) {
+    // the tuner's shapes are the plain CG kernels': nothing to tune otherwise
+    const Geo g0 = make_geo(gr.nx, gr.ny, gr.nz, gr.ccx0 == 0, gr.ccy0 == 0);
+    if (mg_applies(o) && mg_entries(g0) > 0) {
+        // the shape a fall-back to plain CG would take
+        int kz_c = 0, vx_c = 0;
+        if (autotune_) cached_shape(gr.nx, gr.ny, gr.nz, o.mixed, &kz_c, &vx_c);
+        if (kz == 0) kz = kz_c;
+        if (vx == 0) vx = vx_c;
+    } else if ((kz == 0 || vx == 0) && autotune_ && no_alloc_active()) {
         // tuning allocates a scratch problem: take what is recorded instead
         int kz_c = 0, vx_c = 0;
         cached_shape(gr.nx, gr.ny, gr.nz, o.mixed, &kz_c, &vx_c);
@@ -326,27 +367,62 @@ int Engine::admit(const suli_ps_grid &gr, const SetupIn &in, double *prd1_out, c
         if (kz == 0) kz = kz_t;
         if (vx == 0) vx = vx_t;
     }
-    sl.g = make_geo(gr.nx, gr.ny, gr.nz, gr.ccx0 == 0, gr.ccy0 == 0, kz, o.mixed ? vx : 1);
-    sl.g.dtop = gr.top_bc == 1 ? 1 : 0;
+    sl.grid = gr;
+    sl.in = in;
     sl.o = o;
-    sl.o.kz = sl.g.kz;
-    sl.o.vx = lane_code(sl.g);
-    const int nt3 = spmv_tiles(sl.g), nt1 = vec_tiles(sl.g.n);
+    sl.o.kz = kz;
+    sl.o.vx = vx;
     sl.bytes = problem_bytes(gr.nx, gr.ny, gr.nz, o.mixed);
     sl.own_block = block == nullptr;
     sl.block = block ? block : pool_.get(sl.bytes, err_);
     if (!sl.block) return SULI_PS_ENOMEM;
-    Carver cv{static_cast<char *>(sl.block)};
+    sl.prd1_out = prd1_out;
+    sl.solid = in.solid;
+    sl.user = user;
+    sl.used = true;
+    sl.active = true;
+    const int rc = setup_slot(si, true, wait_ev);
+    if (rc) return rc;
+    if (slot_out) *slot_out = si;
+    return 0;
+}
+
+int Engine::setup_slot(int si, bool multi, hipEvent_t wait_ev)
+{
+    Slot &sl = slots_[si];
+    const suli_ps_grid &gr = sl.grid;
+    const SetupIn &in = sl.in;
+    const SolveOpts &o = sl.o;
     ProbDev &pd = sl.pd;
-    pd = ProbDev{};
-    pd.g = sl.g;
-    carve(cv, sl.g, o.mixed, nt3, nt1, pd);
+    int nt3 = 0, nt1 = 0;
+    // the multigrid kernels have a tiling of their own: the replacement's
+    // kernels, which walk one cell per lane, take the default shape
+    sl.mg = false;
+    for (const bool mg : {true, false}) {
+        if (mg && !(multi && mg_applies(o))) continue;
+        sl.g = make_geo(gr.nx, gr.ny, gr.nz, gr.ccx0 == 0, gr.ccy0 == 0, mg ? 0 : o.kz, mg ? 1 : o.mixed ? o.vx : 1);
+        sl.g.dtop = gr.top_bc == 1 ? 1 : 0;
+        nt3 = spmv_tiles(sl.g);
+        nt1 = vec_tiles(sl.g.n);
+        Carver cv{static_cast<char *>(sl.block)};
+        pd = ProbDev{};
+        pd.g = sl.g;
+        carve(cv, sl.g, o.mixed, nt3, nt1, pd);
+        if (mg) {
+            sl.mg = mg_plan(sl.g, o.mixed, pd.p32 + 2 * pd.pslot, reinterpret_cast<float *>(pd.r),
+                            2 * (size_t)sl.g.n, pd) &&
+                    3 * pd.ntm <= 8 * nt3;
+            if (sl.mg) break;
+        }
+    }
     // constant density (IPA, 9_grad.f90:109-116) and no solid mask: the
-    // iteration kernels read per-plane tables instead of the face arrays
+    // iteration kernels read per-plane tables instead of the face arrays (the
+    // multigrid ones the row tables, whose rows then all hold the plane's
+    // values)
     if (gr.t_press != 2 || in.solid) {
         pd.tx = pd.ty = pd.tz = nullptr;
         pd.tx32 = pd.ty32 = pd.tz32 = nullptr;
-    } else {
+    } else if (!sl.mg) {
         pd.rx32 = pd.ry32 = pd.rz32 = nullptr;
         pd.rowreg = nullptr;
     }
@@ -355,13 +431,8 @@ int Engine::admit(const suli_ps_grid &gr, const SetupIn &in, double *prd1_out, c
     pd.mixed = o.mixed ? 1 : 0;
     pd.store_r = o.mixed && o.store_r ? 1 : 0;
     pd.S = d_status_ + si;
-    sl.n0 = step_ + 1;   // iteration 1 runs at the next global step
+    sl.n0 = (sl.mg ? mstep_ : step_) + 1;   // iteration 1 runs at the next step
     pd.n0 = sl.n0;
-    sl.prd1_out = prd1_out;
-    sl.solid = in.solid;
-    sl.user = user;
-    sl.used = true;
-    sl.active = true;
 
     // initial scalars and the descriptor, staged through pinned memory
     CgScalars s0{};
@@ -382,7 +453,8 @@ int Engine::admit(const suli_ps_grid &gr, const SetupIn &in, double *prd1_out, c
     }
     s0.done_at = kNotDone;
     s0.skip_e_at = -1;
-    s0.next_refresh = kFirstRefresh;
+    s0.next_refresh = sl.mg ? kNotDone : kFirstRefresh;
+    s0.mg = sl.mg ? 1 : 0;
     sl.status = s0;
     const size_t need = sizeof(CgScalars) + sizeof(ProbDev);
     int stg;
@@ -420,14 +492,14 @@ int Engine::admit(const suli_ps_grid &gr, const SetupIn &in, double *prd1_out, c
         launch_face_tables(sl.g, pd.sx, pd.sy, pd.sz, pd.sx32, pd.sy32, pd.sz32, const_cast<double *>(pd.tx),
                            const_cast<double *>(pd.ty), const_cast<double *>(pd.tz), const_cast<float *>(pd.tx32),
                            const_cast<float *>(pd.ty32), const_cast<float *>(pd.tz32), s_);
-    else if (pd.rowreg)
+    if (pd.rowreg)
         launch_row_tables(sl.g, pd.sx32, pd.sy32, pd.sz32, const_cast<float *>(pd.rx32), const_cast<float *>(pd.ry32),
                           const_cast<float *>(pd.rz32), const_cast<unsigned *>(pd.rowreg), s_);
     launch_init(sl.g, in, Op<double>{pd.sx, pd.sy, pd.sz}, pd.d, pd.b, pd.e, pd.r, o.mixed ? nullptr : pd.r,
                 pd.r32, pd.c32, pd.P, init_blocks(sl.g), pd.S, s_);
+    if (sl.mg) launch_mg_setup(pd, d_probs_ + si, in, s_);
     ECHK(hipGetLastError());
     tables_dirty_ = true;
-    if (slot_out) *slot_out = si;
     return rc;
 }
 
@@ -447,10 +519,22 @@ int Engine::rebuild_tables()
     tab_.t3_32.clear();
     tab_.t1_32.clear();
     tab_.mixed_probs.clear();
+    tab_.mg_fine.clear();
+    tab_.mg_t3.clear();
+    tab_.mg_t1.clear();
+    tab_.mg_lev.clear();
+    tab_.mg_probs.clear();
     table_cells_ = 0;
     for (int i = 0; i < max_slots_; ++i) {
         const Slot &sl = slots_[i];
         if (!sl.active || sl.finished) continue;
+        if (sl.mg) {
+            for (int t = 0; t < sl.pd.ntm; ++t) tab_.mg_fine.push_back({i, t});
+            for (int t = 0; t < sl.pd.nt3; ++t) tab_.mg_t3.push_back({i, t});
+            for (int t = 0; t < sl.pd.nt1; ++t) tab_.mg_t1.push_back({i, t});
+            tab_.mg_probs.push_back(i);
+            continue;
+        }
         table_cells_ += sl.g.n;
         auto &t1 = sl.o.mixed ? tab_.t1_32 : tab_.t1_64;
         if (!sl.o.mixed)
@@ -463,7 +547,7 @@ int Engine::rebuild_tables()
         sub_t3_32[w] = (int)tab_.t3_32.size();
         for (int i = 0; i < max_slots_; ++i) {
             const Slot &sl = slots_[i];
-            if (!sl.active || sl.finished || !sl.o.mixed || lane_kind(sl.g) != w) continue;
+            if (!sl.active || sl.finished || sl.mg || !sl.o.mixed || lane_kind(sl.g) != w) continue;
             for (int t = 0; t < sl.pd.nt3; ++t) tab_.t3_32.push_back({i, t});
         }
         cnt_t3_32[w] = (int)tab_.t3_32.size() - sub_t3_32[w];
@@ -472,8 +556,23 @@ int Engine::rebuild_tables()
     off_t1_64 = off_t3_64 + (int)tab_.t3_64.size();
     off_t3_32 = off_t1_64 + (int)tab_.t1_64.size();
     off_t1_32 = off_t3_32 + (int)tab_.t3_32.size();
-    const size_t ntab = off_t1_32 + tab_.t1_32.size();
-    const size_t nprobs = tab_.mixed_probs.size();
+    // multigrid: coarse levels' entries, each level's down and up tables
+    int off_lev[2][kMgLevels] = {};
+    for (int l = 1; l < kMgLevels; ++l)
+        for (int up = 0; up < 2; ++up) {
+            off_lev[up][l] = (int)tab_.mg_lev.size();
+            for (int i : tab_.mg_probs) {
+                const int nt = up ? mg_up_tiles(slots_[i].pd, l) : mg_down_tiles(slots_[i].pd, l);
+                for (int t = 0; t < nt; ++t) tab_.mg_lev.push_back({i, t});
+            }
+            (up ? mgt_.nup : mgt_.ndown)[l] = (int)tab_.mg_lev.size() - off_lev[up][l];
+        }
+    const int off_mg = off_t1_32 + (int)tab_.t1_32.size();
+    off_mg_t3_ = off_mg + (int)tab_.mg_fine.size();
+    off_mg_t1_ = off_mg_t3_ + (int)tab_.mg_t3.size();
+    const int off_mg_lev = off_mg_t1_ + (int)tab_.mg_t1.size();
+    const size_t ntab = off_mg_lev + tab_.mg_lev.size();
+    const size_t nprobs = tab_.mixed_probs.size() + tab_.mg_probs.size();
     if (ntab > tab_cap_ || nprobs > probs_cap_ || !d_tab_) {
         NO_ALLOC_HERE("grow the launch tables");
         // grow: buffers still read by queued kernels are freed after a sync
@@ -506,6 +605,19 @@ int Engine::rebuild_tables()
     std::copy(tab_.t1_32.begin(), tab_.t1_32.end(), ht + off_t1_32);
     int *hp = reinterpret_cast<int *>(h + align_up(sizeof(TileRef) * ntab, 64));
     std::copy(tab_.mixed_probs.begin(), tab_.mixed_probs.end(), hp);
+    std::copy(tab_.mg_probs.begin(), tab_.mg_probs.end(), hp + tab_.mixed_probs.size());
+    std::copy(tab_.mg_fine.begin(), tab_.mg_fine.end(), ht + off_mg);
+    std::copy(tab_.mg_t3.begin(), tab_.mg_t3.end(), ht + off_mg_t3_);
+    std::copy(tab_.mg_t1.begin(), tab_.mg_t1.end(), ht + off_mg_t1_);
+    std::copy(tab_.mg_lev.begin(), tab_.mg_lev.end(), ht + off_mg_lev);
+    mgt_.fine = d_tab_ + off_mg;
+    mgt_.nfine = (int)tab_.mg_fine.size();
+    mgt_.probs = d_probs_list_ + tab_.mixed_probs.size();
+    mgt_.nprobs = (int)tab_.mg_probs.size();
+    for (int l = 1; l < kMgLevels; ++l) {
+        mgt_.down[l] = d_tab_ + off_mg_lev + off_lev[0][l];
+        mgt_.up[l] = d_tab_ + off_mg_lev + off_lev[1][l];
+    }
     if (ntab) ECHK(hipMemcpyAsync(d_tab_, ht, sizeof(TileRef) * ntab, hipMemcpyHostToDevice, s_));
     if (nprobs) ECHK(hipMemcpyAsync(d_probs_list_, hp, sizeof(int) * nprobs, hipMemcpyHostToDevice, s_));
     ECHK(hipEventRecord(ev_stage_[stg], s_));
@@ -521,6 +633,7 @@ int Engine::rebuild_tables()
 // every iteration and only need the host to notice it.
 int Engine::next_chunk_len() const
 {
+    if (plain_count() == 0) return chunk_ > 0 ? chunk_ : kMgChunk;
     if (chunk_ > 0) return (chunk_ + kRefreshGrain - 1) / kRefreshGrain * kRefreshGrain;
     bool any_mixed = false;
     long long biggest = 0;
@@ -528,6 +641,7 @@ int Engine::next_chunk_len() const
     for (int i = 0; i < max_slots_; ++i) {
         const Slot &sl = slots_[i];
         if (!sl.active || sl.finished) continue;
+        if (sl.mg) continue;
         biggest = std::max(biggest, sl.g.n);
         if (!sl.o.mixed) continue;
         any_mixed = true;
@@ -548,7 +662,7 @@ bool Engine::refresh_may_be_due(int s) const
 {
     for (int i = 0; i < max_slots_; ++i) {
         const Slot &sl = slots_[i];
-        if (!sl.active || sl.finished || !sl.o.mixed) continue;
+        if (!sl.active || sl.finished || sl.mg || !sl.o.mixed) continue;
         const int n = s - sl.n0 + 1;
         if (n >= sl.status.next_refresh || n > sl.o.max_iter || sl.status.done_at != kNotDone) return true;
     }
@@ -585,13 +699,15 @@ int Engine::enqueue_steps_direct(int nsteps, bool timing)
 {
     const int n3_64 = (int)tab_.t3_64.size(), n1_64 = (int)tab_.t1_64.size();
     const int n3_32 = (int)tab_.t3_32.size(), n1_32 = (int)tab_.t1_32.size();
-    const int nmix = (int)tab_.mixed_probs.size();
+    const int nmix = (int)tab_.mixed_probs.size(), nmg = (int)tab_.mg_probs.size();
+    const bool plain = n3_64 || n3_32;
     for (int it = 0; it < nsteps; ++it) {
-        ++step_;
+        if (plain || !nmg) ++step_;
+        if (nmg) ++mstep_;
         const StepRef sr{nullptr, step_, nullptr};
         // timing windows of kTimeSteps consecutive steps (events only at
         // their ends, so the per-step figure is the launches' own time)
-        const int ph = step_ % kTimeStride;
+        const int ph = (plain || !nmg ? step_ : mstep_) % kTimeStride;
         const bool t_open = timing && ph == 1 && ntimed_ < kMaxTimed;
         const bool t_close = timing && ph == kTimeSteps && ntimed_ < kMaxTimed;
         int *ran = t_open ? d_ran_ + 2 * ntimed_ : t_close ? d_ran_ + 2 * ntimed_ + 1 : nullptr;
@@ -600,6 +716,15 @@ int Engine::enqueue_steps_direct(int nsteps, bool timing)
         if (n3_32) {
             const int rc = launch_steps_m(sr, ran, true);
             if (rc) return rc;
+        }
+        if (nmg) {
+            const StepRef sm{nullptr, mstep_, nullptr};
+            launch_mg_step(d_probs_, mgt_, kMaxGrid, sm, ran, s_);
+            bool even = false;
+            for (int i : tab_.mg_probs) even = even || ((mstep_ - slots_[i].n0 + 1) & 1) == 0;
+            if (even)
+                launch_mg_refresh(d_probs_, d_tab_ + off_mg_t1_, (int)tab_.mg_t1.size(), d_tab_ + off_mg_t3_,
+                                  (int)tab_.mg_t3.size(), mgt_.probs, nmg, kMaxGrid, sm, s_);
         }
         if (t_close) {
             ECHK(hipEventRecord(ev_spmv_[2 * ntimed_ + 1], s_));
@@ -610,7 +735,7 @@ int Engine::enqueue_steps_direct(int nsteps, bool timing)
             launch_refresh(d_probs_, d_tab_ + off_t1_32, n1_32, d_tab_ + off_t3_32, n3_32, d_probs_list_, nmix,
                            kMaxGrid, sr, s_);
     }
-    dstep_valid_ = false;   // the device counters no longer follow step_
+    if (plain) dstep_valid_ = false;   // the device counters no longer follow step_
     ECHK(hipGetLastError());
     return 0;
 }
@@ -728,7 +853,7 @@ int Engine::enqueue_chunk(int K, bool timing)
 {
     int rc;
     // capture and instantiation allocate: a no-allocation call launches directly
-    if (graphs_ && !timing && table_cells_ < kDirectCells && !no_alloc_active()) {
+    if (graphs_ && !timing && table_cells_ < kDirectCells && !no_alloc_active() && tab_.mg_probs.empty()) {
         for (int it = 0; it < K; it += kRefreshGrain)
             if ((rc = enqueue_group_graph())) return rc;
     } else if ((rc = enqueue_steps_direct(K, timing))) {
@@ -742,6 +867,7 @@ int Engine::enqueue_chunk(int K, bool timing)
                         hipMemcpyDeviceToHost, s_));
     ECHK(hipEventRecord(ev_status_[slot], s_));
     status_step_[slot] = step_;
+    status_mstep_[slot] = mstep_;
     ++chunk_idx_;
     return 0;
 }
@@ -811,15 +937,22 @@ int Engine::pump(bool timing, std::vector<int> &finished)
     --npend_;
     ECHK(hipEventSynchronize(ev_status_[which]));
     const CgScalars *h = h_status_ + (size_t)which * max_slots_;
-    const int last_step = status_step_[which];
     std::vector<int> &done = done_;
     done.clear();
     for (int i = 0; i < max_slots_; ++i) {
         Slot &sl = slots_[i];
         // problems admitted after this chunk was queued took no part in it
-        if (!sl.used || !sl.active || sl.finished || sl.n0 > last_step) continue;
+        if (!sl.used || !sl.active || sl.finished) continue;
+        if (sl.n0 > (sl.mg ? status_mstep_ : status_step_)[which] || h[i].mg != (sl.mg ? 1 : 0)) continue;
         sl.status = h[i];
-        if (h[i].final_) done.push_back(i);
+        if (!h[i].final_) continue;
+        if (sl.mg && h[i].giveup) {
+            // the multigrid iteration broke down: the whole solve again by
+            // plain CG (its inputs and prd1 still stand)
+            if ((rc = setup_slot(i, false, nullptr))) return rc;
+            continue;
+        }
+        done.push_back(i);
     }
     if ((rc = finish(done))) return rc;
     for (int i : done) finished.push_back(i);

@@ -39,6 +39,27 @@ constexpr int kFold = 4;
 static_assert(kRefreshGrain % kFold == 0 && kFirstRefresh % kFold == 0, "replacements must end fold groups");
 static_assert((kFold & (kFold - 1)) == 0, "kFold is a power of two");
 
+// Multigrid-preconditioned CG (ps_mg.hip), the mixed solver's iteration from
+// kMgMinCells cells on.
+//
+// kMgMinCells: smaller problems keep plain CG, whose iterates the options
+// stored_residual and a small max_iter are specified on.
+constexpr long long kMgMinCells = 49153;
+// A cap below this keeps plain CG: a capped solve returns CG's iterate.
+constexpr int kMgMinCap = 256;
+constexpr int kMgLevels = 20;
+constexpr int kMgBottomCells = 8192;   // the bottom kernel's largest level
+constexpr int kMgBottomLds = 12288;    // cells of all its levels (two floats each in LDS)
+constexpr int kMgCoarsestCells = 8;
+constexpr int kMgCoarsestSweeps = 8;
+constexpr int kMgTiles = 768;          // workgroups the fine kernels' tiling aims at
+constexpr int kMgChunk = 4;            // iterations between host polls
+// Residual replacement: once the FP32 r.r has fallen by this factor since
+// the last one (or to the threshold), and at the latest after kMgMaxGap
+// iterations; always after an even iteration.
+constexpr double kMgCycleDrop = 1e-7;
+constexpr int kMgMaxGap = 40;
+
 // Grid geometry as the kernels see it.  Cells are 0-based (i, j, k) with x
 // fastest; a cell vector holds nx*ny*nz values with no halo.  Ghost values
 // follow the reference's mirror (Neumann) or periodic rule per direction,
@@ -107,6 +128,11 @@ struct CgScalars {
     double beta_after;  // beta of the step after a replacement (mixed)
     double alph[kFold];   // mixed: alpha_k in slot k % kFold, for the correction c
     double bet[2];    // mixed: beta_n in slot n & 1, the factor that formed p_n
+    double rz[2];     // multigrid: r.z of iteration n in slot n & 1
+    int mg;           // 1: multigrid-preconditioned
+    int giveup;       // 1: the multigrid iteration broke down; solved again by CG
+    int parts;        // connected parts of a masked problem's fluid
+    int stalls;       // replacements in a row that did not halve r.r
     int lag_stop;     // 1: the FP64 stop test reads the r.r that entered the previous
                       // iteration (SuLi-IT's loop, SuLi-IT/9_grad.f90:165-177)
 };
@@ -120,6 +146,17 @@ struct Partials {
     double *proj;     // [2*ni]     setup after projection: r0.r0, FP32 r0.r0
     double *m4;       // [2][nt3][4] one-launch FP32 iteration n, slot n & 1:
                       //            p_n.q_n, q_n.r_{n-1}, q_n.q_n, r_{n-1}.r_{n-1}
+};
+
+// One level of the multigrid hierarchy (level 0: the problem itself, whose
+// faces are sx32 .. and whose r and e stand elsewhere).  Scaled faces in the
+// face arrays' layouts, 0 at walls on the coarse levels; w = sqrt(diagonal),
+// 0 in cells without faces; r the scaled restricted residual; e the
+// correction, un-scaled; ex the diagonal's extra term on the top plane (the
+// p = 0 lid, SuLi-IT's free surface).
+struct MgLevel {
+    int nx, ny, nz, px, py;
+    float *sx, *sy, *sz, *w, *r, *e, *ex;
 };
 
 // Device descriptor of one problem of a batch: geometry, tiling, where its
@@ -167,6 +204,15 @@ struct ProbDev {
     const unsigned *rowreg;
     Partials P;
     CgScalars *S;
+    // multigrid (mg set): tiles of the fine kernels (mtx x mty x planes of
+    // mkz, 1 << mlrs lanes per row), the hierarchy, level 0's weights.  p_k
+    // is in ring slot k & 1 (slot 2 holds w32), q_k in q32, z_k in q32b, r_k
+    // in r32 (k even) or r32b (k odd); the coarse levels are in r, which the
+    // set-up has done with by then.
+    int mg, mtx, mty, mkz, mlrs, ntm, medge;
+    int nlev, lbot;
+    float *w32;
+    MgLevel lv[kMgLevels];
 };
 
 // Global step of a launch: *base + off when base is set (kernels replayed
@@ -294,6 +340,8 @@ void launch_cg_m(const ProbDev *P, const TileRef *t3, int nt3, int grid, StepRef
 // recurrence; decide converged / capped / continue.
 void launch_refresh(const ProbDev *P, const TileRef *t1, int nt1, const TileRef *t3, int nt3, const int *probs,
                     int nprobs, int grid, StepRef step, hipStream_t s);
+// The FP64 true residual of launch_refresh alone.
+void launch_true_residual(const ProbDev *P, const TileRef *t3, int nt3, int grid, StepRef step, hipStream_t s);
 // *base = value: sets a device step counter.
 void launch_set_step(int *base, int value, hipStream_t s);
 // After a problem's solve: FP64 true residual r.r into S->rr_true and the
@@ -302,6 +350,28 @@ void launch_finish(const ProbDev *P, const TileRef *t3, int nt3, const int *prob
                    hipStream_t s);
 // Stand-alone SpMV q = A p of one problem (no vector updates), for timing.
 void launch_spmv_only(bool fp32, const ProbDev *P, const TileRef *t3, int nt3, int grid, hipStream_t s);
+
+// ---- multigrid-preconditioned CG (ps_mg.hip) ----
+// Lays the hierarchy of a problem out in `space` (`floats` of them; w32 holds
+// level 0's weights) and fills pd's multigrid fields; false where it does not apply (size, or the
+// hierarchy does not fit), pd.mg then stays 0.
+bool mg_plan(const Geo &g, bool mixed, float *w32, float *space, size_t floats, ProbDev &pd);
+// Table entries of levels l -> l + 1 (down) and l + 1 -> l (up).
+int mg_down_tiles(const ProbDev &pd, int l);
+int mg_up_tiles(const ProbDev &pd, int l);
+// Weights and coarse operators, after launch_init; dev: pd on the device.
+void launch_mg_setup(const ProbDev &pd, const ProbDev *dev, const SetupIn &in, hipStream_t s);
+struct MgTables {
+    const TileRef *fine = nullptr, *down[kMgLevels] = {}, *up[kMgLevels] = {};
+    int nfine = 0, ndown[kMgLevels] = {}, nup[kMgLevels] = {};
+    const int *probs = nullptr;
+    int nprobs = 0;
+};
+// Iteration step - n0 + 1 of every problem in the tables.
+void launch_mg_step(const ProbDev *P, const MgTables &T, int maxgrid, StepRef step, int *ran, hipStream_t s);
+// Residual replacement after an even iteration, as launch_refresh.
+void launch_mg_refresh(const ProbDev *P, const TileRef *t1, int nt1, const TileRef *t3, int nt3, const int *probs,
+                       int nprobs, int maxgrid, StepRef step, hipStream_t s);
 
 // Plain copy of n16 16-byte vectors (measurement only).
 void launch_copy(const void *src, void *dst, long long n16, hipStream_t s);

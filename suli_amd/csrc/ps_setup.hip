@@ -500,7 +500,7 @@ __global__ __launch_bounds__(kThreads) void k_init_finalize(Partials P, int np, 
         S->refreshes = 0;
         S->gshift = 0.0;
         S->skip_e_at = -1;
-        S->next_refresh = kFirstRefresh;
+        S->next_refresh = S->mg ? kNotDone : kFirstRefresh;
         S->prev_iters = 0;
         S->prev_rr = 0.0;
         S->slope = 0.0;

@@ -34,7 +34,7 @@ namespace {
 constexpr int kMaxSlots = 256;   // problems resident at once per context
 // Launch-table entries reserved by every context for the no-allocation entry
 // point (3-D and 1-D tiles of its one problem).
-constexpr int kNoAllocEntries = 32768;
+constexpr int kNoAllocEntries = 65536;
 constexpr int kMaxDevices = 64;
 
 struct ScratchTable {
@@ -570,7 +570,12 @@ int suli_ps_graddin_noalloc_dev(suli_ps_ctx *ctx, const suli_ps_grid *g, const d
     if (ctx->opts.autotune) ctx->eng.cached_shape(g->nx, g->ny, g->nz, mixed, &kz, &vx);
     const Geo geo = make_geo(g->nx, g->ny, g->nz, g->ccx0 == 0, g->ccy0 == 0, kz > 0 ? std::max(kz, kMinKz) : 0,
                              mixed ? vx : 1);
-    const long long entries = (long long)spmv_tiles(geo) + vec_tiles(geo.n);
+    long long entries = (long long)spmv_tiles(geo) + vec_tiles(geo.n);
+    if (mg_applies(solve_opts(ctx->opts))) {
+        const Geo def = make_geo(g->nx, g->ny, g->nz, g->ccx0 == 0, g->ccy0 == 0);
+        const long long mg = mg_entries(def);
+        if (mg > 0) entries = std::max(entries, (long long)spmv_tiles(def) + vec_tiles(def.n) + mg);
+    }
     if (entries > ctx->eng.reserved_entries())
         return fail(ctx, SULI_PS_EINVAL, "no-allocation solve: %lld launch-table entries needed, %d reserved",
                     entries, ctx->eng.reserved_entries());

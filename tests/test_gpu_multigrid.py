@@ -1,0 +1,199 @@
+"""The mixed solver's multigrid-preconditioned iteration (grids of more than
+49152 cells) against the CPU oracle.
+
+Sizes where its kernels can go wrong: the first size it serves, rows of 16,
+32 and 64 lanes with whole and partial last lanes, rows of several segments,
+an odd number of rows and planes (half-filled coarse cells), thin grids (coarse
+levels one cell wide), every boundary and operator kind.  Both solve to a
+1e-11 relative residual (oracle 1e-12); the pressure agrees within 1e-8 as in
+the plain CG tests.  The options that name properties of plain CG keep it.
+"""
+import numpy as np
+import pytest
+
+import oracle
+from suli_amd import cases
+from tests import helpers
+
+pytestmark = pytest.mark.gpu
+
+PRESSURE_RTOL = 1e-8
+
+
+@pytest.fixture(scope="module")
+def solver():
+    from suli_amd.solver import PressureSolver
+    s = PressureSolver(precision="mixed", stop_rule="relative", tol=1e-11, verbose=False)
+    yield s
+    s.close()
+
+
+def lid(c):
+    c.grid.top_bc = 1
+    return c
+
+
+def ipa(c):
+    c.grid.t_press, c.grid.rho_f1 = 2, 1000.0
+    return c
+
+
+def cylinder(nx, ny, nz, seed):
+    c = cases.config3(seed=seed, nx=nx, ny=ny, nz=nz)
+    cases.make_stretched_compatible(c)
+    return c
+
+
+def two_parts(nx, ny, nz, seed):
+    """A solid wall one cell thick cuts the fluid in two."""
+    c = cases.random_case(nx, ny, nz, seed)
+    c.fields.solid = np.zeros((nx, ny, nz), np.uint8, order="F")
+    c.fields.solid[nx // 3, :, :] = 1
+    return c
+
+
+R = cases.random_case
+CASES = [
+    ("first_size", lambda: R(37, 37, 36, 1)),             # 49284 cells, partial lanes, 16 per row
+    ("rows_of_64", lambda: R(64, 33, 25, 2)),
+    ("rows_of_65", lambda: R(65, 40, 21, 3, periodic_x=True)),
+    ("rows_of_130", lambda: R(130, 21, 20, 4)),
+    ("two_segments", lambda: R(257, 17, 13, 5)),
+    ("three_segments_px", lambda: R(515, 11, 10, 6, periodic_x=True, periodic_y=True)),
+    ("four_aligned_px", lambda: R(128, 24, 18, 7, periodic_x=True)),
+    ("py", lambda: R(52, 40, 25, 8, periodic_y=True)),
+    ("thin_z", lambda: R(160, 160, 2, 9)),
+    ("thin_y", lambda: R(200, 2, 130, 10)),
+    ("thin_x", lambda: R(3, 130, 128, 11, periodic_x=True)),
+    ("ratio_1", lambda: R(48, 41, 31, 12, ratio=1.0)),
+    ("lid", lambda: lid(R(50, 40, 33, 13))),
+    ("ipa", lambda: ipa(R(63, 31, 29, 14))),
+    ("ibm_rhs", lambda: R(56, 48, 24, 15, ibm=True)),
+    ("cylinder", lambda: cylinder(72, 40, 24, 16)),
+    ("flat_cells", lambda: R(64, 48, 20, 17, dx=5e-3)),
+]
+
+
+@pytest.mark.parametrize("name,make", CASES, ids=[n for n, _ in CASES])
+def test_vs_oracle(solver, name, make):
+    c = make()
+    if name == "flat_cells":
+        c.grid.dx = c.grid.dy = 4e-2     # 8 times as wide as high
+    print(f"multigrid {name}", flush=True)
+    p_or, _, rc = oracle.graddin(c.grid, c.fields, stop_rule=oracle.STOP_RELATIVE, tol=1e-12, project_null=True)
+    assert rc == 0
+    solver.configure(precision="mixed", stop_rule="relative", tol=1e-11, verbose=False)
+    df = solver.upload(c.grid, c.fields)
+    try:
+        st = solver.graddin_dev(c.grid, df)
+        p = df.download("prd1")
+    finally:
+        df.free()
+    print(f"  {st.iters} iterations", flush=True)
+    assert st.status == 0 and st.rel_true <= 1e-11, st.as_dict()
+    # far fewer than plain CG's several hundred: the iteration itself ran
+    assert st.iters < 150 or name in ("thin_z", "thin_y", "thin_x", "flat_cells"), st.iters
+    assert helpers.rel_diff(p, p_or, helpers.face_mask(p.shape)) <= PRESSURE_RTOL
+
+
+@pytest.mark.parametrize("shape", [(40, 37, 36), (130, 40, 11)])
+def test_suli_it_vs_oracle(solver, shape):
+    g, f = cases.it_case(*shape, seed=21)
+    print(f"multigrid suli-it {shape}", flush=True)
+    f_or = f.copy()
+    p_or, _, rc = oracle.it_graddin(g, f_or, stop_rule=oracle.STOP_RELATIVE, tol=1e-12)
+    assert rc == 0
+    solver.configure(precision="mixed", stop_rule="relative", tol=1e-11, verbose=False)
+    st = solver.it_graddin(g, f)
+    assert st.status == 0 and st.iters < 150, st.as_dict()
+    assert helpers.rel_diff(f.prd1, p_or, helpers.face_mask(f.prd1.shape)) <= PRESSURE_RTOL
+
+
+def test_two_parts_keep_their_gauges(solver):
+    """Fluid cut in two by a solid wall: each part's pressure keeps the mean
+    that plain CG (the FP64 solver) gives it."""
+    c = two_parts(48, 40, 30, 31)
+    print("multigrid two parts", flush=True)
+    out = {}
+    for precision, tol in (("fp64", 1e-12), ("mixed", 1e-11)):
+        solver.configure(precision=precision, stop_rule="relative", tol=tol, verbose=False)
+        df = solver.upload(c.grid, c.fields)
+        try:
+            st = solver.graddin_dev(c.grid, df)
+            out[precision] = df.download("prd1")
+        finally:
+            df.free()
+        assert st.status == 0, st.as_dict()
+    assert helpers.rel_diff(out["mixed"], out["fp64"], helpers.face_mask(out["fp64"].shape)) <= PRESSURE_RTOL
+
+
+def test_options_that_keep_plain_cg(solver):
+    """A small iteration cap returns plain CG's iterate, also at this size;
+    keep_null and stored_residual take plain CG's iteration counts."""
+    c = cases.random_case(48, 40, 30, 41)
+    print("multigrid options", flush=True)
+
+    def run(**kw):
+        solver.configure(stop_rule="relative", verbose=False, **kw)
+        df = solver.upload(c.grid, c.fields)
+        try:
+            st = solver.graddin_dev(c.grid, df)
+            return df.download("prd1"), st
+        finally:
+            df.free()
+
+    p64, _ = run(precision="fp64", tol=1e-14, max_iter=37)
+    p32, st = run(precision="mixed", tol=1e-14, max_iter=37)
+    assert st.status == 1 and st.iters == 37
+    assert helpers.rel_diff(p32, p64, helpers.face_mask(p64.shape)) <= 1e-5
+    _, st64 = run(precision="fp64", tol=1e-8)
+    for kw in (dict(keep_null=True), dict(stored_residual=True)):
+        _, st = run(precision="mixed", tol=1e-8, **kw)
+        assert st.status == 0 and st.iters >= 0.5 * st64.iters, (kw, st.iters, st64.iters)
+
+
+def test_batch_and_server_equal_alone():
+    """Problems of both iterations in one batch, and through the server: each
+    bit for bit as alone."""
+    from suli_amd.server import PressureServer
+    from suli_amd.solver import PressureSolver
+    cs = [R(40, 24, 16, 51), R(66, 40, 30, 52), cylinder(72, 40, 24, 53), ipa(R(61, 33, 31, 54)),
+          R(130, 40, 33, 55, periodic_x=True), R(24, 20, 16, 56)]
+    with PressureSolver(precision="mixed", stop_rule="relative", tol=1e-11, verbose=False) as s:
+        alone = []
+        for c in cs:
+            df = s.upload(c.grid, c.fields)
+            st = s.graddin_dev(c.grid, df)
+            assert st.status == 0
+            alone.append((df.download("prd1"), st.iters))
+            df.free()
+        dfs = [s.upload(c.grid, c.fields) for c in cs]
+        sts = s.graddin_batch_dev([(c.grid, df) for c, df in zip(cs, dfs)])
+        for i, (df, st) in enumerate(zip(dfs, sts)):
+            assert st.iters == alone[i][1], i
+            np.testing.assert_array_equal(df.download("prd1"), alone[i][0])
+            df.free()
+    with PressureServer(precision="mixed", stop_rule="relative", tol=1e-11) as srv:
+        todo = [i for i, c in enumerate(cs) if c.fields.solid is None]
+        fields = [cs[i].fields.copy() for i in todo]
+        tickets = [srv.submit(cs[i].grid, f) for i, f in zip(todo, fields)]
+        for i, f, t in zip(todo, fields, tickets):
+            st = srv.wait(t)
+            assert st.status == 0 and st.iters == alone[i][1], i
+            np.testing.assert_array_equal(f.prd1, alone[i][0])
+
+
+def test_noalloc_equals_alone(solver):
+    c = R(72, 50, 40, 61)
+    print("multigrid noalloc", flush=True)
+    solver.configure(precision="mixed", stop_rule="relative", tol=1e-11, verbose=False)
+    out = []
+    for noalloc in (False, True):
+        df = solver.upload(c.grid, c.fields)
+        try:
+            st = solver.graddin_noalloc_dev(c.grid, df) if noalloc else solver.graddin_dev(c.grid, df)
+            out.append((df.download("prd1"), st.iters, st.refreshes))
+        finally:
+            df.free()
+    assert out[0][1:] == out[1][1:]
+    np.testing.assert_array_equal(out[0][0], out[1][0])
