@@ -1161,8 +1161,10 @@ __global__ __launch_bounds__(kThreads) void k_true_residual(const ProbDev *__res
         const gptr<const double> __restrict__ e = glob((const double *)pd.e);
         const gptr<const double> __restrict__ b = glob(pd.b);
         const gptr<const double> __restrict__ d = glob(pd.d);
-        // the replaced residual goes where the next cg_m reads r_{n}
-        const gptr<float> __restrict__ r32 = WRITE32 ? glob(pd.r32) : nullptr;
+        // the replaced residual goes where the next cg_m, or multigrid step,
+        // reads it
+        const bool odd = pd.mg && ((step - pd.n0 + 1) & 1);
+        const gptr<float> __restrict__ r32 = WRITE32 ? glob(odd ? pd.r32b : pd.r32) : nullptr;
         double acc = 0.0, acc32 = 0.0, acc_en = 0.0;
         // a tile of vx cells per lane is walked as vx one-cell-per-lane
         // sub-tiles, so that every load is coalesced

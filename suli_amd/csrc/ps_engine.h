@@ -206,13 +206,13 @@ private:
     struct Tables {
         std::vector<TileRef> t3_64, t1_64, t3_32, t1_32;
         std::vector<int> mixed_probs;
-        // multigrid problems: fine tiles, 3-D and 1-D tiles of the
-        // replacement, coarse levels
-        std::vector<TileRef> mg_fine, mg_t3, mg_t1, mg_lev;
+        // multigrid problems: fine tiles, 3-D tiles of the replacement,
+        // coarse levels
+        std::vector<TileRef> mg_fine, mg_t3, mg_lev;
         std::vector<int> mg_probs;
     } tab_;
     MgTables mgt_;                     // the same on the device
-    int off_mg_t3_ = 0, off_mg_t1_ = 0;
+
     TileRef *d_tab_ = nullptr;
     int *d_probs_list_ = nullptr;
     size_t tab_cap_ = 0, probs_cap_ = 0;

@@ -274,7 +274,6 @@ int Engine::reserve(int entries)
     tab_.mixed_probs.reserve(max_slots_);
     tab_.mg_fine.reserve(ntab);
     tab_.mg_t3.reserve(ntab);
-    tab_.mg_t1.reserve(ntab);
     tab_.mg_lev.reserve(ntab);
     tab_.mg_probs.reserve(max_slots_);
     pool_.reserve(max_slots_);
@@ -326,7 +325,7 @@ long long mg_entries(const Geo &g)
     carve(cv, g, true, nt3, vec_tiles(g.n), pd);
     if (!mg_plan(g, true, nullptr, nullptr, 2 * (size_t)g.n, pd) || 3 * pd.ntm > 8 * nt3) return 0;
     long long n = pd.ntm;
-    for (int l = 1; l < pd.lbot; ++l) n += mg_down_tiles(pd, l) + mg_up_tiles(pd, l);
+    for (int l = 1; l < pd.lbot; ++l) n += mg_level_tiles(pd, l);
     return n;
 }
 
@@ -521,7 +520,6 @@ int Engine::rebuild_tables()
     tab_.mixed_probs.clear();
     tab_.mg_fine.clear();
     tab_.mg_t3.clear();
-    tab_.mg_t1.clear();
     tab_.mg_lev.clear();
     tab_.mg_probs.clear();
     table_cells_ = 0;
@@ -531,7 +529,6 @@ int Engine::rebuild_tables()
         if (sl.mg) {
             for (int t = 0; t < sl.pd.ntm; ++t) tab_.mg_fine.push_back({i, t});
             for (int t = 0; t < sl.pd.nt3; ++t) tab_.mg_t3.push_back({i, t});
-            for (int t = 0; t < sl.pd.nt1; ++t) tab_.mg_t1.push_back({i, t});
             tab_.mg_probs.push_back(i);
             continue;
         }
@@ -556,21 +553,19 @@ int Engine::rebuild_tables()
     off_t1_64 = off_t3_64 + (int)tab_.t3_64.size();
     off_t3_32 = off_t1_64 + (int)tab_.t1_64.size();
     off_t1_32 = off_t3_32 + (int)tab_.t3_32.size();
-    // multigrid: coarse levels' entries, each level's down and up tables
-    int off_lev[2][kMgLevels] = {};
-    for (int l = 1; l < kMgLevels; ++l)
-        for (int up = 0; up < 2; ++up) {
-            off_lev[up][l] = (int)tab_.mg_lev.size();
-            for (int i : tab_.mg_probs) {
-                const int nt = up ? mg_up_tiles(slots_[i].pd, l) : mg_down_tiles(slots_[i].pd, l);
-                for (int t = 0; t < nt; ++t) tab_.mg_lev.push_back({i, t});
-            }
-            (up ? mgt_.nup : mgt_.ndown)[l] = (int)tab_.mg_lev.size() - off_lev[up][l];
+    // multigrid: coarse levels' entries
+    int off_lev[kMgLevels] = {};
+    for (int l = 1; l < kMgLevels; ++l) {
+        off_lev[l] = (int)tab_.mg_lev.size();
+        for (int i : tab_.mg_probs) {
+            const int nt = mg_level_tiles(slots_[i].pd, l);
+            for (int t = 0; t < nt; ++t) tab_.mg_lev.push_back({i, t});
         }
+        mgt_.nlev[l] = (int)tab_.mg_lev.size() - off_lev[l];
+    }
     const int off_mg = off_t1_32 + (int)tab_.t1_32.size();
-    off_mg_t3_ = off_mg + (int)tab_.mg_fine.size();
-    off_mg_t1_ = off_mg_t3_ + (int)tab_.mg_t3.size();
-    const int off_mg_lev = off_mg_t1_ + (int)tab_.mg_t1.size();
+    const int off_mg_t3 = off_mg + (int)tab_.mg_fine.size();
+    const int off_mg_lev = off_mg_t3 + (int)tab_.mg_t3.size();
     const size_t ntab = off_mg_lev + tab_.mg_lev.size();
     const size_t nprobs = tab_.mixed_probs.size() + tab_.mg_probs.size();
     if (ntab > tab_cap_ || nprobs > probs_cap_ || !d_tab_) {
@@ -607,17 +602,15 @@ int Engine::rebuild_tables()
     std::copy(tab_.mixed_probs.begin(), tab_.mixed_probs.end(), hp);
     std::copy(tab_.mg_probs.begin(), tab_.mg_probs.end(), hp + tab_.mixed_probs.size());
     std::copy(tab_.mg_fine.begin(), tab_.mg_fine.end(), ht + off_mg);
-    std::copy(tab_.mg_t3.begin(), tab_.mg_t3.end(), ht + off_mg_t3_);
-    std::copy(tab_.mg_t1.begin(), tab_.mg_t1.end(), ht + off_mg_t1_);
+    std::copy(tab_.mg_t3.begin(), tab_.mg_t3.end(), ht + off_mg_t3);
     std::copy(tab_.mg_lev.begin(), tab_.mg_lev.end(), ht + off_mg_lev);
     mgt_.fine = d_tab_ + off_mg;
     mgt_.nfine = (int)tab_.mg_fine.size();
+    mgt_.t3 = d_tab_ + off_mg_t3;
+    mgt_.nt3 = (int)tab_.mg_t3.size();
     mgt_.probs = d_probs_list_ + tab_.mixed_probs.size();
     mgt_.nprobs = (int)tab_.mg_probs.size();
-    for (int l = 1; l < kMgLevels; ++l) {
-        mgt_.down[l] = d_tab_ + off_mg_lev + off_lev[0][l];
-        mgt_.up[l] = d_tab_ + off_mg_lev + off_lev[1][l];
-    }
+    for (int l = 1; l < kMgLevels; ++l) mgt_.lev[l] = d_tab_ + off_mg_lev + off_lev[l];
     if (ntab) ECHK(hipMemcpyAsync(d_tab_, ht, sizeof(TileRef) * ntab, hipMemcpyHostToDevice, s_));
     if (nprobs) ECHK(hipMemcpyAsync(d_probs_list_, hp, sizeof(int) * nprobs, hipMemcpyHostToDevice, s_));
     ECHK(hipEventRecord(ev_stage_[stg], s_));
@@ -720,11 +713,6 @@ int Engine::enqueue_steps_direct(int nsteps, bool timing)
         if (nmg) {
             const StepRef sm{nullptr, mstep_, nullptr};
             launch_mg_step(d_probs_, mgt_, kMaxGrid, sm, ran, s_);
-            bool even = false;
-            for (int i : tab_.mg_probs) even = even || ((mstep_ - slots_[i].n0 + 1) & 1) == 0;
-            if (even)
-                launch_mg_refresh(d_probs_, d_tab_ + off_mg_t1_, (int)tab_.mg_t1.size(), d_tab_ + off_mg_t3_,
-                                  (int)tab_.mg_t3.size(), mgt_.probs, nmg, kMaxGrid, sm, s_);
         }
         if (t_close) {
             ECHK(hipEventRecord(ev_spmv_[2 * ntimed_ + 1], s_));

@@ -48,16 +48,16 @@ constexpr long long kMgMinCells = 49153;
 // A cap below this keeps plain CG: a capped solve returns CG's iterate.
 constexpr int kMgMinCap = 256;
 constexpr int kMgLevels = 20;
-constexpr int kMgBottomCells = 8192;   // the bottom kernel's largest level
-constexpr int kMgBottomLds = 12288;    // cells of all its levels (two floats each in LDS)
+constexpr int kMgBottomCells = 6144;   // the bottom kernel's largest level
+constexpr int kMgBottomLds = 38912;    // floats of LDS it has (152 KiB)
 constexpr int kMgCoarsestCells = 8;
 constexpr int kMgCoarsestSweeps = 8;
-constexpr int kMgTiles = 768;          // workgroups the fine kernels' tiling aims at
-constexpr int kMgChunk = 4;            // iterations between host polls
-// Residual replacement: once the FP32 r.r has fallen by this factor since
-// the last one (or to the threshold), and at the latest after kMgMaxGap
-// iterations; always after an even iteration.
-constexpr double kMgCycleDrop = 1e-7;
+constexpr int kMgChunk = 2;            // iterations between host polls
+// Residual replacement: once the FP32 r.r has fallen by kMgCycleDrop since the
+// last one, or to kMgMargin of the threshold, and at the latest after kMgMaxGap
+// iterations.
+constexpr double kMgCycleDrop = 1e-9;
+constexpr double kMgMargin = 0.5;
 constexpr int kMgMaxGap = 40;
 
 // Grid geometry as the kernels see it.  Cells are 0-based (i, j, k) with x
@@ -149,14 +149,14 @@ struct Partials {
 };
 
 // One level of the multigrid hierarchy (level 0: the problem itself, whose
-// faces are sx32 .. and whose r and e stand elsewhere).  Scaled faces in the
+// faces are sx32 .. and whose vectors stand elsewhere).  Scaled faces in the
 // face arrays' layouts, 0 at walls on the coarse levels; w = sqrt(diagonal),
-// 0 in cells without faces; r the scaled restricted residual; e the
-// correction, un-scaled; ex the diagonal's extra term on the top plane (the
+// 0 in cells without faces; r the scaled restricted residual; t, rho and r0
+// the cycle's vectors (ps_mg.hip), t at last the correction, un-scaled; ex the diagonal's extra term on the top plane (the
 // p = 0 lid, SuLi-IT's free surface).
 struct MgLevel {
     int nx, ny, nz, px, py;
-    float *sx, *sy, *sz, *w, *r, *e, *ex;
+    float *sx, *sy, *sz, *w, *r, *t, *rho, *r0, *ex;
 };
 
 // Device descriptor of one problem of a batch: geometry, tiling, where its
@@ -206,11 +206,13 @@ struct ProbDev {
     CgScalars *S;
     // multigrid (mg set): tiles of the fine kernels (mtx x mty x planes of
     // mkz, 1 << mlrs lanes per row), the hierarchy, level 0's weights.  p_k
-    // is in ring slot k & 1 (slot 2 holds w32), q_k in q32, z_k in q32b, r_k
-    // in r32 (k even) or r32b (k odd); the coarse levels are in r, which the
+    // is in ring slot k & 1 (slot 2 holds w32, slot 3 t), q_k in q32, rho and
+    // then z_k in q32b, r_k in r32 (k even) or r32b (k odd), the other one
+    // holding r0; the coarse levels are in r, which the
     // set-up has done with by then.
     int mg, mtx, mty, mkz, mlrs, ntm, medge;
-    int nlev, lbot;
+    int nlev, lbot, nbot;   // nbot: cells of levels lbot and coarser
+    float *bot;             // those cells' coefficients, packed
     float *w32;
     MgLevel lv[kMgLevels];
 };
@@ -356,23 +358,20 @@ void launch_spmv_only(bool fp32, const ProbDev *P, const TileRef *t3, int nt3, i
 // level 0's weights) and fills pd's multigrid fields; false where it does not apply (size, or the
 // hierarchy does not fit), pd.mg then stays 0.
 bool mg_plan(const Geo &g, bool mixed, float *w32, float *space, size_t floats, ProbDev &pd);
-// Table entries of levels l -> l + 1 (down) and l + 1 -> l (up).
-int mg_down_tiles(const ProbDev &pd, int l);
-int mg_up_tiles(const ProbDev &pd, int l);
+// Table entries of level l's kernels.
+int mg_level_tiles(const ProbDev &pd, int l);
 // Weights and coarse operators, after launch_init; dev: pd on the device.
 void launch_mg_setup(const ProbDev &pd, const ProbDev *dev, const SetupIn &in, hipStream_t s);
 struct MgTables {
-    const TileRef *fine = nullptr, *down[kMgLevels] = {}, *up[kMgLevels] = {};
-    int nfine = 0, ndown[kMgLevels] = {}, nup[kMgLevels] = {};
+    const TileRef *fine = nullptr, *lev[kMgLevels] = {};
+    int nfine = 0, nlev[kMgLevels] = {};
+    const TileRef *t3 = nullptr;   // 3-D tiles of the true residual
+    int nt3 = 0;
     const int *probs = nullptr;
     int nprobs = 0;
 };
-// Iteration step - n0 + 1 of every problem in the tables.
+// Step step - n0 + 1 (an iteration or a replacement) of every problem in the tables.
 void launch_mg_step(const ProbDev *P, const MgTables &T, int maxgrid, StepRef step, int *ran, hipStream_t s);
-// Residual replacement after an even iteration, as launch_refresh.
-void launch_mg_refresh(const ProbDev *P, const TileRef *t1, int nt1, const TileRef *t3, int nt3, const int *probs,
-                       int nprobs, int maxgrid, StepRef step, hipStream_t s);
-
 // Plain copy of n16 16-byte vectors (measurement only).
 void launch_copy(const void *src, void *dst, long long n16, hipStream_t s);
 // Plain read of n16 16-byte vectors (measurement only); out holds

@@ -9,8 +9,8 @@
 // FP32 inside FP64 residual replacement, as the CG step: dot products, alpha
 // and beta are FP64 and convergence is judged on the FP64 true residual.
 //
-// The V-cycle: a weighted Jacobi sweep before (from z = 0, so z = omega r)
-// and after the coarse correction on every level.  A coarse cell joins 2x2x2
+// The V-cycle smooths with a Chebyshev polynomial of degree two before and
+// after the coarse correction on every level.  A coarse cell joins 2x2x2
 // cells; restriction sums the children's residuals, prolongation copies the
 // parent's value, and a coarse face's coefficient is half the sum of the fine
 // faces it covers (twice the distance).  The cycle is symmetric positive
@@ -19,21 +19,33 @@
 // with w = sqrt(d): restriction weighs with w, prolongation too, and each
 // coarse level is scaled to a unit diagonal in the same way (its own w).
 //
-// Measured at 256x128x96 from prd1 = 0 to 1e-12 relative: plain CG 37.8 ms
-// (1992 iterations of one 18.5 us launch), this 7.70 ms (54 iterations); the
-// stretched masked cylinder at 384x192x128 248.7 and 24.3 ms, SuLi-IT's
-// 256x128x48 19.9 and 6.0 ms, twelve uneven tanks in a batch 72.1 and 11.7 ms.
+// Degree two against one Jacobi sweep (weight 0.85): 15 iterations to 1e-12
+// on the 256x128x96 tank instead of 49, for five passes over the fine grid
+// instead of three.  Degree two on the coarse levels alone gives 24.
 //
-// One iteration n is 4 + 2 lbot launches (lbot levels before the ones the
-// bottom kernel takes whole):
-//   resid   r_{n-1} = r_{n-2} - alpha q (formed where needed), the residual
-//           left by z = omega r restricted to level 1; partials r.r
-//   down    the same on levels 1 .. lbot-1
+// With the polynomial s(A) = c0 + c1 A, a level's steps are
+//   t = A r                      rho = r - A s(A) r = r - c0 t - c1 A t
+//   (coarse: restrict rho, correct by e)
+//   r0 = rho - A (w e)           z = s(A) r + w e + s(A) r0
+// each a single pass with one application of A.
+//
+// Measured at 256x128x96 from prd1 = 0 to 1e-12 relative: plain CG 37.8 ms
+// (1992 iterations of one 18.5 us launch), this 3.39 ms (17 iterations); the
+// stretched masked cylinder at 384x192x128 238.4 and 10.8 ms, SuLi-IT's
+// 256x128x48 19.4 and 3.1 ms, twelve uneven tanks in a batch 67.7 and 6.0 ms.
+//
+// One iteration n (lbot: the first level of the bottom kernel):
+//   A1      r_{n-1} = r_{n-2} - alpha q (formed where needed), t; partials r.r
+//   A2      rho, restricted to level 1
+//   D1, D2  the same on levels 1 .. lbot-1
 //   bottom  levels lbot and coarser, one workgroup per problem, in LDS
-//   up      coarse correction and post-smoothing on levels lbot-1 .. 1
-//   smooth  the same on level 0: z_n; partials r.z
+//   U1, U2  coarse correction and post-smoothing on levels lbot-1 .. 1
+//   B1, B2  the same on level 0: z_n; partials r.z
 //   dir     beta, c -= alpha_{n-1} p_{n-1}, p_n = z + beta p, q = A p;
 //           partials p.q
+// or, in a step whose A2 finds r_{n-1} small enough, instead of D1 .. dir the
+// residual replacement: dir folds c and alpha p into e, then
+//   k_true_residual, k_mg_decide: converged, or on with the replaced residual
 // Each total is summed by the kernel that needs it from the partials of an
 // earlier launch, as in ps_cg.hip.
 #include <algorithm>
@@ -43,13 +55,19 @@
 namespace sps {
 namespace {
 
-// Weight of the Jacobi sweeps.  The scaled operator's spectrum lies in
-// (0, 2), so any weight below 1 keeps the V-cycle positive definite.
-constexpr float kOmega = 0.85f;
+// Chebyshev polynomial of degree two on [kLmax / 6, kLmax], kLmax = 2 above
+// the scaled operator's spectrum (0, 2): s(x) = kC0 + kC1 x, positive there,
+// as 1 - x s(x) stays within (-1, 1).
+constexpr float kLmax = 2.0f, kLmin = kLmax / 6.0f;
+constexpr float kTheta = 0.5f * (kLmax + kLmin), kDelta = 0.5f * (kLmax - kLmin);
+constexpr float kRho1 = 1.0f / (2.0f * kTheta / kDelta - kDelta / kTheta);
+constexpr float kC0 = (1.0f + kRho1 * kDelta / kTheta) / kTheta + 2.0f * kRho1 / kDelta;
+constexpr float kC1 = -2.0f * kRho1 / (kDelta * kTheta);
+constexpr float kOmega = 0.85f;   // Jacobi sweeps of the coarsest level
 constexpr int kBotThreads = 1024;
 constexpr int kBotPer = kMgBottomCells / kBotThreads;
 
-enum { kResid = 0, kSmooth = 1, kDir = 2 };
+enum { kA1 = 0, kA2 = 1, kB1 = 2, kB2 = 3, kDir = 4 };
 
 __device__ __forceinline__ int step_of(StepRef s) { return s.base ? *s.base + s.off : s.off; }
 
@@ -87,6 +105,9 @@ __device__ __forceinline__ double *part_rr(const ProbDev &pd) { return pd.P.m4 +
 // r_k alternates between two buffers, as p_k does.
 __device__ __forceinline__ float *rbuf(const ProbDev &pd, int k) { return (k & 1) ? pd.r32b : pd.r32; }
 __device__ __forceinline__ float *mpbuf(const ProbDev &pd, int k) { return pd.p32 + (k & 1) * pd.pslot; }
+
+// t of level 0: ring slot 3
+__device__ __forceinline__ float *tbuf(const ProbDev &pd) { return pd.p32 + 3 * pd.pslot; }
 
 typedef float vf4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef float vf2 __attribute__((ext_vector_type(2), aligned(4)));
@@ -147,22 +168,31 @@ __device__ __forceinline__ float from_upper(float v)
 // the 2x2x2 cells of a coarse cell into one lane.  Rows up to 64 (128) cells
 // take 16 (32) lanes, so that short rows share a wave.
 //
-// The stencil value v is formed where it is needed from two operands:
-//   resid   v = a - s b       a = r_{n-2}, b = q          (fresh: v = a)
-//   smooth  v = omega a + w e a = r_{n-1}, e = the parent's correction
-//   dir     v = a + s b       a = z, b = p_{n-1}          (fresh: v = a)
-// then y = (A v) and, on the tile's cells,
-//   resid   r_{n-1} = v; sums w (v - omega y) into the coarse cells
-//   smooth  z = v + omega (a - y)
-//   dir     p_n = v, q = y, c -= s2 b
+// The stencil value v is formed where it is needed, y = (A v), and on the
+// tile's cells
+//   A1   v = a - s b   a = r_{n-2}, b = q (fresh: v = a)   r = v, t = y
+//   A2   v = a         a = t       rho = r - c0 t - c1 y, summed into coarse cells
+//   B1   v = w e       e = the parent's correction         r0 = rho - y
+//   B2   v = a         a = r0      z = c0 r + c1 t + w e + c0 r0 + c1 y
+//   dir  v = a + s b   a = z, b = p_{n-1} (fresh: v = a)   p = v, q = y, c -= s2 b
 // EDGE: rows whose ends need a loaded neighbour (x periodic, or more than one
 // segment of 4 lr cells) or whose length is no multiple of four.
+struct FineArgs {
+    gptr<const float> a, b;       // stencil operands
+    gptr<const float> r, t;       // at the cell: r, t (A2, B2), rho as r (B1)
+    gptr<float> o1, o2, x;        // outputs; x: c (dir)
+    bool fresh, do_x;
+    float s, s2;
+};
+
 template <int KIND, bool EDGE>
-__device__ __forceinline__ double mg_tile(const ProbDev &pd, int tile, gptr<const float> __restrict__ a_,
-                                          gptr<const float> __restrict__ b_, gptr<float> __restrict__ o1,
-                                          gptr<float> __restrict__ o2, gptr<float> __restrict__ x_, bool fresh, float s,
-                                          float s2, bool do_x)
+__device__ __forceinline__ double mg_tile(const ProbDev &pd, int tile, const FineArgs &F)
 {
+    constexpr bool kTwo = KIND == kA1 || KIND == kDir;   // two operands a, b
+    constexpr bool kW = KIND == kA2 || KIND == kB2;      // w at the cell
+    const gptr<const float> a_ = F.a, b_ = F.b;
+    const bool fresh = F.fresh;
+    const float s = F.s;
     const int nx = pd.g.nx, ny = pd.g.ny, nz = pd.g.nz;
     const int px = pd.g.px, py = pd.g.py;
     const int lrs = pd.mlrs, lr = 1 << lrs;
@@ -192,37 +222,36 @@ __device__ __forceinline__ double mg_tile(const ProbDev &pd, int tile, gptr<cons
     const long long cplane = (long long)C.nx * C.ny;
     const unsigned ca = (unsigned)(ja >> 1) * ncx + (ci >> 1), cb = (unsigned)(jb >> 1) * ncx + (ci >> 1);
     const unsigned cs = (unsigned)(js >> 1) * ncx + (ci >> 1), cn = (unsigned)(jn >> 1) * ncx + (ci >> 1);
-    const gptr<const float> e1 = glob((const float *)C.e), w_ = glob((const float *)pd.w32);
+    const gptr<const float> e1 = glob((const float *)C.t), w_ = glob((const float *)pd.w32);
     // cells beyond the segment's ends
     const bool ise = i < nx && (i + 4 >= nx || sl == lr - 1);
     const bool ldw = EDGE && sl == 0 && (i0 > 0 || px), lde = EDGE && ise && (i + 4 < nx || px);
     const int xw = i0 > 0 ? i0 - 1 : nx - 1, xe = i + 4 < nx ? i + 4 : 0;
 
-    auto v_of = [&](float a, float b, float e) -> float {
-        if (KIND == kSmooth) return kOmega * a + b * e;
-        if (KIND == kResid) return fresh ? a : a - s * b;
-        return fresh ? a : a + s * b;
+    auto v_of = [&](float a, float b) -> float {
+        if (KIND == kB1) return a * b;
+        if (KIND == kA1) return fresh ? a : a - s * b;
+        if (KIND == kDir) return fresh ? a : a + s * b;
+        return a;
     };
-    // four values of a row at plane kk, with their operands
-    auto row = [&](int kk, unsigned o, unsigned c, float (&v)[4], float (&a)[4], float (&b)[4]) {
-        const gptr<const float> ap = a_ + kk * plane;
-        ld4(ap, o, a);
-        float e[2] = {0.f, 0.f};
-        if (KIND == kSmooth) {
-            ld4(w_ + kk * plane, o, b);
+    // four values of a row at plane kk, with the second operand
+    auto row = [&](int kk, unsigned o, unsigned c, float (&v)[4], float (&b)[4]) {
+        float a[4], e[2];
+        if (KIND == kB1) {
+            ld4(w_ + kk * plane, o, a);
             ld2(e1 + (kk >> 1) * cplane, c, e);
         } else {
-            ld4(b_ + kk * plane, o, b);
+            ld4(a_ + kk * plane, o, a);
+            if (kTwo) ld4(b_ + kk * plane, o, b);
         }
 #pragma unroll
-        for (int m = 0; m < 4; ++m) v[m] = v_of(a[m], b[m], e[m >> 1]);
+        for (int m = 0; m < 4; ++m) v[m] = v_of(a[m], KIND == kB1 ? e[m >> 1] : kTwo ? b[m] : 0.f);
     };
     auto one = [&](int kk, int jj, int x) -> float {
         const unsigned o = (unsigned)jj * nx + x;
-        const float a = ld1(a_ + kk * plane, o);
-        if (KIND == kSmooth)
-            return v_of(a, ld1(w_ + kk * plane, o), ld1(e1 + (kk >> 1) * cplane, (unsigned)(jj >> 1) * ncx + (x >> 1)));
-        return v_of(a, ld1(b_ + kk * plane, o), 0.f);
+        if (KIND == kB1)
+            return ld1(w_ + kk * plane, o) * ld1(e1 + (kk >> 1) * cplane, (unsigned)(jj >> 1) * ncx + (x >> 1));
+        return v_of(ld1(a_ + kk * plane, o), kTwo ? ld1(b_ + kk * plane, o) : 0.f);
     };
 
     // the rows' table bits for the tile's planes (planes past 32 read the arrays)
@@ -242,13 +271,13 @@ __device__ __forceinline__ double mg_tile(const ProbDev &pd, int tile, gptr<cons
     const int jb1 = min(ja + 1, ny - 1);   // row b for face addresses
     const int jy2 = min(ja + 2, ny);       // y face north of row b
 
-    float vb[2][4], vc[2][4], ac[2][4], bc[2][4];
-    row(k0, oa, ca, vc[0], ac[0], bc[0]);
-    row(k0, ob, cb, vc[1], ac[1], bc[1]);
+    float vb[2][4], vc[2][4], bc[2][4];
+    row(k0, oa, ca, vc[0], bc[0]);
+    row(k0, ob, cb, vc[1], bc[1]);
     if (k0 > 0) {
-        float t0[4], t1[4];
-        row(k0 - 1, oa, ca, vb[0], t0, t1);
-        row(k0 - 1, ob, cb, vb[1], t0, t1);
+        float t1[4];
+        row(k0 - 1, oa, ca, vb[0], t1);
+        row(k0 - 1, ob, cb, vb[1], t1);
     } else {
 #pragma unroll
         for (int m = 0; m < 4; ++m) vb[0][m] = vc[0][m], vb[1][m] = vc[1][m];
@@ -263,11 +292,11 @@ __device__ __forceinline__ double mg_tile(const ProbDev &pd, int tile, gptr<cons
     for (int k = k0; k < k1; ++k) {
         const int ku = k < nz - 1 ? k + 1 : k;
         const bool ra = (k - k0) < 32 && ((bita >> (k - k0)) & 1u), rb = (k - k0) < 32 && ((bitb >> (k - k0)) & 1u);
-        float vt[2][4], at[2][4], bt[2][4], vs[4], vn[4], t0[4], t1[4];
-        row(ku, oa, ca, vt[0], at[0], bt[0]);
-        row(ku, ob, cb, vt[1], at[1], bt[1]);
-        row(k, os, cs, vs, t0, t1);
-        row(k, on, cn, vn, t0, t1);
+        float vt[2][4], bt[2][4], vs[4], vn[4], t1[4];
+        row(ku, oa, ca, vt[0], bt[0]);
+        row(ku, ob, cb, vt[1], bt[1]);
+        row(k, os, cs, vs, t1);
+        row(k, on, cn, vn, t1);
         float sx[2][5], sy0[4], sy1[4], sy2[4], szt[2][4];
         {
             const gptr<const float> xa = ra ? RX + 8 * k : SX + ((long long)k * ny + ja) * (nx + 1) + ci;
@@ -289,14 +318,24 @@ __device__ __forceinline__ double mg_tile(const ProbDev &pd, int tile, gptr<cons
             fld4(rb ? RZ + 4 * (k + 1) : SZ + (long long)(k + 1) * plane + (unsigned)jb1 * nx + ci, szt[1]);
         }
         // operands of the outputs
-        float wx[2][4];
-        if (KIND == kResid) {
+        float wx[2][4], rc[2][4], tc[2][4], ec[2][2];
+        if (kW) {
             ld4(w_ + k * plane, oa, wx[0]);
             ld4(w_ + k * plane, ob, wx[1]);
         }
         if (KIND == kDir) {
-            ld4(x_ + k * plane, oa, wx[0]);
-            ld4(x_ + k * plane, ob, wx[1]);
+            ld4((gptr<const float>)F.x + k * plane, oa, wx[0]);
+            ld4((gptr<const float>)F.x + k * plane, ob, wx[1]);
+        }
+        if (KIND == kA2 || KIND == kB1 || KIND == kB2) {
+            ld4(F.r + k * plane, oa, rc[0]);
+            ld4(F.r + k * plane, ob, rc[1]);
+        }
+        if (KIND == kB2) {
+            ld4(F.t + k * plane, oa, tc[0]);
+            ld4(F.t + k * plane, ob, tc[1]);
+            ld2(e1 + (k >> 1) * cplane, ca, ec[0]);
+            ld2(e1 + (k >> 1) * cplane, cb, ec[1]);
         }
         float ew[2] = {vc[0][0], vc[1][0]}, ee[2];
         if (EDGE) {
@@ -345,39 +384,33 @@ __device__ __forceinline__ double mg_tile(const ProbDev &pd, int tile, gptr<cons
         for (int r = 0; r < 2; ++r) {
             const int nv = r == 0 ? nva : nvb;
             const unsigned o = r == 0 ? oa : ob;
-            if (KIND == kResid) {
+            float o1[4], o2[4];
 #pragma unroll
-                for (int m = 0; m < 4; ++m) {
-                    const bool in = EDGE ? m < nv : nv > 0;
-                    const float v = in ? vc[r][m] : 0.f;
-                    const float rho = vc[r][m] - kOmega * y[r][m];
-                    acc += (double)v * (double)v;
-                    sum[m >> 1] += in ? wx[r][m] * rho : 0.f;
+            for (int m = 0; m < 4; ++m) {
+                const bool in = EDGE ? m < nv : nv > 0;
+                const float v = vc[r][m], av = y[r][m];
+                o1[m] = v;
+                o2[m] = av;
+                if (KIND == kA1) {
+                    acc += in ? (double)v * (double)v : 0.0;
+                } else if (KIND == kA2) {
+                    o1[m] = rc[r][m] - kC0 * v - kC1 * av;
+                    sum[m >> 1] += in ? wx[r][m] * o1[m] : 0.f;
+                } else if (KIND == kB1) {
+                    o1[m] = rc[r][m] - av;
+                } else if (KIND == kB2) {
+                    o1[m] = kC0 * (rc[r][m] + v) + kC1 * (tc[r][m] + av) + wx[r][m] * ec[r][m >> 1];
+                    acc += in ? (double)rc[r][m] * (double)o1[m] : 0.0;
+                } else {
+                    acc += in ? (double)v * (double)av : 0.0;
+                    wx[r][m] = wx[r][m] - F.s2 * bc[r][m];
                 }
-                if (!fresh) st4(o1 + k * plane, o, vc[r], nv);
-            } else if (KIND == kSmooth) {
-                float z[4];
-#pragma unroll
-                for (int m = 0; m < 4; ++m) {
-                    const bool in = EDGE ? m < nv : nv > 0;
-                    z[m] = vc[r][m] + kOmega * (ac[r][m] - y[r][m]);
-                    acc += in ? (double)ac[r][m] * (double)z[m] : 0.0;
-                }
-                st4(o1 + k * plane, o, z, nv);
-            } else {
-                float c[4];
-#pragma unroll
-                for (int m = 0; m < 4; ++m) {
-                    const bool in = EDGE ? m < nv : nv > 0;
-                    acc += in ? (double)vc[r][m] * (double)y[r][m] : 0.0;
-                    c[m] = wx[r][m] - s2 * bc[r][m];
-                }
-                st4(o1 + k * plane, o, vc[r], nv);
-                st4(o2 + k * plane, o, y[r], nv);
-                if (do_x) st4(x_ + k * plane, o, c, nv);
             }
+            if (!(KIND == kA1 && fresh)) st4(F.o1 + k * plane, o, o1, nv);
+            if (KIND == kA1 || KIND == kDir) st4(F.o2 + k * plane, o, o2, nv);
+            if (KIND == kDir && F.do_x) st4(F.x + k * plane, o, wx[r], nv);
         }
-        if (KIND == kResid && ((k & 1) || k == nz - 1)) {
+        if (KIND == kA2 && ((k & 1) || k == nz - 1)) {
             // the coarse cells are complete: scaled residual of level 1
             const unsigned cc = (unsigned)(ja >> 1) * ncx + (ci >> 1);
             const gptr<float> rc = glob(C.r) + (k >> 1) * cplane;
@@ -396,18 +429,43 @@ __device__ __forceinline__ double mg_tile(const ProbDev &pd, int tile, gptr<cons
             for (int m = 0; m < 4; ++m) {
                 vb[r][m] = vc[r][m];
                 vc[r][m] = vt[r][m];
-                ac[r][m] = at[r][m];
-                bc[r][m] = bt[r][m];
+                if (KIND == kDir) bc[r][m] = bt[r][m];
                 szb[r][m] = szt[r][m];
             }
     }
     return acc;
 }
 
+// A tile's share of e += c - al p, c = 0 (all arrays, 16 or 32 bytes a lane).
+__device__ __forceinline__ void fold_correction(const ProbDev &pd, int tile, gptr<float> c, gptr<const float> p,
+                                                float al)
+{
+    typedef double vd4 __attribute__((ext_vector_type(4)));
+    typedef float va4 __attribute__((ext_vector_type(4)));
+    const gptr<double> e = glob(pd.e);
+    const long long len = pd.g.n, nv = len / 4, stride = (long long)pd.ntm * kThreads;
+    for (long long v = (long long)tile * kThreads + threadIdx.x; v < nv; v += stride) {
+        const va4 cv = ((gptr<const va4>)c)[v], pv = ((gptr<const va4>)p)[v];
+        vd4 ev = ((gptr<const vd4>)e)[v];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) ev[m] += (double)(cv[m] - al * pv[m]);
+        ((gptr<vd4>)e)[v] = ev;
+        ((gptr<va4>)c)[v] = va4{0.f, 0.f, 0.f, 0.f};
+    }
+    if (tile == 0) {
+        const long long x = nv * 4 + threadIdx.x;
+        if (x < len) {
+            e[x] += (double)(c[x] - al * p[x]);
+            c[x] = 0.f;
+        }
+    }
+}
+
+// Waves per SIMD: the kinds with one operand fit three, those with two
+// operands need the registers of two.
 template <int KIND>
-__global__ __launch_bounds__(kThreads, 2) void k_mg_fine(const ProbDev *__restrict__ P,
-                                                         const TileRef *__restrict__ tab, int ntab, StepRef sref,
-                                                         int *ran)
+__global__ __launch_bounds__(kThreads, (KIND == kA1 || KIND == kDir) ? 2 : 3) void k_mg_fine(
+    const ProbDev *__restrict__ P, const TileRef *__restrict__ tab, int ntab, StepRef sref, int *ran)
 {
     const Run run = my_run(ntab);
     const int step = step_of(sref);
@@ -418,160 +476,172 @@ __global__ __launch_bounds__(kThreads, 2) void k_mg_fine(const ProbDev *__restri
         const gptr<CgScalars> S = glob(pd.S);
         const int n = step - pd.n0 + 1;
         const int done_at = S->done_at, skip_e_at = S->skip_e_at;
-        if (n < 1 || n > done_at) continue;
+        const bool due = KIND != kA1 && KIND != kA2 && S->next_refresh == n;   // set by A2
+        if (n < 1 || n > done_at || (due && KIND != kDir)) continue;
         const bool fresh = n == 1 || step == skip_e_at;   // r_{n-1} stands in its buffer
-        double acc = 0.0;
-        const bool edge = pd.medge != 0;
-        if (KIND == kResid) {
+        const gptr<float> r = glob(rbuf(pd, n - 1)), r0 = glob(rbuf(pd, n));
+        const gptr<float> tt = glob(tbuf(pd)), rho = glob(pd.q32b), z = rho, q = glob(pd.q32);
+        FineArgs F{};
+        if (KIND == kA1) {
             const double rz = S->rz[(n - 1) & 1];
             const double pq = tot.get(tr.prob, part_pq(pd), pd.ntm);
             const double alpha = fresh || !(pq != 0.0) ? 0.0 : rz / pq;   // 0 / 0 once the residual is 0
             if (tr.tile == 0 && threadIdx.x == 0) S->alpha = alpha;
-            const gptr<const float> a = glob((const float *)rbuf(pd, fresh ? n - 1 : n));
-            const gptr<const float> b = glob((const float *)pd.q32);
-            const gptr<float> o = glob(rbuf(pd, n - 1));
-            acc = edge ? mg_tile<KIND, true>(pd, tr.tile, a, b, o, o, o, fresh, (float)alpha, 0.f, false)
-                       : mg_tile<KIND, false>(pd, tr.tile, a, b, o, o, o, fresh, (float)alpha, 0.f, false);
-        } else if (KIND == kSmooth) {
-            const gptr<const float> a = glob((const float *)rbuf(pd, n - 1));
-            const gptr<float> o = glob(pd.q32b);
-            acc = edge ? mg_tile<KIND, true>(pd, tr.tile, a, a, o, o, o, false, 0.f, 0.f, false)
-                       : mg_tile<KIND, false>(pd, tr.tile, a, a, o, o, o, false, 0.f, 0.f, false);
+            F = FineArgs{fresh ? r : r0, q, nullptr, nullptr, r, tt, nullptr, fresh, false, (float)alpha, 0.f};
+        } else if (KIND == kA2) {
+            if (tr.tile == 0) {
+                // a replacement instead of iteration n once r.r (the FP32
+                // recurrence's) has reached the threshold, or fallen as far
+                // as FP32 carries one cycle, or at the cap
+                const double rr = block_total_of(part_rr(pd), pd.ntm);
+                if (threadIdx.x == 0) {
+                    S->rr[n & 1] = rr;
+                    const double base = S->refreshes ? S->rr_after : S->rr0;
+                    const int iters = S->iters;
+                    if (!fresh && (rr <= kMgMargin * S->thresh || rr <= kMgCycleDrop * base ||
+                                   iters - S->prev_iters >= kMgMaxGap || iters >= S->max_iter))
+                        S->next_refresh = n;
+                }
+            }
+            F = FineArgs{tt, nullptr, r, nullptr, rho, nullptr, nullptr, false, false, 0.f, 0.f};
+        } else if (KIND == kB1) {
+            F = FineArgs{nullptr, nullptr, rho, nullptr, r0, nullptr, nullptr, false, false, 0.f, 0.f};
+        } else if (KIND == kB2) {
+            F = FineArgs{r0, nullptr, r, tt, z, nullptr, nullptr, false, false, 0.f, 0.f};
         } else {
             const double rz_prev = S->rz[(n - 1) & 1], alpha = S->alpha;
-            const int max_iter = S->max_iter;
-            const double rz = tot.get(tr.prob, part_rz(pd), pd.ntm);
+            const double rz = due ? 0.0 : tot.get(tr.prob, part_rz(pd), pd.ntm);
             // a breakdown: r.z and p.q are positive for every operator the
             // V-cycle is definite for, unless a value left FP32's range
             const bool bad = !(rz >= 0.0 && rz < 1e300) || !(alpha >= 0.0 && alpha < 1e300);
-            const bool cap = n - 1 >= max_iter;
-            const double beta = n == 1 || !(rz_prev > 0.0) ? 0.0 : rz / rz_prev;
-            if (tr.tile == 0) {
-                const double rr = block_total_of(part_rr(pd), pd.ntm);
-                if (threadIdx.x == 0) {
+            // a replacement starts the directions afresh: the replaced residual
+            // is no longer r - alpha q, and directions conjugate to it went
+            // on at a third of the rate
+            const double beta = fresh || !(rz_prev > 0.0) ? 0.0 : rz / rz_prev;
+            if (tr.tile == 0 && threadIdx.x == 0) {
+                if (bad) {
+                    S->giveup = 1;
+                    S->final_ = 1;
+                    S->done_at = n;
+                } else if (!due) {
                     S->rz[n & 1] = rz;
-                    S->rr[n & 1] = rr;
-                    S->iters = n - 1;
-                    if (bad) {
-                        S->giveup = 1;
-                        S->final_ = 1;
-                        S->done_at = n;
-                    } else if (cap) {
-                        S->done_at = n;
-                    } else if (S->next_refresh == kNotDone) {
-                        // r.r (FP32 recurrence) has reached the threshold,
-                        // or as far as FP32 carries one cycle
-                        const double base = S->refreshes ? S->rr_after : S->rr0;
-                        if (rr <= S->thresh || rr <= kMgCycleDrop * base || n - S->prev_iters >= kMgMaxGap)
-                            S->next_refresh = n + (n & 1);
-                    }
-                    if (ran && tr.prob == 0 && !bad && !cap) *ran = 1;
+                    S->iters = S->iters + 1;
+                    if (ran && tr.prob == 0) *ran = 1;
                 }
             }
             if (bad) continue;
-            const gptr<const float> z = glob((const float *)pd.q32b), po = glob((const float *)mpbuf(pd, n - 1));
+            const gptr<float> po = glob(mpbuf(pd, n - 1));
             const gptr<float> x = glob(pd.c32);
-            if (cap) {
-                // finish iteration n - 1 only: c -= alpha p
-                if (!fresh) {
-                    const float al = (float)alpha;
-                    for (long long c = (long long)tr.tile * kThreads + threadIdx.x; c < pd.g.n;
-                         c += (long long)pd.ntm * kThreads)
-                        x[c] = x[c] - al * po[c];
-                }
+            if (due) {
+                // e += c - alpha_{n-1} p_{n-1}, c = 0
+                fold_correction(pd, tr.tile, x, po, (float)alpha);
                 continue;
             }
-            const gptr<float> pn = glob(mpbuf(pd, n)), q = glob(pd.q32);
-            acc = edge ? mg_tile<KIND, true>(pd, tr.tile, z, po, pn, q, x, n == 1, (float)beta, (float)alpha, !fresh)
-                       : mg_tile<KIND, false>(pd, tr.tile, z, po, pn, q, x, n == 1, (float)beta, (float)alpha, !fresh);
+            F = FineArgs{z, po, nullptr, nullptr, glob(mpbuf(pd, n)), q, x, fresh, !fresh, (float)beta, (float)alpha};
         }
+        const double acc = pd.medge ? mg_tile<KIND, true>(pd, tr.tile, F) : mg_tile<KIND, false>(pd, tr.tile, F);
+        if (KIND == kA2 || KIND == kB1) continue;
         const double sres = block_sum(acc);
-        if (threadIdx.x == 0) (KIND == kResid ? part_rr(pd) : KIND == kSmooth ? part_rz(pd) : part_pq(pd))[tr.tile] = sres;
+        if (threadIdx.x == 0) (KIND == kA1 ? part_rr(pd) : KIND == kB2 ? part_rz(pd) : part_pq(pd))[tr.tile] = sres;
     }
 }
 
 // ---- coarse levels (l >= 1) -------------------------------------------------
 
 // sum over the six neighbours of s_face f(neighbour); faces at walls hold 0,
-// so a clamped neighbour index only has to be valid
+// so a wrapped neighbour index only has to be valid
 template <class F>
-__device__ __forceinline__ float nb_sum(const MgLevel &L, int i, int j, int k, F &&f)
+__device__ __forceinline__ float nb_sum(const MgLevel &L, int c, int i, int j, int k, F &&f)
 {
-    const int nx = L.nx, ny = L.ny;
-    const int c = (k * ny + j) * nx + i;
-    const gptr<const float> sx = glob((const float *)L.sx) + ((k * ny + j) * (nx + 1) + i);
-    const gptr<const float> sy = glob((const float *)L.sy) + ((k * (ny + 1) + j) * nx + i);
+    const int nx = L.nx, ny = L.ny, nz = L.nz, pl = nx * ny;
+    const gptr<const float> sx = glob((const float *)L.sx) + (c + (k * ny + j));
+    const gptr<const float> sy = glob((const float *)L.sy) + (c + k * nx);
     const gptr<const float> sz = glob((const float *)L.sz) + c;
-    const int cw = c + nb_lo(i, nx, L.px) - i, ce = c + nb_hi(i, nx, L.px) - i;
-    const int cs = c + (nb_lo(j, ny, L.py) - j) * nx, cn = c + (nb_hi(j, ny, L.py) - j) * nx;
-    const int pl = nx * ny, cb = k > 0 ? c - pl : c, ct = k < L.nz - 1 ? c + pl : c;
-    return sx[1] * f(ce, i < nx - 1 ? i + 1 : 0, j, k) + sx[0] * f(cw, i > 0 ? i - 1 : nx - 1, j, k) +
-           sy[nx] * f(cn, i, j < ny - 1 ? j + 1 : 0, k) + sy[0] * f(cs, i, j > 0 ? j - 1 : ny - 1, k) +
-           sz[pl] * f(ct, i, j, k < L.nz - 1 ? k + 1 : k) + sz[0] * f(cb, i, j, k > 0 ? k - 1 : k);
+    const int ie = i < nx - 1 ? i + 1 : 0, iw = i > 0 ? i - 1 : nx - 1;
+    const int jn = j < ny - 1 ? j + 1 : 0, js = j > 0 ? j - 1 : ny - 1;
+    const int kt = k < nz - 1 ? k + 1 : 0, kb = k > 0 ? k - 1 : nz - 1;
+    return sx[1] * f(c + ie - i, ie, j, k) + sx[0] * f(c + iw - i, iw, j, k) + sy[nx] * f(c + (jn - j) * nx, i, jn, k) +
+           sy[0] * f(c + (js - j) * nx, i, js, k) + sz[pl] * f(c + (kt - k) * pl, i, j, kt) +
+           sz[0] * f(c + (kb - k) * pl, i, j, kb);
 }
 
 __device__ __forceinline__ bool running(const ProbDev &pd, int step)
 {
     const gptr<const CgScalars> S = glob((const CgScalars *)pd.S);
     const int n = step - pd.n0 + 1;
-    return n >= 1 && n <= S->done_at;
+    return n >= 1 && n <= S->done_at && n != S->next_refresh;
 }
 
-// Level l -> l + 1: a thread per coarse cell sums its children's weighted
-// residuals after z = omega r.
-__global__ __launch_bounds__(kThreads) void k_mg_down(const ProbDev *__restrict__ P, const TileRef *__restrict__ tab,
-                                                      int ntab, int l, StepRef sref)
+// Bricks of 16 x 4 x 4 cells, one workgroup each and one cell per thread: a
+// brick holds whole coarse cells, and its 2x2x2 sums go through LDS.
+constexpr int kBx = 16, kBy = 4, kBz = 4;
+__host__ __device__ inline int bricks(const MgLevel &L)
 {
+    return ((L.nx + kBx - 1) / kBx) * ((L.ny + kBy - 1) / kBy) * ((L.nz + kBz - 1) / kBz);
+}
+
+// A pass over level l (1 <= l < lbot): D1, D2, U1 or U2 (A1, A2, B1, B2 of
+// the fine kernels; no partial sums, and U2 leaves the un-scaled correction).
+template <int KIND>
+__global__ __launch_bounds__(kThreads) void k_mg_level(const ProbDev *__restrict__ P, const TileRef *__restrict__ tab,
+                                                       int ntab, int l, StepRef sref)
+{
+    __shared__ float sh[kThreads];
     const Run run = my_run(ntab);
     const int step = step_of(sref);
-    for (int t = run.begin; t < run.end; ++t) {
-        const TileRef tr = tab[t];
+    for (int tt = run.begin; tt < run.end; ++tt) {
+        const TileRef tr = tab[tt];
         const ProbDev &pd = P[tr.prob];
         if (!running(pd, step)) continue;
         const MgLevel &L = pd.lv[l], &C = pd.lv[l + 1];
-        const int c = tr.tile * kThreads + threadIdx.x;
-        const int I = c % C.nx, r0 = c / C.nx, J = r0 % C.ny, K = r0 / C.ny;
-        if (K >= C.nz) continue;
-        const gptr<const float> r = glob((const float *)L.r), w = glob((const float *)L.w);
-        float sum = 0.f;
-#pragma unroll
-        for (int m = 0; m < 8; ++m) {
-            const int i = 2 * I + (m & 1), j = 2 * J + ((m >> 1) & 1), k = 2 * K + (m >> 2);
-            if (i < L.nx && j < L.ny && k < L.nz) {
-                const int x = (k * L.ny + j) * L.nx + i;
-                const float nb = nb_sum(L, i, j, k, [&](int y, int, int, int) { return r[y]; });
-                sum += w[x] * ((1.f - kOmega) * r[x] + kOmega * nb);
+        const int bx = (L.nx + kBx - 1) / kBx, by = (L.ny + kBy - 1) / kBy;
+        const int tx = tr.tile % bx, rest = tr.tile / bx, ty = rest % by, tz = rest / by;
+        const int tid = threadIdx.x;
+        const int i = tx * kBx + (tid & 15), j = ty * kBy + ((tid >> 4) & 3), k = tz * kBz + (tid >> 6);
+        const bool in = i < L.nx && j < L.ny && k < L.nz;
+        const int c = (k * L.ny + j) * L.nx + i;
+        const gptr<float> r = glob(L.r), t = glob(L.t), rho = glob(L.rho), r0 = glob(L.r0), w = glob(L.w);
+        const gptr<const float> e = glob((const float *)C.t);
+        auto parent = [&](int a, int b, int d) { return ((d >> 1) * C.ny + (b >> 1)) * C.nx + (a >> 1); };
+        if (KIND == kA1) {
+            if (in) t[c] = r[c] - nb_sum(L, c, i, j, k, [&](int x, int, int, int) { return r[x]; });
+        } else if (KIND == kA2) {
+            float v = 0.f;
+            if (in) {
+                const float tc = t[c];
+                const float y = tc - nb_sum(L, c, i, j, k, [&](int x, int, int, int) { return t[x]; });
+                const float rh = r[c] - kC0 * tc - kC1 * y;
+                rho[c] = rh;
+                v = w[c] * rh;
+            }
+            __syncthreads();
+            sh[tid] = v;
+            __syncthreads();
+            if (tid < kThreads / 8) {
+                const int I = tid & 7, J = (tid >> 3) & 1, K = tid >> 4;
+                const int b = (2 * K) * 64 + (2 * J) * 16 + 2 * I;
+                const float sum = ((sh[b] + sh[b + 1]) + (sh[b + 16] + sh[b + 17])) +
+                                  ((sh[b + 64] + sh[b + 65]) + (sh[b + 80] + sh[b + 81]));
+                const int ic = tx * (kBx / 2) + I, jc = ty * (kBy / 2) + J, kc = tz * (kBz / 2) + K;
+                if (ic < C.nx && jc < C.ny && kc < C.nz) {
+                    const int x = (kc * C.ny + jc) * C.nx + ic;
+                    const float wc = C.w[x];
+                    glob(C.r)[x] = wc > 0.f ? sum / wc : 0.f;
+                }
+            }
+        } else if (KIND == kB1) {
+            if (in) {
+                auto v = [&](int x, int a, int b, int d) { return w[x] * e[parent(a, b, d)]; };
+                r0[c] = rho[c] - v(c, i, j, k) + nb_sum(L, c, i, j, k, v);
+            }
+        } else {
+            if (in) {
+                const float v = r0[c], wc = w[c];
+                const float y = v - nb_sum(L, c, i, j, k, [&](int x, int, int, int) { return r0[x]; });
+                const float z = kC0 * (r[c] + v) + kC1 * (t[c] + y) + wc * e[parent(i, j, k)];
+                t[c] = wc > 0.f ? z / wc : 0.f;
             }
         }
-        const float wc = C.w[c];
-        glob(C.r)[c] = wc > 0.f ? sum / wc : 0.f;
-    }
-}
-
-// Level l: v = omega r + w (parent's correction), one Jacobi sweep, and the
-// correction un-scaled for the level below in the hierarchy.
-__global__ __launch_bounds__(kThreads) void k_mg_up(const ProbDev *__restrict__ P, const TileRef *__restrict__ tab,
-                                                    int ntab, int l, StepRef sref)
-{
-    const Run run = my_run(ntab);
-    const int step = step_of(sref);
-    for (int t = run.begin; t < run.end; ++t) {
-        const TileRef tr = tab[t];
-        const ProbDev &pd = P[tr.prob];
-        if (!running(pd, step)) continue;
-        const MgLevel &L = pd.lv[l], &C = pd.lv[l + 1];
-        const int c = tr.tile * kThreads + threadIdx.x;
-        const int i = c % L.nx, r0 = c / L.nx, j = r0 % L.ny, k = r0 / L.ny;
-        if (k >= L.nz) continue;
-        const gptr<const float> r = glob((const float *)L.r), w = glob((const float *)L.w), e = glob((const float *)C.e);
-        auto v = [&](int x, int a, int b, int d) {
-            return kOmega * r[x] + w[x] * e[((d >> 1) * C.ny + (b >> 1)) * C.nx + (a >> 1)];
-        };
-        const float vc = v(c, i, j, k);
-        const float nb = nb_sum(L, i, j, k, v);
-        const float z = vc + kOmega * (r[c] - vc + nb);
-        const float wc = w[c];
-        glob(L.e)[c] = wc > 0.f ? z / wc : 0.f;
     }
 }
 
@@ -589,189 +659,233 @@ __device__ __forceinline__ double bot_sum(double v)
     return s;
 }
 
-// Takes the constant-pressure component out of a level's scaled residual (v
-// -= (v.w / w.w) w) or un-scaled correction (v -= (v.w^2 / w.w)).  Where the
-// operator has that null space, the coarse levels would amplify the
-// component about fourfold each, and the FP32 operator is not exactly (nor
-// surely not negatively) singular on it: p.q then went negative at 1e-11
-// relative residuals.  Taken out of both sides, the cycle stays symmetric.
-__device__ __forceinline__ void drop_null(const MgLevel &L, float *v, bool unscaled)
+// One cell of a bottom level: its faces (E, W, N, S, T, B), w, and its parent
+// (bits 6 up) and the sides it is on (bits 0 .. 5).  The set-up packs the
+// cells of all bottom levels one after another.
+struct BotCell {
+    float s[6], w;
+    unsigned bits;
+    __device__ __forceinline__ float iw() const { return w > 0.f ? 1.f / w : 0.f; }
+};
+static_assert(sizeof(BotCell) == 32, "two 16-byte loads");
+__device__ __forceinline__ BotCell packed_cell(gptr<const float> pack, int c)
 {
-    const int m = L.nx * L.ny * L.nz;
-    const gptr<const float> w = glob((const float *)L.w);
-    double vw = 0.0, ww = 0.0;
-    for (int c = threadIdx.x; c < m; c += kBotThreads) {
-        const double wc = w[c];
-        vw += (unscaled ? wc * wc : wc) * (double)v[c];
-        ww += wc * wc;
-    }
-    vw = bot_sum(vw);
-    ww = bot_sum(ww);
-    const double f = ww > 0.0 ? vw / ww : 0.0;
-    for (int c = threadIdx.x; c < m; c += kBotThreads) v[c] = (float)((double)v[c] - f * (unscaled ? 1.0 : (double)w[c]));
-    __syncthreads();
+    typedef float va4 __attribute__((ext_vector_type(4)));
+    const va4 u = ((gptr<const va4>)pack)[2 * c], v = ((gptr<const va4>)pack)[2 * c + 1];
+    return BotCell{{u[0], u[1], u[2], u[3], v[0], v[1]}, v[2], __float_as_uint(v[3])};
+}
+__device__ __forceinline__ BotCell bot_cell(const MgLevel &L, int c)
+{
+    const int nx = L.nx, ny = L.ny, nz = L.nz;
+    const int i = c % nx, r0 = c / nx, j = r0 % ny, k = r0 / ny;
+    const float *sx = L.sx + (c + (k * ny + j)), *sy = L.sy + (c + k * nx), *sz = L.sz + c;
+    BotCell b;
+    b.s[0] = sx[1];
+    b.s[1] = sx[0];
+    b.s[2] = sy[nx];
+    b.s[3] = sy[0];
+    b.s[4] = sz[nx * ny];
+    b.s[5] = sz[0];
+    b.w = L.w[c];
+    b.bits = (i == nx - 1) | (i == 0) << 1 | (j == ny - 1) << 2 | (j == 0) << 3 |
+             (unsigned)((i >> 1) + (((nx + 1) >> 1) * ((j >> 1) + ((ny + 1) >> 1) * (k >> 1)))) << 6;
+    return b;
+}
+// The six neighbours' share of A v.  Neighbours across a wall are the next
+// cells in memory: their face is 0, and everything around is finite.  Only
+// periodic sides need the wrapped index.
+struct BotDim {
+    int nx, pl;
+    bool per;
+};
+__device__ __forceinline__ float bot_nb(const BotDim &d, const BotCell &b, int c, const float *v)
+{
+    const int nx = d.nx, pl = d.pl;
+    const float z = b.s[4] * v[c + pl] + b.s[5] * v[c - pl];
+    if (!d.per) return b.s[0] * v[c + 1] + b.s[1] * v[c - 1] + b.s[2] * v[c + nx] + b.s[3] * v[c - nx] + z;
+    const int ny1 = pl - nx;
+    return b.s[0] * v[c + ((b.bits & 1u) ? 1 - nx : 1)] + b.s[1] * v[c + ((b.bits & 2u) ? nx - 1 : -1)] +
+           b.s[2] * v[c + ((b.bits & 4u) ? -ny1 : nx)] + b.s[3] * v[c + ((b.bits & 8u) ? ny1 : -nx)] + z;
 }
 
-// Levels lbot .. nlev - 1 of one problem in one workgroup: residuals and
-// corrections in LDS, coefficients from L2.  zs holds a level's weighted
-// residuals on the way down and its corrections on the way up.
+// Levels lbot .. nlev - 1 of one problem in one workgroup.  Vectors live in
+// LDS; the coefficients of level lbot in registers (kBotPer cells per thread)
+// and the smaller levels' in LDS, all loaded at the start, so that the passes
+// wait on memory once.  Levels of at most kBotWave cells are one wave's, whose
+// LDS accesses need no barrier.
+//
+// The constant-pressure component is taken out of level lbot's residual where
+// the operator has that null space: the coarse levels would amplify it about
+// fourfold each, and the FP32 operator is not exactly (nor surely not
+// negatively) singular on it; p.q then went negative at 1e-11 relative
+// residuals.  (Residuals of a consistent system have that component from
+// rounding alone, so r.z stays that of a symmetric cycle.)
+constexpr int kBotWave = 256;
 __global__ __launch_bounds__(kBotThreads) void k_mg_bottom(const ProbDev *__restrict__ P,
                                                            const int *__restrict__ probs, StepRef sref)
 {
-    __shared__ float rs[kMgBottomLds], zs[kMgBottomLds];
+    __shared__ __align__(16) float lds[kMgBottomLds];
+    __shared__ int lnx[kMgLevels], lny[kMgLevels], lnz[kMgLevels];
     const ProbDev &pd = P[probs[blockIdx.x]];
     if (!running(pd, step_of(sref))) return;
     const int tid = threadIdx.x, lb = pd.lbot, nl = pd.nlev;
-    {
-        const MgLevel &L = pd.lv[lb];
-        const int m = L.nx * L.ny * L.nz;
-        const gptr<const float> r = glob((const float *)L.r);
-        for (int c = tid; c < m; c += kBotThreads) rs[c] = r[c];
+    const bool project = pd.S->project != 0;
+    const MgLevel &L0 = pd.lv[lb];
+    const int m0 = L0.nx * L0.ny * L0.nz, total = pd.nbot;
+    const gptr<const float> pack = glob((const float *)pd.bot);
+    const gptr<const float> r0 = glob((const float *)L0.r);
+    const bool per = L0.px | L0.py;
+    // the coefficients of the levels below lbot, then R, A, B, D (a value
+    // per cell of all levels) with a guard of one plane on both sides
+    const int guard = L0.nx * L0.ny;
+    BotCell *const low = reinterpret_cast<BotCell *>(lds);
+    float *const R = lds + 8 * (total - m0) + guard, *const A = R + total, *const B = A + total, *const D = B + total;
+    BotCell top[kBotPer];
+    double vw = 0.0, ww = 0.0;
+#pragma unroll
+    for (int q = 0; q < kBotPer; ++q) {
+        const int c = tid + q * kBotThreads;
+        if (c < m0) {
+            top[q] = packed_cell(pack, c);
+            const float r = r0[c];
+            R[c] = r;
+            vw += (double)top[q].w * (double)r;
+            ww += (double)top[q].w * (double)top[q].w;
+        }
+    }
+    for (int c = tid; c < total - m0; c += kBotThreads) low[c] = packed_cell(pack, m0 + c);
+    if (tid < nl - lb) {
+        lnx[tid] = pd.lv[lb + tid].nx;
+        lny[tid] = pd.lv[lb + tid].ny;
+        lnz[tid] = pd.lv[lb + tid].nz;
+    }
+    // every value that a wall's neighbour index can reach is finite
+    for (int c = tid; c < guard; c += kBotThreads) R[c - guard] = D[total + c] = 0.f;
+    for (int c = tid; c < total - m0; c += kBotThreads) R[m0 + c] = 0.f;
+    for (int c = tid; c < 3 * total; c += kBotThreads) A[c] = 0.f;
+    if (project) {
+        vw = bot_sum(vw);
+        ww = bot_sum(ww);
+        const double f = ww > 0.0 ? vw / ww : 0.0;
+#pragma unroll
+        for (int q = 0; q < kBotPer; ++q) {
+            const int c = tid + q * kBotThreads;
+            if (c < m0) R[c] = (float)((double)R[c] - f * (double)top[q].w);
+        }
     }
     __syncthreads();
-    if (pd.S->project) drop_null(pd.lv[lb], rs, false);
-    int off = 0;
-    for (int l = lb; l < nl - 1; ++l) {
-        const MgLevel &L = pd.lv[l], &C = pd.lv[l + 1];
-        const int m = L.nx * L.ny * L.nz, mc = C.nx * C.ny * C.nz;
-        const float *r = rs + off;
-        float *z = zs + off;
-        for (int c = tid; c < m; c += kBotThreads) {
-            const int i = c % L.nx, r0 = c / L.nx, j = r0 % L.ny, k = r0 / L.ny;
-            const float nb = nb_sum(L, i, j, k, [&](int y, int, int, int) { return r[y]; });
-            z[c] = L.w[c] * ((1.f - kOmega) * r[c] + kOmega * nb);
-        }
-        __syncthreads();
-        for (int c = tid; c < mc; c += kBotThreads) {
-            const int I = c % C.nx, r0 = c / C.nx, J = r0 % C.ny, K = r0 / C.ny;
-            float sum = 0.f;
+    // f(cell, index in the level) for the cells of level lb + l at off, by
+    // all threads or by the first wave's
+    auto each = [&](bool wave, int l, int off, int m, auto &&f) {
+        if (l == 0) {
 #pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const int i = 2 * I + (q & 1), j = 2 * J + ((q >> 1) & 1), k = 2 * K + (q >> 2);
-                if (i < L.nx && j < L.ny && k < L.nz) sum += z[(k * L.ny + j) * L.nx + i];
+            for (int q = 0; q < kBotPer; ++q) {
+                const int c = tid + q * kBotThreads;
+                if (c < m0) f(top[q], c);
             }
-            const float wc = C.w[c];
-            rs[off + m + c] = wc > 0.f ? sum / wc : 0.f;
+        } else {
+            for (int c = tid; c < m; c += wave ? 64 : kBotThreads) f(low[off - m0 + c], c);
         }
-        __syncthreads();
-        off += m;
-    }
-    {
-        // the coarsest level: Jacobi sweeps from zero
-        const MgLevel &L = pd.lv[nl - 1];
-        const int m = L.nx * L.ny * L.nz;   // <= kBotThreads
-        const int i = tid % L.nx, r0 = tid / L.nx, j = r0 % L.ny, k = r0 / L.ny;
-        const float *r = rs + off;
-        float *z = zs + off;
-        float v = 0.f;
-        if (tid < m) z[tid] = v = kOmega * r[tid];
-        __syncthreads();
-        for (int it = 1; it < kMgCoarsestSweeps; ++it) {
-            if (tid < m) {
-                const float nb = nb_sum(L, i, j, k, [&](int y, int, int, int) { return z[y]; });
-                v = v + kOmega * (r[tid] - v + nb);
+    };
+    auto sync = [&](bool wave) {
+        if (wave)
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        else
+            __syncthreads();
+    };
+    auto dim = [&](int l) {
+        const int nx = lnx[l], ny = lny[l];
+        // a side of a single cell is not periodic (mg_plan), its faces are 0
+        return BotDim{nx, nx * ny, per};
+    };
+    auto down = [&](bool wave, int l, int off) {
+        const BotDim d = dim(l);
+        const int nx = d.nx, ny = lny[l], nz = lnz[l], m = d.pl * nz;
+        float *const r = R + off, *const a = A + off, *const b = B + off, *const w = D + off;
+        each(wave, l, off, m, [&](const BotCell &x, int c) { a[c] = r[c] - bot_nb(d, x, c, r); });
+        sync(wave);
+        each(wave, l, off, m, [&](const BotCell &x, int c) {
+            b[c] = r[c] - kC0 * a[c] - kC1 * (a[c] - bot_nb(d, x, c, a));
+            w[c] = x.w * b[c];
+        });
+        sync(wave);
+        const int cx = lnx[l + 1], cy = lny[l + 1], mc = cx * cy * lnz[l + 1];
+        for (int c = tid; c < mc; c += wave ? 64 : kBotThreads) {
+            const int I = c % cx, q0 = c / cx, J = q0 % cy, K = q0 / cy;
+            const float *x = w + ((2 * K * ny + 2 * J) * nx + 2 * I);
+            const bool i1 = 2 * I + 1 < nx, j1 = 2 * J + 1 < ny, k1 = 2 * K + 1 < nz;
+            float sum = x[0] + (i1 ? x[1] : 0.f);
+            if (j1) sum += x[nx] + (i1 ? x[nx + 1] : 0.f);
+            if (k1) {
+                x += d.pl;
+                sum += x[0] + (i1 ? x[1] : 0.f);
+                if (j1) sum += x[nx] + (i1 ? x[nx + 1] : 0.f);
             }
-            __syncthreads();
-            if (tid < m) z[tid] = v;
-            __syncthreads();
+            R[off + m + c] = sum * low[off + m - m0 + c].iw();
         }
-        if (tid < m) {
-            const float wc = L.w[tid];
-            z[tid] = wc > 0.f ? v / wc : 0.f;
+        sync(wave);
+        return off + m;
+    };
+    auto up = [&](bool wave, int l, int off, int m) {
+        const BotDim dd = dim(l);
+        const float *const e = A + off + m;
+        float *const r = R + off, *const a = A + off, *const b = B + off, *const d = D + off;
+        each(wave, l, off, m, [&](const BotCell &x, int c) { d[c] = x.w * e[x.bits >> 6]; });
+        sync(wave);
+        each(wave, l, off, m, [&](const BotCell &x, int c) { b[c] = b[c] - d[c] + bot_nb(dd, x, c, d); });
+        sync(wave);
+        each(wave, l, off, m, [&](const BotCell &x, int c) {
+            const float y = b[c] - bot_nb(dd, x, c, b);
+            a[c] = (kC0 * (r[c] + b[c]) + kC1 * (a[c] + y) + d[c]) * x.iw();
+        });
+        sync(wave);
+    };
+    const int nb = nl - lb;
+    auto size = [&](int l) { return lnx[l] * lny[l] * lnz[l]; };
+    int l = 0, off = 0;
+    for (; l < nb - 1 && (l == 0 || size(l) > kBotWave); ++l) off = down(false, l, off);
+    const int lw = l, offw = off;
+    if (tid < 64) {
+        for (; l < nb - 1; ++l) off = down(true, l, off);
+        {
+            // the coarsest level (at most 64 cells): Jacobi sweeps from zero
+            const BotDim d = dim(l);
+            const int m = size(l);
+            const BotCell x = nb == 1 ? top[0] : low[off - m0 + min(tid, m - 1)];
+            float *const a = A + off;
+            const float r = tid < m ? R[off + tid] : 0.f;
+            float v = kOmega * r;
+            for (int it = 1; it < kMgCoarsestSweeps; ++it) {
+                if (tid < m) a[tid] = v;
+                sync(true);
+                if (tid < m) v = v + kOmega * (r - v + bot_nb(d, x, tid, a));
+                sync(true);
+            }
+            if (tid < m) a[tid] = v * x.iw();
+            sync(true);
         }
-        __syncthreads();
+        for (--l; l >= lw; --l) {
+            const int m = size(l);
+            off -= m;
+            up(true, l, off, m);
+        }
     }
-    for (int l = nl - 2; l >= lb; --l) {
-        const MgLevel &L = pd.lv[l], &C = pd.lv[l + 1];
-        const int m = L.nx * L.ny * L.nz;
-        const float *ec = zs + off;
+    __syncthreads();
+    off = offw;
+    for (l = lw - 1; l >= 0; --l) {
+        const int m = size(l);
         off -= m;
-        const float *r = rs + off;
-        float *z = zs + off;
-        for (int c = tid; c < m; c += kBotThreads) {
-            const int i = c % L.nx, r0 = c / L.nx, j = r0 % L.ny, k = r0 / L.ny;
-            z[c] = kOmega * r[c] + L.w[c] * ec[((k >> 1) * C.ny + (j >> 1)) * C.nx + (i >> 1)];
-        }
-        __syncthreads();
-        float v[kBotPer];
-#pragma unroll
-        for (int q = 0; q < kBotPer; ++q) {
-            const int c = tid + q * kBotThreads;
-            v[q] = 0.f;
-            if (c < m) {
-                const int i = c % L.nx, r0 = c / L.nx, j = r0 % L.ny, k = r0 / L.ny;
-                const float nb = nb_sum(L, i, j, k, [&](int y, int, int, int) { return z[y]; });
-                const float wc = L.w[c];
-                v[q] = wc > 0.f ? (z[c] + kOmega * (r[c] - z[c] + nb)) / wc : 0.f;
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < kBotPer; ++q) {
-            const int c = tid + q * kBotThreads;
-            if (c < m) z[c] = v[q];
-        }
-        __syncthreads();
+        up(false, l, off, m);
     }
-    if (pd.S->project) drop_null(pd.lv[lb], zs, true);
-    {
-        const MgLevel &L = pd.lv[lb];
-        const int m = L.nx * L.ny * L.nz;
-        const gptr<float> e = glob(L.e);
-        for (int c = tid; c < m; c += kBotThreads) e[c] = zs[c];
+    const gptr<float> e = glob(L0.t);
+#pragma unroll
+    for (int q = 0; q < kBotPer; ++q) {
+        const int c = tid + q * kBotThreads;
+        if (c < m0) e[c] = A[c];
     }
 }
 
 // ---- residual replacement ---------------------------------------------------
-
-// As refresh_due in ps_cg.hip.
-__device__ __forceinline__ bool mg_due(const ProbDev &pd, int step)
-{
-    const gptr<const CgScalars> S = glob((const CgScalars *)pd.S);
-    const int n = step - pd.n0 + 1;
-    return n >= 1 && !S->final_ && (n == S->next_refresh || S->done_at != kNotDone);
-}
-
-// e += c - alpha_n p_n (alpha_n from the partials of iteration n's kernels), c = 0.
-__global__ __launch_bounds__(kThreads) void k_mg_refresh_e(const ProbDev *__restrict__ P,
-                                                           const TileRef *__restrict__ tab, int ntab, StepRef sref)
-{
-    const Run run = my_run(ntab);
-    const int step = step_of(sref);
-    TotalCache tot;
-    for (int t = run.begin; t < run.end; ++t) {
-        const TileRef tr = tab[t];
-        const ProbDev &pd = P[tr.prob];
-        if (!mg_due(pd, step)) continue;
-        const gptr<const CgScalars> S = glob((const CgScalars *)pd.S);
-        const int n = step - pd.n0 + 1;
-        const bool pending = S->done_at == kNotDone;
-        const double pq = tot.get(tr.prob, part_pq(pd), pd.ntm);
-        const float al = pending && pq != 0.0 ? (float)(S->rz[n & 1] / pq) : 0.f;
-        const gptr<const float> p = glob((const float *)mpbuf(pd, n));
-        const gptr<double> e = glob(pd.e);
-        const gptr<float> c = glob(pd.c32);
-        typedef double vd4 __attribute__((ext_vector_type(4)));
-        typedef float va4 __attribute__((ext_vector_type(4)));
-        const long long len = pd.g.n, nv = len / 4, stride = (long long)pd.nt1 * kThreads;
-        for (long long v = (long long)tr.tile * kThreads + threadIdx.x; v < nv; v += stride) {
-            va4 cv = ((gptr<const va4>)c)[v];
-            const va4 pv = ((gptr<const va4>)p)[v];
-            vd4 ev = ((gptr<const vd4>)e)[v];
-#pragma unroll
-            for (int m = 0; m < 4; ++m) ev[m] += (double)(pending ? cv[m] - al * pv[m] : cv[m]);
-            ((gptr<vd4>)e)[v] = ev;
-            ((gptr<va4>)c)[v] = va4{0.f, 0.f, 0.f, 0.f};
-        }
-        if (tr.tile == 0) {
-            const long long x = nv * 4 + threadIdx.x;
-            if (x < len) {
-                e[x] += (double)(pending ? c[x] - al * p[x] : c[x]);
-                c[x] = 0.f;
-            }
-        }
-    }
-}
 
 // After k_true_residual: converged, capped, given up, or on.
 __global__ __launch_bounds__(kThreads) void k_mg_decide(const ProbDev *__restrict__ P, const int *__restrict__ probs,
@@ -780,35 +894,32 @@ __global__ __launch_bounds__(kThreads) void k_mg_decide(const ProbDev *__restric
     const int step = step_of(sref);
     const ProbDev &pd = P[probs[blockIdx.x]];
     CgScalars *S = pd.S;
-    if (!mg_due(pd, step)) return;
     const int n = step - pd.n0 + 1;
+    if (n < 1 || S->final_ || n != S->next_refresh) return;
     const double rrt = block_total_of(pd.P.tres, pd.nt3);
     const double rrs = block_total_of(pd.P.tres + pd.nt3, pd.nt3);
     if (threadIdx.x == 0) {
-        const bool pending = S->done_at == kNotDone;
-        const int iters = pending ? n : S->iters;
         const bool finite = rrt >= 0.0 && rrt < 1e300;
         const bool conv = finite && !(rrt > S->thresh);
-        const bool cap = iters >= S->max_iter;
+        const bool cap = S->iters >= S->max_iter;
         // a cycle that did not halve r.r: counted, and after three in a row
         // the solve goes back to CG from the start
         const double before = S->refreshes ? S->prev_rr : S->rr0;
         S->stalls = rrt < 0.5 * before ? 0 : S->stalls + 1;
         S->rr_true = rrt;
         S->refreshes += 1;
-        S->iters = iters;
         if (!conv && (!finite || S->stalls >= 3)) {
             S->giveup = 1;
             S->final_ = 1;
-            if (pending) S->done_at = n;
+            S->done_at = n;
         } else if (conv || cap) {
             S->final_ = 1;
             S->status = conv ? 0 : 1;
-            if (pending) S->done_at = n;
+            S->done_at = n;
         } else {
             S->skip_e_at = step + 1;
             S->rr_after = rrs;
-            S->prev_iters = n;
+            S->prev_iters = S->iters;
             S->prev_rr = rrt;
             S->next_refresh = kNotDone;
         }
@@ -1034,7 +1145,8 @@ __global__ __launch_bounds__(kThreads) void k_mg_scale(MgLevel C)
     if (c < C.nx * C.ny * C.nz) scale_cell(C, c);
 }
 
-// Levels lbot .. nlev - 1 in one workgroup (each from the one before).
+// Levels l0 .. nlev - 1 in one workgroup (each from the one before), and the
+// bottom levels' cells packed.
 __global__ __launch_bounds__(kBotThreads) void k_mg_coarse_bottom(const ProbDev *__restrict__ P, int l0, int lid, float top)
 {
     const ProbDev &pd = *P;
@@ -1047,6 +1159,14 @@ __global__ __launch_bounds__(kBotThreads) void k_mg_coarse_bottom(const ProbDev 
         for (int c = threadIdx.x; c < m; c += kBotThreads) scale_cell(C, c);
         __threadfence_block();
         __syncthreads();
+    }
+    // the bottom kernel's pack
+    int off = 0;
+    for (int l = pd.lbot; l < pd.nlev; ++l) {
+        const MgLevel L = pd.lv[l];
+        const int m = L.nx * L.ny * L.nz;
+        for (int c = threadIdx.x; c < m; c += kBotThreads) reinterpret_cast<BotCell *>(pd.bot)[off + c] = bot_cell(L, c);
+        off += m;
     }
 }
 
@@ -1094,15 +1214,28 @@ bool mg_plan(const Geo &g, bool mixed, float *w32, float *space, size_t floats, 
         C.sz = take(n + (size_t)C.nx * C.ny);
         C.w = take(n);
         C.r = take(n);
-        C.e = take(n);
+        C.t = take(n);
+        C.rho = take(n);
+        C.r0 = take(n);
         C.ex = take((size_t)C.nx * C.ny);
         ++l;
-        if (!lbot && n <= (size_t)kMgBottomCells) lbot = l;
     }
-    if (!lbot || off > floats) return false;
-    size_t lds = 0;
-    for (int q = lbot; q <= l; ++q) lds += cells(pd.lv[q]);
-    if (lds > (size_t)kMgBottomLds) return false;
+    if (off > floats) return false;
+    // the bottom kernel starts at the first level whose cells its threads hold
+    // and whose hierarchy fits its LDS (four floats per cell, and the
+    // coefficients of the levels below)
+    for (int b = 1; b <= l && !lbot; ++b) {
+        size_t low = 0;
+        for (int q = b + 1; q <= l; ++q) low += cells(pd.lv[q]);
+        const size_t n = cells(pd.lv[b]);
+        if (n <= (size_t)kMgBottomCells && 4 * (n + low) + low * (sizeof(BotCell) / sizeof(float)) + 2 * (size_t)pd.lv[b].nx * pd.lv[b].ny <= (size_t)kMgBottomLds) {
+            lbot = b;
+            pd.nbot = (int)(n + low);
+        }
+    }
+    if (!lbot) return false;
+    pd.bot = take((size_t)pd.nbot * (sizeof(BotCell) / sizeof(float)));
+    if (off > floats) return false;
     pd.nlev = l + 1;
     pd.lbot = lbot;
     // rows: 16, 32 or 64 lanes of four cells
@@ -1111,20 +1244,21 @@ bool mg_plan(const Geo &g, bool mixed, float *w32, float *space, size_t floats, 
     pd.mtx = (g.nx + 4 * lr - 1) / (4 * lr);
     const int rows = 8 << (6 - pd.mlrs);   // rows per workgroup
     pd.mty = (g.ny + rows - 1) / rows;
-    // planes per tile (even, so that coarse cells are whole): thin while that
-    // leaves fewer than kMgTiles workgroups
+    // planes per tile (even, so that coarse cells are whole): 4, or 8 where
+    // that still leaves 512 workgroups, two per CU (a third less z halo: the
+    // passes over 384x192x128 took 258 us against 273), or 2 where 4 would
+    // leave fewer workgroups than CUs
     const long long cols = (long long)pd.mtx * pd.mty;
-    long long kz = cols * g.nz / kMgTiles / 2 * 2;
-    kz = std::max<long long>(2, std::min<long long>(kz, 16));
-    pd.mkz = (int)kz;
-    pd.ntm = (int)(cols * ((g.nz + kz - 1) / kz));
+    auto tiles = [&](int kz) { return cols * ((g.nz + kz - 1) / kz); };
+    const int kz = tiles(8) >= 512 ? 8 : tiles(4) >= 256 ? 4 : 2;
+    pd.mkz = kz;
+    pd.ntm = (int)tiles(kz);
     pd.medge = g.px || pd.mtx > 1 || g.nx % 4 != 0;
     pd.mg = 1;
     return true;
 }
 
-int mg_down_tiles(const ProbDev &pd, int l) { return l >= 1 && l < pd.lbot ? blocks(cells(pd.lv[l + 1])) : 0; }
-int mg_up_tiles(const ProbDev &pd, int l) { return l >= 1 && l < pd.lbot ? blocks(cells(pd.lv[l])) : 0; }
+int mg_level_tiles(const ProbDev &pd, int l) { return l >= 1 && l < pd.lbot ? bricks(pd.lv[l]) : 0; }
 
 void launch_mg_setup(const ProbDev &pd, const ProbDev *dev, const SetupIn &in, hipStream_t s)
 {
@@ -1138,37 +1272,42 @@ void launch_mg_setup(const ProbDev &pd, const ProbDev *dev, const SetupIn &in, h
         hipLaunchKernelGGL(k_mg_parts, dim3(1), dim3(64), 0, s, pd.S);
     }
     hipLaunchKernelGGL(k_mg_weights, dim3(std::min(blocks(n), 4096)), dim3(kThreads), 0, s, n, pd.d, in.solid, pd.w32);
-    for (int l = 1; l < pd.lbot; ++l) {
+    for (int l = 1; l <= pd.lbot; ++l) {
         const int b = blocks(cells(pd.lv[l]));
         hipLaunchKernelGGL(k_mg_coarse, dim3(b), dim3(kThreads), 0, s, pd.lv[l - 1], pd.lv[l], pd.g.dtop, top);
         hipLaunchKernelGGL(k_mg_scale, dim3(b), dim3(kThreads), 0, s, pd.lv[l]);
     }
-    hipLaunchKernelGGL(k_mg_coarse_bottom, dim3(1), dim3(kBotThreads), 0, s, dev, pd.lbot, pd.g.dtop, top);
+    hipLaunchKernelGGL(k_mg_coarse_bottom, dim3(1), dim3(kBotThreads), 0, s, dev, pd.lbot + 1, pd.g.dtop, top);
 }
 
 void launch_mg_step(const ProbDev *P, const MgTables &T, int maxgrid, StepRef step, int *ran, hipStream_t s)
 {
     const int grid = std::min(T.nfine, maxgrid);
-    hipLaunchKernelGGL(k_mg_fine<kResid>, dim3(grid), dim3(kThreads), 0, s, P, T.fine, T.nfine, step, nullptr);
+#define MG_FINE(KIND, RAN) \
+    hipLaunchKernelGGL(k_mg_fine<KIND>, dim3(grid), dim3(kThreads), 0, s, P, T.fine, T.nfine, step, RAN)
+#define MG_LEVEL(KIND, l)                                                                                          \
+    hipLaunchKernelGGL(k_mg_level<KIND>, dim3(std::min(T.nlev[l], 4 * maxgrid)), dim3(kThreads), 0, s, P, T.lev[l], \
+                       T.nlev[l], l, step)
+    MG_FINE(kA1, nullptr);
+    MG_FINE(kA2, nullptr);
     for (int l = 1; l < kMgLevels; ++l)
-        if (T.ndown[l])
-            hipLaunchKernelGGL(k_mg_down, dim3(std::min(T.ndown[l], maxgrid)), dim3(kThreads), 0, s, P, T.down[l],
-                               T.ndown[l], l, step);
+        if (T.nlev[l]) {
+            MG_LEVEL(kA1, l);
+            MG_LEVEL(kA2, l);
+        }
     hipLaunchKernelGGL(k_mg_bottom, dim3(T.nprobs), dim3(kBotThreads), 0, s, P, T.probs, step);
     for (int l = kMgLevels - 1; l >= 1; --l)
-        if (T.nup[l])
-            hipLaunchKernelGGL(k_mg_up, dim3(std::min(T.nup[l], maxgrid)), dim3(kThreads), 0, s, P, T.up[l], T.nup[l],
-                               l, step);
-    hipLaunchKernelGGL(k_mg_fine<kSmooth>, dim3(grid), dim3(kThreads), 0, s, P, T.fine, T.nfine, step, nullptr);
-    hipLaunchKernelGGL(k_mg_fine<kDir>, dim3(grid), dim3(kThreads), 0, s, P, T.fine, T.nfine, step, ran);
-}
-
-void launch_mg_refresh(const ProbDev *P, const TileRef *t1, int nt1, const TileRef *t3, int nt3, const int *probs,
-                       int nprobs, int maxgrid, StepRef step, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_mg_refresh_e, dim3(std::min(maxgrid, nt1)), dim3(kThreads), 0, s, P, t1, nt1, step);
-    launch_true_residual(P, t3, nt3, maxgrid, step, s);
-    hipLaunchKernelGGL(k_mg_decide, dim3(nprobs), dim3(kThreads), 0, s, P, probs, step);
+        if (T.nlev[l]) {
+            MG_LEVEL(kB1, l);
+            MG_LEVEL(kB2, l);
+        }
+    MG_FINE(kB1, nullptr);
+    MG_FINE(kB2, nullptr);
+    MG_FINE(kDir, ran);
+    launch_true_residual(P, T.t3, T.nt3, maxgrid, step, s);
+    hipLaunchKernelGGL(k_mg_decide, dim3(T.nprobs), dim3(kThreads), 0, s, P, T.probs, step);
+#undef MG_FINE
+#undef MG_LEVEL
 }
 
 }  // namespace sps
