@@ -26,6 +26,7 @@
 // mixed-precision one (e is then the FP32 correction c).  Dot products and
 // the CG scalars are always FP64.
 #include <algorithm>
+#include <type_traits>
 
 #include "ps_device.h"
 
@@ -163,10 +164,11 @@ struct TotalCache {
 // FIRST (iteration 1: p_1 = r_0, nothing to finish) and DO_E (apply the
 // deferred e -= alpha p) are template parameters so that the plane loop has
 // no branches: every load of a plane is issued before any is waited for.
-template <typename T, bool FIRST, bool DO_E, class CO>
+// R: the type r is stored in (the multigrid step passes its FP32 z).
+template <typename T, bool FIRST, bool DO_E, class CO, typename R = T>
 __device__ __forceinline__ double cg_a_tile(const Geo &g, const Tile &t, gptr<T> __restrict__ e,
                                             gptr<const T> __restrict__ p_old, gptr<T> __restrict__ p_new,
-                                            gptr<const T> __restrict__ r, const CO &co, gptr<T> __restrict__ q, T b,
+                                            gptr<const R> __restrict__ r, const CO &co, gptr<T> __restrict__ q, T b,
                                             T a_prev)
 {
     const int nx = g.nx, ny = g.ny, nz = g.nz;
@@ -180,9 +182,9 @@ __device__ __forceinline__ double cg_a_tile(const Geo &g, const Tile &t, gptr<T>
     long long fx = ((long long)t.k0 * ny + t.j) * (nx + 1) + t.i;
     long long fy = ((long long)t.k0 * (ny + 1) + t.j) * nx + t.i;
     // p_n = r + beta p_{n-1} (9_grad.f90:518-527), formed where needed
-    auto pn = [&](long long x) -> T { return FIRST ? r[x] : r[x] + b * p_old[x]; };
+    auto pn = [&](long long x) -> T { return FIRST ? (T)r[x] : (T)r[x] + b * p_old[x]; };
     T poc = FIRST ? T(0) : p_old[c];
-    T pc = FIRST ? r[c] : r[c] + b * poc;
+    T pc = FIRST ? (T)r[c] : (T)r[c] + b * poc;
     T pb = t.k0 > 0 ? pn(c - plane) : pc;
     T szb = co.z(c, t.k0);
     for (int k = t.k0; k < t.k1; ++k) {
@@ -190,7 +192,7 @@ __device__ __forceinline__ double cg_a_tile(const Geo &g, const Tile &t, gptr<T>
         // top neighbour; at the lid the mirror ghost is the cell itself
         const long long up = (k < nz - 1) ? plane : 0;
         const T pot = FIRST ? T(0) : p_old[c + up];
-        const T pt = FIRST ? r[c + up] : r[c + up] + b * pot;
+        const T pt = FIRST ? (T)r[c + up] : (T)r[c + up] + b * pot;
         const T szt = co.z(c + plane, k + 1);
         const T pw = pn(r0 + iw), pe = pn(r0 + ie);
         const T ps = pn(c + dS), pnn = pn(c + dN);
@@ -310,6 +312,65 @@ __global__ __launch_bounds__(kThreads) void k_cg_a(const ProbDev *__restrict__ P
             if (first) return cg_a_tile<T, true, false>(pd.g, tl, V.e, p_old, p_new, V.r, co, V.q, b, a_prev);
             if (do_e) return cg_a_tile<T, false, true>(pd.g, tl, V.e, p_old, p_new, V.r, co, V.q, b, a_prev);
             return cg_a_tile<T, false, false>(pd.g, tl, V.e, p_old, p_new, V.r, co, V.q, b, a_prev);
+        });
+        const double s = block_sum(acc);
+        if (threadIdx.x == 0) pd.P.spmv[tr.tile] = s;
+    }
+}
+
+// The FP64 direction step of the multigrid-preconditioned iteration n
+// (ps_mg.hip): cg_a with z in the place of r, and the end of the solve where
+// A2 marked step n (r.r at the threshold, or the cap).
+__global__ __launch_bounds__(kThreads) void k_mg_dir64(const ProbDev *__restrict__ P, const TileRef *__restrict__ tab,
+                                                       int ntab, StepRef sref, int *ran)
+{
+    const Run run = my_run(ntab);
+    const int step = sref.base ? *sref.base + sref.off : sref.off;
+    TotalCache rz_tot;
+    for (int t = run.begin; t < run.end; ++t) {
+        const TileRef tr = tab[t];
+        const ProbDev &pd = P[tr.prob];
+        const gptr<CgScalars> S = glob(pd.S);
+        const int n = step - pd.n0 + 1;
+        const int done_at = S->done_at;
+        const bool due = S->next_refresh == n;
+        const double rz_prev = S->rz[(n - 1) & 1], alpha = S->alpha, rr = S->rr[n & 1], thresh = S->thresh;
+        if (n < 1 || n > done_at) continue;
+        const bool first = n == 1;
+        const double rz = due ? 0.0 : rz_tot.get(tr.prob, pd.P.m4 + pd.ntm, pd.ntm);
+        const bool bad = !(rz >= 0.0 && rz < 1e300) || !(alpha >= 0.0 && alpha < 1e300);
+        const double beta = first || !(rz_prev > 0.0) ? 0.0 : rz / rz_prev;
+        if (tr.tile == 0 && threadIdx.x == 0) {
+            if (bad || due) {
+                S->giveup = bad ? 1 : 0;
+                S->status = rr <= thresh ? 0 : 1;
+                S->final_ = 1;
+                S->done_at = n;
+            } else {
+                S->rz[n & 1] = rz;
+                S->iters = n;
+                if (ran && tr.prob == 0) *ran = 1;
+            }
+        }
+        if (bad) continue;
+        const Vecs<double> V = vecs(pd, 0.0);
+        const gptr<double> p_old = (n & 1) ? V.p0 : V.p1;
+        const gptr<double> p_new = (n & 1) ? V.p1 : V.p0;
+        const Tile tl = tile3(pd.g, tr.tile);
+        if (due) {
+            if (tl.i < pd.g.nx && tl.j < pd.g.ny) {
+                const long long plane = (long long)pd.g.nx * pd.g.ny;
+                long long c = (long long)tl.k0 * plane + (long long)tl.j * pd.g.nx + tl.i;
+                for (int k = tl.k0; k < tl.k1; ++k, c += plane) V.e[c] = V.e[c] - alpha * p_old[c];
+            }
+            continue;
+        }
+        const gptr<const float> z = glob((const float *)pd.q32b);
+        const double acc = with_coefs(V, [&](const auto &co) {
+            using CO = std::decay_t<decltype(co)>;
+            if (first)
+                return cg_a_tile<double, true, false, CO, float>(pd.g, tl, V.e, p_old, p_new, z, co, V.q, beta, alpha);
+            return cg_a_tile<double, false, true, CO, float>(pd.g, tl, V.e, p_old, p_new, z, co, V.q, beta, alpha);
         });
         const double s = block_sum(acc);
         if (threadIdx.x == 0) pd.P.spmv[tr.tile] = s;
@@ -1553,6 +1614,11 @@ void launch_refresh(const ProbDev *P, const TileRef *t1, int nt1, const TileRef 
     hipLaunchKernelGGL(k_refresh_e, dim3(std::min(grid, nt1)), dim3(kThreads), 0, s, P, t1, nt1, step);
     launch_true_residual(P, t3, nt3, grid, step, s);
     hipLaunchKernelGGL(k_refresh_decide, dim3(nprobs), dim3(kThreads), 0, s, P, probs, step);
+}
+
+void launch_mg_dir64(const ProbDev *P, const TileRef *t3, int nt3, int maxgrid, StepRef step, int *ran, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_mg_dir64, dim3(std::min(nt3, maxgrid)), dim3(kThreads), 0, s, P, t3, nt3, step, ran);
 }
 
 void launch_true_residual(const ProbDev *P, const TileRef *t3, int nt3, int grid, StepRef step, hipStream_t s)

@@ -67,10 +67,19 @@ struct Slot {
 // any tile depth kz >= kMinKz).
 size_t problem_bytes(int nx, int ny, int nz, bool mixed);
 
+// The same for the iteration these options choose: an FP64 solve by the
+// multigrid iteration keeps FP32 arrays for it beside its own (about 115
+// instead of 80 B per cell).  A size whose plain state the no-allocation call
+// accepts but whose larger one its array does not hold (SULI_PS_NOALLOC_MAX_BYTES
+// + kNoAllocExtra) stays with plain CG, so that it solves the same way with
+// and without allocation.
+constexpr size_t kNoAllocExtra = (size_t)40 << 20;
+size_t state_bytes(int nx, int ny, int nz, const SolveOpts &o);
+
 // Whether the multigrid iteration serves solves with these options.
 bool mg_applies(const SolveOpts &o);
-// Launch-table entries its kernels need for a mixed problem on this grid
-// beside the replacement's (3-D and 1-D tiles of make_geo's default shape);
+// Launch-table entries its kernels need for a problem on this grid beside the
+// 3-D and 1-D tiles of make_geo's default shape;
 // 0: it does not apply to the grid.
 long long mg_entries(const Geo &g);
 
@@ -111,11 +120,12 @@ public:
     // Admits a problem: allocates its slot, enqueues the setup kernels on the
     // stream and schedules its iteration 1 at the next global step.
     // prd1_out receives the solution (device, reference layout) when done.
-    // block (optional): problem_bytes() of device memory the caller owns, used
-    // instead of the engine's pool; wait_ev (optional): the setup kernels
+    // block (optional): block_bytes of device memory the caller owns, used
+    // instead of the engine's pool: state_bytes() of it, or, for plain CG,
+    // problem_bytes(); wait_ev (optional): the setup kernels
     // wait for it (inputs copied on another stream).
     int admit(const suli_ps_grid &gr, const SetupIn &in, double *prd1_out, const SolveOpts &o, int user,
-              int *slot_out, void *block = nullptr, hipEvent_t wait_ev = nullptr);
+              int *slot_out, void *block = nullptr, size_t block_bytes = 0, hipEvent_t wait_ev = nullptr);
     // Runs chunks until every admitted problem has finished; each finished
     // problem's prd1_out holds its solution and status its final state.
     int run_all(bool timing);
@@ -206,9 +216,9 @@ private:
     struct Tables {
         std::vector<TileRef> t3_64, t1_64, t3_32, t1_32;
         std::vector<int> mixed_probs;
-        // multigrid problems: fine tiles, 3-D tiles of the replacement,
-        // coarse levels
-        std::vector<TileRef> mg_fine, mg_t3, mg_lev;
+        // multigrid problems: fine tiles, 3-D tiles of the replacement (mixed),
+        // 1-D and 3-D tiles (FP64), coarse levels
+        std::vector<TileRef> mg_fine, mg_t3, mg_t1_64, mg_t3_64, mg_lev;
         std::vector<int> mg_probs;
     } tab_;
     MgTables mgt_;                     // the same on the device

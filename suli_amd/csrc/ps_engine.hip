@@ -88,6 +88,30 @@ void carve(Carver &cv, const Geo &g, bool mixed, int nt3, int nt1, ProbDev &pd)
     pd.P.proj = cv.take<double>(2 * (size_t)init_blocks(g));
 }
 
+// The FP32 arrays of an FP64 problem's V-cycle, behind carve()'s (false: the
+// multigrid iteration does not apply to the grid).
+bool carve_mg64(Carver &cv, const Geo &g, ProbDev &pd)
+{
+    const size_t n = (size_t)g.n;
+    size_t floats = 0;
+    ProbDev probe{};
+    if (!mg_plan(g, nullptr, nullptr, (size_t)-1, probe, &floats)) return false;
+    pd.sx32 = cv.take<float>((size_t)(g.nx + 1) * g.ny * g.nz);
+    pd.sy32 = cv.take<float>((size_t)g.nx * (g.ny + 1) * g.nz);
+    pd.sz32 = cv.take<float>((size_t)g.nx * g.ny * (g.nz + 1));
+    pd.r32 = cv.take<float>(n);
+    pd.r32b = cv.take<float>(n);
+    pd.q32b = cv.take<float>(n);
+    pd.t32 = cv.take<float>(n);
+    float *w = cv.take<float>(n), *space = cv.take<float>(floats);
+    pd.rx32 = cv.take<float>(8 * (size_t)g.nz);
+    pd.ry32 = cv.take<float>(4 * (size_t)g.nz);
+    pd.rz32 = cv.take<float>(4 * ((size_t)g.nz + 1));
+    pd.rowreg = cv.take<unsigned>((size_t)(g.ny + 31) / 32 * g.nz);
+    pd.P.m4 = cv.take<double>(3 * (size_t)probe.ntm);
+    return mg_plan(g, w, space, floats, pd);
+}
+
 }  // namespace
 
 // ------------------------------------------------------ allocation guard ----
@@ -152,6 +176,19 @@ size_t problem_bytes(int nx, int ny, int nz, bool mixed)
     ProbDev pd{};
     carve(cv, g, mixed, spmv_tiles(g), vec_tiles(g.n), pd);
     return align_up(cv.off, 2 << 20);
+}
+
+size_t state_bytes(int nx, int ny, int nz, const SolveOpts &o)
+{
+    const size_t plain = problem_bytes(nx, ny, nz, o.mixed);
+    if (o.mixed || !mg_applies(o) || mg_entries(make_geo(nx, ny, nz, 0, 0)) == 0) return plain;
+    const Geo g = make_geo(nx, ny, nz, 0, 0, kMinKz);
+    Carver cv{nullptr};
+    ProbDev pd{};
+    carve(cv, g, false, spmv_tiles(g), vec_tiles(g.n), pd);
+    if (!carve_mg64(cv, g, pd)) return plain;
+    const size_t multi = align_up(cv.off, 2 << 20);
+    return multi > SULI_PS_NOALLOC_MAX_BYTES + kNoAllocExtra && plain <= SULI_PS_NOALLOC_MAX_BYTES ? plain : multi;
 }
 
 // -------------------------------------------------------------- Engine ----
@@ -274,6 +311,8 @@ int Engine::reserve(int entries)
     tab_.mixed_probs.reserve(max_slots_);
     tab_.mg_fine.reserve(ntab);
     tab_.mg_t3.reserve(ntab);
+    tab_.mg_t1_64.reserve(ntab);
+    tab_.mg_t3_64.reserve(ntab);
     tab_.mg_lev.reserve(ntab);
     tab_.mg_probs.reserve(max_slots_);
     pool_.reserve(max_slots_);
@@ -309,28 +348,29 @@ int Engine::active_count() const
     return n;
 }
 
-// The multigrid iteration serves mixed solves that any cap leaves room to
-// converge; keep_null and stored_residual name properties of the plain CG
-// iteration.
+// The multigrid iteration serves mixed solves, and FP64 ones by the relative
+// rule, that any cap leaves room to converge; the reference's rule in FP64,
+// keep_null and stored_residual name properties of the plain CG iteration.
 bool mg_applies(const SolveOpts &o)
 {
-    return o.mixed && !o.keep_null && !o.store_r && o.max_iter >= kMgMinCap;
+    return (o.mixed ? !o.store_r : o.stop_rule == SULI_PS_STOP_RELATIVE) && !o.keep_null && o.max_iter >= kMgMinCap;
 }
 
 long long mg_entries(const Geo &g)
 {
-    Carver cv{nullptr};
     ProbDev pd{};
-    const int nt3 = spmv_tiles(g);
-    carve(cv, g, true, nt3, vec_tiles(g.n), pd);
-    if (!mg_plan(g, true, nullptr, nullptr, 2 * (size_t)g.n, pd) || 3 * pd.ntm > 8 * nt3) return 0;
+    size_t floats = 0;
+    const long long nt3 = spmv_tiles(g);
+    // mixed solves keep the hierarchy in 2 n floats and three partial sums per
+    // fine tile in m4; FP64 ones go by the same rule
+    if (!mg_plan(g, nullptr, nullptr, 2 * (size_t)g.n, pd, &floats) || 3 * pd.ntm > 8 * nt3) return 0;
     long long n = pd.ntm;
     for (int l = 1; l < pd.lbot; ++l) n += mg_level_tiles(pd, l);
     return n;
 }
 
 int Engine::admit(const suli_ps_grid &gr, const SetupIn &in, double *prd1_out, const SolveOpts &o, int user,
-                  int *slot_out, void *block, hipEvent_t wait_ev)
+                  int *slot_out, void *block, size_t block_bytes, hipEvent_t wait_ev)
 {
     int si = -1;
     for (int i = 0; i < max_slots_; ++i)
@@ -346,7 +386,9 @@ int Engine::admit(const suli_ps_grid &gr, const SetupIn &in, double *prd1_out, c
     int vx = o.vx > 0 ? o.vx : 0;
     // the tuner's shapes are the plain CG kernels': nothing to tune otherwise
     const Geo g0 = make_geo(gr.nx, gr.ny, gr.nz, gr.ccx0 == 0, gr.ccy0 == 0);
-    if (mg_applies(o) && mg_entries(g0) > 0) {
+    sl.bytes = state_bytes(gr.nx, gr.ny, gr.nz, o);
+    const size_t plain = problem_bytes(gr.nx, gr.ny, gr.nz, o.mixed);
+    if (mg_applies(o) && mg_entries(g0) > 0 && (o.mixed || sl.bytes > plain)) {
         // the shape a fall-back to plain CG would take
         int kz_c = 0, vx_c = 0;
         if (autotune_) cached_shape(gr.nx, gr.ny, gr.nz, o.mixed, &kz_c, &vx_c);
@@ -371,9 +413,14 @@ int Engine::admit(const suli_ps_grid &gr, const SetupIn &in, double *prd1_out, c
     sl.o = o;
     sl.o.kz = kz;
     sl.o.vx = vx;
-    sl.bytes = problem_bytes(gr.nx, gr.ny, gr.nz, o.mixed);
     sl.own_block = block == nullptr;
+    if (block && block_bytes < sl.bytes) sl.bytes = plain;
     sl.block = block ? block : pool_.get(sl.bytes, err_);
+    if (!sl.block && sl.bytes > plain && !no_alloc_active()) {
+        // plain CG where the V-cycle's arrays do not fit any more
+        sl.bytes = plain;
+        sl.block = pool_.get(sl.bytes, err_);
+    }
     if (!sl.block) return SULI_PS_ENOMEM;
     sl.prd1_out = prd1_out;
     sl.solid = in.solid;
@@ -398,7 +445,8 @@ int Engine::setup_slot(int si, bool multi, hipEvent_t wait_ev)
     // kernels, which walk one cell per lane, take the default shape
     sl.mg = false;
     for (const bool mg : {true, false}) {
-        if (mg && !(multi && mg_applies(o))) continue;
+        if (mg && !(multi && mg_applies(o) && mg_entries(make_geo(gr.nx, gr.ny, gr.nz, 0, 0)) > 0)) continue;
+        if (mg && !o.mixed && sl.bytes <= problem_bytes(gr.nx, gr.ny, gr.nz, false)) continue;
         sl.g = make_geo(gr.nx, gr.ny, gr.nz, gr.ccx0 == 0, gr.ccy0 == 0, mg ? 0 : o.kz, mg ? 1 : o.mixed ? o.vx : 1);
         sl.g.dtop = gr.top_bc == 1 ? 1 : 0;
         nt3 = spmv_tiles(sl.g);
@@ -408,9 +456,10 @@ int Engine::setup_slot(int si, bool multi, hipEvent_t wait_ev)
         pd.g = sl.g;
         carve(cv, sl.g, o.mixed, nt3, nt1, pd);
         if (mg) {
-            sl.mg = mg_plan(sl.g, o.mixed, pd.p32 + 2 * pd.pslot, reinterpret_cast<float *>(pd.r),
-                            2 * (size_t)sl.g.n, pd) &&
-                    3 * pd.ntm <= 8 * nt3;
+            sl.mg = o.mixed ? mg_plan(sl.g, pd.p32 + 2 * pd.pslot, reinterpret_cast<float *>(pd.r),
+                                      2 * (size_t)sl.g.n, pd)
+                            : carve_mg64(cv, sl.g, pd);
+            if (o.mixed) pd.t32 = pd.p32 + 3 * pd.pslot;
             if (sl.mg) break;
         }
     }
@@ -488,14 +537,16 @@ int Engine::setup_slot(int si, bool multi, hipEvent_t wait_ev)
     launch_scale_faces(sl.g, pd.d, sx, sy, sz, const_cast<float *>(pd.sx32), const_cast<float *>(pd.sy32),
                        const_cast<float *>(pd.sz32), s_);
     if (pd.tx)
-        launch_face_tables(sl.g, pd.sx, pd.sy, pd.sz, pd.sx32, pd.sy32, pd.sz32, const_cast<double *>(pd.tx),
+        // (the FP32 tables are the mixed solver's; an FP64 problem has none)
+        launch_face_tables(sl.g, pd.sx, pd.sy, pd.sz, pd.tx32 ? pd.sx32 : nullptr, pd.tx32 ? pd.sy32 : nullptr,
+                           pd.tx32 ? pd.sz32 : nullptr, const_cast<double *>(pd.tx),
                            const_cast<double *>(pd.ty), const_cast<double *>(pd.tz), const_cast<float *>(pd.tx32),
                            const_cast<float *>(pd.ty32), const_cast<float *>(pd.tz32), s_);
     if (pd.rowreg)
         launch_row_tables(sl.g, pd.sx32, pd.sy32, pd.sz32, const_cast<float *>(pd.rx32), const_cast<float *>(pd.ry32),
                           const_cast<float *>(pd.rz32), const_cast<unsigned *>(pd.rowreg), s_);
     launch_init(sl.g, in, Op<double>{pd.sx, pd.sy, pd.sz}, pd.d, pd.b, pd.e, pd.r, o.mixed ? nullptr : pd.r,
-                pd.r32, pd.c32, pd.P, init_blocks(sl.g), pd.S, s_);
+                o.mixed ? pd.r32 : nullptr, pd.c32, pd.P, init_blocks(sl.g), pd.S, s_);
     if (sl.mg) launch_mg_setup(pd, d_probs_ + si, in, s_);
     ECHK(hipGetLastError());
     tables_dirty_ = true;
@@ -520,6 +571,8 @@ int Engine::rebuild_tables()
     tab_.mixed_probs.clear();
     tab_.mg_fine.clear();
     tab_.mg_t3.clear();
+    tab_.mg_t1_64.clear();
+    tab_.mg_t3_64.clear();
     tab_.mg_lev.clear();
     tab_.mg_probs.clear();
     table_cells_ = 0;
@@ -528,7 +581,10 @@ int Engine::rebuild_tables()
         if (!sl.active || sl.finished) continue;
         if (sl.mg) {
             for (int t = 0; t < sl.pd.ntm; ++t) tab_.mg_fine.push_back({i, t});
-            for (int t = 0; t < sl.pd.nt3; ++t) tab_.mg_t3.push_back({i, t});
+            auto &t3 = sl.o.mixed ? tab_.mg_t3 : tab_.mg_t3_64;
+            for (int t = 0; t < sl.pd.nt3; ++t) t3.push_back({i, t});
+            if (!sl.o.mixed)
+                for (int t = 0; t < sl.pd.nt1; ++t) tab_.mg_t1_64.push_back({i, t});
             tab_.mg_probs.push_back(i);
             continue;
         }
@@ -565,7 +621,9 @@ int Engine::rebuild_tables()
     }
     const int off_mg = off_t1_32 + (int)tab_.t1_32.size();
     const int off_mg_t3 = off_mg + (int)tab_.mg_fine.size();
-    const int off_mg_lev = off_mg_t3 + (int)tab_.mg_t3.size();
+    const int off_mg_t3_64 = off_mg_t3 + (int)tab_.mg_t3.size();
+    const int off_mg_t1_64 = off_mg_t3_64 + (int)tab_.mg_t3_64.size();
+    const int off_mg_lev = off_mg_t1_64 + (int)tab_.mg_t1_64.size();
     const size_t ntab = off_mg_lev + tab_.mg_lev.size();
     const size_t nprobs = tab_.mixed_probs.size() + tab_.mg_probs.size();
     if (ntab > tab_cap_ || nprobs > probs_cap_ || !d_tab_) {
@@ -603,11 +661,17 @@ int Engine::rebuild_tables()
     std::copy(tab_.mg_probs.begin(), tab_.mg_probs.end(), hp + tab_.mixed_probs.size());
     std::copy(tab_.mg_fine.begin(), tab_.mg_fine.end(), ht + off_mg);
     std::copy(tab_.mg_t3.begin(), tab_.mg_t3.end(), ht + off_mg_t3);
+    std::copy(tab_.mg_t3_64.begin(), tab_.mg_t3_64.end(), ht + off_mg_t3_64);
+    std::copy(tab_.mg_t1_64.begin(), tab_.mg_t1_64.end(), ht + off_mg_t1_64);
     std::copy(tab_.mg_lev.begin(), tab_.mg_lev.end(), ht + off_mg_lev);
     mgt_.fine = d_tab_ + off_mg;
     mgt_.nfine = (int)tab_.mg_fine.size();
     mgt_.t3 = d_tab_ + off_mg_t3;
     mgt_.nt3 = (int)tab_.mg_t3.size();
+    mgt_.t3_64 = d_tab_ + off_mg_t3_64;
+    mgt_.nt3_64 = (int)tab_.mg_t3_64.size();
+    mgt_.t1_64 = d_tab_ + off_mg_t1_64;
+    mgt_.nt1_64 = (int)tab_.mg_t1_64.size();
     mgt_.probs = d_probs_list_ + tab_.mixed_probs.size();
     mgt_.nprobs = (int)tab_.mg_probs.size();
     for (int l = 1; l < kMgLevels; ++l) mgt_.lev[l] = d_tab_ + off_mg_lev + off_lev[l];

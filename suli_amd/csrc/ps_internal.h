@@ -39,8 +39,8 @@ constexpr int kFold = 4;
 static_assert(kRefreshGrain % kFold == 0 && kFirstRefresh % kFold == 0, "replacements must end fold groups");
 static_assert((kFold & (kFold - 1)) == 0, "kFold is a power of two");
 
-// Multigrid-preconditioned CG (ps_mg.hip), the mixed solver's iteration from
-// kMgMinCells cells on.
+// Multigrid-preconditioned CG (ps_mg.hip), the iteration of mixed solves, and
+// of FP64 solves by the relative rule, from kMgMinCells cells on.
 //
 // kMgMinCells: smaller problems keep plain CG, whose iterates the options
 // stored_residual and a small max_iter are specified on.
@@ -57,8 +57,13 @@ constexpr int kMgChunk = 2;            // iterations between host polls
 // last one, or to kMgMargin of the threshold, and at the latest after kMgMaxGap
 // iterations.
 constexpr double kMgCycleDrop = 1e-9;
-constexpr double kMgMargin = 0.5;
 constexpr int kMgMaxGap = 40;
+// The solve goes on to r.r = kMgMargin of the threshold, a tenth of the
+// tolerance (half an iteration on average), unless that is out of reach: at
+// one residual norm the smooth part of the error is larger here than plain
+// CG leaves it (twice on a 319x46x22 constant-density grid).
+constexpr double kMgMargin = 1e-2;
+constexpr int kMgMarginIters = 4;   // FP64: at most so many iterations below the threshold
 
 // Grid geometry as the kernels see it.  Cells are 0-based (i, j, k) with x
 // fastest; a cell vector holds nx*ny*nz values with no halo.  Ghost values
@@ -204,7 +209,8 @@ struct ProbDev {
     const unsigned *rowreg;
     Partials P;
     CgScalars *S;
-    // multigrid (mg set): tiles of the fine kernels (mtx x mty x planes of
+    // multigrid (mg set; FP64 problems have these FP32 arrays beside their own
+    // then, and P.m4 for the fine kernels' partial sums): tiles of the fine kernels (mtx x mty x planes of
     // mkz, 1 << mlrs lanes per row), the hierarchy, level 0's weights.  p_k
     // is in ring slot k & 1 (slot 2 holds w32, slot 3 t), q_k in q32, rho and
     // then z_k in q32b, r_k in r32 (k even) or r32b (k odd), the other one
@@ -213,7 +219,7 @@ struct ProbDev {
     int mg, mtx, mty, mkz, mlrs, ntm, medge;
     int nlev, lbot, nbot;   // nbot: cells of levels lbot and coarser
     float *bot;             // those cells' coefficients, packed
-    float *w32;
+    float *w32, *t32;
     MgLevel lv[kMgLevels];
 };
 
@@ -357,7 +363,7 @@ void launch_spmv_only(bool fp32, const ProbDev *P, const TileRef *t3, int nt3, i
 // Lays the hierarchy of a problem out in `space` (`floats` of them; w32 holds
 // level 0's weights) and fills pd's multigrid fields; false where it does not apply (size, or the
 // hierarchy does not fit), pd.mg then stays 0.
-bool mg_plan(const Geo &g, bool mixed, float *w32, float *space, size_t floats, ProbDev &pd);
+bool mg_plan(const Geo &g, float *w32, float *space, size_t floats, ProbDev &pd, size_t *used = nullptr);
 // Table entries of level l's kernels.
 int mg_level_tiles(const ProbDev &pd, int l);
 // Weights and coarse operators, after launch_init; dev: pd on the device.
@@ -365,13 +371,20 @@ void launch_mg_setup(const ProbDev &pd, const ProbDev *dev, const SetupIn &in, h
 struct MgTables {
     const TileRef *fine = nullptr, *lev[kMgLevels] = {};
     int nfine = 0, nlev[kMgLevels] = {};
-    const TileRef *t3 = nullptr;   // 3-D tiles of the true residual
+    const TileRef *t3 = nullptr;   // 3-D tiles of the true residual (mixed)
     int nt3 = 0;
+    const TileRef *t1_64 = nullptr, *t3_64 = nullptr;   // 1-D and 3-D tiles of the FP64 problems
+    int nt1_64 = 0, nt3_64 = 0;
     const int *probs = nullptr;
     int nprobs = 0;
 };
 // Step step - n0 + 1 (an iteration or a replacement) of every problem in the tables.
 void launch_mg_step(const ProbDev *P, const MgTables &T, int maxgrid, StepRef step, int *ran, hipStream_t s);
+// FP64 problems' direction step (ps_cg.hip): beta, e -= alpha p_{n-1}, p_n = z +
+// beta p_{n-1}, q = A p_n, p.q partials; or, when A2 marked step n, the end of the solve.
+void launch_mg_dir64(const ProbDev *P, const TileRef *t3, int nt3, int maxgrid, StepRef step, int *ran,
+                     hipStream_t s);
+
 // Plain copy of n16 16-byte vectors (measurement only).
 void launch_copy(const void *src, void *dst, long long n16, hipStream_t s);
 // Plain read of n16 16-byte vectors (measurement only); out holds

@@ -1,13 +1,18 @@
-// Multigrid-preconditioned CG of the mixed-precision solver, batched over
-// problems.
+// Multigrid-preconditioned CG, batched over problems.
 //
 // The scaled system A e = b (unit diagonal, ps_cg.hip) has a condition number
 // that grows with the square of the grid's longest side, so plain CG takes
 // about a thousand iterations on a 256x128x96 two-phase tank.  Here one
 // iteration applies a V-cycle M to the residual first (z = M r, p = z + beta
-// p, beta and alpha from r.z) and takes 25 to 50 on any grid.  Everything is
-// FP32 inside FP64 residual replacement, as the CG step: dot products, alpha
-// and beta are FP64 and convergence is judged on the FP64 true residual.
+// p, beta and alpha from r.z) and takes 10 to 25 on any grid.
+//
+// Mixed solves: everything is FP32 inside FP64 residual replacement, as the CG
+// step: dot products, alpha and beta are FP64 and convergence is judged on
+// the FP64 true residual.  FP64 solves by the relative rule: the iterate, the
+// residual, the directions, the operator and the stop test are FP64 as in
+// plain CG (ps_cg.hip), and only the V-cycle works on an FP32 copy of the
+// residual; which z it returns changes the number of iterations, not what
+// r = A e - b reaches.
 //
 // The V-cycle smooths with a Chebyshev polynomial of degree two before and
 // after the coarse correction on every level.  A coarse cell joins 2x2x2
@@ -46,6 +51,9 @@
 // or, in a step whose A2 finds r_{n-1} small enough, instead of D1 .. dir the
 // residual replacement: dir folds c and alpha p into e, then
 //   k_true_residual, k_mg_decide: converged, or on with the replaced residual
+// FP64: before A1, upd64 (r -= alpha q, its FP32 copy, partials r.r); instead
+// of dir, dir64 (ps_cg.hip; e -= alpha p), which ends the solve when A2 found
+// r.r at the threshold.
 // Each total is summed by the kernel that needs it from the partials of an
 // earlier launch, as in ps_cg.hip.
 #include <algorithm>
@@ -106,8 +114,6 @@ __device__ __forceinline__ double *part_rr(const ProbDev &pd) { return pd.P.m4 +
 __device__ __forceinline__ float *rbuf(const ProbDev &pd, int k) { return (k & 1) ? pd.r32b : pd.r32; }
 __device__ __forceinline__ float *mpbuf(const ProbDev &pd, int k) { return pd.p32 + (k & 1) * pd.pslot; }
 
-// t of level 0: ring slot 3
-__device__ __forceinline__ float *tbuf(const ProbDev &pd) { return pd.p32 + 3 * pd.pslot; }
 
 typedef float vf4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef float vf2 __attribute__((ext_vector_type(2), aligned(4)));
@@ -478,29 +484,42 @@ __global__ __launch_bounds__(kThreads, (KIND == kA1 || KIND == kDir) ? 2 : 3) vo
         const int done_at = S->done_at, skip_e_at = S->skip_e_at;
         const bool due = KIND != kA1 && KIND != kA2 && S->next_refresh == n;   // set by A2
         if (n < 1 || n > done_at || (due && KIND != kDir)) continue;
-        const bool fresh = n == 1 || step == skip_e_at;   // r_{n-1} stands in its buffer
-        const gptr<float> r = glob(rbuf(pd, n - 1)), r0 = glob(rbuf(pd, n));
-        const gptr<float> tt = glob(tbuf(pd)), rho = glob(pd.q32b), z = rho, q = glob(pd.q32);
+        const bool mixed = pd.mixed != 0;
+        if (KIND == kDir && !mixed) continue;
+        // r_{n-1} stands in its buffer (FP64: always the one FP32 copy)
+        const bool fresh = n == 1 || step == skip_e_at || !mixed;
+        const gptr<float> r = glob(mixed ? rbuf(pd, n - 1) : pd.r32), r0 = glob(mixed ? rbuf(pd, n) : pd.r32b);
+        const gptr<float> tt = glob(pd.t32), rho = glob(pd.q32b), z = rho, q = glob(pd.q32);
         FineArgs F{};
         if (KIND == kA1) {
-            const double rz = S->rz[(n - 1) & 1];
-            const double pq = tot.get(tr.prob, part_pq(pd), pd.ntm);
-            const double alpha = fresh || !(pq != 0.0) ? 0.0 : rz / pq;   // 0 / 0 once the residual is 0
-            if (tr.tile == 0 && threadIdx.x == 0) S->alpha = alpha;
-            F = FineArgs{fresh ? r : r0, q, nullptr, nullptr, r, tt, nullptr, fresh, false, (float)alpha, 0.f};
+            double alpha = 0.0;
+            if (mixed) {
+                const double rz = S->rz[(n - 1) & 1];
+                const double pq = tot.get(tr.prob, part_pq(pd), pd.ntm);
+                alpha = fresh || !(pq != 0.0) ? 0.0 : rz / pq;   // 0 / 0 once the residual is 0
+                if (tr.tile == 0 && threadIdx.x == 0) S->alpha = alpha;
+            }
+            // (the second operand is loaded whether used or not)
+            F = FineArgs{fresh ? r : r0, mixed ? q : r, nullptr, nullptr, r, tt, nullptr, fresh, false, (float)alpha, 0.f};
         } else if (KIND == kA2) {
             if (tr.tile == 0) {
-                // a replacement instead of iteration n once r.r (the FP32
-                // recurrence's) has reached the threshold, or fallen as far
-                // as FP32 carries one cycle, or at the cap
-                const double rr = block_total_of(part_rr(pd), pd.ntm);
+                // mixed: a replacement instead of iteration n once r.r (the
+                // FP32 recurrence's) has reached the threshold, or fallen as
+                // far as FP32 carries one cycle, or at the cap; FP64: the end
+                const double rr = mixed ? block_total_of(part_rr(pd), pd.ntm) : block_total_of(pd.P.upd, pd.nt1);
                 if (threadIdx.x == 0) {
                     S->rr[n & 1] = rr;
                     const double base = S->refreshes ? S->rr_after : S->rr0;
                     const int iters = S->iters;
-                    if (!fresh && (rr <= kMgMargin * S->thresh || rr <= kMgCycleDrop * base ||
-                                   iters - S->prev_iters >= kMgMaxGap || iters >= S->max_iter))
+                    if (!mixed) {
+                        if (n > 1 && rr <= S->thresh && S->prev_iters == 0) S->prev_iters = n;
+                        if (n > 1 && (rr <= kMgMargin * S->thresh || iters >= S->max_iter ||
+                                      (rr <= S->thresh && n - S->prev_iters >= kMgMarginIters)))
+                            S->next_refresh = n;
+                    } else if (!fresh && (rr <= kMgMargin * S->thresh || rr <= kMgCycleDrop * base ||
+                                          iters - S->prev_iters >= kMgMaxGap || iters >= S->max_iter)) {
                         S->next_refresh = n;
+                    }
                 }
             }
             F = FineArgs{tt, nullptr, r, nullptr, rho, nullptr, nullptr, false, false, 0.f, 0.f};
@@ -543,6 +562,62 @@ __global__ __launch_bounds__(kThreads, (KIND == kA1 || KIND == kDir) ? 2 : 3) vo
         if (KIND == kA2 || KIND == kB1) continue;
         const double sres = block_sum(acc);
         if (threadIdx.x == 0) (KIND == kA1 ? part_rr(pd) : KIND == kB2 ? part_rz(pd) : part_pq(pd))[tr.tile] = sres;
+    }
+}
+
+// FP64: r_{n-1} = r_{n-2} - alpha_{n-1} q_{n-1} and its FP32 copy for the
+// V-cycle, r.r partials (1-D tiles).
+__global__ __launch_bounds__(kThreads) void k_mg_upd64(const ProbDev *__restrict__ P, const TileRef *__restrict__ tab,
+                                                       int ntab, StepRef sref)
+{
+    typedef double vd4 __attribute__((ext_vector_type(4)));
+    typedef float va4 __attribute__((ext_vector_type(4)));
+    const Run run = my_run(ntab);
+    const int step = step_of(sref);
+    TotalCache tot;
+    for (int t = run.begin; t < run.end; ++t) {
+        const TileRef tr = tab[t];
+        const ProbDev &pd = P[tr.prob];
+        const gptr<CgScalars> S = glob(pd.S);
+        const int n = step - pd.n0 + 1;
+        if (n < 1 || n > S->done_at) continue;
+        const bool first = n == 1;
+        const double rz = S->rz[(n - 1) & 1];
+        const double pq = first ? 0.0 : tot.get(tr.prob, pd.P.spmv, pd.nt3);
+        const double alpha = pq != 0.0 ? rz / pq : 0.0;
+        if (tr.tile == 0 && threadIdx.x == 0) S->alpha = alpha;
+        const gptr<double> r = glob(pd.r);
+        const gptr<const double> q = glob((const double *)pd.q);
+        const gptr<float> r32 = glob(pd.r32);
+        const long long len = pd.g.n, nv = len / 4, stride = (long long)pd.nt1 * kThreads;
+        double acc = 0.0;
+        for (long long v = (long long)tr.tile * kThreads + threadIdx.x; v < nv; v += stride) {
+            vd4 rv = ((gptr<const vd4>)r)[v];
+            va4 f;
+            if (!first) {
+                const vd4 qv = ((gptr<const vd4>)q)[v];
+#pragma unroll
+                for (int m = 0; m < 4; ++m) rv[m] = rv[m] - alpha * qv[m];
+                ((gptr<vd4>)r)[v] = rv;
+            }
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                acc += rv[m] * rv[m];
+                f[m] = (float)rv[m];
+            }
+            ((gptr<va4>)r32)[v] = f;
+        }
+        if (tr.tile == 0) {
+            const long long c = nv * 4 + threadIdx.x;
+            if (c < len) {
+                const double rv = first ? r[c] : r[c] - alpha * q[c];
+                r[c] = rv;
+                r32[c] = (float)rv;
+                acc += rv * rv;
+            }
+        }
+        const double s = block_sum(acc);
+        if (threadIdx.x == 0) pd.P.upd[tr.tile] = s;
     }
 }
 
@@ -714,12 +789,13 @@ __device__ __forceinline__ float bot_nb(const BotDim &d, const BotCell &b, int c
 // wait on memory once.  Levels of at most kBotWave cells are one wave's, whose
 // LDS accesses need no barrier.
 //
-// The constant-pressure component is taken out of level lbot's residual where
-// the operator has that null space: the coarse levels would amplify it about
-// fourfold each, and the FP32 operator is not exactly (nor surely not
-// negatively) singular on it; p.q then went negative at 1e-11 relative
-// residuals.  (Residuals of a consistent system have that component from
-// rounding alone, so r.z stays that of a symmetric cycle.)
+// The constant-pressure component is taken out of level lbot's residual and
+// correction where the operator has that null space: the coarse levels would
+// amplify the residual's about fourfold each, and leave one in the correction
+// that is 99 % of z at a density ratio of 1000; the FP32 operator is not exactly
+// (nor surely not negatively) singular on it, and p.q or r.z then went
+// negative at small residuals.  Taken out of both sides, the cycle stays
+// symmetric.
 constexpr int kBotWave = 256;
 __global__ __launch_bounds__(kBotThreads) void k_mg_bottom(const ProbDev *__restrict__ P,
                                                            const int *__restrict__ probs, StepRef sref)
@@ -877,11 +953,22 @@ __global__ __launch_bounds__(kBotThreads) void k_mg_bottom(const ProbDev *__rest
         off -= m;
         up(false, l, off, m);
     }
+    double f = 0.0;
+    if (project) {
+        double ew = 0.0;
+#pragma unroll
+        for (int q = 0; q < kBotPer; ++q) {
+            const int c = tid + q * kBotThreads;
+            if (c < m0) ew += (double)top[q].w * (double)top[q].w * (double)A[c];
+        }
+        ew = bot_sum(ew);
+        f = ww > 0.0 ? ew / ww : 0.0;
+    }
     const gptr<float> e = glob(L0.t);
 #pragma unroll
     for (int q = 0; q < kBotPer; ++q) {
         const int c = tid + q * kBotThreads;
-        if (c < m0) e[c] = A[c];
+        if (c < m0) e[c] = (float)((double)A[c] - f);
     }
 }
 
@@ -895,16 +982,18 @@ __global__ __launch_bounds__(kThreads) void k_mg_decide(const ProbDev *__restric
     const ProbDev &pd = P[probs[blockIdx.x]];
     CgScalars *S = pd.S;
     const int n = step - pd.n0 + 1;
-    if (n < 1 || S->final_ || n != S->next_refresh) return;
+    if (n < 1 || S->final_ || n != S->next_refresh || !pd.mixed) return;
     const double rrt = block_total_of(pd.P.tres, pd.nt3);
     const double rrs = block_total_of(pd.P.tres + pd.nt3, pd.nt3);
     if (threadIdx.x == 0) {
         const bool finite = rrt >= 0.0 && rrt < 1e300;
-        const bool conv = finite && !(rrt > S->thresh);
+        const double before = S->refreshes ? S->prev_rr : S->rr0;
         const bool cap = S->iters >= S->max_iter;
+        // one more cycle when only the margin is missing
+        const bool conv = finite && (rrt <= kMgMargin * S->thresh ||
+                                     (rrt <= S->thresh && (before <= S->thresh || cap)));
         // a cycle that did not halve r.r: counted, and after three in a row
         // the solve goes back to CG from the start
-        const double before = S->refreshes ? S->prev_rr : S->rr0;
         S->stalls = rrt < 0.5 * before ? 0 : S->stalls + 1;
         S->rr_true = rrt;
         S->refreshes += 1;
@@ -1175,9 +1264,9 @@ int blocks(long long n) { return (int)((n + kThreads - 1) / kThreads); }
 
 }  // namespace
 
-bool mg_plan(const Geo &g, bool mixed, float *w32, float *space, size_t floats, ProbDev &pd)
+bool mg_plan(const Geo &g, float *w32, float *space, size_t floats, ProbDev &pd, size_t *used)
 {
-    if (!mixed || g.n < kMgMinCells || (long long)g.nx * g.ny >= (1LL << 29)) return false;
+    if (g.n < kMgMinCells || (long long)g.nx * g.ny >= (1LL << 29)) return false;
     size_t off = 0;
     auto take = [&](size_t count) {
         float *p = space + off;
@@ -1235,6 +1324,7 @@ bool mg_plan(const Geo &g, bool mixed, float *w32, float *space, size_t floats, 
     }
     if (!lbot) return false;
     pd.bot = take((size_t)pd.nbot * (sizeof(BotCell) / sizeof(float)));
+    if (used) *used = off;
     if (off > floats) return false;
     pd.nlev = l + 1;
     pd.lbot = lbot;
@@ -1288,6 +1378,9 @@ void launch_mg_step(const ProbDev *P, const MgTables &T, int maxgrid, StepRef st
 #define MG_LEVEL(KIND, l)                                                                                          \
     hipLaunchKernelGGL(k_mg_level<KIND>, dim3(std::min(T.nlev[l], 4 * maxgrid)), dim3(kThreads), 0, s, P, T.lev[l], \
                        T.nlev[l], l, step)
+    if (T.nt1_64)
+        hipLaunchKernelGGL(k_mg_upd64, dim3(std::min(T.nt1_64, maxgrid)), dim3(kThreads), 0, s, P, T.t1_64, T.nt1_64,
+                           step);
     MG_FINE(kA1, nullptr);
     MG_FINE(kA2, nullptr);
     for (int l = 1; l < kMgLevels; ++l)
@@ -1303,9 +1396,12 @@ void launch_mg_step(const ProbDev *P, const MgTables &T, int maxgrid, StepRef st
         }
     MG_FINE(kB1, nullptr);
     MG_FINE(kB2, nullptr);
-    MG_FINE(kDir, ran);
-    launch_true_residual(P, T.t3, T.nt3, maxgrid, step, s);
-    hipLaunchKernelGGL(k_mg_decide, dim3(T.nprobs), dim3(kThreads), 0, s, P, T.probs, step);
+    if (T.nt3) {
+        MG_FINE(kDir, ran);
+        launch_true_residual(P, T.t3, T.nt3, maxgrid, step, s);
+        hipLaunchKernelGGL(k_mg_decide, dim3(T.nprobs), dim3(kThreads), 0, s, P, T.probs, step);
+    }
+    if (T.nt3_64) launch_mg_dir64(P, T.t3_64, T.nt3_64, maxgrid, step, ran, s);
 #undef MG_FINE
 #undef MG_LEVEL
 }

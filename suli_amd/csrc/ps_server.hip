@@ -347,7 +347,7 @@ void suli_ps_server::dev_loop()
             int slot = -1;
             const int rc = broken ? SULI_PS_EHIP
                                   : eng.admit(r->g, in, r->dprd1, so, (int)(r->ticket & 0x7fffffff), &slot,
-                                              r->state_block, r->ev_up);
+                                              r->state_block, r->bytes - r->field_bytes, r->ev_up);
             std::lock_guard<std::mutex> lk(m);
             if (rc) {
                 fail_resident(r, rc, broken ? err : eng.error());
@@ -500,7 +500,11 @@ int64_t suli_ps_server_submit(suli_ps_server *srv, const suli_ps_grid *g, const 
     r->dzz = dzz;
     r->prd1 = prd1;
     r->field_bytes = carve_fields(*r, nullptr);
-    r->bytes = r->field_bytes + problem_bytes(g->nx, g->ny, g->nz, srv->opts.solve.precision == SULI_PS_MIXED);
+    // a request whose larger state (state_bytes) is beyond the budget is solved
+    // by plain CG in the smaller one
+    r->bytes = r->field_bytes + state_bytes(g->nx, g->ny, g->nz, solve_opts(srv->opts.solve));
+    if (r->bytes > srv->budget)
+        r->bytes = r->field_bytes + problem_bytes(g->nx, g->ny, g->nz, srv->opts.solve.precision == SULI_PS_MIXED);
     std::lock_guard<std::mutex> lk(srv->m);
     for (auto pr : {std::make_pair(&r->ev_up, &srv->spare_up), std::make_pair(&r->ev_done, &srv->spare_done)}) {
         if (!pr.second->empty()) {

@@ -27,7 +27,10 @@ using namespace sps;
 // only a stand-in for the device array: its device address is looked up
 // once per device (scratch_address) and that address is what the engine
 // and the kernels are given.
-static __device__ __align__(256) unsigned char scratch[SULI_PS_NOALLOC_MAX_BYTES];
+// kNoAllocExtra bytes more than the accepted state hold the FP32 arrays of an
+// FP64 problem's V-cycle (about 35 B per cell beside the 80 that are
+// accepted), so that it iterates as with allocation.
+static __device__ __align__(256) unsigned char scratch[SULI_PS_NOALLOC_MAX_BYTES + kNoAllocExtra];
 
 namespace {
 
@@ -218,8 +221,8 @@ void warn_capped(const suli_ps_ctx *ctx, const suli_ps_stats &st)
     }
 }
 
-// block: device memory for the problem's solver state (problem_bytes), or
-// NULL for the engine's pool.
+// block: the fixed array for the problem's solver state, or NULL for the
+// engine's pool.
 int run_graddin_dev(suli_ps_ctx *ctx, const suli_ps_grid *gr, const double *u, const double *v, const double *w,
                     const double *rho, const double *ox, const double *oy, const double *oz, const double *dz,
                     const double *dzz, double *prd1, suli_ps_stats *stats, const uint8_t *solid = nullptr,
@@ -232,7 +235,8 @@ int run_graddin_dev(suli_ps_ctx *ctx, const suli_ps_grid *gr, const double *u, c
     HIPCHK(ctx, hipEventRecord(ctx->ev[0], s));
     const SetupIn in = make_setup(gr, u, v, w, rho, prd1, ox, oy, oz, dz, dzz, solid);
     int slot = -1;
-    if ((rc = ctx->eng.admit(*gr, in, prd1, solve_opts(ctx->opts), 0, &slot, block)))
+    if ((rc = ctx->eng.admit(*gr, in, prd1, solve_opts(ctx->opts), 0, &slot, block,
+                             block ? SULI_PS_NOALLOC_MAX_BYTES + kNoAllocExtra : 0)))
         return fail(ctx, rc, "%s", ctx->eng.error().c_str());
     ctx->last_slots.push_back(slot);
     if ((rc = ctx->eng.run_all(ctx->opts.timing != 0))) return fail(ctx, rc, "%s", ctx->eng.error().c_str());
