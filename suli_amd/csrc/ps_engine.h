@@ -74,7 +74,8 @@ size_t problem_bytes(int nx, int ny, int nz, bool mixed);
 // + kNoAllocExtra) stays with plain CG, so that it solves the same way with
 // and without allocation.
 constexpr size_t kNoAllocExtra = (size_t)40 << 20;
-size_t state_bytes(int nx, int ny, int nz, const SolveOpts &o);
+// multi (optional): whether the multigrid iteration serves such a problem.
+size_t state_bytes(int nx, int ny, int nz, const SolveOpts &o, bool *multi = nullptr);
 
 // Whether the multigrid iteration serves solves with these options.
 bool mg_applies(const SolveOpts &o);
@@ -179,7 +180,7 @@ private:
     int fail(int code, const std::string &msg);
     int rebuild_tables();
     // Descriptor and set-up kernels of a slot whose geometry and block stand;
-    // multi: by the multigrid iteration where it applies.
+    // multi: by the multigrid iteration (state_bytes() of memory).
     int setup_slot(int si, bool multi, hipEvent_t wait_ev);
     int enqueue_chunk(int K, bool timing);
     int enqueue_steps_direct(int nsteps, bool timing);
@@ -255,6 +256,7 @@ private:
     struct Tuned {
         int kz, vx;   // vx: lane code
         double us;
+        bool fixed;   // by set_tiles: the size is then solved by plain CG
     };
     std::map<std::tuple<int, int, int, bool>, Tuned> tuned_;
     int chunk_ = 0;

@@ -95,7 +95,7 @@ bool carve_mg64(Carver &cv, const Geo &g, ProbDev &pd)
     const size_t n = (size_t)g.n;
     size_t floats = 0;
     ProbDev probe{};
-    if (!mg_plan(g, nullptr, nullptr, (size_t)-1, probe, &floats)) return false;
+    if (!mg_plan(g, nullptr, nullptr, (size_t)-1, nullptr, probe, &floats)) return false;
     pd.sx32 = cv.take<float>((size_t)(g.nx + 1) * g.ny * g.nz);
     pd.sy32 = cv.take<float>((size_t)g.nx * (g.ny + 1) * g.nz);
     pd.sz32 = cv.take<float>((size_t)g.nx * g.ny * (g.nz + 1));
@@ -109,7 +109,7 @@ bool carve_mg64(Carver &cv, const Geo &g, ProbDev &pd)
     pd.rz32 = cv.take<float>(4 * ((size_t)g.nz + 1));
     pd.rowreg = cv.take<unsigned>((size_t)(g.ny + 31) / 32 * g.nz);
     pd.P.m4 = cv.take<double>(3 * (size_t)probe.ntm);
-    return mg_plan(g, w, space, floats, pd);
+    return mg_plan(g, w, space, floats, pd.q32b, pd);
 }
 
 }  // namespace
@@ -178,17 +178,21 @@ size_t problem_bytes(int nx, int ny, int nz, bool mixed)
     return align_up(cv.off, 2 << 20);
 }
 
-size_t state_bytes(int nx, int ny, int nz, const SolveOpts &o)
+size_t state_bytes(int nx, int ny, int nz, const SolveOpts &o, bool *multi)
 {
     const size_t plain = problem_bytes(nx, ny, nz, o.mixed);
-    if (o.mixed || !mg_applies(o) || mg_entries(make_geo(nx, ny, nz, 0, 0)) == 0) return plain;
+    const bool can = mg_applies(o) && mg_entries(make_geo(nx, ny, nz, 0, 0)) > 0;
+    if (multi) *multi = can;
+    if (o.mixed || !can) return plain;
     const Geo g = make_geo(nx, ny, nz, 0, 0, kMinKz);
     Carver cv{nullptr};
     ProbDev pd{};
     carve(cv, g, false, spmv_tiles(g), vec_tiles(g.n), pd);
-    if (!carve_mg64(cv, g, pd)) return plain;
-    const size_t multi = align_up(cv.off, 2 << 20);
-    return multi > SULI_PS_NOALLOC_MAX_BYTES + kNoAllocExtra && plain <= SULI_PS_NOALLOC_MAX_BYTES ? plain : multi;
+    const bool ok = carve_mg64(cv, g, pd);
+    const size_t bytes = align_up(cv.off, 2 << 20);
+    if (ok && !(bytes > SULI_PS_NOALLOC_MAX_BYTES + kNoAllocExtra && plain <= SULI_PS_NOALLOC_MAX_BYTES)) return bytes;
+    if (multi) *multi = false;
+    return plain;
 }
 
 // -------------------------------------------------------------- Engine ----
@@ -363,7 +367,7 @@ long long mg_entries(const Geo &g)
     const long long nt3 = spmv_tiles(g);
     // mixed solves keep the hierarchy in 2 n floats and three partial sums per
     // fine tile in m4; FP64 ones go by the same rule
-    if (!mg_plan(g, nullptr, nullptr, 2 * (size_t)g.n, pd, &floats) || 3 * pd.ntm > 8 * nt3) return 0;
+    if (!mg_plan(g, nullptr, nullptr, 2 * (size_t)g.n, nullptr, pd, &floats) || 3 * pd.ntm > 8 * nt3) return 0;
     long long n = pd.ntm;
     for (int l = 1; l < pd.lbot; ++l) n += mg_level_tiles(pd, l);
     return n;
@@ -384,11 +388,16 @@ int Engine::admit(const suli_ps_grid &gr, const SetupIn &in, double *prd1_out, c
     sl = Slot{};
     int kz = o.kz > 0 ? std::max(o.kz, kMinKz) : 0;
     int vx = o.vx > 0 ? o.vx : 0;
-    // the tuner's shapes are the plain CG kernels': nothing to tune otherwise
-    const Geo g0 = make_geo(gr.nx, gr.ny, gr.nz, gr.ccx0 == 0, gr.ccy0 == 0);
-    sl.bytes = state_bytes(gr.nx, gr.ny, gr.nz, o);
+    // a tile shape fixed by the caller names plain CG's kernels
+    const auto fixed = tuned_.find(std::make_tuple(gr.nx, gr.ny, gr.nz, o.mixed));
+    bool multi = false;
     const size_t plain = problem_bytes(gr.nx, gr.ny, gr.nz, o.mixed);
-    if (mg_applies(o) && mg_entries(g0) > 0 && (o.mixed || sl.bytes > plain)) {
+    sl.bytes = state_bytes(gr.nx, gr.ny, gr.nz, o, &multi);
+    if (autotune_ && fixed != tuned_.end() && fixed->second.fixed) multi = false;
+    if (block && block_bytes < sl.bytes) multi = false;
+    if (!multi) sl.bytes = plain;
+    // the tuner's shapes are the plain CG kernels': nothing to tune otherwise
+    if (multi) {
         // the shape a fall-back to plain CG would take
         int kz_c = 0, vx_c = 0;
         if (autotune_) cached_shape(gr.nx, gr.ny, gr.nz, o.mixed, &kz_c, &vx_c);
@@ -414,10 +423,10 @@ int Engine::admit(const suli_ps_grid &gr, const SetupIn &in, double *prd1_out, c
     sl.o.kz = kz;
     sl.o.vx = vx;
     sl.own_block = block == nullptr;
-    if (block && block_bytes < sl.bytes) sl.bytes = plain;
     sl.block = block ? block : pool_.get(sl.bytes, err_);
     if (!sl.block && sl.bytes > plain && !no_alloc_active()) {
         // plain CG where the V-cycle's arrays do not fit any more
+        multi = false;
         sl.bytes = plain;
         sl.block = pool_.get(sl.bytes, err_);
     }
@@ -427,7 +436,7 @@ int Engine::admit(const suli_ps_grid &gr, const SetupIn &in, double *prd1_out, c
     sl.user = user;
     sl.used = true;
     sl.active = true;
-    const int rc = setup_slot(si, true, wait_ev);
+    const int rc = setup_slot(si, multi, wait_ev);
     if (rc) return rc;
     if (slot_out) *slot_out = si;
     return 0;
@@ -445,8 +454,7 @@ int Engine::setup_slot(int si, bool multi, hipEvent_t wait_ev)
     // kernels, which walk one cell per lane, take the default shape
     sl.mg = false;
     for (const bool mg : {true, false}) {
-        if (mg && !(multi && mg_applies(o) && mg_entries(make_geo(gr.nx, gr.ny, gr.nz, 0, 0)) > 0)) continue;
-        if (mg && !o.mixed && sl.bytes <= problem_bytes(gr.nx, gr.ny, gr.nz, false)) continue;
+        if (mg && !multi) continue;
         sl.g = make_geo(gr.nx, gr.ny, gr.nz, gr.ccx0 == 0, gr.ccy0 == 0, mg ? 0 : o.kz, mg ? 1 : o.mixed ? o.vx : 1);
         sl.g.dtop = gr.top_bc == 1 ? 1 : 0;
         nt3 = spmv_tiles(sl.g);
@@ -457,7 +465,7 @@ int Engine::setup_slot(int si, bool multi, hipEvent_t wait_ev)
         carve(cv, sl.g, o.mixed, nt3, nt1, pd);
         if (mg) {
             sl.mg = o.mixed ? mg_plan(sl.g, pd.p32 + 2 * pd.pslot, reinterpret_cast<float *>(pd.r),
-                                      2 * (size_t)sl.g.n, pd)
+                                      2 * (size_t)sl.g.n, pd.q32b, pd)
                             : carve_mg64(cv, sl.g, pd);
             if (o.mixed) pd.t32 = pd.p32 + 3 * pd.pslot;
             if (sl.mg) break;
@@ -1066,7 +1074,7 @@ int Engine::run_all(bool timing)
 void Engine::set_tiles(int nx, int ny, int nz, bool mixed, int kz, int vx)
 {
     const Geo g = make_geo(nx, ny, nz, 0, 0, std::max(kz, kMinKz), mixed ? vx : 1);
-    tuned_[std::make_tuple(nx, ny, nz, mixed)] = Tuned{g.kz, lane_code(g), 0.0};
+    tuned_[std::make_tuple(nx, ny, nz, mixed)] = Tuned{g.kz, lane_code(g), 0.0, true};
 }
 
 int Engine::tune(int nx, int ny, int nz, bool mixed, int *kz_out, int *vx_out, double *us_out)
@@ -1196,7 +1204,7 @@ int Engine::tune(int nx, int ny, int nz, bool mixed, int *kz_out, int *vx_out, d
     }
 #undef TCHK
     cleanup();
-    tuned_[key] = Tuned{best_kz, best_vx, best_us};
+    tuned_[key] = Tuned{best_kz, best_vx, best_us, false};
     *kz_out = best_kz;
     *vx_out = best_vx;
     *us_out = best_us;

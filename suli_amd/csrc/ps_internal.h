@@ -42,9 +42,10 @@ static_assert((kFold & (kFold - 1)) == 0, "kFold is a power of two");
 // Multigrid-preconditioned CG (ps_mg.hip), the iteration of mixed solves, and
 // of FP64 solves by the relative rule, from kMgMinCells cells on.
 //
-// kMgMinCells: smaller problems keep plain CG, whose iterates the options
-// stored_residual and a small max_iter are specified on.
-constexpr long long kMgMinCells = 49153;
+// kMgMinCells: below, the hierarchy does not fit the memory it shares.  Plain
+// CG against this from prd1 = 0 to 1e-12 relative, mixed: 4096 cells 2.20 and
+// 0.96 ms, 15360 cells 3.25 and 1.00, 46080 cells 4.51 and 1.20.
+constexpr long long kMgMinCells = 4096;
 // A cap below this keeps plain CG: a capped solve returns CG's iterate.
 constexpr int kMgMinCap = 256;
 constexpr int kMgLevels = 20;
@@ -363,7 +364,8 @@ void launch_spmv_only(bool fp32, const ProbDev *P, const TileRef *t3, int nt3, i
 // Lays the hierarchy of a problem out in `space` (`floats` of them; w32 holds
 // level 0's weights) and fills pd's multigrid fields; false where it does not apply (size, or the
 // hierarchy does not fit), pd.mg then stays 0.
-bool mg_plan(const Geo &g, float *w32, float *space, size_t floats, ProbDev &pd, size_t *used = nullptr);
+bool mg_plan(const Geo &g, float *w32, float *space, size_t floats, float *scratch, ProbDev &pd,
+             size_t *used = nullptr);
 // Table entries of level l's kernels.
 int mg_level_tiles(const ProbDev &pd, int l);
 // Weights and coarse operators, after launch_init; dev: pd on the device.

@@ -1264,15 +1264,20 @@ int blocks(long long n) { return (int)((n + kThreads - 1) / kThreads); }
 
 }  // namespace
 
-bool mg_plan(const Geo &g, float *w32, float *space, size_t floats, ProbDev &pd, size_t *used)
+bool mg_plan(const Geo &g, float *w32, float *space, size_t floats, float *scratch, ProbDev &pd, size_t *used)
 {
     if (g.n < kMgMinCells || (long long)g.nx * g.ny >= (1LL << 29)) return false;
-    size_t off = 0;
-    auto take = [&](size_t count) {
-        float *p = space + off;
-        off += (count + 63) / 64 * 64 + 64;   // 256-byte aligned; short reads past a row's end stay inside
-        return p;
-    };
+    // 256-byte aligned; short reads past a row's end stay inside
+    struct Take {
+        float *p;
+        size_t off = 0;
+        float *operator()(size_t count)
+        {
+            float *q = p + off;
+            off += (count + 63) / 64 * 64 + 64;
+            return q;
+        }
+    } keep{space}, setup{scratch};
     pd.w32 = w32;
     MgLevel &L0 = pd.lv[0];
     L0 = MgLevel{};
@@ -1289,7 +1294,7 @@ bool mg_plan(const Geo &g, float *w32, float *space, size_t floats, ProbDev &pd,
     while (cells(pd.lv[l]) > kMgCoarsestCells) {
         if (l + 1 >= kMgLevels) return false;
         const MgLevel &F = pd.lv[l];
-        MgLevel &C = pd.lv[l + 1];
+        MgLevel &C = pd.lv[++l];
         C = MgLevel{};
         C.nx = (F.nx + 1) / 2;
         C.ny = (F.ny + 1) / 2;
@@ -1297,35 +1302,45 @@ bool mg_plan(const Geo &g, float *w32, float *space, size_t floats, ProbDev &pd,
         // a single cell around has no neighbour but itself
         C.px = F.px && C.nx > 1;
         C.py = F.py && C.ny > 1;
-        const size_t n = (size_t)cells(C);
-        C.sx = take((size_t)(C.nx + 1) * C.ny * C.nz);
-        C.sy = take((size_t)C.nx * (C.ny + 1) * C.nz);
-        C.sz = take(n + (size_t)C.nx * C.ny);
-        C.w = take(n);
-        C.r = take(n);
-        C.t = take(n);
-        C.rho = take(n);
-        C.r0 = take(n);
-        C.ex = take((size_t)C.nx * C.ny);
-        ++l;
     }
-    if (off > floats) return false;
     // the bottom kernel starts at the first level whose cells its threads hold
-    // and whose hierarchy fits its LDS (four floats per cell, and the
-    // coefficients of the levels below)
+    // and whose hierarchy fits its LDS (four floats per cell, the coefficients
+    // of the levels below, two guards)
     for (int b = 1; b <= l && !lbot; ++b) {
         size_t low = 0;
         for (int q = b + 1; q <= l; ++q) low += cells(pd.lv[q]);
         const size_t n = cells(pd.lv[b]);
-        if (n <= (size_t)kMgBottomCells && 4 * (n + low) + low * (sizeof(BotCell) / sizeof(float)) + 2 * (size_t)pd.lv[b].nx * pd.lv[b].ny <= (size_t)kMgBottomLds) {
+        if (n <= (size_t)kMgBottomCells &&
+            4 * (n + low) + 8 * low + 2 * (size_t)pd.lv[b].nx * pd.lv[b].ny <= (size_t)kMgBottomLds) {
             lbot = b;
             pd.nbot = (int)(n + low);
         }
     }
     if (!lbot) return false;
-    pd.bot = take((size_t)pd.nbot * (sizeof(BotCell) / sizeof(float)));
-    if (used) *used = off;
-    if (off > floats) return false;
+    // faces and weights of the bottom levels are packed at the end of the
+    // set-up: only w of level lbot, its r and its t are read again
+    for (int q = 1; q <= l; ++q) {
+        MgLevel &C = pd.lv[q];
+        const size_t n = (size_t)cells(C);
+        Take &t = q < lbot ? keep : setup;
+        C.sx = t((size_t)(C.nx + 1) * C.ny * C.nz);
+        C.sy = t((size_t)C.nx * (C.ny + 1) * C.nz);
+        C.sz = t(n + (size_t)C.nx * C.ny);
+        C.ex = t((size_t)C.nx * C.ny);
+        C.w = q <= lbot ? keep(n) : setup(n);
+        if (q <= lbot) {
+            C.r = keep(n);
+            C.t = keep(n);
+        }
+        if (q < lbot) {
+            C.rho = keep(n);
+            C.r0 = keep(n);
+        }
+    }
+    static_assert(sizeof(BotCell) == 8 * sizeof(float), "the pack's size");
+    pd.bot = keep(8 * (size_t)pd.nbot);
+    if (used) *used = keep.off;
+    if (keep.off > floats || setup.off > (size_t)g.n) return false;
     pd.nlev = l + 1;
     pd.lbot = lbot;
     // rows: 16, 32 or 64 lanes of four cells

@@ -1,5 +1,5 @@
 """The multigrid-preconditioned iteration (mixed solves, and FP64 ones by the
-relative rule, on grids of more than 49152 cells) against the CPU oracle.
+relative rule, on grids of 4096 cells or more) against the CPU oracle.
 
 Sizes where its kernels can go wrong: the first size it serves, rows of 16,
 32 and 64 lanes with whole and partial last lanes, rows of several segments,
@@ -56,7 +56,9 @@ def two_parts(nx, ny, nz, seed):
 
 R = cases.random_case
 CASES = [
-    ("first_size", lambda: R(37, 37, 36, 1)),             # 49284 cells, partial lanes, 16 per row
+    ("first_size", lambda: R(16, 16, 16, 1)),             # the bottom kernel takes every coarse level
+    ("one_coarse_grid", lambda: R(37, 37, 33, 23)),       # 6137 cells on level 1
+    ("two_coarse_grids", lambda: R(37, 37, 36, 24)),      # 6498: one more level of its own
     ("rows_of_64", lambda: R(64, 33, 25, 2)),
     ("rows_of_65", lambda: R(65, 40, 21, 3, periodic_x=True)),
     ("rows_of_130", lambda: R(130, 21, 20, 4)),
