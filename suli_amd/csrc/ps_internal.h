@@ -51,8 +51,13 @@ constexpr int kMgMinCap = 256;
 constexpr int kMgLevels = 20;
 constexpr int kMgBottomCells = 6144;   // the bottom kernel's largest level
 constexpr int kMgBottomLds = 38912;    // floats of LDS it has (152 KiB)
-constexpr int kMgCoarsestCells = 8;
-constexpr int kMgCoarsestSweeps = 8;
+// The coarsest level: at most a cell per lane of one wave and kMgCoarsestSide
+// around (the sweeps must reach from end to end).  At 64 cells and 16 sweeps a
+// cycle over 64x64x32 takes as many iterations as at 8 cells and 8 sweeps, with
+// one level less: 1.25 -> 1.19 ms; at 8 sweeps it took one iteration more.
+constexpr int kMgCoarsestCells = 64;
+constexpr int kMgCoarsestSide = 8;
+constexpr int kMgCoarsestSweeps = 16;
 constexpr int kMgChunk = 2;            // iterations between host polls
 // Residual replacement: once the FP32 r.r has fallen by kMgCycleDrop since the
 // last one, or to kMgMargin of the threshold, and at the latest after kMgMaxGap

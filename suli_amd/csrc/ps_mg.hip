@@ -720,18 +720,24 @@ __global__ __launch_bounds__(kThreads) void k_mg_level(const ProbDev *__restrict
     }
 }
 
-// Sum over the bottom kernel's workgroup, to every thread.
-__device__ __forceinline__ double bot_sum(double v)
+// Sums over the bottom kernel's workgroup, to every thread.
+template <int N>
+__device__ __forceinline__ void bot_sum(double (&v)[N])
 {
-    __shared__ double red[kBotThreads / 64];
-    v = wave_sum(v);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    double s = red[0];
+    __shared__ double red[N][kBotThreads / 64];
 #pragma unroll
-    for (int w = 1; w < kBotThreads / 64; ++w) s += red[w];
-    return s;
+    for (int i = 0; i < N; ++i) v[i] = wave_sum(v[i]);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+        if ((threadIdx.x & 63) == 0) red[i][threadIdx.x >> 6] = v[i];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        v[i] = red[i][0];
+#pragma unroll
+        for (int w = 1; w < kBotThreads / 64; ++w) v[i] += red[i][w];
+    }
 }
 
 // One cell of a bottom level: its faces (E, W, N, S, T, B), w, and its parent
@@ -796,7 +802,7 @@ __device__ __forceinline__ float bot_nb(const BotDim &d, const BotCell &b, int c
 // (nor surely not negatively) singular on it, and p.q or r.z then went
 // negative at small residuals.  Taken out of both sides, the cycle stays
 // symmetric.
-constexpr int kBotWave = 256;
+constexpr int kBotWave = 128;
 __global__ __launch_bounds__(kBotThreads) void k_mg_bottom(const ProbDev *__restrict__ P,
                                                            const int *__restrict__ probs, StepRef sref)
 {
@@ -817,7 +823,7 @@ __global__ __launch_bounds__(kBotThreads) void k_mg_bottom(const ProbDev *__rest
     BotCell *const low = reinterpret_cast<BotCell *>(lds);
     float *const R = lds + 8 * (total - m0) + guard, *const A = R + total, *const B = A + total, *const D = B + total;
     BotCell top[kBotPer];
-    double vw = 0.0, ww = 0.0;
+    double pr[2] = {0.0, 0.0};   // w.r, w.w
 #pragma unroll
     for (int q = 0; q < kBotPer; ++q) {
         const int c = tid + q * kBotThreads;
@@ -825,8 +831,8 @@ __global__ __launch_bounds__(kBotThreads) void k_mg_bottom(const ProbDev *__rest
             top[q] = packed_cell(pack, c);
             const float r = r0[c];
             R[c] = r;
-            vw += (double)top[q].w * (double)r;
-            ww += (double)top[q].w * (double)top[q].w;
+            pr[0] += (double)top[q].w * (double)r;
+            pr[1] += (double)top[q].w * (double)top[q].w;
         }
     }
     for (int c = tid; c < total - m0; c += kBotThreads) low[c] = packed_cell(pack, m0 + c);
@@ -840,9 +846,8 @@ __global__ __launch_bounds__(kBotThreads) void k_mg_bottom(const ProbDev *__rest
     for (int c = tid; c < total - m0; c += kBotThreads) R[m0 + c] = 0.f;
     for (int c = tid; c < 3 * total; c += kBotThreads) A[c] = 0.f;
     if (project) {
-        vw = bot_sum(vw);
-        ww = bot_sum(ww);
-        const double f = ww > 0.0 ? vw / ww : 0.0;
+        bot_sum(pr);
+        const double f = pr[1] > 0.0 ? pr[0] / pr[1] : 0.0;
 #pragma unroll
         for (int q = 0; q < kBotPer; ++q) {
             const int c = tid + q * kBotThreads;
@@ -955,14 +960,14 @@ __global__ __launch_bounds__(kBotThreads) void k_mg_bottom(const ProbDev *__rest
     }
     double f = 0.0;
     if (project) {
-        double ew = 0.0;
+        double ew[1] = {0.0};
 #pragma unroll
         for (int q = 0; q < kBotPer; ++q) {
             const int c = tid + q * kBotThreads;
-            if (c < m0) ew += (double)top[q].w * (double)top[q].w * (double)A[c];
+            if (c < m0) ew[0] += (double)top[q].w * (double)top[q].w * (double)A[c];
         }
-        ew = bot_sum(ew);
-        f = ww > 0.0 ? ew / ww : 0.0;
+        bot_sum(ew);
+        f = pr[1] > 0.0 ? ew[0] / pr[1] : 0.0;
     }
     const gptr<float> e = glob(L0.t);
 #pragma unroll
@@ -1291,7 +1296,10 @@ bool mg_plan(const Geo &g, float *w32, float *space, size_t floats, float *scrat
     L0.sz = const_cast<float *>(pd.sz32);
     L0.w = pd.w32;
     int l = 0, lbot = 0;
-    while (cells(pd.lv[l]) > kMgCoarsestCells) {
+    auto coarsest = [&](const MgLevel &L) {
+        return cells(L) <= kMgCoarsestCells && std::max({L.nx, L.ny, L.nz}) <= kMgCoarsestSide;
+    };
+    while (!coarsest(pd.lv[l])) {
         if (l + 1 >= kMgLevels) return false;
         const MgLevel &F = pd.lv[l];
         MgLevel &C = pd.lv[++l];
