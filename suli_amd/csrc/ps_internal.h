@@ -162,12 +162,12 @@ struct Partials {
 // One level of the multigrid hierarchy (level 0: the problem itself, whose
 // faces are sx32 .. and whose vectors stand elsewhere).  Scaled faces in the
 // face arrays' layouts, 0 at walls on the coarse levels; w = sqrt(diagonal),
-// 0 in cells without faces; r the scaled restricted residual; t, rho and r0
-// the cycle's vectors (ps_mg.hip), t at last the correction, un-scaled; ex the diagonal's extra term on the top plane (the
-// p = 0 lid, SuLi-IT's free surface).
+// 0 in cells without faces; r the scaled restricted residual; t and rho the
+// cycle's vectors (ps_mg.hip), t at last the correction, un-scaled; ex the
+// diagonal's extra term on the top plane (the p = 0 lid, SuLi-IT's free surface).
 struct MgLevel {
     int nx, ny, nz, px, py;
-    float *sx, *sy, *sz, *w, *r, *t, *rho, *r0, *ex;
+    float *sx, *sy, *sz, *w, *r, *t, *rho, *ex;
 };
 
 // Device descriptor of one problem of a batch: geometry, tiling, where its

@@ -32,7 +32,8 @@
 //   t = A r                      rho = r - A s(A) r = r - c0 t - c1 A t
 //   (coarse: restrict rho, correct by e)
 //   r0 = rho - A (w e)           z = s(A) r + w e + s(A) r0
-// each a single pass with one application of A.
+// each a single pass with one application of A on the fine grid; below it the
+// two on either side of the coarser levels are one pass.
 //
 // Measured at 256x128x96 from prd1 = 0 to 1e-12 relative: plain CG 37.8 ms
 // (1992 iterations of one 18.5 us launch), this 3.39 ms (17 iterations); the
@@ -42,13 +43,13 @@
 // One iteration n (lbot: the first level of the bottom kernel):
 //   A1      r_{n-1} = r_{n-2} - alpha q (formed where needed), t; partials r.r
 //   A2      rho, restricted to level 1
-//   D1, D2  the same on levels 1 .. lbot-1
+//   D       the same on levels 1 .. lbot-1
 //   bottom  levels lbot and coarser, one workgroup per problem, in LDS
-//   U1, U2  coarse correction and post-smoothing on levels lbot-1 .. 1
+//   U       coarse correction and post-smoothing on levels lbot-1 .. 1
 //   B1, B2  the same on level 0: z_n; partials r.z
 //   dir     beta, c -= alpha_{n-1} p_{n-1}, p_n = z + beta p, q = A p;
 //           partials p.q
-// or, in a step whose A2 finds r_{n-1} small enough, instead of D1 .. dir the
+// or, in a step whose A2 finds r_{n-1} small enough, instead of D .. dir the
 // residual replacement: dir folds c and alpha p into e, then
 //   k_true_residual, k_mg_decide: converged, or on with the replaced residual
 // FP64: before A1, upd64 (r -= alpha q, its FP32 copy, partials r.r); instead
@@ -623,23 +624,6 @@ __global__ __launch_bounds__(kThreads) void k_mg_upd64(const ProbDev *__restrict
 
 // ---- coarse levels (l >= 1) -------------------------------------------------
 
-// sum over the six neighbours of s_face f(neighbour); faces at walls hold 0,
-// so a wrapped neighbour index only has to be valid
-template <class F>
-__device__ __forceinline__ float nb_sum(const MgLevel &L, int c, int i, int j, int k, F &&f)
-{
-    const int nx = L.nx, ny = L.ny, nz = L.nz, pl = nx * ny;
-    const gptr<const float> sx = glob((const float *)L.sx) + (c + (k * ny + j));
-    const gptr<const float> sy = glob((const float *)L.sy) + (c + k * nx);
-    const gptr<const float> sz = glob((const float *)L.sz) + c;
-    const int ie = i < nx - 1 ? i + 1 : 0, iw = i > 0 ? i - 1 : nx - 1;
-    const int jn = j < ny - 1 ? j + 1 : 0, js = j > 0 ? j - 1 : ny - 1;
-    const int kt = k < nz - 1 ? k + 1 : 0, kb = k > 0 ? k - 1 : nz - 1;
-    return sx[1] * f(c + ie - i, ie, j, k) + sx[0] * f(c + iw - i, iw, j, k) + sy[nx] * f(c + (jn - j) * nx, i, jn, k) +
-           sy[0] * f(c + (js - j) * nx, i, js, k) + sz[pl] * f(c + (kt - k) * pl, i, j, kt) +
-           sz[0] * f(c + (kb - k) * pl, i, j, kb);
-}
-
 __device__ __forceinline__ bool running(const ProbDev &pd, int step)
 {
     const gptr<const CgScalars> S = glob((const CgScalars *)pd.S);
@@ -648,20 +632,99 @@ __device__ __forceinline__ bool running(const ProbDev &pd, int step)
 }
 
 // Bricks of 16 x 4 x 4 cells, one workgroup each and one cell per thread: a
-// brick holds whole coarse cells, and its 2x2x2 sums go through LDS.
+// brick holds whole coarse cells.  With two cells around, a brick's vectors are
+// in LDS, and both matrix products of a half of the cycle are done there: the
+// first on the brick and its 288 face neighbours, the second on the brick.  These
+// passes wait on their launch and on memory's latency, not its rate: the two
+// products as launches of their own took 4.9 us each over 128x64x48 cells and 4.0
+// over 64x32x24, together they take 8.5 to 9.1 and 5.4 to 6.6 (a 64x64x32 solve
+// 1.20 -> 1.14 ms, 256x128x96 3.52 -> 3.44, 384x192x128 11.33 -> 11.09).
 constexpr int kBx = 16, kBy = 4, kBz = 4;
+constexpr int kHx = kBx + 4, kHy = kBy + 4, kHz = kBz + 4;   // with halo
+constexpr int kShell = 2 * (kBx * kBy + kBx * kBz + kBy * kBz);
+static_assert(kBx * kBy * kBz == kThreads && kHx * kHy * kHz % kThreads == 0 && kBx * kBy == 64 && kBx * kBz == 64,
+              "brick");
 __host__ __device__ inline int bricks(const MgLevel &L)
 {
     return ((L.nx + kBx - 1) / kBx) * ((L.ny + kBy - 1) / kBy) * ((L.nz + kBz - 1) / kBz);
 }
 
-// A pass over level l (1 <= l < lbot): D1, D2, U1 or U2 (A1, A2, B1, B2 of
-// the fine kernels; no partial sums, and U2 leaves the un-scaled correction).
-template <int KIND>
+struct Brick {
+    int x0, y0, z0;      // cell (0, 0, 0) of the halo box
+    int nx, ny, nz;
+    bool px, py;
+    __device__ __forceinline__ Brick(const MgLevel &L, int tile) : nx(L.nx), ny(L.ny), nz(L.nz), px(L.px), py(L.py)
+    {
+        const int bx = (nx + kBx - 1) / kBx, by = (ny + kBy - 1) / kBy;
+        const int rest = tile / bx;
+        x0 = (tile % bx) * kBx - 2;
+        y0 = (rest % by) * kBy - 2;
+        z0 = (rest / by) * kBz - 2;
+    }
+    // The grid cell at box position (a, b, d), wrapped around periodic sides;
+    // false where there is none.
+    __device__ __forceinline__ bool cell(int a, int b, int d, int &i, int &j, int &k) const
+    {
+        i = x0 + a;
+        j = y0 + b;
+        k = z0 + d;
+        if (px) i += i < 0 ? nx : i >= nx ? -nx : 0;
+        if (py) j += j < 0 ? ny : j >= ny ? -ny : 0;
+        return (unsigned)i < (unsigned)nx && (unsigned)j < (unsigned)ny && (unsigned)k < (unsigned)nz;
+    }
+    __device__ __forceinline__ int index(int i, int j, int k) const { return (k * ny + j) * nx + i; }
+    static __device__ __forceinline__ int box(int a, int b, int d) { return (d * kHy + b) * kHx + a; }
+};
+// Box position of shell cell h: below, above, south, north, west, east.
+__device__ __forceinline__ void shell_cell(int h, int &a, int &b, int &d)
+{
+    const int u = h & 63;
+    if (h < 128) {
+        a = 2 + (u & 15);
+        b = 2 + (u >> 4);
+        d = h < 64 ? 1 : 2 + kBz;
+    } else if (h < 256) {
+        a = 2 + (u & 15);
+        b = h < 192 ? 1 : 2 + kBy;
+        d = 2 + (u >> 4);
+    } else {
+        a = h < 272 ? 1 : 2 + kBx;
+        b = 2 + (u & 3);
+        d = 2 + ((u >> 2) & 3);
+    }
+}
+struct Faces {
+    float e, w, n, s, t, b;
+    __device__ __forceinline__ void load(const MgLevel &L, bool ok, int c, int j, int k)
+    {
+        e = w = n = s = t = b = 0.f;
+        if (!ok) return;
+        const gptr<const float> sx = glob((const float *)L.sx) + (c + (k * L.ny + j));
+        const gptr<const float> sy = glob((const float *)L.sy) + (c + k * L.nx);
+        const gptr<const float> sz = glob((const float *)L.sz) + c;
+        e = sx[1];
+        w = sx[0];
+        n = sy[L.nx];
+        s = sy[0];
+        t = sz[L.nx * L.ny];
+        b = sz[0];
+    }
+    // the six neighbours' share of A v at box cell x
+    __device__ __forceinline__ float sum(const float *v, int x) const
+    {
+        return e * v[x + 1] + w * v[x - 1] + n * v[x + kHx] + s * v[x - kHx] + t * v[x + kHx * kHy] +
+               b * v[x - kHx * kHy];
+    }
+};
+
+// Half a cycle on level l (1 <= l < lbot): down (A1 and A2 of the fine
+// kernels) or up (B1 and B2); no partial sums, and up leaves the un-scaled
+// correction.
+template <bool UP>
 __global__ __launch_bounds__(kThreads) void k_mg_level(const ProbDev *__restrict__ P, const TileRef *__restrict__ tab,
                                                        int ntab, int l, StepRef sref)
 {
-    __shared__ float sh[kThreads];
+    __shared__ float va[kHx * kHy * kHz], vb[kHx * kHy * kHz], sh[kThreads];
     const Run run = my_run(ntab);
     const int step = step_of(sref);
     for (int tt = run.begin; tt < run.end; ++tt) {
@@ -669,52 +732,85 @@ __global__ __launch_bounds__(kThreads) void k_mg_level(const ProbDev *__restrict
         const ProbDev &pd = P[tr.prob];
         if (!running(pd, step)) continue;
         const MgLevel &L = pd.lv[l], &C = pd.lv[l + 1];
-        const int bx = (L.nx + kBx - 1) / kBx, by = (L.ny + kBy - 1) / kBy;
-        const int tx = tr.tile % bx, rest = tr.tile / bx, ty = rest % by, tz = rest / by;
+        const Brick B(L, tr.tile);
         const int tid = threadIdx.x;
-        const int i = tx * kBx + (tid & 15), j = ty * kBy + ((tid >> 4) & 3), k = tz * kBz + (tid >> 6);
-        const bool in = i < L.nx && j < L.ny && k < L.nz;
-        const int c = (k * L.ny + j) * L.nx + i;
-        const gptr<float> r = glob(L.r), t = glob(L.t), rho = glob(L.rho), r0 = glob(L.r0), w = glob(L.w);
-        const gptr<const float> e = glob((const float *)C.t);
-        auto parent = [&](int a, int b, int d) { return ((d >> 1) * C.ny + (b >> 1)) * C.nx + (a >> 1); };
-        if (KIND == kA1) {
-            if (in) t[c] = r[c] - nb_sum(L, c, i, j, k, [&](int x, int, int, int) { return r[x]; });
-        } else if (KIND == kA2) {
-            float v = 0.f;
-            if (in) {
-                const float tc = t[c];
-                const float y = tc - nb_sum(L, c, i, j, k, [&](int x, int, int, int) { return t[x]; });
-                const float rh = r[c] - kC0 * tc - kC1 * y;
-                rho[c] = rh;
-                v = w[c] * rh;
+        const gptr<float> t = glob(L.t), rho = glob(L.rho);
+        const gptr<const float> r = glob((const float *)L.r), w = glob((const float *)L.w),
+                                e = glob((const float *)C.t);
+        const int Cx = C.nx, Cy = C.ny;
+        auto parent = [&](int i, int j, int k) { return ((k >> 1) * Cy + (j >> 1)) * Cx + (i >> 1); };
+        // the thread's own cell and its shell cell
+        const int a0 = 2 + (tid & 15), b0 = 2 + ((tid >> 4) & 3), d0 = 2 + (tid >> 6);
+        int i, j, k;
+        const bool ok = B.cell(a0, b0, d0, i, j, k);
+        const bool in = ok && i == B.x0 + a0 && j == B.y0 + b0;   // not around a periodic side
+        const int c = B.index(i, j, k), x0 = Brick::box(a0, b0, d0);
+        Faces f0;
+        f0.load(L, ok, c, j, k);
+        float va0[kHx * kHy * kHz / kThreads];
+#pragma unroll
+        for (int q = 0; q < kHx * kHy * kHz / kThreads; ++q) {
+            const int h = tid + q * kThreads, a = h % kHx, b = h / kHx % kHy, d = h / (kHx * kHy);
+            int ii, jj, kk;
+            va0[q] = 0.f;
+            if (B.cell(a, b, d, ii, jj, kk)) {
+                const int x = B.index(ii, jj, kk);
+                va0[q] = UP ? w[x] * e[parent(ii, jj, kk)] : r[x];
             }
-            __syncthreads();
-            sh[tid] = v;
+        }
+        float rho0 = 0.f, r_c = 0.f, t_c = 0.f, w_c = 0.f;
+        if (ok) w_c = w[c];
+        if (UP && ok) {
+            rho0 = rho[c];
+            r_c = r[c];
+            t_c = t[c];
+        }
+        __syncthreads();   // the last tile's reads of va
+#pragma unroll
+        for (int q = 0; q < kHx * kHy * kHz / kThreads; ++q) va[tid + q * kThreads] = va0[q];
+        __syncthreads();
+        const float own = va[x0];
+        const float u0 = UP ? rho0 - own + f0.sum(va, x0) : own - f0.sum(va, x0);
+        vb[x0] = u0;
+        for (int h = tid; h < kShell; h += kThreads) {
+            int a, b, d, ii, jj, kk;
+            shell_cell(h, a, b, d);
+            float u = 0.f;
+            const int x = Brick::box(a, b, d);
+            if (B.cell(a, b, d, ii, jj, kk)) {
+                const int cc = B.index(ii, jj, kk);
+                Faces f;
+                f.load(L, true, cc, jj, kk);
+                u = UP ? rho[cc] - va[x] + f.sum(va, x) : va[x] - f.sum(va, x);
+            }
+            vb[x] = u;
+        }
+        __syncthreads();
+        const float y = u0 - f0.sum(vb, x0);
+        if (UP) {
+            if (in) {
+                const float z = kC0 * (r_c + u0) + kC1 * (t_c + y) + own;
+                t[c] = w_c > 0.f ? z / w_c : 0.f;
+            }
+        } else {
+            const float rh = own - kC0 * u0 - kC1 * y;
+            if (in) {
+                t[c] = u0;
+                rho[c] = rh;
+            }
+            sh[tid] = in ? w_c * rh : 0.f;
             __syncthreads();
             if (tid < kThreads / 8) {
                 const int I = tid & 7, J = (tid >> 3) & 1, K = tid >> 4;
                 const int b = (2 * K) * 64 + (2 * J) * 16 + 2 * I;
                 const float sum = ((sh[b] + sh[b + 1]) + (sh[b + 16] + sh[b + 17])) +
                                   ((sh[b + 64] + sh[b + 65]) + (sh[b + 80] + sh[b + 81]));
-                const int ic = tx * (kBx / 2) + I, jc = ty * (kBy / 2) + J, kc = tz * (kBz / 2) + K;
+                const int ic = (B.x0 + 2) / 2 + I, jc = (B.y0 + 2) / 2 + J, kc = (B.z0 + 2) / 2 + K;
                 if (ic < C.nx && jc < C.ny && kc < C.nz) {
                     const int x = (kc * C.ny + jc) * C.nx + ic;
                     const float wc = C.w[x];
                     glob(C.r)[x] = wc > 0.f ? sum / wc : 0.f;
                 }
-            }
-        } else if (KIND == kB1) {
-            if (in) {
-                auto v = [&](int x, int a, int b, int d) { return w[x] * e[parent(a, b, d)]; };
-                r0[c] = rho[c] - v(c, i, j, k) + nb_sum(L, c, i, j, k, v);
-            }
-        } else {
-            if (in) {
-                const float v = r0[c], wc = w[c];
-                const float y = v - nb_sum(L, c, i, j, k, [&](int x, int, int, int) { return r0[x]; });
-                const float z = kC0 * (r[c] + v) + kC1 * (t[c] + y) + wc * e[parent(i, j, k)];
-                t[c] = wc > 0.f ? z / wc : 0.f;
             }
         }
     }
@@ -1342,7 +1438,6 @@ bool mg_plan(const Geo &g, float *w32, float *space, size_t floats, float *scrat
         }
         if (q < lbot) {
             C.rho = keep(n);
-            C.r0 = keep(n);
         }
     }
     static_assert(sizeof(BotCell) == 8 * sizeof(float), "the pack's size");
@@ -1398,8 +1493,8 @@ void launch_mg_step(const ProbDev *P, const MgTables &T, int maxgrid, StepRef st
     const int grid = std::min(T.nfine, maxgrid);
 #define MG_FINE(KIND, RAN) \
     hipLaunchKernelGGL(k_mg_fine<KIND>, dim3(grid), dim3(kThreads), 0, s, P, T.fine, T.nfine, step, RAN)
-#define MG_LEVEL(KIND, l)                                                                                          \
-    hipLaunchKernelGGL(k_mg_level<KIND>, dim3(std::min(T.nlev[l], 4 * maxgrid)), dim3(kThreads), 0, s, P, T.lev[l], \
+#define MG_LEVEL(UP, l)                                                                                          \
+    hipLaunchKernelGGL(k_mg_level<UP>, dim3(std::min(T.nlev[l], 4 * maxgrid)), dim3(kThreads), 0, s, P, T.lev[l], \
                        T.nlev[l], l, step)
     if (T.nt1_64)
         hipLaunchKernelGGL(k_mg_upd64, dim3(std::min(T.nt1_64, maxgrid)), dim3(kThreads), 0, s, P, T.t1_64, T.nt1_64,
@@ -1407,16 +1502,10 @@ void launch_mg_step(const ProbDev *P, const MgTables &T, int maxgrid, StepRef st
     MG_FINE(kA1, nullptr);
     MG_FINE(kA2, nullptr);
     for (int l = 1; l < kMgLevels; ++l)
-        if (T.nlev[l]) {
-            MG_LEVEL(kA1, l);
-            MG_LEVEL(kA2, l);
-        }
+        if (T.nlev[l]) MG_LEVEL(false, l);
     hipLaunchKernelGGL(k_mg_bottom, dim3(T.nprobs), dim3(kBotThreads), 0, s, P, T.probs, step);
     for (int l = kMgLevels - 1; l >= 1; --l)
-        if (T.nlev[l]) {
-            MG_LEVEL(kB1, l);
-            MG_LEVEL(kB2, l);
-        }
+        if (T.nlev[l]) MG_LEVEL(true, l);
     MG_FINE(kB1, nullptr);
     MG_FINE(kB2, nullptr);
     if (T.nt3) {
