@@ -322,15 +322,15 @@ __global__ __launch_bounds__(kThreads) void k_cg_a(const ProbDev *__restrict__ P
 // (ps_mg.hip): cg_a with z in the place of r, and the end of the solve where
 // A2 marked step n (r.r at the threshold, or the cap).
 __global__ __launch_bounds__(kThreads) void k_mg_dir64(const ProbDev *__restrict__ P, const TileRef *__restrict__ tab,
-                                                       int ntab, StepRef sref, int *ran)
+                                                       int ntab, MgStep st, int *ran)
 {
     const Run run = my_run(ntab);
-    const int step = sref.base ? *sref.base + sref.off : sref.off;
+    const int step = st.step;
     TotalCache rz_tot;
     for (int t = run.begin; t < run.end; ++t) {
-        const TileRef tr = tab[t];
+        const TileRef tr = st.one >= 0 ? TileRef{st.one, t} : tab[t];
         const ProbDev &pd = P[tr.prob];
-        const gptr<CgScalars> S = glob(pd.S);
+        const gptr<CgScalars> S = glob(st.S + tr.prob);
         const int n = step - pd.n0 + 1;
         const int done_at = S->done_at;
         const bool due = S->next_refresh == n;
@@ -1616,7 +1616,7 @@ void launch_refresh(const ProbDev *P, const TileRef *t1, int nt1, const TileRef 
     hipLaunchKernelGGL(k_refresh_decide, dim3(nprobs), dim3(kThreads), 0, s, P, probs, step);
 }
 
-void launch_mg_dir64(const ProbDev *P, const TileRef *t3, int nt3, int maxgrid, StepRef step, int *ran, hipStream_t s)
+void launch_mg_dir64(const ProbDev *P, const TileRef *t3, int nt3, int maxgrid, const MgStep &step, int *ran, hipStream_t s)
 {
     hipLaunchKernelGGL(k_mg_dir64, dim3(std::min(nt3, maxgrid)), dim3(kThreads), 0, s, P, t3, nt3, step, ran);
 }

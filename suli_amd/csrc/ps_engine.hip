@@ -783,7 +783,7 @@ int Engine::enqueue_steps_direct(int nsteps, bool timing)
             if (rc) return rc;
         }
         if (nmg) {
-            const StepRef sm{nullptr, mstep_, nullptr};
+            const MgStep sm{mstep_, nmg == 1 ? tab_.mg_probs[0] : -1, d_status_};
             launch_mg_step(d_probs_, mgt_, kMaxGrid, sm, ran, s_);
         }
         if (t_close) {

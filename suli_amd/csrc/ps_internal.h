@@ -240,6 +240,15 @@ struct StepRef {
     int *next;
 };
 
+// A multigrid step's launches: the step, the problems' scalars (of problem i
+// at S + i), and the problem where the tables hold only one, else -1.  A short
+// pass waits on its chain of dependent reads: one problem's tile needs no
+// table entry, and its scalars and descriptor are read side by side.
+struct MgStep {
+    int step, one;
+    CgScalars *S;
+};
+
 // Entry of a launch table: tile `tile` of problem `prob`.
 struct TileRef {
     int prob;
@@ -386,10 +395,10 @@ struct MgTables {
     int nprobs = 0;
 };
 // Step step - n0 + 1 (an iteration or a replacement) of every problem in the tables.
-void launch_mg_step(const ProbDev *P, const MgTables &T, int maxgrid, StepRef step, int *ran, hipStream_t s);
+void launch_mg_step(const ProbDev *P, const MgTables &T, int maxgrid, const MgStep &step, int *ran, hipStream_t s);
 // FP64 problems' direction step (ps_cg.hip): beta, e -= alpha p_{n-1}, p_n = z +
 // beta p_{n-1}, q = A p_n, p.q partials; or, when A2 marked step n, the end of the solve.
-void launch_mg_dir64(const ProbDev *P, const TileRef *t3, int nt3, int maxgrid, StepRef step, int *ran,
+void launch_mg_dir64(const ProbDev *P, const TileRef *t3, int nt3, int maxgrid, const MgStep &step, int *ran,
                      hipStream_t s);
 
 // Plain copy of n16 16-byte vectors (measurement only).

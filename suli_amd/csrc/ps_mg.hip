@@ -78,7 +78,10 @@ constexpr int kBotPer = kMgBottomCells / kBotThreads;
 
 enum { kA1 = 0, kA2 = 1, kB1 = 2, kB2 = 3, kDir = 4 };
 
-__device__ __forceinline__ int step_of(StepRef s) { return s.base ? *s.base + s.off : s.off; }
+__device__ __forceinline__ TileRef tile_of(const MgStep &st, const TileRef *tab, int t)
+{
+    return st.one >= 0 ? TileRef{st.one, t} : tab[t];
+}
 
 struct Run {
     int begin, end;
@@ -472,15 +475,15 @@ __device__ __forceinline__ void fold_correction(const ProbDev &pd, int tile, gpt
 // operands need the registers of two.
 template <int KIND>
 __global__ __launch_bounds__(kThreads, (KIND == kA1 || KIND == kDir) ? 2 : 3) void k_mg_fine(
-    const ProbDev *__restrict__ P, const TileRef *__restrict__ tab, int ntab, StepRef sref, int *ran)
+    const ProbDev *__restrict__ P, const TileRef *__restrict__ tab, int ntab, MgStep st, int *ran)
 {
     const Run run = my_run(ntab);
-    const int step = step_of(sref);
+    const int step = st.step;
     TotalCache tot;
     for (int t = run.begin; t < run.end; ++t) {
-        const TileRef tr = tab[t];
+        const TileRef tr = tile_of(st, tab, t);
         const ProbDev &pd = P[tr.prob];
-        const gptr<CgScalars> S = glob(pd.S);
+        const gptr<CgScalars> S = glob(st.S + tr.prob);
         const int n = step - pd.n0 + 1;
         const int done_at = S->done_at, skip_e_at = S->skip_e_at;
         const bool due = KIND != kA1 && KIND != kA2 && S->next_refresh == n;   // set by A2
@@ -569,17 +572,17 @@ __global__ __launch_bounds__(kThreads, (KIND == kA1 || KIND == kDir) ? 2 : 3) vo
 // FP64: r_{n-1} = r_{n-2} - alpha_{n-1} q_{n-1} and its FP32 copy for the
 // V-cycle, r.r partials (1-D tiles).
 __global__ __launch_bounds__(kThreads) void k_mg_upd64(const ProbDev *__restrict__ P, const TileRef *__restrict__ tab,
-                                                       int ntab, StepRef sref)
+                                                       int ntab, MgStep st)
 {
     typedef double vd4 __attribute__((ext_vector_type(4)));
     typedef float va4 __attribute__((ext_vector_type(4)));
     const Run run = my_run(ntab);
-    const int step = step_of(sref);
+    const int step = st.step;
     TotalCache tot;
     for (int t = run.begin; t < run.end; ++t) {
-        const TileRef tr = tab[t];
+        const TileRef tr = tile_of(st, tab, t);
         const ProbDev &pd = P[tr.prob];
-        const gptr<CgScalars> S = glob(pd.S);
+        const gptr<CgScalars> S = glob(st.S + tr.prob);
         const int n = step - pd.n0 + 1;
         if (n < 1 || n > S->done_at) continue;
         const bool first = n == 1;
@@ -624,10 +627,10 @@ __global__ __launch_bounds__(kThreads) void k_mg_upd64(const ProbDev *__restrict
 
 // ---- coarse levels (l >= 1) -------------------------------------------------
 
-__device__ __forceinline__ bool running(const ProbDev &pd, int step)
+__device__ __forceinline__ bool running(const ProbDev &pd, const MgStep &st, int prob)
 {
-    const gptr<const CgScalars> S = glob((const CgScalars *)pd.S);
-    const int n = step - pd.n0 + 1;
+    const gptr<const CgScalars> S = glob((const CgScalars *)st.S + prob);
+    const int n = st.step - pd.n0 + 1;
     return n >= 1 && n <= S->done_at && n != S->next_refresh;
 }
 
@@ -722,15 +725,15 @@ struct Faces {
 // correction.
 template <bool UP>
 __global__ __launch_bounds__(kThreads) void k_mg_level(const ProbDev *__restrict__ P, const TileRef *__restrict__ tab,
-                                                       int ntab, int l, StepRef sref)
+                                                       int ntab, int l, MgStep st)
 {
     __shared__ float va[kHx * kHy * kHz], vb[kHx * kHy * kHz], sh[kThreads];
     const Run run = my_run(ntab);
-    const int step = step_of(sref);
+    const int step = st.step;
     for (int tt = run.begin; tt < run.end; ++tt) {
-        const TileRef tr = tab[tt];
+        const TileRef tr = tile_of(st, tab, tt);
         const ProbDev &pd = P[tr.prob];
-        if (!running(pd, step)) continue;
+        if (!running(pd, st, tr.prob)) continue;
         const MgLevel &L = pd.lv[l], &C = pd.lv[l + 1];
         const Brick B(L, tr.tile);
         const int tid = threadIdx.x;
@@ -900,14 +903,15 @@ __device__ __forceinline__ float bot_nb(const BotDim &d, const BotCell &b, int c
 // symmetric.
 constexpr int kBotWave = 128;
 __global__ __launch_bounds__(kBotThreads) void k_mg_bottom(const ProbDev *__restrict__ P,
-                                                           const int *__restrict__ probs, StepRef sref)
+                                                           const int *__restrict__ probs, MgStep st)
 {
     __shared__ __align__(16) float lds[kMgBottomLds];
     __shared__ int lnx[kMgLevels], lny[kMgLevels], lnz[kMgLevels];
-    const ProbDev &pd = P[probs[blockIdx.x]];
-    if (!running(pd, step_of(sref))) return;
+    const int prob = st.one >= 0 ? st.one : probs[blockIdx.x];
+    const ProbDev &pd = P[prob];
+    if (!running(pd, st, prob)) return;
     const int tid = threadIdx.x, lb = pd.lbot, nl = pd.nlev;
-    const bool project = pd.S->project != 0;
+    const bool project = st.S[prob].project != 0;
     const MgLevel &L0 = pd.lv[lb];
     const int m0 = L0.nx * L0.ny * L0.nz, total = pd.nbot;
     const gptr<const float> pack = glob((const float *)pd.bot);
@@ -1077,11 +1081,12 @@ __global__ __launch_bounds__(kBotThreads) void k_mg_bottom(const ProbDev *__rest
 
 // After k_true_residual: converged, capped, given up, or on.
 __global__ __launch_bounds__(kThreads) void k_mg_decide(const ProbDev *__restrict__ P, const int *__restrict__ probs,
-                                                        StepRef sref)
+                                                        MgStep st)
 {
-    const int step = step_of(sref);
-    const ProbDev &pd = P[probs[blockIdx.x]];
-    CgScalars *S = pd.S;
+    const int step = st.step;
+    const int prob = st.one >= 0 ? st.one : probs[blockIdx.x];
+    const ProbDev &pd = P[prob];
+    CgScalars *S = st.S + prob;
     const int n = step - pd.n0 + 1;
     if (n < 1 || S->final_ || n != S->next_refresh || !pd.mixed) return;
     const double rrt = block_total_of(pd.P.tres, pd.nt3);
@@ -1488,7 +1493,7 @@ void launch_mg_setup(const ProbDev &pd, const ProbDev *dev, const SetupIn &in, h
     hipLaunchKernelGGL(k_mg_coarse_bottom, dim3(1), dim3(kBotThreads), 0, s, dev, pd.lbot + 1, pd.g.dtop, top);
 }
 
-void launch_mg_step(const ProbDev *P, const MgTables &T, int maxgrid, StepRef step, int *ran, hipStream_t s)
+void launch_mg_step(const ProbDev *P, const MgTables &T, int maxgrid, const MgStep &step, int *ran, hipStream_t s)
 {
     const int grid = std::min(T.nfine, maxgrid);
 #define MG_FINE(KIND, RAN) \
@@ -1510,7 +1515,7 @@ void launch_mg_step(const ProbDev *P, const MgTables &T, int maxgrid, StepRef st
     MG_FINE(kB2, nullptr);
     if (T.nt3) {
         MG_FINE(kDir, ran);
-        launch_true_residual(P, T.t3, T.nt3, maxgrid, step, s);
+        launch_true_residual(P, T.t3, T.nt3, maxgrid, StepRef{nullptr, step.step, nullptr}, s);
         hipLaunchKernelGGL(k_mg_decide, dim3(T.nprobs), dim3(kThreads), 0, s, P, T.probs, step);
     }
     if (T.nt3_64) launch_mg_dir64(P, T.t3_64, T.nt3_64, maxgrid, step, ran, s);
