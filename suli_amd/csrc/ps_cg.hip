@@ -365,7 +365,7 @@ __global__ __launch_bounds__(kThreads) void k_mg_dir64(const ProbDev *__restrict
             }
             continue;
         }
-        const gptr<const float> z = glob((const float *)pd.q32b);
+        const gptr<const float> z = glob((const float *)(pd.brick ? pd.r32b : pd.q32b));
         const double acc = with_coefs(V, [&](const auto &co) {
             using CO = std::decay_t<decltype(co)>;
             if (first)

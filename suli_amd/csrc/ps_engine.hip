@@ -108,7 +108,7 @@ bool carve_mg64(Carver &cv, const Geo &g, ProbDev &pd)
     pd.ry32 = cv.take<float>(4 * (size_t)g.nz);
     pd.rz32 = cv.take<float>(4 * ((size_t)g.nz + 1));
     pd.rowreg = cv.take<unsigned>((size_t)(g.ny + 31) / 32 * g.nz);
-    pd.P.m4 = cv.take<double>(3 * (size_t)probe.ntm);
+    if (!probe.brick) pd.P.m4 = cv.take<double>(3 * (size_t)probe.ntm);
     return mg_plan(g, w, space, floats, pd.q32b, pd);
 }
 
@@ -367,7 +367,8 @@ long long mg_entries(const Geo &g)
     const long long nt3 = spmv_tiles(g);
     // mixed solves keep the hierarchy in 2 n floats and three partial sums per
     // fine tile in m4; FP64 ones go by the same rule
-    if (!mg_plan(g, nullptr, nullptr, 2 * (size_t)g.n, nullptr, pd, &floats) || 3 * pd.ntm > 8 * nt3) return 0;
+    if (!mg_plan(g, nullptr, nullptr, 2 * (size_t)g.n, nullptr, pd, &floats) || (!pd.brick && 3 * pd.ntm > 8 * nt3))
+        return 0;
     long long n = pd.ntm;
     for (int l = 1; l < pd.lbot; ++l) n += mg_level_tiles(pd, l);
     return n;
@@ -588,7 +589,8 @@ int Engine::rebuild_tables()
         const Slot &sl = slots_[i];
         if (!sl.active || sl.finished) continue;
         if (sl.mg) {
-            for (int t = 0; t < sl.pd.ntm; ++t) tab_.mg_fine.push_back({i, t});
+            if (!sl.pd.brick)
+                for (int t = 0; t < sl.pd.ntm; ++t) tab_.mg_fine.push_back({i, t});
             auto &t3 = sl.o.mixed ? tab_.mg_t3 : tab_.mg_t3_64;
             for (int t = 0; t < sl.pd.nt3; ++t) t3.push_back({i, t});
             if (!sl.o.mixed)
@@ -619,7 +621,7 @@ int Engine::rebuild_tables()
     off_t1_32 = off_t3_32 + (int)tab_.t3_32.size();
     // multigrid: coarse levels' entries
     int off_lev[kMgLevels] = {};
-    for (int l = 1; l < kMgLevels; ++l) {
+    for (int l = 0; l < kMgLevels; ++l) {
         off_lev[l] = (int)tab_.mg_lev.size();
         for (int i : tab_.mg_probs) {
             const int nt = mg_level_tiles(slots_[i].pd, l);
@@ -682,7 +684,7 @@ int Engine::rebuild_tables()
     mgt_.nt1_64 = (int)tab_.mg_t1_64.size();
     mgt_.probs = d_probs_list_ + tab_.mixed_probs.size();
     mgt_.nprobs = (int)tab_.mg_probs.size();
-    for (int l = 1; l < kMgLevels; ++l) mgt_.lev[l] = d_tab_ + off_mg_lev + off_lev[l];
+    for (int l = 0; l < kMgLevels; ++l) mgt_.lev[l] = d_tab_ + off_mg_lev + off_lev[l];
     if (ntab) ECHK(hipMemcpyAsync(d_tab_, ht, sizeof(TileRef) * ntab, hipMemcpyHostToDevice, s_));
     if (nprobs) ECHK(hipMemcpyAsync(d_probs_list_, hp, sizeof(int) * nprobs, hipMemcpyHostToDevice, s_));
     ECHK(hipEventRecord(ev_stage_[stg], s_));

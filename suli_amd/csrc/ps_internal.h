@@ -58,6 +58,16 @@ constexpr int kMgBottomLds = 38912;    // floats of LDS it has (152 KiB)
 constexpr int kMgCoarsestCells = 64;
 constexpr int kMgCoarsestSide = 8;
 constexpr int kMgCoarsestSweeps = 16;
+// Problems up to this many cells do both matrix products of a half cycle in one
+// launch on the fine level too, in bricks; larger ones march through tiles, which
+// read each value fewer times.  Alone, mixed from prd1 = 0 to 1e-12: 5120 cells
+// 0.94 -> 0.71 ms, 40960 1.10 -> 0.86, 131072 1.28 -> 1.03, 245760 1.37 -> 1.16, 786432
+// 1.92 -> 1.81, 983040 2.21 -> 2.09.  But many together fill the chip either way
+// (64 problems of 92000 cells 12.0 -> 11.8 ms, 128 of them 23.1 -> 24.2), and a batch
+// with problems on both sides of the line holds launches of both kinds: twelve
+// of 32 to 128 cells a side, 4.5 million cells, took 5.93 ms marching, 5.90 with
+// the line here and 6.12 with it at 2^18.
+constexpr long long kMgBrickCells = 1LL << 17;
 constexpr int kMgChunk = 2;            // iterations between host polls
 // Residual replacement: once the FP32 r.r has fallen by kMgCycleDrop since the
 // last one, or to kMgMargin of the threshold, and at the latest after kMgMaxGap
@@ -223,6 +233,7 @@ struct ProbDev {
     // holding r0; the coarse levels are in r, which the
     // set-up has done with by then.
     int mg, mtx, mty, mkz, mlrs, ntm, medge;
+    int brick;              // the fine kernels work on bricks (ntm of them), z_n then in the place of r0
     int nlev, lbot, nbot;   // nbot: cells of levels lbot and coarser
     float *bot;             // those cells' coefficients, packed
     float *w32, *t32;

@@ -86,15 +86,16 @@ __device__ __forceinline__ TileRef tile_of(const MgStep &st, const TileRef *tab,
 struct Run {
     int begin, end;
 };
-__device__ __forceinline__ Run my_run(int ntab)
+__device__ __forceinline__ Run my_run(int ntab, int block, int G)
 {
-    const int G = gridDim.x;
-    const long long L = xcd_tile(blockIdx.x, G);
+    const long long L = xcd_tile(block, G);
     Run r;
     r.begin = (int)(L * ntab / G);
     r.end = (int)((L + 1) * ntab / G);
     return r;
 }
+
+__device__ __forceinline__ Run my_run(int ntab) { return my_run(ntab, blockIdx.x, gridDim.x); }
 
 // Per-workgroup cache of a problem's partial-sum total.
 struct TotalCache {
@@ -471,13 +472,63 @@ __device__ __forceinline__ void fold_correction(const ProbDev &pd, int tile, gpt
     }
 }
 
-// Waves per SIMD: the kinds with one operand fit three, those with two
-// operands need the registers of two.
-template <int KIND>
-__global__ __launch_bounds__(kThreads, (KIND == kA1 || KIND == kDir) ? 2 : 3) void k_mg_fine(
-    const ProbDev *__restrict__ P, const TileRef *__restrict__ tab, int ntab, MgStep st, int *ran)
+// The total r.r entering iteration n is known: whether the step ends otherwise
+// (S->next_refresh = n, stored by one thread).  Mixed: a replacement instead of
+// iteration n once r.r (the FP32 recurrence's) has reached the threshold, or
+// fallen as far as FP32 carries one cycle, or at the cap; FP64: the end.
+__device__ __forceinline__ bool judge(gptr<CgScalars> S, bool mixed, bool fresh, int n, double rr, bool store)
 {
-    const Run run = my_run(ntab);
+    const double thresh = S->thresh, base = S->refreshes ? S->rr_after : S->rr0;
+    const int iters = S->iters, max_iter = S->max_iter;
+    int prev = S->prev_iters;
+    bool due;
+    if (!mixed) {
+        const bool below = n > 1 && rr <= thresh;
+        if (below && prev == 0) {
+            prev = n;
+            if (store) S->prev_iters = n;
+        }
+        due = n > 1 && (rr <= kMgMargin * thresh || iters >= max_iter || (below && n - prev >= kMgMarginIters));
+    } else {
+        due = !fresh && (rr <= kMgMargin * thresh || rr <= kMgCycleDrop * base || iters - prev >= kMgMaxGap ||
+                         iters >= max_iter);
+    }
+    if (store) {
+        S->rr[n & 1] = rr;
+        if (due) S->next_refresh = n;
+    }
+    return due;
+}
+
+// alpha and beta of a mixed problem's direction step; false at a breakdown:
+// r.z and p.q are positive for every operator the V-cycle is definite for,
+// unless a value left FP32's range.  A replacement starts the directions
+// afresh: the replaced residual is no longer r - alpha q, and directions
+// conjugate to it went on at a third of the rate.
+__device__ __forceinline__ bool direction(gptr<CgScalars> S, bool fresh, bool due, int n, double rz, bool store,
+                                          double &alpha, double &beta)
+{
+    const double rz_prev = S->rz[(n - 1) & 1];
+    alpha = S->alpha;
+    const bool bad = !(rz >= 0.0 && rz < 1e300) || !(alpha >= 0.0 && alpha < 1e300);
+    beta = fresh || !(rz_prev > 0.0) ? 0.0 : rz / rz_prev;
+    if (store) {
+        if (bad) {
+            S->giveup = 1;
+            S->final_ = 1;
+            S->done_at = n;
+        } else if (!due) {
+            S->rz[n & 1] = rz;
+            S->iters = S->iters + 1;
+        }
+    }
+    return !bad;
+}
+
+template <int KIND>
+__device__ __forceinline__ void fine_tiles(const ProbDev *__restrict__ P, const TileRef *__restrict__ tab, Run run,
+                                           const MgStep &st, int *ran)
+{
     const int step = st.step;
     TotalCache tot;
     for (int t = run.begin; t < run.end; ++t) {
@@ -507,24 +558,8 @@ __global__ __launch_bounds__(kThreads, (KIND == kA1 || KIND == kDir) ? 2 : 3) vo
             F = FineArgs{fresh ? r : r0, mixed ? q : r, nullptr, nullptr, r, tt, nullptr, fresh, false, (float)alpha, 0.f};
         } else if (KIND == kA2) {
             if (tr.tile == 0) {
-                // mixed: a replacement instead of iteration n once r.r (the
-                // FP32 recurrence's) has reached the threshold, or fallen as
-                // far as FP32 carries one cycle, or at the cap; FP64: the end
                 const double rr = mixed ? block_total_of(part_rr(pd), pd.ntm) : block_total_of(pd.P.upd, pd.nt1);
-                if (threadIdx.x == 0) {
-                    S->rr[n & 1] = rr;
-                    const double base = S->refreshes ? S->rr_after : S->rr0;
-                    const int iters = S->iters;
-                    if (!mixed) {
-                        if (n > 1 && rr <= S->thresh && S->prev_iters == 0) S->prev_iters = n;
-                        if (n > 1 && (rr <= kMgMargin * S->thresh || iters >= S->max_iter ||
-                                      (rr <= S->thresh && n - S->prev_iters >= kMgMarginIters)))
-                            S->next_refresh = n;
-                    } else if (!fresh && (rr <= kMgMargin * S->thresh || rr <= kMgCycleDrop * base ||
-                                          iters - S->prev_iters >= kMgMaxGap || iters >= S->max_iter)) {
-                        S->next_refresh = n;
-                    }
-                }
+                judge(S, mixed, fresh, n, rr, threadIdx.x == 0);
             }
             F = FineArgs{tt, nullptr, r, nullptr, rho, nullptr, nullptr, false, false, 0.f, 0.f};
         } else if (KIND == kB1) {
@@ -532,27 +567,10 @@ __global__ __launch_bounds__(kThreads, (KIND == kA1 || KIND == kDir) ? 2 : 3) vo
         } else if (KIND == kB2) {
             F = FineArgs{r0, nullptr, r, tt, z, nullptr, nullptr, false, false, 0.f, 0.f};
         } else {
-            const double rz_prev = S->rz[(n - 1) & 1], alpha = S->alpha;
             const double rz = due ? 0.0 : tot.get(tr.prob, part_rz(pd), pd.ntm);
-            // a breakdown: r.z and p.q are positive for every operator the
-            // V-cycle is definite for, unless a value left FP32's range
-            const bool bad = !(rz >= 0.0 && rz < 1e300) || !(alpha >= 0.0 && alpha < 1e300);
-            // a replacement starts the directions afresh: the replaced residual
-            // is no longer r - alpha q, and directions conjugate to it went
-            // on at a third of the rate
-            const double beta = fresh || !(rz_prev > 0.0) ? 0.0 : rz / rz_prev;
-            if (tr.tile == 0 && threadIdx.x == 0) {
-                if (bad) {
-                    S->giveup = 1;
-                    S->final_ = 1;
-                    S->done_at = n;
-                } else if (!due) {
-                    S->rz[n & 1] = rz;
-                    S->iters = S->iters + 1;
-                    if (ran && tr.prob == 0) *ran = 1;
-                }
-            }
-            if (bad) continue;
+            double alpha, beta;
+            if (!direction(S, fresh, due, n, rz, tr.tile == 0 && threadIdx.x == 0, alpha, beta)) continue;
+            if (ran && !due && tr.tile == 0 && threadIdx.x == 0 && tr.prob == 0) *ran = 1;
             const gptr<float> po = glob(mpbuf(pd, n - 1));
             const gptr<float> x = glob(pd.c32);
             if (due) {
@@ -567,6 +585,17 @@ __global__ __launch_bounds__(kThreads, (KIND == kA1 || KIND == kDir) ? 2 : 3) vo
         const double sres = block_sum(acc);
         if (threadIdx.x == 0) (KIND == kA1 ? part_rr(pd) : KIND == kB2 ? part_rz(pd) : part_pq(pd))[tr.tile] = sres;
     }
+}
+
+// Waves per SIMD: the kinds with one operand fit three, those with two
+// operands need the registers of two.
+constexpr int fine_waves(int kind) { return kind == kA1 || kind == kDir ? 2 : 3; }
+template <int KIND>
+__global__ __launch_bounds__(kThreads, fine_waves(KIND)) void k_mg_fine(const ProbDev *__restrict__ P,
+                                                                        const TileRef *__restrict__ tab, int ntab,
+                                                                        MgStep st, int *ran)
+{
+    fine_tiles<KIND>(P, tab, my_run(ntab), st, ran);
 }
 
 // FP64: r_{n-1} = r_{n-2} - alpha_{n-1} q_{n-1} and its FP32 copy for the
@@ -634,29 +663,50 @@ __device__ __forceinline__ bool running(const ProbDev &pd, const MgStep &st, int
     return n >= 1 && n <= S->done_at && n != S->next_refresh;
 }
 
-// Bricks of 16 x 4 x 4 cells, one workgroup each and one cell per thread: a
-// brick holds whole coarse cells.  With two cells around, a brick's vectors are
-// in LDS, and both matrix products of a half of the cycle are done there: the
-// first on the brick and its 288 face neighbours, the second on the brick.  These
-// passes wait on their launch and on memory's latency, not its rate: the two
-// products as launches of their own took 4.9 us each over 128x64x48 cells and 4.0
-// over 64x32x24, together they take 8.5 to 9.1 and 5.4 to 6.6 (a 64x64x32 solve
-// 1.20 -> 1.14 ms, 256x128x96 3.52 -> 3.44, 384x192x128 11.33 -> 11.09).
-constexpr int kBx = 16, kBy = 4, kBz = 4;
-constexpr int kHx = kBx + 4, kHy = kBy + 4, kHz = kBz + 4;   // with halo
-constexpr int kShell = 2 * (kBx * kBy + kBx * kBz + kBy * kBz);
-static_assert(kBx * kBy * kBz == kThreads && kHx * kHy * kHz % kThreads == 0 && kBx * kBy == 64 && kBx * kBz == 64,
-              "brick");
+// Bricks of 16x8x8 cells, one workgroup each; a brick holds whole coarse cells.
+// With two cells around, a brick's vectors are in LDS, and both matrix products
+// of a half of the cycle are done there: the first on the brick and its face
+// neighbours, the second on the brick.  A thread loads one column of the box and
+// owns kOwn cells in z, so that a cell's place is worked out once for its column.
+//
+// On the coarse levels and on small grids a pass waits on its launch and on
+// memory's latency, not its rate, so two products a launch pay: on the coarse
+// levels two launches took 4.9 us each over 128x64x48 cells and 4.0 over
+// 64x32x24, one takes 8.5 to 9.1 and 5.4 to 6.6 (a 64x64x32 solve 1.20 -> 1.14 ms,
+// 256x128x96 3.52 -> 3.44, 384x192x128 11.33 -> 11.09).
+//
+// The brick's shape weighs latency (more, smaller bricks) against the halo: 16x4x4
+// took 0.72 ms for a 32x24x20 solve and 28.4 ms for 128 problems of 40 to 50 cells
+// a side, 16x8x4 0.75 and 26.2, 16x8x8 0.78 and 24.2 (marched tiles on the fine
+// level: 1.00 and 23.1).
+constexpr int kBx = 16, kBy = 8, kBz = 8;
+constexpr int kHx = kBx + 4, kHy = kBy + 4, kHz = kBz + 4;   // the box
+constexpr int kOwn = kBx * kBy * kBz / kThreads;
+constexpr int kCols = kBx * kBy;
+static_assert(kThreads % kCols == 0 && kOwn * (kThreads / kCols) == kBz && kHx * kHy <= kThreads && kOwn > 0, "brick");
 __host__ __device__ inline int bricks(const MgLevel &L)
 {
     return ((L.nx + kBx - 1) / kBx) * ((L.ny + kBy - 1) / kBy) * ((L.nz + kBz - 1) / kBz);
 }
 
+// A box column's or plane's place in the grid: wrapped around periodic sides;
+// beyond a wall it is the mirror image inside (the coarse levels' faces there
+// are 0), at box position + shift, and above the top its values count sg times
+// (the p = 0 lid: -1).
+struct Col {
+    int i, j, shift;
+};
+struct Plane {
+    int k, shift;
+    float sg;
+};
 struct Brick {
-    int x0, y0, z0;      // cell (0, 0, 0) of the halo box
+    int x0, y0, z0;      // cell (0, 0, 0) of the box
     int nx, ny, nz;
     bool px, py;
-    __device__ __forceinline__ Brick(const MgLevel &L, int tile) : nx(L.nx), ny(L.ny), nz(L.nz), px(L.px), py(L.py)
+    float top;
+    __device__ __forceinline__ Brick(const MgLevel &L, int tile, float lid)
+        : nx(L.nx), ny(L.ny), nz(L.nz), px(L.px), py(L.py), top(lid)
     {
         const int bx = (nx + kBx - 1) / kBx, by = (ny + kBy - 1) / kBy;
         const int rest = tile / bx;
@@ -664,44 +714,33 @@ struct Brick {
         y0 = (rest % by) * kBy - 2;
         z0 = (rest / by) * kBz - 2;
     }
-    // The grid cell at box position (a, b, d), wrapped around periodic sides;
-    // false where there is none.
-    __device__ __forceinline__ bool cell(int a, int b, int d, int &i, int &j, int &k) const
+    __device__ __forceinline__ Col col(int a, int b) const
     {
-        i = x0 + a;
-        j = y0 + b;
-        k = z0 + d;
+        int i = x0 + a, j = y0 + b;
         if (px) i += i < 0 ? nx : i >= nx ? -nx : 0;
         if (py) j += j < 0 ? ny : j >= ny ? -ny : 0;
-        return (unsigned)i < (unsigned)nx && (unsigned)j < (unsigned)ny && (unsigned)k < (unsigned)nz;
+        Col c;
+        c.i = min(max(i, 0), nx - 1);
+        c.j = min(max(j, 0), ny - 1);
+        c.shift = (c.i - i) + (c.j - j) * kHx;
+        return c;
     }
-    __device__ __forceinline__ int index(int i, int j, int k) const { return (k * ny + j) * nx + i; }
-    static __device__ __forceinline__ int box(int a, int b, int d) { return (d * kHy + b) * kHx + a; }
+    __device__ __forceinline__ Plane plane(int d) const
+    {
+        const int k = z0 + d;
+        Plane p;
+        p.k = min(max(k, 0), nz - 1);
+        p.shift = (p.k - k) * (kHx * kHy);
+        p.sg = k >= nz ? top : 1.f;
+        return p;
+    }
+    __device__ __forceinline__ int index(const Col &c, const Plane &p) const { return (p.k * ny + c.j) * nx + c.i; }
+    static __device__ __forceinline__ int pos(int a, int b, int d) { return (d * kHy + b) * kHx + a; }
 };
-// Box position of shell cell h: below, above, south, north, west, east.
-__device__ __forceinline__ void shell_cell(int h, int &a, int &b, int &d)
-{
-    const int u = h & 63;
-    if (h < 128) {
-        a = 2 + (u & 15);
-        b = 2 + (u >> 4);
-        d = h < 64 ? 1 : 2 + kBz;
-    } else if (h < 256) {
-        a = 2 + (u & 15);
-        b = h < 192 ? 1 : 2 + kBy;
-        d = 2 + (u >> 4);
-    } else {
-        a = h < 272 ? 1 : 2 + kBx;
-        b = 2 + (u & 3);
-        d = 2 + ((u >> 2) & 3);
-    }
-}
 struct Faces {
     float e, w, n, s, t, b;
-    __device__ __forceinline__ void load(const MgLevel &L, bool ok, int c, int j, int k)
+    __device__ __forceinline__ void load(const MgLevel &L, int c, int j, int k)
     {
-        e = w = n = s = t = b = 0.f;
-        if (!ok) return;
         const gptr<const float> sx = glob((const float *)L.sx) + (c + (k * L.ny + j));
         const gptr<const float> sy = glob((const float *)L.sy) + (c + k * L.nx);
         const gptr<const float> sz = glob((const float *)L.sz) + c;
@@ -712,13 +751,142 @@ struct Faces {
         t = sz[L.nx * L.ny];
         b = sz[0];
     }
-    // the six neighbours' share of A v at box cell x
+    // the six neighbours' share of A v at box position x
     __device__ __forceinline__ float sum(const float *v, int x) const
     {
         return e * v[x + 1] + w * v[x - 1] + n * v[x + kHx] + s * v[x - kHx] + t * v[x + kHx * kHy] +
                b * v[x - kHx * kHy];
     }
 };
+// f(box position (a, b, d)) for the brick's face neighbours, below and above,
+// south and north, west and east
+template <class F>
+__device__ __forceinline__ void each_shell(F &&f)
+{
+    const int tid = threadIdx.x;
+#pragma unroll
+    for (int h = 0; h < 2 * kCols; h += kThreads) {
+        const int u = h + tid;
+        if (2 * kCols % kThreads == 0 || u < 2 * kCols)
+            f(2 + (u & 15), 2 + (u >> 4) % kBy, u < kCols ? 1 : 2 + kBz);
+    }
+#pragma unroll
+    for (int h = 0; h < 2 * kBx * kBz; h += kThreads) {
+        const int u = h + tid;
+        if (2 * kBx * kBz % kThreads == 0 || u < 2 * kBx * kBz)
+            f(2 + (u & 15), u < kBx * kBz ? 1 : 2 + kBy, 2 + (u >> 4) % kBz);
+    }
+    if (tid < 2 * kBy * kBz) f(tid < kBy * kBz ? 1 : 2 + kBx, 2 + tid % kBy, 2 + tid / kBy % kBz);
+}
+// The thread's own cells of a brick: (a, b, d + q), q < kOwn.
+struct Own {
+    int a, b, d;
+    Col col;
+    Plane pl[kOwn];
+    int c[kOwn];
+    bool in[kOwn];   // a cell of the grid, and this brick's
+    __device__ __forceinline__ explicit Own(const Brick &B)
+    {
+        const int tid = threadIdx.x;
+        a = 2 + (tid & 15);
+        b = 2 + (tid >> 4) % kBy;
+        d = 2 + tid / kCols * kOwn;
+        col = B.col(a, b);
+        const bool inc = B.x0 + a < B.nx && B.y0 + b < B.ny;
+#pragma unroll
+        for (int q = 0; q < kOwn; ++q) {
+            pl[q] = B.plane(d + q);
+            c[q] = B.index(col, pl[q]);
+            in[q] = inc && B.z0 + d + q < B.nz;
+        }
+    }
+    __device__ __forceinline__ int pos(int q) const { return Brick::pos(a, b, d + q); }
+};
+// The thread's column of the box.
+struct BoxCol {
+    bool any;
+    int pos;
+    Col col;
+    __device__ __forceinline__ explicit BoxCol(const Brick &B)
+    {
+        const int tid = threadIdx.x;
+        any = tid < kHx * kHy;
+        pos = tid;
+        col = B.col(tid % kHx, any ? tid / kHx : 0);
+    }
+};
+
+struct HalfBox {
+    float va[kHx * kHy * kHz], vb[kHx * kHy * kHz];
+};
+// Both products of a half cycle, from the box column's values v0:
+//   down  v = r:    u = A v,        y = A u
+//   up    v = w e:  u = rho - A v,  y = A u
+template <bool UP>
+__device__ __forceinline__ void half_cycle(const MgLevel &L, const Brick &B, const Own &o, const BoxCol &bc,
+                                           HalfBox &s, const float (&v0)[kHz], gptr<const float> rho,
+                                           float (&v)[kOwn], float (&u)[kOwn], float (&y)[kOwn])
+{
+    Faces f0[kOwn];
+    float rho0[kOwn];
+#pragma unroll
+    for (int q = 0; q < kOwn; ++q) {
+        f0[q].load(L, o.c[q], o.col.j, o.pl[q].k);
+        rho0[q] = UP ? rho[o.c[q]] : 0.f;
+    }
+    __syncthreads();   // reads of the last tile
+    if (bc.any) {
+#pragma unroll
+        for (int d = 0; d < kHz; ++d) s.va[bc.pos + d * kHx * kHy] = v0[d];
+    }
+    __syncthreads();
+    // u at a box cell: its mirror image's, times sg
+    auto first = [&](const Faces &f, int x, float sg, float rh) {
+        const float av = s.va[x] - f.sum(s.va, x);
+        return sg * (UP ? rh - av : av);
+    };
+#pragma unroll
+    for (int q = 0; q < kOwn; ++q) {
+        const int x = o.pos(q);
+        v[q] = s.va[x];
+        u[q] = first(f0[q], x + o.col.shift + o.pl[q].shift, o.pl[q].sg, rho0[q]);
+        s.vb[x] = u[q];
+    }
+    each_shell([&](int a, int b, int d) {
+        const Col col = B.col(a, b);
+        const Plane p = B.plane(d);
+        const int c = B.index(col, p), x = Brick::pos(a, b, d);
+        Faces f;
+        f.load(L, c, col.j, p.k);
+        s.vb[x] = first(f, x + col.shift + p.shift, p.sg, UP ? rho[c] : 0.f);
+    });
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kOwn; ++q) y[q] = u[q] - f0[q].sum(s.vb, o.pos(q));
+}
+
+// The brick's coarse cells: the restricted residual, scaled, from w rho at the
+// own cells.  (va is read no more.)
+__device__ __forceinline__ void restrict_brick(const MgLevel &C, const Brick &B, const Own &o, float *va,
+                                               const float (&wr)[kOwn])
+{
+    const int tid = threadIdx.x;
+#pragma unroll
+    for (int q = 0; q < kOwn; ++q) va[o.pos(q)] = wr[q];
+    __syncthreads();
+    if (tid < kOwn * kThreads / 8) {
+        const int I = tid % (kBx / 2), J = tid / (kBx / 2) % (kBy / 2), K = tid / (kBx / 2 * kBy / 2);
+        const float *x = va + Brick::pos(2 + 2 * I, 2 + 2 * J, 2 + 2 * K);
+        const float *z = x + kHx * kHy;
+        const float sum = ((x[0] + x[1]) + (x[kHx] + x[kHx + 1])) + ((z[0] + z[1]) + (z[kHx] + z[kHx + 1]));
+        const int ic = (B.x0 + 2) / 2 + I, jc = (B.y0 + 2) / 2 + J, kc = (B.z0 + 2) / 2 + K;
+        if (ic < C.nx && jc < C.ny && kc < C.nz) {
+            const int c = (kc * C.ny + jc) * C.nx + ic;
+            const float wc = C.w[c];
+            glob(C.r)[c] = wc > 0.f ? sum / wc : 0.f;
+        }
+    }
+}
 
 // Half a cycle on level l (1 <= l < lbot): down (A1 and A2 of the fine
 // kernels) or up (B1 and B2); no partial sums, and up leaves the un-scaled
@@ -727,96 +895,219 @@ template <bool UP>
 __global__ __launch_bounds__(kThreads) void k_mg_level(const ProbDev *__restrict__ P, const TileRef *__restrict__ tab,
                                                        int ntab, int l, MgStep st)
 {
-    __shared__ float va[kHx * kHy * kHz], vb[kHx * kHy * kHz], sh[kThreads];
+    __shared__ HalfBox box;
     const Run run = my_run(ntab);
-    const int step = st.step;
     for (int tt = run.begin; tt < run.end; ++tt) {
         const TileRef tr = tile_of(st, tab, tt);
         const ProbDev &pd = P[tr.prob];
         if (!running(pd, st, tr.prob)) continue;
         const MgLevel &L = pd.lv[l], &C = pd.lv[l + 1];
-        const Brick B(L, tr.tile);
-        const int tid = threadIdx.x;
+        const Brick B(L, tr.tile, 1.f);
+        const Own o(B);
+        const BoxCol bc(B);
         const gptr<float> t = glob(L.t), rho = glob(L.rho);
         const gptr<const float> r = glob((const float *)L.r), w = glob((const float *)L.w),
                                 e = glob((const float *)C.t);
-        const int Cx = C.nx, Cy = C.ny;
-        auto parent = [&](int i, int j, int k) { return ((k >> 1) * Cy + (j >> 1)) * Cx + (i >> 1); };
-        // the thread's own cell and its shell cell
-        const int a0 = 2 + (tid & 15), b0 = 2 + ((tid >> 4) & 3), d0 = 2 + (tid >> 6);
-        int i, j, k;
-        const bool ok = B.cell(a0, b0, d0, i, j, k);
-        const bool in = ok && i == B.x0 + a0 && j == B.y0 + b0;   // not around a periodic side
-        const int c = B.index(i, j, k), x0 = Brick::box(a0, b0, d0);
-        Faces f0;
-        f0.load(L, ok, c, j, k);
-        float va0[kHx * kHy * kHz / kThreads];
+        float v0[kHz], wc[kOwn], rc[kOwn], tc[kOwn];
 #pragma unroll
-        for (int q = 0; q < kHx * kHy * kHz / kThreads; ++q) {
-            const int h = tid + q * kThreads, a = h % kHx, b = h / kHx % kHy, d = h / (kHx * kHy);
-            int ii, jj, kk;
-            va0[q] = 0.f;
-            if (B.cell(a, b, d, ii, jj, kk)) {
-                const int x = B.index(ii, jj, kk);
-                va0[q] = UP ? w[x] * e[parent(ii, jj, kk)] : r[x];
-            }
+        for (int d = 0; d < kHz; ++d) {
+            const Plane p = B.plane(d);
+            const int c = B.index(bc.col, p);
+            v0[d] = UP ? w[c] * e[((p.k >> 1) * C.ny + (bc.col.j >> 1)) * C.nx + (bc.col.i >> 1)] : r[c];
         }
-        float rho0 = 0.f, r_c = 0.f, t_c = 0.f, w_c = 0.f;
-        if (ok) w_c = w[c];
-        if (UP && ok) {
-            rho0 = rho[c];
-            r_c = r[c];
-            t_c = t[c];
-        }
-        __syncthreads();   // the last tile's reads of va
 #pragma unroll
-        for (int q = 0; q < kHx * kHy * kHz / kThreads; ++q) va[tid + q * kThreads] = va0[q];
-        __syncthreads();
-        const float own = va[x0];
-        const float u0 = UP ? rho0 - own + f0.sum(va, x0) : own - f0.sum(va, x0);
-        vb[x0] = u0;
-        for (int h = tid; h < kShell; h += kThreads) {
-            int a, b, d, ii, jj, kk;
-            shell_cell(h, a, b, d);
-            float u = 0.f;
-            const int x = Brick::box(a, b, d);
-            if (B.cell(a, b, d, ii, jj, kk)) {
-                const int cc = B.index(ii, jj, kk);
-                Faces f;
-                f.load(L, true, cc, jj, kk);
-                u = UP ? rho[cc] - va[x] + f.sum(va, x) : va[x] - f.sum(va, x);
-            }
-            vb[x] = u;
+        for (int q = 0; q < kOwn; ++q) {
+            wc[q] = w[o.c[q]];
+            rc[q] = UP ? r[o.c[q]] : 0.f;
+            tc[q] = UP ? t[o.c[q]] : 0.f;
         }
-        __syncthreads();
-        const float y = u0 - f0.sum(vb, x0);
-        if (UP) {
-            if (in) {
-                const float z = kC0 * (r_c + u0) + kC1 * (t_c + y) + own;
-                t[c] = w_c > 0.f ? z / w_c : 0.f;
+        float v[kOwn], u[kOwn], y[kOwn];
+        half_cycle<UP>(L, B, o, bc, box, v0, rho, v, u, y);
+#pragma unroll
+        for (int q = 0; q < kOwn; ++q) {
+            const int c = o.c[q];
+            if (UP) {
+                const float z = kC0 * (rc[q] + u[q]) + kC1 * (tc[q] + y[q]) + v[q];
+                if (o.in[q]) t[c] = wc[q] > 0.f ? z / wc[q] : 0.f;
+            } else {
+                const float rh = v[q] - kC0 * u[q] - kC1 * y[q];
+                if (o.in[q]) {
+                    t[c] = u[q];
+                    rho[c] = rh;
+                }
+                wc[q] = o.in[q] ? wc[q] * rh : 0.f;
             }
-        } else {
-            const float rh = own - kC0 * u0 - kC1 * y;
-            if (in) {
-                t[c] = u0;
-                rho[c] = rh;
+        }
+        if (!UP) restrict_brick(C, B, o, box.va, wc);
+    }
+}
+
+// The fine level of a problem with pd.brick set, the same way.
+//   down  A1 and A2 (r_{n-1}, t, rho, the restriction; partials r.r)
+//   up    B1 and B2 (z in the place of r0; partials r.z)
+//   dir   as in k_mg_fine
+// r.r is judged by the bottom kernel.
+enum { kDown = 0, kUp = 1, kDirB = 2 };
+template <int KIND>
+__device__ __forceinline__ void brick_tiles(const ProbDev *__restrict__ P, const TileRef *__restrict__ tab, Run run,
+                                            const MgStep &st, int *ran)
+{
+    __shared__ HalfBox box;
+    const int step = st.step;
+    TotalCache tot;
+    for (int tt = run.begin; tt < run.end; ++tt) {
+        const TileRef tr = tile_of(st, tab, tt);
+        const ProbDev &pd = P[tr.prob];
+        const gptr<CgScalars> S = glob(st.S + tr.prob);
+        const int n = step - pd.n0 + 1;
+        const int done_at = S->done_at, skip_e_at = S->skip_e_at;
+        const bool due = KIND != kDown && S->next_refresh == n;   // set by the bottom kernel
+        if (n < 1 || n > done_at || (due && KIND != kDirB)) continue;
+        const bool mixed = pd.mixed != 0;
+        if (KIND == kDirB && !mixed) continue;
+        const bool fresh = n == 1 || step == skip_e_at || !mixed;
+        const bool lead = tr.tile == 0 && threadIdx.x == 0;
+        const MgLevel &L = pd.lv[0], &C = pd.lv[1];
+        const Brick B(L, tr.tile, pd.g.dtop ? -1.f : 1.f);
+        const Own o(B);
+        const gptr<float> r = glob(mixed ? rbuf(pd, n - 1) : pd.r32), r0 = glob(mixed ? rbuf(pd, n) : pd.r32b);
+        const gptr<float> t = glob(pd.t32), rho = glob(pd.q32b), z = r0, qv = glob(pd.q32);
+        const gptr<const float> w = glob((const float *)pd.w32);
+        double acc = 0.0;
+        float v[kOwn], u[kOwn], y[kOwn];
+        if (KIND == kDown) {
+            const BoxCol bc(B);
+            // the second operand is loaded whether used or not
+            const gptr<const float> a_ = fresh ? r : r0, b_ = mixed ? qv : r;
+            float v0[kHz], b0[kHz], wc[kOwn];
+#pragma unroll
+            for (int d = 0; d < kHz; ++d) {
+                const int c = B.index(bc.col, B.plane(d));
+                v0[d] = a_[c];
+                b0[d] = b_[c];
             }
-            sh[tid] = in ? w_c * rh : 0.f;
-            __syncthreads();
-            if (tid < kThreads / 8) {
-                const int I = tid & 7, J = (tid >> 3) & 1, K = tid >> 4;
-                const int b = (2 * K) * 64 + (2 * J) * 16 + 2 * I;
-                const float sum = ((sh[b] + sh[b + 1]) + (sh[b + 16] + sh[b + 17])) +
-                                  ((sh[b + 64] + sh[b + 65]) + (sh[b + 80] + sh[b + 81]));
-                const int ic = (B.x0 + 2) / 2 + I, jc = (B.y0 + 2) / 2 + J, kc = (B.z0 + 2) / 2 + K;
-                if (ic < C.nx && jc < C.ny && kc < C.nz) {
-                    const int x = (kc * C.ny + jc) * C.nx + ic;
-                    const float wc = C.w[x];
-                    glob(C.r)[x] = wc > 0.f ? sum / wc : 0.f;
+#pragma unroll
+            for (int q = 0; q < kOwn; ++q) wc[q] = w[o.c[q]];
+            double alpha = 0.0;
+            if (mixed) {
+                const double rz = S->rz[(n - 1) & 1];
+                const double pq = tot.get(tr.prob, part_pq(pd), pd.ntm);
+                alpha = fresh || !(pq != 0.0) ? 0.0 : rz / pq;   // 0 / 0 once the residual is 0
+                if (lead) S->alpha = alpha;
+            }
+#pragma unroll
+            for (int d = 0; d < kHz; ++d) v0[d] = B.plane(d).sg * (fresh ? v0[d] : v0[d] - (float)alpha * b0[d]);
+            half_cycle<false>(L, B, o, bc, box, v0, nullptr, v, u, y);
+#pragma unroll
+            for (int q = 0; q < kOwn; ++q) {
+                const int c = o.c[q];
+                const float rh = v[q] - kC0 * u[q] - kC1 * y[q];
+                if (o.in[q]) {
+                    if (!fresh) r[c] = v[q];
+                    t[c] = u[q];
+                    rho[c] = rh;
+                    acc += (double)v[q] * (double)v[q];
+                }
+                wc[q] = o.in[q] ? wc[q] * rh : 0.f;
+            }
+            restrict_brick(C, B, o, box.va, wc);
+        } else if (KIND == kUp) {
+            const BoxCol bc(B);
+            const gptr<const float> e = glob((const float *)C.t);
+            float v0[kHz], rc[kOwn], tc[kOwn];
+#pragma unroll
+            for (int d = 0; d < kHz; ++d) {
+                const Plane p = B.plane(d);
+                v0[d] = p.sg * (w[B.index(bc.col, p)] *
+                                e[((p.k >> 1) * C.ny + (bc.col.j >> 1)) * C.nx + (bc.col.i >> 1)]);
+            }
+#pragma unroll
+            for (int q = 0; q < kOwn; ++q) {
+                rc[q] = r[o.c[q]];
+                tc[q] = t[o.c[q]];
+            }
+            half_cycle<true>(L, B, o, bc, box, v0, rho, v, u, y);
+#pragma unroll
+            for (int q = 0; q < kOwn; ++q) {
+                const float zc = kC0 * (rc[q] + u[q]) + kC1 * (tc[q] + y[q]) + v[q];
+                if (o.in[q]) {
+                    z[o.c[q]] = zc;
+                    acc += (double)rc[q] * (double)zc;
                 }
             }
+        } else {
+            const gptr<const float> po = glob(mpbuf(pd, n - 1));
+            const gptr<float> x = glob(pd.c32);
+            float zc[kOwn], pc[kOwn], xc[kOwn];
+            Faces f[kOwn];
+#pragma unroll
+            for (int q = 0; q < kOwn; ++q) {
+                const int c = o.c[q];
+                zc[q] = z[c];
+                pc[q] = po[c];
+                xc[q] = x[c];
+                f[q].load(L, c, o.col.j, o.pl[q].k);
+            }
+            const double rz = due ? 0.0 : tot.get(tr.prob, part_rz(pd), pd.ntm);
+            double alpha, beta;
+            if (!direction(S, fresh, due, n, rz, lead, alpha, beta)) continue;
+            if (ran && !due && lead && tr.prob == 0) *ran = 1;
+            if (due) {
+                // e += c - alpha_{n-1} p_{n-1}, c = 0
+                fold_correction(pd, tr.tile, x, po, (float)alpha);
+                continue;
+            }
+            auto p_of = [&](float zv, float pv) { return fresh ? zv : zv + (float)beta * pv; };
+            __syncthreads();   // reads of the last tile
+            each_shell([&](int a, int b, int d) {
+                const Plane p = B.plane(d);
+                const int c = B.index(B.col(a, b), p);
+                box.va[Brick::pos(a, b, d)] = p.sg * p_of(z[c], po[c]);
+            });
+            // (beyond the grid, the own cells' places hold mirror images too)
+#pragma unroll
+            for (int q = 0; q < kOwn; ++q) {
+                v[q] = p_of(zc[q], pc[q]);
+                box.va[o.pos(q)] = o.pl[q].sg * v[q];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < kOwn; ++q)
+                if (o.in[q]) {
+                    const int c = o.c[q];
+                    const float av = v[q] - f[q].sum(box.va, o.pos(q));
+                    glob(mpbuf(pd, n))[c] = v[q];
+                    qv[c] = av;
+                    if (!fresh) x[c] = xc[q] - (float)alpha * pc[q];
+                    acc += (double)v[q] * (double)av;
+                }
         }
+        if (KIND == kDown && !mixed) continue;
+        const double sres = block_sum(acc);
+        if (threadIdx.x == 0) (KIND == kDown ? part_rr(pd) : KIND == kUp ? part_rz(pd) : part_pq(pd))[tr.tile] = sres;
     }
+}
+
+template <int KIND>
+__global__ __launch_bounds__(kThreads) void k_mg_brick(const ProbDev *__restrict__ P, const TileRef *__restrict__ tab,
+                                                       int ntab, MgStep st, int *ran)
+{
+    brick_tiles<KIND>(P, tab, my_run(ntab), st, ran);
+}
+
+// Both kinds of problems in the tables: the first gb workgroups take the
+// bricks, the others the marched tiles, in one launch.
+template <int KIND, int BRICK>
+__global__ __launch_bounds__(kThreads, fine_waves(KIND)) void k_mg_both(const ProbDev *__restrict__ P,
+                                                                        const TileRef *__restrict__ fine, int nfine,
+                                                                        int gb, const TileRef *__restrict__ brick,
+                                                                        int nbrick, MgStep st, int *ran)
+{
+    const int b = blockIdx.x;
+    if (b < gb)
+        brick_tiles<BRICK>(P, brick, my_run(nbrick, b, gb), st, ran);
+    else
+        fine_tiles<KIND>(P, fine, my_run(nfine, b - gb, gridDim.x - gb), st, ran);
 }
 
 // Sums over the bottom kernel's workgroup, to every thread.
@@ -911,7 +1202,8 @@ __global__ __launch_bounds__(kBotThreads) void k_mg_bottom(const ProbDev *__rest
     const ProbDev &pd = P[prob];
     if (!running(pd, st, prob)) return;
     const int tid = threadIdx.x, lb = pd.lbot, nl = pd.nlev;
-    const bool project = st.S[prob].project != 0;
+    const gptr<CgScalars> S = glob(st.S + prob);
+    const bool project = S->project != 0, judged = pd.brick != 0;
     const MgLevel &L0 = pd.lv[lb];
     const int m0 = L0.nx * L0.ny * L0.nz, total = pd.nbot;
     const gptr<const float> pack = glob((const float *)pd.bot);
@@ -923,7 +1215,12 @@ __global__ __launch_bounds__(kBotThreads) void k_mg_bottom(const ProbDev *__rest
     BotCell *const low = reinterpret_cast<BotCell *>(lds);
     float *const R = lds + 8 * (total - m0) + guard, *const A = R + total, *const B = A + total, *const D = B + total;
     BotCell top[kBotPer];
-    double pr[2] = {0.0, 0.0};   // w.r, w.w
+    double pr[3] = {0.0, 0.0, 0.0};   // w.r, w.w, and r.r of the fine grid
+    if (judged) {
+        const gptr<const double> part = glob((const double *)(pd.mixed ? part_rr(pd) : pd.P.upd));
+        const int np = pd.mixed ? pd.ntm : pd.nt1;
+        for (int i = tid; i < np; i += kBotThreads) pr[2] += part[i];
+    }
 #pragma unroll
     for (int q = 0; q < kBotPer; ++q) {
         const int c = tid + q * kBotThreads;
@@ -945,8 +1242,12 @@ __global__ __launch_bounds__(kBotThreads) void k_mg_bottom(const ProbDev *__rest
     for (int c = tid; c < guard; c += kBotThreads) R[c - guard] = D[total + c] = 0.f;
     for (int c = tid; c < total - m0; c += kBotThreads) R[m0 + c] = 0.f;
     for (int c = tid; c < 3 * total; c += kBotThreads) A[c] = 0.f;
+    if (project || judged) bot_sum(pr);
+    if (judged) {
+        const int n = st.step - pd.n0 + 1;
+        if (judge(S, pd.mixed != 0, n == 1 || st.step == S->skip_e_at || !pd.mixed, n, pr[2], tid == 0)) return;
+    }
     if (project) {
-        bot_sum(pr);
         const double f = pr[1] > 0.0 ? pr[0] / pr[1] : 0.0;
 #pragma unroll
         for (int q = 0; q < kBotPer; ++q) {
@@ -1447,6 +1748,10 @@ bool mg_plan(const Geo &g, float *w32, float *space, size_t floats, float *scrat
     }
     static_assert(sizeof(BotCell) == 8 * sizeof(float), "the pack's size");
     pd.bot = keep(8 * (size_t)pd.nbot);
+    // bricks on the fine level (ps_mg.hip: k_mg_brick)
+    const int nb = g.n <= kMgBrickCells ? bricks(L0) : 0;
+    pd.brick = nb && keep.off + 6 * (size_t)nb + 128 <= 2 * (size_t)g.n;
+    if (pd.brick) pd.P.m4 = reinterpret_cast<double *>(keep(6 * (size_t)nb));
     if (used) *used = keep.off;
     if (keep.off > floats || setup.off > (size_t)g.n) return false;
     pd.nlev = l + 1;
@@ -1465,13 +1770,13 @@ bool mg_plan(const Geo &g, float *w32, float *space, size_t floats, float *scrat
     auto tiles = [&](int kz) { return cols * ((g.nz + kz - 1) / kz); };
     const int kz = tiles(8) >= 512 ? 8 : tiles(4) >= 256 ? 4 : 2;
     pd.mkz = kz;
-    pd.ntm = (int)tiles(kz);
+    pd.ntm = pd.brick ? nb : (int)tiles(kz);
     pd.medge = g.px || pd.mtx > 1 || g.nx % 4 != 0;
     pd.mg = 1;
     return true;
 }
 
-int mg_level_tiles(const ProbDev &pd, int l) { return l >= 1 && l < pd.lbot ? bricks(pd.lv[l]) : 0; }
+int mg_level_tiles(const ProbDev &pd, int l) { return l < pd.lbot && (l || pd.brick) ? bricks(pd.lv[l]) : 0; }
 
 void launch_mg_setup(const ProbDev &pd, const ProbDev *dev, const SetupIn &in, hipStream_t s)
 {
@@ -1495,31 +1800,43 @@ void launch_mg_setup(const ProbDev &pd, const ProbDev *dev, const SetupIn &in, h
 
 void launch_mg_step(const ProbDev *P, const MgTables &T, int maxgrid, const MgStep &step, int *ran, hipStream_t s)
 {
-    const int grid = std::min(T.nfine, maxgrid);
-#define MG_FINE(KIND, RAN) \
-    hipLaunchKernelGGL(k_mg_fine<KIND>, dim3(grid), dim3(kThreads), 0, s, P, T.fine, T.nfine, step, RAN)
-#define MG_LEVEL(UP, l)                                                                                          \
+    const int gf = std::min(T.nfine, maxgrid), nb = T.nlev[0], gb = std::min(nb, 4 * maxgrid);
+#define MG_FINE(KIND) \
+    hipLaunchKernelGGL(k_mg_fine<KIND>, dim3(gf), dim3(kThreads), 0, s, P, T.fine, T.nfine, step, ran)
+#define MG_BRICK(KIND) \
+    hipLaunchKernelGGL(k_mg_brick<KIND>, dim3(gb), dim3(kThreads), 0, s, P, T.lev[0], nb, step, ran)
+#define MG_BOTH(KIND, BRICK)                                                                                        \
+    if (gf && gb)                                                                                                   \
+        hipLaunchKernelGGL((k_mg_both<KIND, BRICK>), dim3(gf + gb), dim3(kThreads), 0, s, P, T.fine, T.nfine, gb,   \
+                           T.lev[0], nb, step, ran);                                                                \
+    else if (gf)                                                                                                    \
+        MG_FINE(KIND);                                                                                              \
+    else                                                                                                            \
+        MG_BRICK(BRICK)
+#define MG_LEVEL(UP, l)                                                                                           \
     hipLaunchKernelGGL(k_mg_level<UP>, dim3(std::min(T.nlev[l], 4 * maxgrid)), dim3(kThreads), 0, s, P, T.lev[l], \
                        T.nlev[l], l, step)
     if (T.nt1_64)
         hipLaunchKernelGGL(k_mg_upd64, dim3(std::min(T.nt1_64, maxgrid)), dim3(kThreads), 0, s, P, T.t1_64, T.nt1_64,
                            step);
-    MG_FINE(kA1, nullptr);
-    MG_FINE(kA2, nullptr);
+    MG_BOTH(kA1, kDown);
+    if (gf) MG_FINE(kA2);
     for (int l = 1; l < kMgLevels; ++l)
         if (T.nlev[l]) MG_LEVEL(false, l);
     hipLaunchKernelGGL(k_mg_bottom, dim3(T.nprobs), dim3(kBotThreads), 0, s, P, T.probs, step);
     for (int l = kMgLevels - 1; l >= 1; --l)
         if (T.nlev[l]) MG_LEVEL(true, l);
-    MG_FINE(kB1, nullptr);
-    MG_FINE(kB2, nullptr);
+    if (gf) MG_FINE(kB1);
+    MG_BOTH(kB2, kUp);
     if (T.nt3) {
-        MG_FINE(kDir, ran);
+        MG_BOTH(kDir, kDirB);
         launch_true_residual(P, T.t3, T.nt3, maxgrid, StepRef{nullptr, step.step, nullptr}, s);
         hipLaunchKernelGGL(k_mg_decide, dim3(T.nprobs), dim3(kThreads), 0, s, P, T.probs, step);
     }
     if (T.nt3_64) launch_mg_dir64(P, T.t3_64, T.nt3_64, maxgrid, step, ran, s);
 #undef MG_FINE
+#undef MG_BRICK
+#undef MG_BOTH
 #undef MG_LEVEL
 }
 
