@@ -76,6 +76,13 @@ CASES = [
     ("ibm_rhs", lambda: R(56, 48, 24, 15, ibm=True)),
     ("cylinder", lambda: cylinder(72, 40, 24, 16)),
     ("flat_cells", lambda: R(64, 48, 20, 17, dx=5e-3)),
+    ("last_brick", lambda: R(64, 64, 32, 25, periodic_x=True)),      # 131072 cells: up to here bricks
+    ("brick_edges", lambda: R(17, 9, 41, 26, periodic_y=True)),
+    ("first_march", lambda: lid(R(61, 43, 50, 27))),                 # 131150
+    ("march_two_segments", lambda: R(257, 27, 19, 28)),
+    ("march_three_segments_px", lambda: R(515, 17, 15, 29, periodic_x=True, periodic_y=True)),
+    ("march_four_aligned_px", lambda: R(128, 33, 32, 30, periodic_x=True)),
+    ("march_cylinder", lambda: cylinder(96, 44, 33, 32)),
 ]
 
 
