@@ -190,6 +190,7 @@ private:
     void reap_graphs(bool wait);
     int finish(const std::vector<int> &done);
     int next_chunk_len() const;
+    int mg_steps_ahead() const;
     int plain_count() const;
     bool refresh_may_be_due(int step) const;
 
@@ -209,6 +210,7 @@ private:
     int max_slots_ = 0;
     int step_ = 0;                     // global step of the last enqueued iteration
     int mstep_ = 0;                    // multigrid problems' own step count
+    int status_seen_ = 0;              // its value when the last state read was queued
     int chunk_idx_ = 0;
     bool tables_dirty_ = true;
     void *d_fin_ = nullptr;            // tables of the problems being finished

@@ -700,7 +700,7 @@ int Engine::rebuild_tables()
 // every iteration and only need the host to notice it.
 int Engine::next_chunk_len() const
 {
-    if (plain_count() == 0) return chunk_ > 0 ? chunk_ : kMgChunk;
+    if (plain_count() == 0) return chunk_ > 0 ? chunk_ : std::max(1, std::min(kMgChunk, mg_steps_ahead()));
     if (chunk_ > 0) return (chunk_ + kRefreshGrain - 1) / kRefreshGrain * kRefreshGrain;
     bool any_mixed = false;
     long long biggest = 0;
@@ -719,6 +719,33 @@ int Engine::next_chunk_len() const
     if (!any_mixed) return biggest <= 200000 ? 64 : 32;
     best = std::max(best, kRefreshGrain);
     return (best + kRefreshGrain - 1) / kRefreshGrain * kRefreshGrain;
+}
+
+// Multigrid steps still to queue, as the last states read foretell: to the end
+// of the slowest problem at the rate at which r.r has fallen so far, one step
+// for each replacement on the way.  kMgChunk until a state tells.  A step queued after the end costs its
+// launches (25 us at 64x64x32, 40 us at 256x128x96), and there were three; one
+// short of it costs the host's turn, about as much.
+int Engine::mg_steps_ahead() const
+{
+    int most = 0;
+    for (int i = 0; i < max_slots_; ++i) {
+        const Slot &sl = slots_[i];
+        if (!sl.active || sl.finished || !sl.mg) continue;
+        const CgScalars &c = sl.status;
+        const int seen = status_seen_ - sl.n0 + 1;   // steps the state has taken
+        if (c.iters < 2 || seen < 1) return kMgChunk;
+        const double now = c.rr[seen & 1];           // r.r entering its last step
+        const double target = kMgMargin * c.thresh;
+        if (!(now > 0.0 && target > 0.0 && now < c.rr0)) return kMgChunk;
+        const double rate = std::log(c.rr0 / now) / (c.iters > 1 ? c.iters - 1 : 1);
+        const double base = c.refreshes ? c.rr_after : c.rr0;
+        int left = now > target ? (int)std::ceil(std::log(now / target) / rate) : 0;
+        left += 1;                                   // its end
+        if (c.mixed && base > 0.0) left += std::max(0, (int)std::ceil(std::log(base / target) / -std::log(kMgCycleDrop)) - 1);
+        most = std::max(most, left - (mstep_ - status_seen_));
+    }
+    return most;
 }
 
 // Could a mixed problem's residual replacement be due after global step s?
@@ -989,6 +1016,7 @@ int Engine::pump(bool timing, std::vector<int> &finished)
     // keep two chunks in flight: the host reads one chunk's state while the
     // next runs
     while (active_count() > 0 && npend_ < 2) {
+        if (npend_ == 1 && plain_count() == 0 && chunk_ <= 0 && mg_steps_ahead() <= 0) break;
         if ((rc = enqueue_chunk(next_chunk_len(), timing))) return rc;
         pend_[(pend_head_ + npend_) & 1] = (chunk_idx_ - 1) & 1;
         ++npend_;
@@ -999,6 +1027,7 @@ int Engine::pump(bool timing, std::vector<int> &finished)
     --npend_;
     ECHK(hipEventSynchronize(ev_status_[which]));
     const CgScalars *h = h_status_ + (size_t)which * max_slots_;
+    status_seen_ = status_mstep_[which];
     std::vector<int> &done = done_;
     done.clear();
     for (int i = 0; i < max_slots_; ++i) {
