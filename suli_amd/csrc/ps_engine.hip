@@ -483,6 +483,7 @@ int Engine::setup_slot(int si, bool multi, hipEvent_t wait_ev)
         pd.rx32 = pd.ry32 = pd.rz32 = nullptr;
         pd.rowreg = nullptr;
     }
+    if (sl.mg && pd.brick) pd.rowreg = nullptr;   // bricks read the arrays
     pd.nt3 = nt3;
     pd.nt1 = nt1;
     pd.mixed = o.mixed ? 1 : 0;

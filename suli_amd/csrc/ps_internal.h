@@ -52,12 +52,14 @@ constexpr int kMgLevels = 20;
 constexpr int kMgBottomCells = 6144;   // the bottom kernel's largest level
 constexpr int kMgBottomLds = 38912;    // floats of LDS it has (152 KiB)
 // The coarsest level: at most a cell per lane of one wave and kMgCoarsestSide
-// around (the sweeps must reach from end to end).  At 64 cells and 16 sweeps a
-// cycle over 64x64x32 takes as many iterations as at 8 cells and 8 sweeps, with
-// one level less: 1.25 -> 1.19 ms; at 8 sweeps it took one iteration more.
+// around, solved by a Chebyshev semi-iteration.  (64 cells instead of 8, with 16
+// Jacobi sweeps, took as many iterations over 64x64x32 and a level less: 1.25 ->
+// 1.19 ms; with 8 sweeps one iteration more.  Degree 8 contracts the slowest error
+// of an 8x8x1 level to 0.5, 16 sweeps to 0.7.)
 constexpr int kMgCoarsestCells = 64;
 constexpr int kMgCoarsestSide = 8;
-constexpr int kMgCoarsestSweeps = 16;
+constexpr int kMgCoarsestDegree = 8;
+constexpr float kCoarsestMin = 0.05f;
 // Problems up to this many cells do both matrix products of a half cycle in one
 // launch on the fine level too, in bricks; larger ones march through tiles, which
 // read each value fewer times.  Alone, mixed from prd1 = 0 to 1e-12: 5120 cells

@@ -72,7 +72,6 @@ constexpr float kTheta = 0.5f * (kLmax + kLmin), kDelta = 0.5f * (kLmax - kLmin)
 constexpr float kRho1 = 1.0f / (2.0f * kTheta / kDelta - kDelta / kTheta);
 constexpr float kC0 = (1.0f + kRho1 * kDelta / kTheta) / kTheta + 2.0f * kRho1 / kDelta;
 constexpr float kC1 = -2.0f * kRho1 / (kDelta * kTheta);
-constexpr float kOmega = 0.85f;   // Jacobi sweeps of the coarsest level
 constexpr int kBotThreads = 1024;
 constexpr int kBotPer = kMgBottomCells / kBotThreads;
 
@@ -1330,17 +1329,23 @@ __global__ __launch_bounds__(kBotThreads) void k_mg_bottom(const ProbDev *__rest
     if (tid < 64) {
         for (; l < nb - 1; ++l) off = down(true, l, off);
         {
-            // the coarsest level (at most 64 cells): Jacobi sweeps from zero
+            // the coarsest level (at most 64 cells): Chebyshev semi-iteration
+            // from zero on [kCoarsestMin, kLmax]
+            constexpr float theta = 0.5f * (kLmax + kCoarsestMin), delta = 0.5f * (kLmax - kCoarsestMin);
             const BotDim d = dim(l);
             const int m = size(l);
             const BotCell x = nb == 1 ? top[0] : low[off - m0 + min(tid, m - 1)];
             float *const a = A + off;
             const float r = tid < m ? R[off + tid] : 0.f;
-            float v = kOmega * r;
-            for (int it = 1; it < kMgCoarsestSweeps; ++it) {
+            float v = r / theta, dv = v, rho = delta / theta;
+#pragma unroll
+            for (int it = 1; it < kMgCoarsestDegree; ++it) {
                 if (tid < m) a[tid] = v;
                 sync(true);
-                if (tid < m) v = v + kOmega * (r - v + bot_nb(d, x, tid, a));
+                const float rho1 = 1.f / (2.f * theta / delta - rho);
+                if (tid < m) dv = rho1 * rho * dv + 2.f * rho1 / delta * (r - v + bot_nb(d, x, tid, a));
+                v += dv;
+                rho = rho1;
                 sync(true);
             }
             if (tid < m) a[tid] = v * x.iw();
