@@ -611,66 +611,93 @@ __global__ __launch_bounds__(kThreads) void k_posdin(Geo g, SetupIn in, double *
     for_cells(g, [&](int i, int j, int k) { posdin_cell(g, in, u, v, w, with_z, i, j, k, aux1, aux2); });
 }
 
-// Planes whose loads a column sweep (k_pressh, k_posdin_hydro_w) issues
-// together before it runs its recurrence over them.
-constexpr int kColumnAhead = 8;
+// The column sweeps (k_pressh, k_posdin_hydro_w): a workgroup takes 64 columns
+// and a chunk of planes at a time.  Its waves load and work out the planes' terms
+// side by side, the first wave runs the recurrence over them in LDS, and all
+// store.  Lanes that walked a column each, eight planes' loads ahead, waited on a
+// round trip per eight planes and on the divisions, and half the CUs had no
+// column.  At 256x128x96 k_pressh (50 MB) 22.0 -> 14.4 us, k_posdin_hydro_w (100
+// MB) 30.8 -> 26.5; with chunks of 64 planes 15.3 and 33.1 (the LDS and registers
+// then leave two workgroups per CU).
+constexpr int kPressThreads = 512, kPressWaves = kPressThreads / 64, kPressChunk = 32;
+constexpr int kPressPer = kPressChunk / kPressWaves;
+constexpr int kWThreads = 256, kWWaves = kWThreads / 64, kWChunk = 16, kWPer = kWChunk / kWWaves;
 
 // pressh, the hydrostatic pressure of t_press = 0 (SuLi-IC/9_grad.f90:
-// 667-702; dz(k) weights: SuLi-ICdz/9_grad.f90:665-700).  One lane per
-// (i, j) column walks k from the top: the top cell takes dz g rho, the one
-// below the trapezoid of the top two, every other cell Simpson's rule over
-// the two cells above it plus prd1(k+2).  The two values above stay in
-// registers; lanes of a wavefront are consecutive i, so every k step reads
-// and writes contiguous rows.  Only prd1's interior is written.
-__global__ __launch_bounds__(kThreads) void k_pressh(Geo g, const double *__restrict__ rho, const double *dz, double dzu,
-                                                     double gz, double *__restrict__ prd1)
+// 667-702; dz(k) weights: SuLi-ICdz/9_grad.f90:665-700).  Each (i, j) column
+// goes from the top: the top cell takes dz g rho, the one below the trapezoid of
+// the top two, every other cell Simpson's rule over the two cells above it plus
+// prd1(k+2).  Only prd1's interior is written.
+__global__ __launch_bounds__(kPressThreads) void k_pressh(Geo g, const double *__restrict__ rho, const double *dz,
+                                                        double dzu, double gz, double *__restrict__ prd1)
 {
+    __shared__ double r[kPressChunk + 2][64];   // rho from two planes above the chunk on
+    __shared__ double t[kPressChunk][64];       // terms, then pressures
     const int nx = g.nx, ny = g.ny, nz = g.nz;
-    const long long col = (long long)blockIdx.x * kThreads + threadIdx.x;
-    if (col >= (long long)nx * ny) return;
-    const int i = (int)(col % nx), j = (int)(col / nx);
-    const long long plane = (long long)nx * ny;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const long long plane = (long long)nx * ny, col = (long long)blockIdx.x * 64 + lane;
+    const bool act = col < plane;
+    const long long cc = act ? col : plane - 1;
     const long long pbb = (long long)(nx + 2) * (ny + 2);
-    const double *rc = rho + col;
-    double *pc = prd1 + (i + 1) + (long long)(nx + 2) * (j + 1);
-    double p1 = 0.0, p2 = 0.0;  // prd1 at k+1, k+2
-    double r1 = 0.0, r2 = 0.0;  // rho at k+1, k+2
-    // rho of kColumnAhead planes loaded together, then the recurrence over
-    // them: one round trip per block of planes instead of one per plane
-    for (int K0 = nz; K0 >= 1; K0 -= kColumnAhead) {
-        double rb[kColumnAhead];
+    const double *rc = rho + cc;
+    double *pc = prd1 + ((int)(cc % nx) + 1) + (long long)(nx + 2) * ((int)(cc / nx) + 1);
+    double p1 = 0.0, p2 = 0.0;   // prd1 at k+1, k+2 (the first wave's)
+    for (int K0 = nz; K0 >= 1; K0 -= kPressChunk) {
+        const int planes = min(kPressChunk, K0);
+        double rb[kPressPer];
 #pragma unroll
-        for (int m = 0; m < kColumnAhead; ++m) rb[m] = K0 - m >= 1 ? rc[(long long)(K0 - m - 1) * plane] : 0.0;
+        for (int q = 0; q < kPressPer; ++q) rb[q] = rc[(long long)(max(K0 - (wave + q * kPressWaves), 1) - 1) * plane];
 #pragma unroll
-        for (int m = 0; m < kColumnAhead; ++m) {
-            const int K = K0 - m;
+        for (int q = 0; q < kPressPer; ++q) r[2 + wave + q * kPressWaves][lane] = rb[q];
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < kPressPer; ++q) {
+            const int m = wave + q * kPressWaves, K = K0 - m;
             if (K < 1) break;
-            const double r0 = rb[m];
-            double p;
+            const double r0 = rb[q], r1 = r[m + 1][lane], r2 = r[m][lane];
+            double v;
             if (dz) {
-                if (K == nz) {
-                    p = dz[K] * gz * r0;
-                } else if (K == nz - 1) {
-                    p = gz * (r0 * dz[K] + r1 * dz[K + 1]) * 0.5 + p1;
-                } else {
-                    const double intz = (r0 * dz[K] + 4. * r1 * dz[K + 1] + r2 * dz[K + 2]) / 3.;
-                    p = gz * intz + p2;
-                }
+                if (K == nz)
+                    v = dz[K] * gz * r0;
+                else if (K == nz - 1)
+                    v = gz * (r0 * dz[K] + r1 * dz[K + 1]) * 0.5;
+                else
+                    v = (r0 * dz[K] + 4. * r1 * dz[K + 1] + r2 * dz[K + 2]) / 3.;
             } else {
-                if (K == nz) {
-                    p = dzu * gz * r0;
-                } else if (K == nz - 1) {
-                    p = dzu * gz * (r0 + r1) * 0.5 + p1;
-                } else {
-                    const double intz = dzu * (r0 + 4. * r1 + r2) / 3.;
-                    p = gz * intz + p2;
+                if (K == nz)
+                    v = dzu * gz * r0;
+                else if (K == nz - 1)
+                    v = dzu * gz * (r0 + r1) * 0.5;
+                else
+                    v = dzu * (r0 + 4. * r1 + r2) / 3.;
+            }
+            t[m][lane] = v;
+        }
+        __syncthreads();
+        if (wave == 0) {
+            for (int m0 = 0; m0 < planes; m0 += 8) {
+                double v[8];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) v[q] = t[m0 + q][lane];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    const int K = K0 - m0 - q;
+                    const double p = K == nz ? v[q] : K == nz - 1 ? v[q] + p1 : gz * v[q] + p2;
+                    p2 = p1;
+                    p1 = p;
+                    t[m0 + q][lane] = p;
                 }
             }
-            pc[(long long)K * pbb] = p;
-            p2 = p1;
-            p1 = p;
-            r2 = r1;
-            r1 = r0;
+        } else if (wave == 1) {
+            const double a = r[kPressChunk][lane], b = r[kPressChunk + 1][lane];
+            r[0][lane] = a;
+            r[1][lane] = b;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < kPressPer; ++q) {
+            const int m = wave + q * kPressWaves, K = K0 - m;
+            if (K >= 1 && act) pc[(long long)K * pbb] = t[m][lane];
         }
     }
 }
@@ -678,60 +705,84 @@ __global__ __launch_bounds__(kThreads) void k_pressh(Geo g, const double *__rest
 // posdin's hydrostatic branch, after the shared u, v correction
 // (SuLi-IC/10_pos.f90:48-57; dz(k): SuLi-ICdz/10_pos.f90:52): w(:,:,1) = 0
 // over the whole bottom plane, then w(k+1) = w(k) - du dz/dx - dv dz/dy up
-// each interior column from the corrected u, v.  The same lane then zeroes
-// its column's w faces where the face value of hs is below 1e-4 (:84-91);
-// the chain itself runs on the values before zeroing, as in the reference,
-// where the zeroing is a later sweep.  Lanes over the (nx+2)(ny+2) plane;
-// the ring only clears its bottom face.
+// each interior column from the corrected u, v.  The w faces where the face
+// value of hs is below 1e-4 are zeroed with it (:84-91); the chain itself runs on
+// the values before zeroing, as in the reference, where the zeroing is a later
+// sweep.  Lanes over the (nx+2)(ny+2) plane; the ring only clears its bottom face.
 template <bool DZ>
-__global__ __launch_bounds__(kThreads) void k_posdin_hydro_w(Geo g, const double *u, const double *v,
-                                                             const double *hs, const double *dz, double dzu,
-                                                             double dx, double dy, double *w)
+__global__ __launch_bounds__(kWThreads) void k_posdin_hydro_w(Geo g, const double *u, const double *v,
+                                                                const double *hs, const double *dz, double dzu,
+                                                                double dx, double dy, double *w)
 {
+    __shared__ double ta[kWChunk][64], tb[kWChunk][64];   // du dz/dx and then w; dv dz/dy
     const int nx = g.nx, ny = g.ny, nz = g.nz;
-    const long long t = (long long)blockIdx.x * kThreads + threadIdx.x;
-    if (t >= (long long)(nx + 2) * (ny + 2)) return;
-    const int I = (int)(t % (nx + 2)), J = (int)(t / (nx + 2));
-    const long long wbb = (long long)(nx + 2) * (ny + 2);
-    double *wc = w + t;
-    wc[wbb] = 0.;  // w(:,:,1) = 0
-    if (I < 1 || I > nx || J < 1 || J > ny) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const long long wbb = (long long)(nx + 2) * (ny + 2), t = (long long)blockIdx.x * 64 + lane;
+    const bool box = t < wbb;
+    const long long tt = box ? t : wbb - 1;
+    const int I = (int)(tt % (nx + 2)), J = (int)(tt / (nx + 2));
+    const bool act = box && I >= 1 && I <= nx && J >= 1 && J <= ny;
+    const int Ic = min(max(I, 1), nx), Jc = min(max(J, 1), ny);   // the ring reads its neighbour's column
     const long long ubb = (long long)(nx + 3) * (ny + 2), vbb = (long long)(nx + 2) * (ny + 3);
-    const double *uc = u + I + (long long)(nx + 3) * J;
-    const double *vc = v + I + (long long)(nx + 2) * J;
-    double wk = 0.;
-    if (face_z(g, hs, dz, I - 1, J - 1, 0) < 0.0001) wc[wbb] = 0.;
-    // u, v and the two hs cells of the z face of kColumnAhead planes loaded
-    // together (no branch between the loads), then the chain over them
-    // (DZ: the stretched grid's dz(K) and the face weights too)
+    const double *uc = u + Ic + (long long)(nx + 3) * Jc;
+    const double *vc = v + Ic + (long long)(nx + 2) * Jc;
     const long long plane = (long long)nx * ny;
-    const double *hc = hs + (long long)(J - 1) * nx + (I - 1);
-    for (int K0 = 1; K0 <= nz; K0 += kColumnAhead) {
-        double u0[kColumnAhead], u1[kColumnAhead], v0[kColumnAhead], v1[kColumnAhead];
-        double h1[kColumnAhead], h0[kColumnAhead], dk[kColumnAhead], d1[kColumnAhead], d0[kColumnAhead];
+    const double *hc = hs + (long long)(Jc - 1) * nx + (Ic - 1);
+    double *wc = w + tt;
+    if (wave == 0 && box) wc[wbb] = 0.;   // w(:,:,1) = 0, whatever hs is there
+    double wk = 0.;                       // (the first wave's)
+    for (int K0 = 1; K0 <= nz; K0 += kWChunk) {
+        const int planes = min(kWChunk, nz - K0 + 1);
+        // u, v and the two hs cells of the z face of the wave's planes loaded
+        // together, no branch between the loads (DZ: the stretched grid's dz(K)
+        // and the face weights too)
+        double u0[kWPer], u1[kWPer], v0[kWPer], v1[kWPer], h1[kWPer], h0[kWPer];
+        double dk[kWPer], d1[kWPer], d0[kWPer];
 #pragma unroll
-        for (int m = 0; m < kColumnAhead; ++m) {
-            const int K = K0 + m <= nz ? K0 + m : nz;
+        for (int q = 0; q < kWPer; ++q) {
+            const int K = min(K0 + wave + q * kWWaves, nz);
             const int a = face_z_upper(g, K);
-            u1[m] = uc[(long long)K * ubb + 1];
-            u0[m] = uc[(long long)K * ubb];
-            v1[m] = vc[(long long)K * vbb + (nx + 2)];
-            v0[m] = vc[(long long)K * vbb];
-            h1[m] = hc[a * plane];
-            h0[m] = hc[(a - 1) * plane];
-            dk[m] = DZ ? dz[K] : dzu;
-            d1[m] = DZ ? dz[a + 1] : 0.0;
-            d0[m] = DZ ? dz[a] : 0.0;
+            u1[q] = uc[(long long)K * ubb + 1];
+            u0[q] = uc[(long long)K * ubb];
+            v1[q] = vc[(long long)K * vbb + (nx + 2)];
+            v0[q] = vc[(long long)K * vbb];
+            h1[q] = hc[a * plane];
+            h0[q] = hc[(a - 1) * plane];
+            dk[q] = DZ ? dz[K] : dzu;
+            d1[q] = DZ ? dz[a + 1] : 0.0;
+            d0[q] = DZ ? dz[a] : 0.0;
         }
+        unsigned dry = 0;
 #pragma unroll
-        for (int m = 0; m < kColumnAhead; ++m) {
-            const int K = K0 + m;
-            if (K > nz) break;
-            const double dzk = dk[m];
-            const double du = u1[m] - u0[m], dv = v1[m] - v0[m];
-            wk = wk - du * dzk / dx - dv * dzk / dy;
-            const double hf = DZ ? face_z_weighted(h1[m], h0[m], d1[m], d0[m]) : (h1[m] + h0[m]) * 0.5;
-            wc[(long long)(K + 1) * wbb] = hf < 0.0001 ? 0. : wk;
+        for (int q = 0; q < kWPer; ++q) {
+            const int m = wave + q * kWWaves;
+            const double du = u1[q] - u0[q], dv = v1[q] - v0[q];
+            ta[m][lane] = du * dk[q] / dx;
+            tb[m][lane] = dv * dk[q] / dy;
+            const double hf = DZ ? face_z_weighted(h1[q], h0[q], d1[q], d0[q]) : (h1[q] + h0[q]) * 0.5;
+            dry |= (hf < 0.0001 ? 1u : 0u) << q;
+        }
+        __syncthreads();
+        if (wave == 0) {
+            for (int m0 = 0; m0 < planes; m0 += 8) {
+                double a[8], b[8];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    a[q] = ta[m0 + q][lane];
+                    b[q] = tb[m0 + q][lane];
+                }
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    wk = wk - a[q] - b[q];
+                    ta[m0 + q][lane] = wk;
+                }
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < kWPer; ++q) {
+            const int m = wave + q * kWWaves, K = K0 + m;
+            if (K <= nz && act) wc[(long long)(K + 1) * wbb] = (dry >> q & 1u) ? 0. : ta[m][lane];
         }
     }
 }
@@ -1301,7 +1352,7 @@ void launch_pressh(const Geo &g, const double *rho, const double *dz, double dzu
                    hipStream_t s)
 {
     const long long ncol = (long long)g.nx * g.ny;
-    hipLaunchKernelGGL(k_pressh, dim3((unsigned)((ncol + kThreads - 1) / kThreads)), dim3(kThreads), 0, s, g, rho,
+    hipLaunchKernelGGL(k_pressh, dim3((unsigned)((ncol + 63) / 64)), dim3(kPressThreads), 0, s, g, rho,
                        dz, dzu, gz, prd1);
 }
 
@@ -1310,12 +1361,12 @@ void launch_posdin_hydro(const Geo &g, const SetupIn &in, const double *hs, doub
 {
     hipLaunchKernelGGL(k_posdin, cell_grid(g), dim3(kThreads), 0, s, g, in, u, v, w, false);
     const long long nplane = (long long)(g.nx + 2) * (g.ny + 2);
-    const dim3 grid((unsigned)((nplane + kThreads - 1) / kThreads));
+    const dim3 grid((unsigned)((nplane + 63) / 64));
     if (in.dz)
-        hipLaunchKernelGGL(k_posdin_hydro_w<true>, grid, dim3(kThreads), 0, s, g, u, v, hs, in.dz, in.dzu, in.dx, in.dy,
+        hipLaunchKernelGGL(k_posdin_hydro_w<true>, grid, dim3(kWThreads), 0, s, g, u, v, hs, in.dz, in.dzu, in.dx, in.dy,
                            w);
     else
-        hipLaunchKernelGGL(k_posdin_hydro_w<false>, grid, dim3(kThreads), 0, s, g, u, v, hs, in.dz, in.dzu, in.dx,
+        hipLaunchKernelGGL(k_posdin_hydro_w<false>, grid, dim3(kWThreads), 0, s, g, u, v, hs, in.dz, in.dzu, in.dx,
                            in.dy, w);
     hipLaunchKernelGGL(k_posdin_hydro_uv, cell_grid(g), dim3(kThreads), 0, s, g, hs, u, v);
 }
