@@ -21,17 +21,15 @@ exp_press, SuLi-IT's solve and posdin), each with its time per call and the
 bytes it moves.  With --only both it also times the device-resident posdin
 (`posdin_dev`).
 
-`roofline` is for the dominant kernel, k_cg_m, the whole FP32 CG iteration of
-the mixed solver in one launch.  `achieved` counts the algorithmic bytes of
-one CG iteration, 14 FP32 words per cell (SpMV 5: p and the three face
-coefficients read, Ap written; iterate, residual and direction 3 each), i.e.
-56 B/cell, divided by the kernel's mean launch time, which HIP events on the
-solver's stream measure around windows of 8 consecutive launches (one window
-per 16 steps) during two directly launched solves; a window's time includes
-the gaps between its launches.  The fused kernel moves fewer bytes than
-that: `traffic` is its HBM bytes per launch from rocprofv3's FETCH_SIZE and
-WRITE_SIZE counters (profiles/hbm_traffic.json, calibrated on the copy
-kernel k_copy), and `traffic_achieved` those bytes at the same launch rate.
+`roofline` is for one multigrid-preconditioned FP32 iteration of the mixed
+solver (the solve is nearly all iterations).  `achieved` counts the bytes its
+five passes over the fine grid read and write, 22 FP32 words per cell: r -=
+alpha q and t = A r (4 words), the residual behind the smoother (4), the
+coarse correction's residual (3), z (5), the direction step (6); faces, which
+regular rows take from small tables, and the coarse levels, about a seventh of
+the cells, are not counted.  The time is the step's mean over windows of 2
+consecutive steps between HIP events on the solver's stream during two
+solves, all of its launches and the gaps between them included.
 `copy_kernel` and `read_kernel` give what a plain 256 MiB copy and a plain
 read reach on the same GPU in the same run: the HBM rates a kernel that
 mixes reads and writes can be held against.
@@ -63,7 +61,11 @@ HBM_PEAK_GBS = 8000.0
 GRAPHS = True
 
 METRIC = "pressure solves/s + p99 latency at 1e-8 residual, mixed vs FP64 CG"
-CG_WORDS = 14          # algorithmic FP32/FP64 words per cell of one CG iteration
+CG_WORDS = 14          # algorithmic words per cell of one plain CG iteration (the CPU's)
+MG_WORDS = 22          # FP32 words per cell of a multigrid iteration's fine passes
+# bytes per cell of an FP64 iteration's: r -= alpha q with its FP32 copy (28), the
+# cycle's four passes (56), the direction step with e and the face arrays (68)
+MG_FP64_BYTES = 152
 SPMV_WORDS = 5         # algorithmic words per cell of the SpMV
 REF_WORDS = 17         # words per cell per iteration of the reference's sweeps
 
@@ -574,29 +576,25 @@ def main():
         return
 
     launch_ms = mixed["step_ms"]
-    alg = CG_WORDS * 4 * n                 # one CG iteration in FP32: 56 B/cell
+    alg = MG_WORDS * 4 * n
     achieved = alg / (launch_ms * 1e-3) / 1e9
-    traffic = load_traffic(f"k_cg_m {g.nx}x{g.ny}x{g.nz}")
     spmv_gbs = SPMV_WORDS * 4 * n / (mixed["spmv_only_ms"] * 1e-3) / 1e9
     fp64_step = fp64["step_ms"]
     roofline = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": achieved / HBM_PEAK_GBS,
-                "traffic": traffic,
-                "kernel": "k_cg_m", "launch_ms": launch_ms,
+                "traffic": load_traffic(f"multigrid iteration {g.nx}x{g.ny}x{g.nz}"),
+                "kernel": "multigrid iteration (k_mg_fine, k_mg_level, k_mg_bottom)", "launch_ms": launch_ms,
                 "algorithmic_bytes_per_launch": alg,
-                "algorithmic_basis": "one FP32 CG iteration, 14 words/cell (SpMV 5 + x, r, p 3 each)",
-                # the bytes the fused step actually moves (profiled HBM traffic) at its launch rate
-                "traffic_achieved": traffic / (launch_ms * 1e-3) / 1e9 if traffic else None,
-                "traffic_frac": traffic / (launch_ms * 1e-3) / 1e9 / HBM_PEAK_GBS if traffic else None,
-                "launch_ms_basis": "HIP events around windows of 8 consecutive launches (gaps included)",
+                "algorithmic_basis": "one FP32 iteration's passes over the fine grid, 22 words/cell",
+                "launch_ms_basis": "HIP events around windows of 2 consecutive steps (all launches, gaps included)",
                 "spmv": {"kernel": "k_spmv<float>", "words_per_cell": SPMV_WORDS,
                          "launch_ms": mixed["spmv_only_ms"], "achieved": spmv_gbs,
                          "frac": spmv_gbs / HBM_PEAK_GBS,
                          "fp64_launch_ms": fp64["spmv_only_ms"],
                          "fp64_achieved": SPMV_WORDS * 8 * n / (fp64["spmv_only_ms"] * 1e-3) / 1e9},
-                "fp64_step": {"kernels": "k_cg_a<double> + k_cg_b<double>", "step_ms": fp64_step,
-                              "achieved": CG_WORDS * 8 * n / (fp64_step * 1e-3) / 1e9 if fp64_step else None,
-                              "kernel_achieved": 12 * 8 * n / (fp64_step * 1e-3) / 1e9 if fp64_step else None}}
+                "fp64_step": {"kernels": "k_mg_upd64, k_mg_fine, k_mg_level, k_mg_bottom, k_mg_dir64",
+                              "step_ms": fp64_step,
+                              "achieved": MG_FP64_BYTES * n / (fp64_step * 1e-3) / 1e9 if fp64_step else None}}
 
     cpu = checks = None
     if not args.no_cpu:

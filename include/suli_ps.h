@@ -32,8 +32,14 @@ extern "C" {
 #define SULI_PS_ABI_VERSION 2
 
 enum suli_ps_precision {
-    SULI_PS_FP64 = 0,   /* FP64 CG, as the reference */
-    SULI_PS_MIXED = 1   /* FP32 SpMV/axpy inside FP64 residual replacement */
+    SULI_PS_FP64 = 0,   /* FP64 CG, as the reference; by the relative rule
+                           preconditioned with an FP32 multigrid V-cycle */
+    SULI_PS_MIXED = 1   /* FP32 CG, preconditioned likewise, inside FP64
+                           residual replacement */
+    /* The plain CG iteration instead: FP64 by the reference rule, keep_null,
+     * stored_residual, 0 < max_iter < 256, grids of fewer than 4096 cells, a
+     * tile shape fixed with suli_ps_set_tiles (and autotune), and masks that
+     * cut the fluid into parts. */
 };
 
 enum suli_ps_stop_rule {
@@ -111,8 +117,9 @@ typedef struct suli_ps_stats {
     double rel_true;       /* FP64 ||b - A e|| / ||b|| recomputed at exit */
     double solve_ms;       /* device time of the solve, setup included */
     double spmv_ms;        /* mean time of one CG step (its launches, SpMV
-                              included) over windows of 8 consecutive steps,
-                              HIP events on the context stream (opts.timing) */
+                              included) over windows of 8 consecutive steps
+                              (multigrid: 2), HIP events on the context stream
+                              (opts.timing) */
     int32_t graph_replays; /* captured HIP graphs launched during the call (each
                               runs 8 CG steps); 0 when every kernel was
                               launched directly.  0 for served requests. */

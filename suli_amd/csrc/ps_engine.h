@@ -272,6 +272,7 @@ private:
     // timing
     std::vector<hipEvent_t> ev_spmv_;
     int *d_ran_ = nullptr;
+    std::vector<int> timed_steps_;   // steps of each window
     int ntimed_ = 0;
     double spmv_ms_ = 0.0;
     int spmv_n_ = 0;

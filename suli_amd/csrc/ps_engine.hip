@@ -11,6 +11,7 @@ namespace {
 
 constexpr int kMaxGrid = 2048;     // persistent workgroups (8 per CU)
 constexpr int kMaxTimed = 256;     // timing windows per run_all
+constexpr int kMgTimeStride = 4, kMgTimeSteps = 2;   // multigrid problems alone: steps 4k+1, 4k+2
 constexpr int kTimeStride = 16;    // one window per 16 steps ...
 constexpr int kTimeSteps = 8;      // ... over steps 16k+1 .. 16k+8 (no replacement inside;
                                     // an even count: the mixed step alternates two kinds)
@@ -262,6 +263,7 @@ int Engine::init(hipStream_t stream, int max_slots)
     for (auto &e : ev_status_) ECHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     for (auto &e : ev_stage_) ECHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     ev_spmv_.resize(2 * kMaxTimed);
+    timed_steps_.resize(kMaxTimed);
     for (auto &e : ev_spmv_) ECHK(hipEventCreate(&e));
     ECHK(hipMalloc(&d_ran_, sizeof(int) * 2 * kMaxTimed));
     ECHK(hipMalloc(&d_step_, 2 * sizeof(int)));
@@ -802,9 +804,13 @@ int Engine::enqueue_steps_direct(int nsteps, bool timing)
         const StepRef sr{nullptr, step_, nullptr};
         // timing windows of kTimeSteps consecutive steps (events only at
         // their ends, so the per-step figure is the launches' own time)
-        const int ph = (plain || !nmg ? step_ : mstep_) % kTimeStride;
+        // (multigrid problems iterate ten to twenty times and replace in between:
+        // two steps)
+        const bool mg_only = nmg && !plain;
+        const int ph = mg_only ? mstep_ % kMgTimeStride : step_ % kTimeStride;
+        const int span = mg_only ? kMgTimeSteps : kTimeSteps;
         const bool t_open = timing && ph == 1 && ntimed_ < kMaxTimed;
-        const bool t_close = timing && ph == kTimeSteps && ntimed_ < kMaxTimed;
+        const bool t_close = timing && ph == span && ntimed_ < kMaxTimed;
         int *ran = t_open ? d_ran_ + 2 * ntimed_ : t_close ? d_ran_ + 2 * ntimed_ + 1 : nullptr;
         if (t_open) ECHK(hipEventRecord(ev_spmv_[2 * ntimed_], s_));
         if (n3_64) launch_cg_a(false, d_probs_, d_tab_ + off_t3_64, n3_64, std::min(n3_64, kMaxGrid), sr, ran, s_);
@@ -818,6 +824,7 @@ int Engine::enqueue_steps_direct(int nsteps, bool timing)
         }
         if (t_close) {
             ECHK(hipEventRecord(ev_spmv_[2 * ntimed_ + 1], s_));
+            timed_steps_[ntimed_] = span;
             ++ntimed_;
         }
         if (n1_64) launch_cg_b(false, d_probs_, d_tab_ + off_t1_64, n1_64, std::min(n1_64, kMaxGrid), sr, s_);
@@ -1095,7 +1102,7 @@ int Engine::run_all(bool timing)
             if (!ran[2 * t] || !ran[2 * t + 1]) continue;
             float ms = 0.f;
             ECHK(hipEventElapsedTime(&ms, ev_spmv_[2 * t], ev_spmv_[2 * t + 1]));
-            sum += ms / kTimeSteps;
+            sum += ms / timed_steps_[t];
             ++spmv_n_;
         }
         spmv_ms_ = spmv_n_ ? sum / spmv_n_ : 0.0;

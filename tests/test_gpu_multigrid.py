@@ -224,3 +224,20 @@ def test_noalloc_equals_alone(solver, shape, precision, tol):
     assert out[0][1:] == out[1][1:]
     assert out[0][1] < 150
     np.testing.assert_array_equal(out[0][0], out[1][0])
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("shape", [(40, 32, 24), (70, 60, 40)], ids=["bricks", "marched"])
+def test_step_is_timed(solver, shape, precision):
+    """opts.timing measures the step however few of them a solve takes."""
+    c = R(*shape, 71)
+    print(f"multigrid timing {shape} {precision}", flush=True)
+    solver.configure(precision=precision, stop_rule="relative", tol=1e-8, verbose=False, timing=True)
+    df = solver.upload(c.grid, c.fields)
+    try:
+        for _ in range(2):   # windows at both alignments of the step counter
+            df.zero("prd1")
+            st = solver.graddin_dev(c.grid, df)
+            assert st.spmv_timed > 0 and 0.0 < st.spmv_ms < st.solve_ms, st.as_dict()
+    finally:
+        df.free()
