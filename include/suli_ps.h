@@ -172,12 +172,12 @@ int suli_ps_posdin_dev(suli_ps_ctx *ctx, const suli_ps_grid *g, double *u, doubl
  * allocation).  Same arguments, options, arithmetic and results as
  * suli_ps_graddin_dev, except that the problem's solver state (scaled face
  * coefficients, diagonal, right-hand side, iterate, Krylov vectors, partial
- * sums) lives in one fixed device array of SULI_PS_NOALLOC_MAX_BYTES per GPU,
- * which the library holds from the first context on that GPU until the
- * process ends.  The call allocates and frees nothing, creates no event and
+ * sums) lives in one fixed device array per GPU, of SULI_PS_NOALLOC_MAX_BYTES
+ * and 40 MiB for the multigrid iteration's arrays of an FP64 solve, which the
+ * library holds from the first context on that GPU until the process ends.  The call allocates and frees nothing, creates no event and
  * captures no graph (it launches every kernel directly); the launch tables
  * and host lists it needs are reserved by suli_ps_create.  A problem whose
- * state does not fit (problem bytes beyond the maximum: about 80 B per cell
+ * plain CG state is beyond SULI_PS_NOALLOC_MAX_BYTES (about 80 B per cell
  * in FP64, 104 B in mixed precision, so up to about 0.8 M / 0.64 M cells) is
  * rejected with SULI_PS_EINVAL and a message giving both sizes; with
  * opts.autotune it uses a tile shape already tuned for the size, or the
@@ -394,7 +394,8 @@ int suli_ps_graddin_batch_dev(suli_ps_ctx *ctx, suli_ps_problem *probs, int32_t 
  *
  * A server owns a device stream, a copy stream and two threads.  Requests
  * (host arrays in the layouts above) are admitted in arrival order while
- * their device memory (fields plus solver state) fits the HBM budget; their
+ * their device memory (fields plus solver state: in FP64 about 115 B per cell, or
+ * 80 and plain CG where the budget holds no more) fits the HBM budget; their
  * inputs are copied while other requests iterate, and every admitted
  * request joins the running batch at the next chunk of CG steps (the
  * kernels of suli_ps_graddin_batch_dev).  Each result is bit-identical to
@@ -464,7 +465,8 @@ int suli_ps_time_spmv(suli_ps_ctx *ctx, int32_t precision, int32_t reps, double 
  * that size then use it when opts.autotune is set.  A result depends on
  * the tiling (the order of its sums), so solves of one size agree bit for
  * bit only under the same choice.  suli_ps_set_tiles fixes a shape
- * instead (vx 1, 2 or 4; 1 for FP64 and where nx is not a multiple).
+ * instead, and solves of that size then iterate by plain CG, whose kernels it
+ * shapes (vx 1, 2 or 4; 1 for FP64 and where nx is not a multiple).
  *
  * With two or four cells per lane the FP32 step comes in two kinds: its
  * plane walk issued plane by plane, or pipelined (each plane's loads issued

@@ -36,9 +36,9 @@
 // two on either side of the coarser levels are one pass.
 //
 // Measured at 256x128x96 from prd1 = 0 to 1e-12 relative: plain CG 37.8 ms
-// (1992 iterations of one 18.5 us launch), this 3.39 ms (17 iterations); the
-// stretched masked cylinder at 384x192x128 238.4 and 10.8 ms, SuLi-IT's
-// 256x128x48 19.4 and 3.1 ms, twelve uneven tanks in a batch 67.7 and 6.0 ms.
+// (1992 iterations of one 18.5 us launch), this 3.3 ms (18 iterations); the
+// stretched masked cylinder at 384x192x128 238.4 and 10.4 ms, SuLi-IT's
+// 256x128x48 19.4 and 3.0 ms, twelve uneven tanks in a batch 67.7 and 6.1 ms.
 //
 // One iteration n (lbot: the first level of the bottom kernel):
 //   A1      r_{n-1} = r_{n-2} - alpha q (formed where needed), t; partials r.r
@@ -54,7 +54,8 @@
 //   k_true_residual, k_mg_decide: converged, or on with the replaced residual
 // FP64: before A1, upd64 (r -= alpha q, its FP32 copy, partials r.r); instead
 // of dir, dir64 (ps_cg.hip; e -= alpha p), which ends the solve when A2 found
-// r.r at the threshold.
+// r.r at the threshold.  Problems in bricks (pd.brick): A1 and A2 in one launch
+// (down), r.r judged by the bottom kernel, B1 and B2 in one (up).
 // Each total is summed by the kernel that needs it from the partials of an
 // earlier launch, as in ps_cg.hip.
 #include <algorithm>
