@@ -743,10 +743,12 @@ int Engine::mg_steps_ahead() const
         if (!(now > 0.0 && target > 0.0 && now < c.rr0)) return kMgChunk;
         const double rate = std::log(c.rr0 / now) / (c.iters > 1 ? c.iters - 1 : 1);
         const double base = c.refreshes ? c.rr_after : c.rr0;
-        int left = now > target ? (int)std::ceil(std::log(now / target) / rate) : 0;
-        left += 1;                                   // its end
-        if (c.mixed && base > 0.0) left += std::max(0, (int)std::ceil(std::log(base / target) / -std::log(kMgCycleDrop)) - 1);
-        most = std::max(most, left - (mstep_ - status_seen_));
+        double left = now > target ? std::ceil(std::log(now / target) / rate) : 0.0;
+        if (c.mixed && base > target)                // replacements on the way
+            left += std::max(0.0, std::ceil(std::log(base / target) / -std::log(kMgCycleDrop)) - 1.0);
+        if (!(left < 1000.0)) return kMgChunk;
+        left += 1.0;                                 // its end
+        most = std::max(most, (int)left - (mstep_ - status_seen_));
     }
     return most;
 }

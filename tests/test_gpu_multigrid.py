@@ -241,3 +241,51 @@ def test_step_is_timed(solver, shape, precision):
             assert st.spmv_timed > 0 and 0.0 < st.spmv_ms < st.solve_ms, st.as_dict()
     finally:
         df.free()
+
+
+def masked(name):
+    """(case, number of connected fluid parts)"""
+    nx, ny, nz = 70, 26, 20
+    px = name.endswith("_px")
+    c = cases.random_case(nx, ny, nz, 81, periodic_x=px)
+    m = np.zeros((nx, ny, nz), np.uint8, order="F")
+    base = name.removesuffix("_px")
+    if base == "wall_x_at_64":
+        m[64] = 1
+    elif base == "wall_y":
+        m[:, 12] = 1
+    elif base == "wall_z":
+        m[:, :, 9] = 1
+    elif base == "gap_in_x":       # two runs of a row, joined by its last rows
+        m[31, :ny - 4] = 1
+    elif base == "gap_in_y":       # two stretches, joined in the last columns
+        m[:nx - 5, 12] = 1
+    elif base == "gap_in_z":
+        m[:, :ny - 4, 9] = 1
+    elif base == "blocks":
+        m[10:20, 5:15, 3:12] = m[40:66, 10:22, 6:20] = 1
+    c.fields.solid = m
+    parts = 2 if base in ("wall_y", "wall_z") or name == "wall_x_at_64" else 1
+    return c, parts
+
+
+@pytest.mark.parametrize("name", ["wall_x_at_64", "wall_x_at_64_px", "wall_y", "wall_z", "gap_in_x", "gap_in_x_px",
+                                  "gap_in_y", "gap_in_z", "blocks", "blocks_px"])
+def test_parts_of_a_mask(solver, name):
+    """Fluid in one part is solved by the multigrid iteration, in several by
+    plain CG (hundreds of iterations); either agrees with the oracle.  (In FP64:
+    plain CG's mixed iteration lets each part's mean drift with FP32's rounding,
+    3e-7 of the pressure over wall_z.)"""
+    c, parts = masked(name)
+    print(f"multigrid mask {name}", flush=True)
+    p_or, _, rc = oracle.graddin(c.grid, c.fields, stop_rule=oracle.STOP_RELATIVE, tol=1e-12, project_null=True)
+    assert rc == 0
+    solver.configure(precision="fp64", stop_rule="relative", tol=1e-12, verbose=False)
+    df = solver.upload(c.grid, c.fields)
+    try:
+        st = solver.graddin_dev(c.grid, df)
+        p = df.download("prd1")
+    finally:
+        df.free()
+    assert st.status == 0 and (st.iters < 60) == (parts == 1), (name, st.as_dict())
+    assert helpers.rel_diff(p, p_or, helpers.face_mask(p.shape)) <= PRESSURE_RTOL
