@@ -1618,39 +1618,47 @@ __device__ __forceinline__ void coarse_cell(const MgLevel &F, const MgLevel &C, 
         return F.sy[(k * (ny + 1) + f) * nx + i] * F.w[at(i, a, k)] * F.w[at(i, b, k)];
     };
     auto fz = [&](int i, int j, int f) {
-        return F.sz[(f * ny + j) * nx + i] * F.w[at(i, j, f)] * F.w[at(i, j, f - 1)];
+        return F.sz[(f * ny + j) * nx + i] * F.w[at(i, j, f)] * F.w[at(i, j, max(f - 1, 0))];
     };
-    const int j1 = min(2 * J + 2, ny), k1 = min(2 * K + 2, nz), i1 = min(2 * I + 2, nx);
+    // the two fine cells of a coarse one in each direction; a side of odd
+    // length repeats its last, which then does not count.  No load waits for
+    // another: with loops over the cells that are there each waited for the one
+    // before (a level of 16384 cells 9.3 us, of 2048 8.2; so 5.4 and 5.6).
+    const int is[2] = {2 * I, min(2 * I + 1, nx - 1)}, js[2] = {2 * J, min(2 * J + 1, ny - 1)};
+    const int ks[2] = {2 * K, min(2 * K + 1, nz - 1)};
+    const bool i2 = 2 * I + 1 < nx, j2 = 2 * J + 1 < ny, k2 = 2 * K + 1 < nz;
+    // sum of f(0 .. 1, 0 .. 1), second index fastest
+    auto quad = [](bool a2, bool b2, auto &&f) {
+        const float v00 = f(0, 0), v01 = f(0, 1), v10 = f(1, 0), v11 = f(1, 1);
+        float s = v00;
+        if (b2) s += v01;
+        if (a2) s += v10;
+        if (a2 && b2) s += v11;
+        return s;
+    };
     auto SX = [&](int If) -> float {   // coarse x face If (0 .. C.nx)
         const bool wall = If == 0 || If == C.nx;
-        if (wall && !C.px) return 0.f;
         const int f = If == C.nx ? nx : 2 * If;
-        float s = 0.f;
-        for (int k = 2 * K; k < k1; ++k)
-            for (int j = 2 * J; j < j1; ++j) s += fx(f, j, k);
-        return 0.5f * s;
+        const float s = quad(k2, j2, [&](int k, int j) { return fx(f, js[j], ks[k]); });
+        return wall && !C.px ? 0.f : 0.5f * s;
     };
     auto SY = [&](int Jf) -> float {
         const bool wall = Jf == 0 || Jf == C.ny;
-        if (wall && !C.py) return 0.f;
         const int f = Jf == C.ny ? ny : 2 * Jf;
-        float s = 0.f;
-        for (int k = 2 * K; k < k1; ++k)
-            for (int i = 2 * I; i < i1; ++i) s += fy(i, f, k);
-        return 0.5f * s;
+        const float s = quad(k2, i2, [&](int k, int i) { return fy(is[i], f, ks[k]); });
+        return wall && !C.py ? 0.f : 0.5f * s;
     };
     auto SZ = [&](int Kf) -> float {
-        if (Kf == 0 || Kf == C.nz) return 0.f;
-        float s = 0.f;
-        for (int j = 2 * J; j < j1; ++j)
-            for (int i = 2 * I; i < i1; ++i) s += fz(i, j, 2 * Kf);
-        return 0.5f * s;
+        const bool wall = Kf == 0 || Kf == C.nz;
+        const int f = wall ? 0 : 2 * Kf;
+        const float s = quad(j2, i2, [&](int j, int i) { return fz(is[i], js[j], f); });
+        return wall ? 0.f : 0.5f * s;
     };
     const float x0 = SX(I), x1 = SX(I + 1), y0 = SY(J), y1 = SY(J + 1), z0 = SZ(K), z1 = SZ(K + 1);
     float ex = 0.f;
     if (K == C.nz - 1) {
-        for (int j = 2 * J; j < j1; ++j)
-            for (int i = 2 * I; i < i1; ++i) {
+        for (int j = 2 * J; j < min(2 * J + 2, ny); ++j)
+            for (int i = 2 * I; i < min(2 * I + 2, nx); ++i) {
                 if (F.ex) {
                     ex += F.ex[j * nx + i];
                 } else if (lid) {
@@ -1718,7 +1726,16 @@ __global__ __launch_bounds__(kBotThreads) void k_mg_coarse_bottom(const ProbDev 
     for (int l = pd.lbot; l < pd.nlev; ++l) {
         const MgLevel L = pd.lv[l];
         const int m = L.nx * L.ny * L.nz;
-        for (int c = threadIdx.x; c < m; c += kBotThreads) reinterpret_cast<BotCell *>(pd.bot)[off + c] = bot_cell(L, c);
+        BotCell *const out = reinterpret_cast<BotCell *>(pd.bot) + off;
+        constexpr int kAhead = 3;   // cells whose loads go together
+        for (int c = threadIdx.x; c < m; c += kAhead * kBotThreads) {
+            BotCell b[kAhead];
+#pragma unroll
+            for (int q = 0; q < kAhead; ++q) b[q] = bot_cell(L, min(c + q * kBotThreads, m - 1));
+#pragma unroll
+            for (int q = 0; q < kAhead; ++q)
+                if (c + q * kBotThreads < m) out[c + q * kBotThreads] = b[q];
+        }
         off += m;
     }
 }
