@@ -453,6 +453,19 @@ int Engine::setup_slot(int si, bool multi, hipEvent_t wait_ev)
     const SolveOpts &o = sl.o;
     ProbDev &pd = sl.pd;
     int nt3 = 0, nt1 = 0;
+    if (wait_ev) ECHK(hipStreamWaitEvent(s_, wait_ev, 0));   // the inputs have arrived
+    if (multi && in.solid) {
+        // plain CG where a mask cuts the fluid into parts.  The host waits for
+        // the count (20 us): set up first and found out by the kernels, such a
+        // problem was set up twice and ran idle steps (31x156x109, FP64: 16.5
+        // ms instead of 16.0)
+        const Geo g = make_geo(gr.nx, gr.ny, gr.nz, gr.ccx0 == 0, gr.ccy0 == 0);
+        int *lab = static_cast<int *>(sl.block), *count = lab + g.n, *h = reinterpret_cast<int *>(h_final_ + si);
+        launch_mg_parts(g, in.solid, lab, count, s_);
+        ECHK(hipMemcpyAsync(h, count, sizeof(int), hipMemcpyDeviceToHost, s_));
+        ECHK(hipStreamSynchronize(s_));
+        multi = *h <= 1;
+    }
     // the multigrid kernels have a tiling of their own: the replacement's
     // kernels, which walk one cell per lane, take the default shape
     sl.mg = false;
@@ -541,8 +554,7 @@ int Engine::setup_slot(int si, bool multi, hipEvent_t wait_ev)
         ECHK(hipEventRecord(ev_stage_[stg], s_));
     }
 
-    // setup kernels (ps_setup.hip), after the inputs have arrived
-    if (wait_ev) ECHK(hipStreamWaitEvent(s_, wait_ev, 0));
+    // setup kernels (ps_setup.hip)
     double *sx = const_cast<double *>(pd.sx), *sy = const_cast<double *>(pd.sy), *sz = const_cast<double *>(pd.sz);
     launch_face_coefs(sl.g, in, sx, sy, sz, s_);
     launch_diag_rhs(sl.g, in, sx, sy, sz, const_cast<double *>(pd.d), pd.b, pd.e, s_);

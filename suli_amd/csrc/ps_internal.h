@@ -154,7 +154,6 @@ struct CgScalars {
     double rz[2];     // multigrid: r.z of iteration n in slot n & 1
     int mg;           // 1: multigrid-preconditioned
     int giveup;       // 1: the multigrid iteration broke down; solved again by CG
-    int parts;        // connected parts of a masked problem's fluid
     int stalls;       // replacements in a row that did not halve r.r
     int lag_stop;     // 1: the FP64 stop test reads the r.r that entered the previous
                       // iteration (SuLi-IT's loop, SuLi-IT/9_grad.f90:165-177)
@@ -396,6 +395,8 @@ bool mg_plan(const Geo &g, float *w32, float *space, size_t floats, float *scrat
 // Table entries of level l's kernels.
 int mg_level_tiles(const ProbDev &pd, int l);
 // Weights and coarse operators, after launch_init; dev: pd on the device.
+// Connected parts of a masked grid's fluid into *count (labels in lab, a word a cell).
+void launch_mg_parts(const Geo &g, const uint8_t *solid, int *lab, int *count, hipStream_t s);
 void launch_mg_setup(const ProbDev &pd, const ProbDev *dev, const SetupIn &in, hipStream_t s);
 struct MgTables {
     const TileRef *fine = nullptr, *lev[kMgLevels] = {};

@@ -1488,11 +1488,13 @@ __device__ __forceinline__ void join(int *p, int a, int b)
 // point at the strip's root at once; where a run finds two, they are joined.
 // With runs joined row by row instead, the paths grew as long as the grid is
 // wide: 444 us over 384x192x128, this and k_mg_join 103 and 67.
-__global__ __launch_bounds__(kThreads) void k_mg_label(Geo g, const uint8_t *__restrict__ solid, int *__restrict__ p)
+__global__ __launch_bounds__(kThreads) void k_mg_label(Geo g, const uint8_t *__restrict__ solid, int *__restrict__ p,
+                                                       int *count)
 {
     const int nx = g.nx, ny = g.ny, parts = (nx + 63) / 64, lane = threadIdx.x & 63;
     const int t = blockIdx.x * (kThreads / 64) + threadIdx.x / 64;
-    if (t >= parts * g.nz) return;   // the whole wave
+    if (t == 0 && lane == 0) *count = 0;   // for k_mg_roots
+    if (t >= parts * g.nz) return;         // the whole wave
     const int i = t % parts * 64 + lane;
     const long long base = (long long)(t / parts) * ny * nx + i;
     const bool col = i < nx;
@@ -1586,16 +1588,6 @@ __global__ __launch_bounds__(kThreads) void k_mg_roots(long long n, const int *p
     int roots = 0;
     for (long long c = (long long)blockIdx.x * kThreads + threadIdx.x; c < n; c += stride) roots += p[c] == (int)c;
     if (roots) atomicAdd(count, roots);
-}
-
-// More than one part: the solve ends here and is set up again as plain CG.
-__global__ void k_mg_parts(CgScalars *S)
-{
-    if (threadIdx.x == 0 && S->parts > 1 && !S->final_) {
-        S->giveup = 1;
-        S->final_ = 1;
-        S->done_at = 0;
-    }
 }
 
 // One coarse cell: its un-scaled low faces (and the far ones of the last
@@ -1852,18 +1844,18 @@ bool mg_plan(const Geo &g, float *w32, float *space, size_t floats, float *scrat
 
 int mg_level_tiles(const ProbDev &pd, int l) { return l < pd.lbot && (l || pd.brick) ? bricks(pd.lv[l]) : 0; }
 
+void launch_mg_parts(const Geo &g, const uint8_t *solid, int *lab, int *count, hipStream_t s)
+{
+    const int strips = (g.nx + 63) / 64 * g.nz, grid = (strips + kThreads / 64 - 1) / (kThreads / 64);
+    hipLaunchKernelGGL(k_mg_label, dim3(grid), dim3(kThreads), 0, s, g, solid, lab, count);
+    hipLaunchKernelGGL(k_mg_join, dim3(grid), dim3(kThreads), 0, s, g, lab);
+    hipLaunchKernelGGL(k_mg_roots, dim3(std::min(blocks(g.n), 2048)), dim3(kThreads), 0, s, g.n, lab, count);
+}
+
 void launch_mg_setup(const ProbDev &pd, const ProbDev *dev, const SetupIn &in, hipStream_t s)
 {
     const long long n = pd.g.n;
     const float top = in.it ? (float)(1.0 / (in.gz * in.tetah * in.dt)) : 0.f;
-    if (in.solid) {
-        int *lab = reinterpret_cast<int *>(pd.q32b);
-        const int strips = (pd.g.nx + 63) / 64 * pd.g.nz, grid = (strips + kThreads / 64 - 1) / (kThreads / 64);
-        hipLaunchKernelGGL(k_mg_label, dim3(grid), dim3(kThreads), 0, s, pd.g, in.solid, lab);
-        hipLaunchKernelGGL(k_mg_join, dim3(grid), dim3(kThreads), 0, s, pd.g, lab);
-        hipLaunchKernelGGL(k_mg_roots, dim3(std::min(blocks(n), 2048)), dim3(kThreads), 0, s, n, lab, &pd.S->parts);
-        hipLaunchKernelGGL(k_mg_parts, dim3(1), dim3(64), 0, s, pd.S);
-    }
     hipLaunchKernelGGL(k_mg_weights, dim3(std::min(blocks(n), 4096)), dim3(kThreads), 0, s, n, pd.d, in.solid, pd.w32);
     for (int l = 1; l <= pd.lbot; ++l) {
         const int b = blocks(cells(pd.lv[l]));
