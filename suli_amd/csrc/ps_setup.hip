@@ -790,22 +790,40 @@ __global__ __launch_bounds__(kWThreads) void k_posdin_hydro_w(Geo g, const doubl
 // posdin's hydrostatic branch, last: u and v zeroed on the faces where hs
 // is below 1e-4 (SuLi-IC/10_pos.f90:64-82).  Runs after the w sweep, which
 // reads the values before zeroing.
+// Two planes a thread, at 256x128x96: 16.8 us; one 19.7, four 18.0, eight 20.1.
+constexpr int kUvPlanes = 2;
 __global__ __launch_bounds__(kThreads) void k_posdin_hydro_uv(Geo g, const double *hs, double *u, double *v)
 {
-    const int nx = g.nx, ny = g.ny;
-    // one thread per cell of the cell tiles: its low x and y faces, and in
-    // the last column and row the high one too
-    for_cells(g, [&](int i, int j, int k) {
-        const long long iu = (i + 1) + (long long)(nx + 3) * ((j + 1) + (long long)(g.ny + 2) * (k + 1));
-        const long long iv = (i + 1) + (long long)(nx + 2) * ((j + 1) + (long long)(g.ny + 3) * (k + 1));
-        const bool cx0 = face_x(g, hs, i, j, k) < 0.0001, cy0 = face_y(g, hs, i, j, k) < 0.0001;
+    const int nx = g.nx, ny = g.ny, nz = g.nz;
+    // one thread per column of a tile of 64 x 4 cells and kUvPlanes planes: its
+    // cells' low x and y faces, and in the last column and row the high ones
+    // too; all planes' loads before the first store
+    const int tx = (nx + 63) / 64, ty = (ny + 3) / 4;
+    const int row = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int t = xcd_tile(blockIdx.x, gridDim.x), r = t / tx;
+    const int i = t % tx * 64 + (threadIdx.x & 63), j = r % ty * 4 + row, k0 = r / ty * kUvPlanes;
+    if (i >= nx || j >= ny) return;
+    double x0[kUvPlanes], x1[kUvPlanes], y0[kUvPlanes], y1[kUvPlanes];
+#pragma unroll
+    for (int q = 0; q < kUvPlanes; ++q) {
+        const int k = min(k0 + q, nz - 1);
+        x0[q] = face_x(g, hs, i, j, k);
         // face i + 1 is in range for every lane; the last column acts on it
-        const bool cx1 = face_x(g, hs, i + 1, j, k) < 0.0001;
-        if (cx0) u[iu] = 0.;
-        if (i == nx - 1 && cx1) u[iu + 1] = 0.;
-        if (cy0) v[iv] = 0.;
-        if (j == ny - 1 && face_y(g, hs, i, ny, k) < 0.0001) v[iv + (nx + 2)] = 0.;
-    });
+        x1[q] = face_x(g, hs, i + 1, j, k);
+        y0[q] = face_y(g, hs, i, j, k);
+        y1[q] = j == ny - 1 ? face_y(g, hs, i, ny, k) : 1.0;
+    }
+#pragma unroll
+    for (int q = 0; q < kUvPlanes; ++q) {
+        const int k = k0 + q;
+        if (k >= nz) break;
+        const long long iu = (i + 1) + (long long)(nx + 3) * ((j + 1) + (long long)(ny + 2) * (k + 1));
+        const long long iv = (i + 1) + (long long)(nx + 2) * ((j + 1) + (long long)(ny + 3) * (k + 1));
+        if (x0[q] < 0.0001) u[iu] = 0.;
+        if (i == nx - 1 && x1[q] < 0.0001) u[iu + 1] = 0.;
+        if (y0[q] < 0.0001) v[iv] = 0.;
+        if (y1[q] < 0.0001) v[iv + (nx + 2)] = 0.;
+    }
 }
 
 // heaviside with t_tens = 0 (SuLi-IC/14_level_set.f90:555-590): the
@@ -1368,7 +1386,8 @@ void launch_posdin_hydro(const Geo &g, const SetupIn &in, const double *hs, doub
     else
         hipLaunchKernelGGL(k_posdin_hydro_w<false>, grid, dim3(kWThreads), 0, s, g, u, v, hs, in.dz, in.dzu, in.dx,
                            in.dy, w);
-    hipLaunchKernelGGL(k_posdin_hydro_uv, cell_grid(g), dim3(kThreads), 0, s, g, hs, u, v);
+    const int uv_tiles = (g.nx + 63) / 64 * ((g.ny + 3) / 4) * ((g.nz + kUvPlanes - 1) / kUvPlanes);
+    hipLaunchKernelGGL(k_posdin_hydro_uv, dim3(uv_tiles), dim3(kThreads), 0, s, g, hs, u, v);
 }
 
 }  // namespace sps
