@@ -164,12 +164,13 @@ struct TotalCache {
 // FIRST (iteration 1: p_1 = r_0, nothing to finish) and DO_E (apply the
 // deferred e -= alpha p) are template parameters so that the plane loop has
 // no branches: every load of a plane is issued before any is waited for.
-// R: the type r is stored in (the multigrid step passes its FP32 z).
+// R: the type r is stored in, r = rs r as stored (the multigrid step passes its
+// scaled FP32 z; rs is not used where the types agree).
 template <typename T, bool FIRST, bool DO_E, class CO, typename R = T>
 __device__ __forceinline__ double cg_a_tile(const Geo &g, const Tile &t, gptr<T> __restrict__ e,
                                             gptr<const T> __restrict__ p_old, gptr<T> __restrict__ p_new,
                                             gptr<const R> __restrict__ r, const CO &co, gptr<T> __restrict__ q, T b,
-                                            T a_prev)
+                                            T a_prev, T rs = T(1))
 {
     const int nx = g.nx, ny = g.ny, nz = g.nz;
     const long long plane = (long long)nx * ny;
@@ -182,9 +183,15 @@ __device__ __forceinline__ double cg_a_tile(const Geo &g, const Tile &t, gptr<T>
     long long fx = ((long long)t.k0 * ny + t.j) * (nx + 1) + t.i;
     long long fy = ((long long)t.k0 * (ny + 1) + t.j) * nx + t.i;
     // p_n = r + beta p_{n-1} (9_grad.f90:518-527), formed where needed
-    auto pn = [&](long long x) -> T { return FIRST ? (T)r[x] : (T)r[x] + b * p_old[x]; };
+    auto dir = [&](long long x, T po) -> T {
+        if constexpr (std::is_same_v<R, T>)
+            return FIRST ? r[x] : r[x] + b * po;
+        else   // (rs is a power of two: the one rounding is fma's)
+            return FIRST ? rs * (T)r[x] : fma(b, po, rs * (T)r[x]);
+    };
+    auto pn = [&](long long x) -> T { return dir(x, FIRST ? T(0) : p_old[x]); };
     T poc = FIRST ? T(0) : p_old[c];
-    T pc = FIRST ? (T)r[c] : (T)r[c] + b * poc;
+    T pc = dir(c, poc);
     T pb = t.k0 > 0 ? pn(c - plane) : pc;
     T szb = co.z(c, t.k0);
     for (int k = t.k0; k < t.k1; ++k) {
@@ -192,7 +199,7 @@ __device__ __forceinline__ double cg_a_tile(const Geo &g, const Tile &t, gptr<T>
         // top neighbour; at the lid the mirror ghost is the cell itself
         const long long up = (k < nz - 1) ? plane : 0;
         const T pot = FIRST ? T(0) : p_old[c + up];
-        const T pt = FIRST ? (T)r[c + up] : (T)r[c + up] + b * pot;
+        const T pt = dir(c + up, pot);
         const T szt = co.z(c + plane, k + 1);
         const T pw = pn(r0 + iw), pe = pn(r0 + ie);
         const T ps = pn(c + dS), pnn = pn(c + dN);
@@ -335,10 +342,13 @@ __global__ __launch_bounds__(kThreads) void k_mg_dir64(const ProbDev *__restrict
         const int done_at = S->done_at;
         const bool due = S->next_refresh == n;
         const double rz_prev = S->rz[(n - 1) & 1], alpha = S->alpha, rr = S->rr[n & 1], thresh = S->thresh;
+        const double rr_prev = S->rr[(n - 1) & 1];
         if (n < 1 || n > done_at) continue;
         const bool first = n == 1;
-        const double rz = due ? 0.0 : rz_tot.get(tr.prob, pd.P.m4 + pd.ntm, pd.ntm);
-        const bool bad = !(rz >= 0.0 && rz < 1e300) || !(alpha >= 0.0 && alpha < 1e300);
+        // z, and so r.z, as the V-cycle was given r
+        const double zs = ldexp(1.0, mg_shift(rr_prev));
+        const double rz = due ? 0.0 : rz_tot.get(tr.prob, pd.P.m4 + pd.ntm, pd.ntm) * zs * zs;
+        const bool bad = mg_breakdown(first, due, rz, alpha);
         const double beta = first || !(rz_prev > 0.0) ? 0.0 : rz / rz_prev;
         if (tr.tile == 0 && threadIdx.x == 0) {
             if (bad || due) {
@@ -369,8 +379,8 @@ __global__ __launch_bounds__(kThreads) void k_mg_dir64(const ProbDev *__restrict
         const double acc = with_coefs(V, [&](const auto &co) {
             using CO = std::decay_t<decltype(co)>;
             if (first)
-                return cg_a_tile<double, true, false, CO, float>(pd.g, tl, V.e, p_old, p_new, z, co, V.q, beta, alpha);
-            return cg_a_tile<double, false, true, CO, float>(pd.g, tl, V.e, p_old, p_new, z, co, V.q, beta, alpha);
+                return cg_a_tile<double, true, false, CO, float>(pd.g, tl, V.e, p_old, p_new, z, co, V.q, beta, alpha, zs);
+            return cg_a_tile<double, false, true, CO, float>(pd.g, tl, V.e, p_old, p_new, z, co, V.q, beta, alpha, zs);
         });
         const double s = block_sum(acc);
         if (threadIdx.x == 0) pd.P.spmv[tr.tile] = s;

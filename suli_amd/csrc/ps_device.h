@@ -176,6 +176,20 @@ __device__ __forceinline__ int xcd_tile(int b, int n)
     return xcd * per + min(xcd, rem) + local;
 }
 
+// FP64 multigrid iterations hand the V-cycle r 2^-e in FP32, with e from the r.r
+// that entered the iteration before (S->rr), so that its size is about 1 whatever r's
+// is: unscaled, an r below FP32's range became 0, z with it, and the solve ran idle
+// steps to its cap.  Powers of two change no rounding: within FP32's range z 2^e has
+// the bits that r's own copy gives.
+__device__ __forceinline__ int mg_shift(double rr) { return rr > 0.0 && rr < 1e300 ? ilogb(rr) / 2 : 0; }
+
+// Whether a direction step's r.z or alpha = r.z / p.q says that the iteration broke
+// down (first: of the directions, alpha is 0; due: no direction is formed).
+__device__ __forceinline__ bool mg_breakdown(bool first, bool due, double rz, double alpha)
+{
+    return !(alpha >= 0.0 && alpha < 1e300) || (!due && (!(rz > 0.0 && rz < 1e300) || (!first && alpha == 0.0)));
+}
+
 // Neighbour index along one direction with the reference's ghost rule:
 // mirror (ghost = first interior cell, 9_grad.f90:531-579) or periodic.
 __device__ __forceinline__ int nb_lo(int i, int n, int periodic) { return i > 0 ? i - 1 : (periodic ? n - 1 : 0); }

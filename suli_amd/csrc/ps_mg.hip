@@ -11,8 +11,8 @@
 // the FP64 true residual.  FP64 solves by the relative rule: the iterate, the
 // residual, the directions, the operator and the stop test are FP64 as in
 // plain CG (ps_cg.hip), and only the V-cycle works on an FP32 copy of the
-// residual; which z it returns changes the number of iterations, not what
-// r = A e - b reaches.
+// residual (scaled by a power of two, mg_shift); which z it returns changes the
+// number of iterations, not what r = A e - b reaches.
 //
 // The V-cycle smooths with a Chebyshev polynomial of degree two before and
 // after the coarse correction on every level.  A coarse cell joins 2x2x2
@@ -503,7 +503,8 @@ __device__ __forceinline__ bool judge(gptr<CgScalars> S, bool mixed, bool fresh,
 
 // alpha and beta of a mixed problem's direction step; false at a breakdown:
 // r.z and p.q are positive for every operator the V-cycle is definite for,
-// unless a value left FP32's range.  A replacement starts the directions
+// unless a value left FP32's range (upwards: infinities and NaN; downwards: a
+// sum of 0 with r.r above its threshold).  A replacement starts the directions
 // afresh: the replaced residual is no longer r - alpha q, and directions
 // conjugate to it went on at a third of the rate.
 __device__ __forceinline__ bool direction(gptr<CgScalars> S, bool fresh, bool due, int n, double rz, bool store,
@@ -511,7 +512,7 @@ __device__ __forceinline__ bool direction(gptr<CgScalars> S, bool fresh, bool du
 {
     const double rz_prev = S->rz[(n - 1) & 1];
     alpha = S->alpha;
-    const bool bad = !(rz >= 0.0 && rz < 1e300) || !(alpha >= 0.0 && alpha < 1e300);
+    const bool bad = mg_breakdown(fresh, due, rz, alpha);
     beta = fresh || !(rz_prev > 0.0) ? 0.0 : rz / rz_prev;
     if (store) {
         if (bad) {
@@ -599,7 +600,7 @@ __global__ __launch_bounds__(kThreads, fine_waves(KIND)) void k_mg_fine(const Pr
     fine_tiles<KIND>(P, tab, my_run(ntab), st, ran);
 }
 
-// FP64: r_{n-1} = r_{n-2} - alpha_{n-1} q_{n-1} and its FP32 copy for the
+// FP64: r_{n-1} = r_{n-2} - alpha_{n-1} q_{n-1} and its scaled FP32 copy for the
 // V-cycle, r.r partials (1-D tiles).
 __global__ __launch_bounds__(kThreads) void k_mg_upd64(const ProbDev *__restrict__ P, const TileRef *__restrict__ tab,
                                                        int ntab, MgStep st)
@@ -616,8 +617,9 @@ __global__ __launch_bounds__(kThreads) void k_mg_upd64(const ProbDev *__restrict
         const int n = step - pd.n0 + 1;
         if (n < 1 || n > S->done_at) continue;
         const bool first = n == 1;
-        const double rz = S->rz[(n - 1) & 1];
+        const double rz = S->rz[(n - 1) & 1], rr = S->rr[(n - 1) & 1];
         const double pq = first ? 0.0 : tot.get(tr.prob, pd.P.spmv, pd.nt3);
+        const double scale = ldexp(1.0, -mg_shift(rr));
         const double alpha = pq != 0.0 ? rz / pq : 0.0;
         if (tr.tile == 0 && threadIdx.x == 0) S->alpha = alpha;
         const gptr<double> r = glob(pd.r);
@@ -637,7 +639,7 @@ __global__ __launch_bounds__(kThreads) void k_mg_upd64(const ProbDev *__restrict
 #pragma unroll
             for (int m = 0; m < 4; ++m) {
                 acc += rv[m] * rv[m];
-                f[m] = (float)rv[m];
+                f[m] = (float)(scale * rv[m]);
             }
             ((gptr<va4>)r32)[v] = f;
         }
@@ -646,7 +648,7 @@ __global__ __launch_bounds__(kThreads) void k_mg_upd64(const ProbDev *__restrict
             if (c < len) {
                 const double rv = first ? r[c] : r[c] - alpha * q[c];
                 r[c] = rv;
-                r32[c] = (float)rv;
+                r32[c] = (float)(scale * rv);
                 acc += rv * rv;
             }
         }
