@@ -5,7 +5,9 @@ of two give the same bits, scaled.
 import numpy as np
 import pytest
 
+import oracle
 from suli_amd import cases
+from tests import helpers
 
 pytestmark = pytest.mark.gpu
 
@@ -39,3 +41,57 @@ def test_fp64_residuals_beyond_fp32(solver, shape):
         p, st = solve(solver, c, cases.scale_velocity(c.fields, 2.0 ** e))
         assert st.status == 0 and st.iters == st0.iters, (e, st.as_dict())
         np.testing.assert_array_equal(p, p0 * 2.0 ** e)
+
+
+def breaking(shape, seed):
+    """A density so small that the operator's diagonal is beyond FP32 (2^280): the
+    V-cycle's weights are infinite and the iteration breaks down in its first step.
+    The velocity is scaled so that the scaled system's vectors are the plain case's,
+    and the pressure is 2^-140 times its."""
+    c = cases.random_case(*shape, seed)
+    fields = cases.scale_velocity(c.fields, 2.0 ** 140)
+    fields.rho = np.asfortranarray(fields.rho * 2.0 ** -280)
+    c.plain, c.fields = c.fields, fields
+    return c
+
+
+BREAKING = [(40, 32, 24), (70, 60, 40)]   # bricks, marched
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("mixed", 1e-11)], ids=["fp64", "mixed"])
+def test_breakdown_is_solved_again_by_plain_cg(solver, precision, tol):
+    """Alone, without allocation, in a batch beside problems that do not break
+    down, and through the server: plain CG's solution, and every neighbour as it
+    is alone.  (The second set-up happens with another chunk of steps in flight.)"""
+    from suli_amd.server import PressureServer
+    cs = [breaking(BREAKING[0], 92), cases.random_case(48, 40, 36, 93), breaking(BREAKING[1], 94),
+          cases.random_case(66, 50, 44, 95), cases.random_case(20, 16, 12, 96)]
+    print(f"multigrid breakdown {precision}", flush=True)
+    solver.configure(precision=precision, stop_rule="relative", tol=tol, verbose=False)
+    alone = [solve(solver, c, c.fields) for c in cs]
+    for c, (p, st) in zip(cs, alone):
+        assert st.status == 0, st.as_dict()
+        if hasattr(c, "plain"):
+            p_or, _, rc = oracle.graddin(c.grid, c.plain, stop_rule=oracle.STOP_RELATIVE, tol=1e-12,
+                                         project_null=True)
+            assert rc == 0 and st.iters > 150   # plain CG's count
+            assert helpers.rel_diff(p * 2.0 ** 140, p_or, helpers.face_mask(p.shape)) <= 1e-8
+    df = solver.upload(cs[0].grid, cs[0].fields)
+    st = solver.graddin_noalloc_dev(cs[0].grid, df)
+    assert st.iters == alone[0][1].iters
+    np.testing.assert_array_equal(df.download("prd1"), alone[0][0])
+    df.free()
+    for _ in range(2):   # the slots serve again
+        dfs = [solver.upload(c.grid, c.fields) for c in cs]
+        sts = solver.graddin_batch_dev([(c.grid, df) for c, df in zip(cs, dfs)])
+        for i, (df, st) in enumerate(zip(dfs, sts)):
+            assert st.status == 0 and st.iters == alone[i][1].iters, (i, st.as_dict())
+            np.testing.assert_array_equal(df.download("prd1"), alone[i][0])
+            df.free()
+    with PressureServer(precision=precision, stop_rule="relative", tol=tol) as srv:
+        fields = [c.fields.copy() for c in cs]
+        tickets = [srv.submit(c.grid, f) for c, f in zip(cs, fields)]
+        for i, (f, t) in enumerate(zip(fields, tickets)):
+            st = srv.wait(t)
+            assert st.status == 0 and st.iters == alone[i][1].iters, i
+            np.testing.assert_array_equal(f.prd1, alone[i][0])
