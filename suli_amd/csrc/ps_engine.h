@@ -15,6 +15,11 @@
 
 namespace sps {
 
+// hipMalloc whose failure the caller reports or gets round: the runtime keeps the
+// error until it is read, through later successful calls, and the next check of a
+// launch would find it.
+hipError_t device_alloc(void **p, size_t bytes);
+
 // Device memory handed out in whole blocks and kept for reuse by size.
 class Pool {
 public:

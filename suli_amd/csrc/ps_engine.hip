@@ -124,6 +124,13 @@ bool no_alloc_active() { return t_no_alloc; }
 NoAllocScope::NoAllocScope() : prev_(t_no_alloc) { t_no_alloc = true; }
 NoAllocScope::~NoAllocScope() { t_no_alloc = prev_; }
 
+hipError_t device_alloc(void **p, size_t bytes)
+{
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
+
 // ---------------------------------------------------------------- Pool ----
 Pool::~Pool() { release_all(); }
 
@@ -141,12 +148,12 @@ void *Pool::get(size_t bytes, std::string &err)
         return nullptr;
     }
     void *p = nullptr;
-    hipError_t e = hipMalloc(&p, bytes);
+    hipError_t e = device_alloc(&p, bytes);
     if (e != hipSuccess) {
         // give back cached blocks of other sizes and retry once
         for (auto &kv : free_) (void)hipFree(kv.second), held_ -= kv.first;
         free_.clear();
-        e = hipMalloc(&p, bytes);
+        e = device_alloc(&p, bytes);
         if (e != hipSuccess) {
             err = std::string("hipMalloc failed: ") + hipGetErrorString(e);
             return nullptr;

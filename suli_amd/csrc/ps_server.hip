@@ -169,7 +169,7 @@ void *suli_ps_server::alloc_block(size_t bytes, std::string &e)
         // device thread is capturing
         std::lock_guard<std::mutex> cl(mcap);
         for (auto &d : drop) (void)hipFree(d.second);
-        he = hipMalloc(&p, bytes);
+        he = device_alloc(&p, bytes);
     }
     if (he != hipSuccess) {
         std::lock_guard<std::mutex> lk(m);

@@ -467,7 +467,7 @@ int ensure_staging(suli_ps_ctx *ctx, int nx, int ny, int nz)
         off[i] = total;
         total += (sizes[i] * sizeof(double) + 255) / 256 * 256;
     }
-    hipError_t e = hipMalloc(&st.block, total);
+    hipError_t e = device_alloc(&st.block, total);
     if (e != hipSuccess) return fail(ctx, SULI_PS_ENOMEM, "hipMalloc(%zu) failed: %s", total, hipGetErrorString(e));
     double **ptrs[18] = {&st.u,   &st.v,   &st.w,   &st.rho, &st.prd1, &st.obsx,   &st.obsy, &st.obsz, &st.dz,
                          &st.dzz, &st.hs,  &st.dzx, &st.dzy, &st.dz3,  &st.eta1, &st.deltah, &st.box2, &st.eta0};
@@ -959,7 +959,7 @@ int suli_ps_graddin_batch_dev(suli_ps_ctx *ctx, suli_ps_problem *probs, int32_t 
 void *suli_ps_dev_alloc(suli_ps_ctx *ctx, size_t bytes)
 {
     void *p = nullptr;
-    if (hipMalloc(&p, std::max<size_t>(bytes, 1)) != hipSuccess) {
+    if (device_alloc(&p, std::max<size_t>(bytes, 1)) != hipSuccess) {
         if (ctx) ctx->err = "hipMalloc failed";
         return nullptr;
     }
@@ -1045,8 +1045,8 @@ int suli_ps_copy_bench(suli_ps_ctx *ctx, size_t bytes, int32_t reps, double *ms)
     if (!ctx || !ms || reps <= 0 || bytes < 16) return SULI_PS_EINVAL;
     const size_t n16 = bytes / 16;
     void *a = nullptr, *b = nullptr;
-    if (hipMalloc(&a, n16 * 16) != hipSuccess) return fail(ctx, SULI_PS_ENOMEM, "hipMalloc(%zu) failed", bytes);
-    if (hipMalloc(&b, n16 * 16) != hipSuccess) {
+    if (device_alloc(&a, n16 * 16) != hipSuccess) return fail(ctx, SULI_PS_ENOMEM, "hipMalloc(%zu) failed", bytes);
+    if (device_alloc(&b, n16 * 16) != hipSuccess) {
         (void)hipFree(a);
         return fail(ctx, SULI_PS_ENOMEM, "hipMalloc(%zu) failed", bytes);
     }
@@ -1073,8 +1073,8 @@ int suli_ps_read_bench(suli_ps_ctx *ctx, size_t bytes, int32_t reps, double *ms)
     const size_t n16 = bytes / 16;
     void *a = nullptr;
     float *out = nullptr;
-    if (hipMalloc(&a, n16 * 16) != hipSuccess) return fail(ctx, SULI_PS_ENOMEM, "hipMalloc(%zu) failed", bytes);
-    if (hipMalloc(&out, sizeof(float) * kReadGrid * kThreads) != hipSuccess) {
+    if (device_alloc(&a, n16 * 16) != hipSuccess) return fail(ctx, SULI_PS_ENOMEM, "hipMalloc(%zu) failed", bytes);
+    if (device_alloc((void **)&out, sizeof(float) * kReadGrid * kThreads) != hipSuccess) {
         (void)hipFree(a);
         return fail(ctx, SULI_PS_ENOMEM, "hipMalloc of the read bench's sums failed");
     }

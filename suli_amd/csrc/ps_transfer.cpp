@@ -90,6 +90,7 @@ hipError_t HostPipe::ensure(int device)
         }
     if (e != hipSuccess) {
         release();
+        (void)hipGetLastError();   // the caller copies without pinned memory
         return e;
     }
     ready_ = true;
