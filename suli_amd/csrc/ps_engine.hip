@@ -447,7 +447,12 @@ int Engine::admit(const suli_ps_grid &gr, const SetupIn &in, double *prd1_out, c
     sl.used = true;
     sl.active = true;
     const int rc = setup_slot(si, multi, wait_ev);
-    if (rc) return rc;
+    if (rc) {
+        // the caller never learns of the slot; what is queued still uses its block
+        (void)hipStreamSynchronize(s_);
+        release(si);
+        return rc;
+    }
     if (slot_out) *slot_out = si;
     return 0;
 }

@@ -29,7 +29,7 @@ struct Device {
     CgScalars *status = nullptr;
     int slots = kSlots;
     int launches = 0, waits = 0;
-    int fail_copies = 0;   // asynchronous copies still to fail
+    int skip_copies = 0, fail_copies = 0;   // asynchronous copies: pass these, then fail these
 } dev;
 
 hipError_t fault(hipError_t e)
@@ -77,7 +77,7 @@ hipError_t hipHostFree(void *p)
 }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t)
 {
-    if (dev.fail_copies > 0) return --dev.fail_copies, fault(hipErrorInvalidValue);
+    if (dev.fail_copies > 0 && dev.skip_copies-- <= 0) return --dev.fail_copies, fault(hipErrorInvalidValue);
     std::memmove(d, s, n);
     return hipSuccess;
 }
@@ -224,11 +224,33 @@ void cached()
     CHECK(b.eng.run_all(false) == 0);
 }
 
+// A set-up that fails on the way leaves no problem behind, and its slot and memory
+// serve the next one.
+void failed_setup()
+{
+    Bench b;
+    for (int n : {0, 1}) {   // the scalars' copy to the device, the descriptor's
+        CHECK(b.admit() == 0);   // (takes slot 0)
+        dev.skip_copies = n;
+        dev.fail_copies = 1;
+        int si = -1;
+        CHECK(b.admit(&si) == SULI_PS_EHIP && si < 0);
+        CHECK(dev.fail_copies == 0 && b.eng.active_count() == 1 && !b.eng.slot(1).used);
+        CHECK(hipGetLastError() != hipSuccess);
+        const size_t held = dev.held;
+        CHECK(b.admit(&si) == 0 && si == 1);
+        CHECK(dev.held == held);   // the failed one's block
+        CHECK(b.eng.run_all(false) == 0);
+        b.eng.release(0);
+        b.eng.release(1);
+    }
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
 {
-    const std::map<std::string, void (*)()> scenarios = {{"fallback", fallback}, {"cached", cached}};
+    const std::map<std::string, void (*)()> scenarios = {{"fallback", fallback}, {"cached", cached}, {"failed_setup", failed_setup}};
     const auto it = scenarios.find(argc > 1 ? argv[1] : "");
     if (it == scenarios.end()) return 2;
     it->second();
