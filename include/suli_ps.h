@@ -384,7 +384,9 @@ typedef struct suli_ps_problem {
 /* graddin on `count` independent problems (device pointers, any mix of
  * sizes), solved together: each CG phase is one launch over the tiles of
  * every problem still iterating.  Each problem stops by its own rule and
- * its result is bit-identical to solving it alone with suli_ps_graddin_dev.
+ * its result is bit-identical to solving it alone with suli_ps_graddin_dev
+ * (where device memory does not hold all of them, those that fit are solved
+ * before the next are admitted).
  * The reference solves one grid per call (9_grad.f90:10); this is the same
  * operation applied to many.  Returns the largest per-problem status (0 or
  * 1) or an error; stats.solve_ms is the time of the whole batch. */
@@ -399,8 +401,8 @@ int suli_ps_graddin_batch_dev(suli_ps_ctx *ctx, suli_ps_problem *probs, int32_t 
  * inputs are copied while other requests iterate, and every admitted
  * request joins the running batch at the next chunk of CG steps (the
  * kernels of suli_ps_graddin_batch_dev).  Each result is bit-identical to
- * solving the request alone.  The reference has no counterpart: it solves
- * the one grid of its time loop (1_principal.f90:102). */
+ * solving the request alone under the same budget.  The reference has no
+ * counterpart: it solves the one grid of its time loop (1_principal.f90:102). */
 typedef struct suli_ps_server suli_ps_server;
 
 typedef struct suli_ps_server_opts {

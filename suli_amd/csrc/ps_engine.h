@@ -125,6 +125,8 @@ public:
 
     // Admits a problem: allocates its slot, enqueues the setup kernels on the
     // stream and schedules its iteration 1 at the next global step.
+    // SULI_PS_ENOMEM beside other problems: there may be room once they are
+    // released.
     // prd1_out receives the solution (device, reference layout) when done.
     // block (optional): block_bytes of device memory the caller owns, used
     // instead of the engine's pool: state_bytes() of it, or, for plain CG,

@@ -434,8 +434,11 @@ int Engine::admit(const suli_ps_grid &gr, const SetupIn &in, double *prd1_out, c
     sl.o.vx = vx;
     sl.own_block = block == nullptr;
     sl.block = block ? block : pool_.get(sl.bytes, err_);
-    if (!sl.block && sl.bytes > plain && !no_alloc_active()) {
-        // plain CG where the V-cycle's arrays do not fit any more
+    const bool beside = std::any_of(slots_.begin(), slots_.end(), [](const Slot &t) { return t.used && t.own_block; });
+    if (!sl.block && sl.bytes > plain && !no_alloc_active() && !beside) {
+        // plain CG where the V-cycle's arrays do not fit the device at all.  (Beside
+        // other problems the caller waits for their memory: which iteration a
+        // problem takes does not depend on what it is solved with.)
         multi = false;
         sl.bytes = plain;
         sl.block = pool_.get(sl.bytes, err_);

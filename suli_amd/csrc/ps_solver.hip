@@ -929,28 +929,40 @@ int suli_ps_graddin_batch_dev(suli_ps_ctx *ctx, suli_ps_problem *probs, int32_t 
     HIPCHK(ctx, hipEventRecord(ctx->ev[0], s));
     const SolveOpts so = solve_opts(ctx->opts);
     std::vector<int> slots(count, -1);
+    int first = 0, replays = 0;   // problems first .. i - 1 are resident
+    auto solve = [&](int end) {
+        if ((rc = ctx->eng.run_all(false))) return fail(ctx, rc, "%s", ctx->eng.error().c_str());
+        for (int i = first; i < end; ++i) fill_stats(ctx->eng.slot(slots[i]), &probs[i].stats);
+        replays += ctx->eng.graph_replays();
+        first = end;
+        return 0;
+    };
     for (int i = 0; i < count; ++i) {
         const suli_ps_problem &p = probs[i];
         const SetupIn in = make_setup(&p.grid, p.u, p.v, p.w, p.rho, p.prd1, p.obs_lsx, p.obs_lsy, p.obs_lsz, p.dz,
                                       p.dzz, p.solid);
-        if ((rc = ctx->eng.admit(p.grid, in, p.prd1, so, i, &slots[i]))) {
+        rc = ctx->eng.admit(p.grid, in, p.prd1, so, i, &slots[i]);
+        if (rc == SULI_PS_ENOMEM && i > first) {
+            // no room beside the resident ones: they are solved first
+            if ((rc = solve(i))) return rc;
             release_last(ctx);
-            for (int s2 : slots)
-                if (s2 >= 0) ctx->eng.release(s2);
+            rc = ctx->eng.admit(p.grid, in, p.prd1, so, i, &slots[i]);
+        }
+        if (rc) {
+            release_last(ctx);
             return fail(ctx, rc, "problem %d: %s", i, ctx->eng.error().c_str());
         }
         ctx->last_slots.push_back(slots[i]);
     }
-    if ((rc = ctx->eng.run_all(false))) return fail(ctx, rc, "%s", ctx->eng.error().c_str());
+    if ((rc = solve(count))) return rc;
     HIPCHK(ctx, hipEventRecord(ctx->ev[1], s));
     HIPCHK(ctx, hipEventSynchronize(ctx->ev[1]));
     float ms = 0.f;
     HIPCHK(ctx, hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[1]));
     int worst = SULI_PS_OK;
     for (int i = 0; i < count; ++i) {
-        fill_stats(ctx->eng.slot(slots[i]), &probs[i].stats);
         probs[i].stats.solve_ms = ms;
-        probs[i].stats.graph_replays = ctx->eng.graph_replays();
+        probs[i].stats.graph_replays = replays;
         worst = std::max(worst, probs[i].stats.status);
     }
     return worst;

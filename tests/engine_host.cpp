@@ -24,6 +24,7 @@ struct Device {
     size_t limit = (size_t)-1, held = 0;
     std::map<void *, size_t> blocks;
     std::vector<size_t> refused;
+    std::map<size_t, int> given;   // how many of a size
     // as the runtime's: kept until it is read, successful calls leave it
     hipError_t last = hipSuccess;
     CgScalars *status = nullptr;
@@ -56,6 +57,7 @@ hipError_t hipMalloc(void **p, size_t n)
     }
     *p = std::calloc(n, 1);
     dev.blocks[*p] = n;
+    ++dev.given[n];
     dev.held += n;
     if (n == sizeof(CgScalars) * dev.slots) dev.status = static_cast<CgScalars *>(*p);
     return hipSuccess;
@@ -246,11 +248,61 @@ void failed_setup()
     }
 }
 
+// Beside another problem, one whose multigrid state does not fit waits for memory
+// instead of taking plain CG's.
+void beside()
+{
+    Bench b;
+    dev.limit = dev.held + multi + plain + tables;
+    int si = -1;
+    CHECK(b.admit() == 0);
+    CHECK(b.admit(&si) == SULI_PS_ENOMEM && si < 0);
+    CHECK(b.eng.run_all(false) == 0);
+    b.eng.release(0);
+    CHECK(b.admit(&si) == 0 && b.eng.slot(si).mg);
+    CHECK(b.eng.run_all(false) == 0);
+}
+
+// A batch that does not fit at once is solved in parts, every problem by the
+// iteration that it takes alone.
+void batch()
+{
+    suli_ps_opts o{};
+    o.precision = SULI_PS_FP64;
+    o.stop_rule = SULI_PS_STOP_RELATIVE;
+    o.tol = 1e-8;
+    o.no_graphs = 1;
+    suli_ps_ctx *ctx = suli_ps_create(&o);
+    CHECK(ctx);
+    dev.limit = dev.held + 2 * multi + plain + tables;
+    dev.given.clear();
+    suli_ps_problem p[5] = {};
+    for (auto &q : p) {
+        q.grid = grid();
+        q.u = q.v = q.w = q.rho = q.prd1 = field;
+        q.stats.status = -1;
+    }
+    CHECK(suli_ps_graddin_batch_dev(ctx, p, 5) == 0);
+    for (auto &q : p) CHECK(q.stats.status == 0);
+    CHECK(!dev.given.count(plain) && dev.given[multi] == 2);
+    // none fits
+    dev.limit = 0;
+    suli_ps_destroy(ctx);
+    dev.limit = (size_t)-1;
+    ctx = suli_ps_create(&o);
+    dev.limit = dev.held;
+    CHECK(suli_ps_graddin_batch_dev(ctx, p, 2) == SULI_PS_ENOMEM);
+    suli_ps_destroy(ctx);
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
 {
-    const std::map<std::string, void (*)()> scenarios = {{"fallback", fallback}, {"cached", cached}, {"failed_setup", failed_setup}};
+    const std::map<std::string, void (*)()> scenarios = {
+        {"fallback", fallback},         {"cached", cached}, {"failed_setup", failed_setup},
+        {"beside", beside},             {"batch", batch},
+    };
     const auto it = scenarios.find(argc > 1 ? argv[1] : "");
     if (it == scenarios.end()) return 2;
     it->second();
