@@ -75,7 +75,8 @@ typedef struct suli_ps_opts {
     int32_t stop_rule;     /* enum suli_ps_stop_rule */
     double tol;            /* relative tolerance for SULI_PS_STOP_RELATIVE */
     int32_t max_iter;      /* <= 0: 10000, the reference cap (9_grad.f90:398) */
-    int32_t chunk;         /* CG iterations between host polls; <= 0: automatic */
+    int32_t chunk;         /* CG iterations between host polls (multigrid: at most
+                              2); <= 0: automatic */
     int32_t verbose;       /* 1: print the reference's non-convergence line */
     int32_t timing;        /* 1: time CG steps with HIP events (stats) */
     int32_t keep_null;     /* 1: keep the initial residual's component along the

@@ -295,13 +295,29 @@ void batch()
     suli_ps_destroy(ctx);
 }
 
+// A chunk length chosen for plain CG's steps does not queue as many multigrid steps,
+// of up to a dozen launches each, past the end of a solve.
+void chunk()
+{
+    int launches[3], k = 0;
+    for (int steps : {0, 1, 512}) {
+        Bench b;
+        b.eng.set_chunk(steps);
+        CHECK(b.admit() == 0 && b.eng.slot(0).mg);
+        const int before = dev.launches;
+        CHECK(b.eng.run_all(false) == 0);
+        launches[k++] = dev.launches - before;
+    }
+    CHECK(launches[1] <= launches[0] && launches[2] == launches[0]);
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
 {
     const std::map<std::string, void (*)()> scenarios = {
         {"fallback", fallback},         {"cached", cached}, {"failed_setup", failed_setup},
-        {"beside", beside},             {"batch", batch},
+        {"beside", beside},             {"batch", batch},   {"chunk", chunk},
     };
     const auto it = scenarios.find(argc > 1 ? argv[1] : "");
     if (it == scenarios.end()) return 2;
