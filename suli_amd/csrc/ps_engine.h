@@ -61,6 +61,7 @@ struct Slot {
     double *prd1_out = nullptr;  // device prd1 (halo box) written at the end
     const uint8_t *solid = nullptr;  // solid-cell mask (device), if any
     bool mg = false;           // multigrid-preconditioned: n0 counts multigrid steps
+    bool counting = false;     // the set-up waits for the count of the mask's fluid parts
     suli_ps_grid grid{};       // what it was admitted with, for a second set-up
     SetupIn in{};
     int n0 = 0;
@@ -132,8 +133,14 @@ public:
     // instead of the engine's pool: state_bytes() of it, or, for plain CG,
     // problem_bytes(); wait_ev (optional): the setup kernels
     // wait for it (inputs copied on another stream).
+    // defer: the caller admits more problems and calls set_up_counted() before it
+    // runs any (masked problems then share one wait).
     int admit(const suli_ps_grid &gr, const SetupIn &in, double *prd1_out, const SolveOpts &o, int user,
-              int *slot_out, void *block = nullptr, size_t block_bytes = 0, hipEvent_t wait_ev = nullptr);
+              int *slot_out, void *block = nullptr, size_t block_bytes = 0, hipEvent_t wait_ev = nullptr,
+              bool defer = false);
+    // Sets up the problems that wait for the count of their fluid parts; on an
+    // error those not set up are released.
+    int set_up_counted();
     // Runs chunks until every admitted problem has finished; each finished
     // problem's prd1_out holds its solution and status its final state.
     int run_all(bool timing);
@@ -188,7 +195,9 @@ private:
     int rebuild_tables();
     // Descriptor and set-up kernels of a slot whose geometry and block stand;
     // multi: by the multigrid iteration (state_bytes() of memory).
-    int setup_slot(int si, bool multi, hipEvent_t wait_ev);
+    int setup_slot(int si, bool multi);
+    // Queues the count of a masked problem's fluid parts.
+    int count_parts(int si);
     int enqueue_chunk(int K, bool timing);
     int enqueue_steps_direct(int nsteps, bool timing);
     int enqueue_group_graph();

@@ -384,7 +384,7 @@ long long mg_entries(const Geo &g)
 }
 
 int Engine::admit(const suli_ps_grid &gr, const SetupIn &in, double *prd1_out, const SolveOpts &o, int user,
-                  int *slot_out, void *block, size_t block_bytes, hipEvent_t wait_ev)
+                  int *slot_out, void *block, size_t block_bytes, hipEvent_t wait_ev, bool defer)
 {
     int si = -1;
     for (int i = 0; i < max_slots_; ++i)
@@ -449,7 +449,14 @@ int Engine::admit(const suli_ps_grid &gr, const SetupIn &in, double *prd1_out, c
     sl.user = user;
     sl.used = true;
     sl.active = true;
-    const int rc = setup_slot(si, multi, wait_ev);
+    int rc = 0;
+    if (wait_ev && hipStreamWaitEvent(s_, wait_ev, 0) != hipSuccess)   // the inputs have arrived
+        rc = fail(SULI_PS_EHIP, "admit: hipStreamWaitEvent failed");
+    else if (multi && in.solid)
+        rc = count_parts(si);
+    else
+        rc = setup_slot(si, multi);
+    if (!rc && !defer) rc = set_up_counted();
     if (rc) {
         // the caller never learns of the slot; what is queued still uses its block
         (void)hipStreamSynchronize(s_);
@@ -460,7 +467,40 @@ int Engine::admit(const suli_ps_grid &gr, const SetupIn &in, double *prd1_out, c
     return 0;
 }
 
-int Engine::setup_slot(int si, bool multi, hipEvent_t wait_ev)
+// A mask that cuts the fluid into parts is for plain CG.  The host waits for the
+// count, once for all the problems that are admitted together: set up first and
+// found out by the kernels, such a problem was set up twice and ran idle steps
+// (31x156x109, FP64: 16.5 ms instead of 16.0).
+int Engine::count_parts(int si)
+{
+    Slot &sl = slots_[si];
+    const suli_ps_grid &gr = sl.grid;
+    const Geo g = make_geo(gr.nx, gr.ny, gr.nz, gr.ccx0 == 0, gr.ccy0 == 0);
+    int *lab = static_cast<int *>(sl.block), *count = lab + g.n;
+    launch_mg_parts(g, sl.in.solid, lab, count, s_);
+    ECHK(hipMemcpyAsync(h_final_ + si, count, sizeof(int), hipMemcpyDeviceToHost, s_));
+    sl.counting = true;
+    return 0;
+}
+
+int Engine::set_up_counted()
+{
+    const auto counting = [](const Slot &sl) { return sl.used && sl.counting; };
+    if (std::none_of(slots_.begin(), slots_.end(), counting)) return 0;
+    int rc = hipStreamSynchronize(s_) == hipSuccess ? 0 : fail(SULI_PS_EHIP, "hipStreamSynchronize failed");
+    for (int i = 0; i < max_slots_; ++i) {
+        if (!counting(slots_[i])) continue;
+        slots_[i].counting = false;
+        if (!rc) rc = setup_slot(i, *reinterpret_cast<const int *>(h_final_ + i) <= 1);
+        if (rc) {
+            (void)hipStreamSynchronize(s_);
+            release(i);
+        }
+    }
+    return rc;
+}
+
+int Engine::setup_slot(int si, bool multi)
 {
     Slot &sl = slots_[si];
     const suli_ps_grid &gr = sl.grid;
@@ -468,19 +508,6 @@ int Engine::setup_slot(int si, bool multi, hipEvent_t wait_ev)
     const SolveOpts &o = sl.o;
     ProbDev &pd = sl.pd;
     int nt3 = 0, nt1 = 0;
-    if (wait_ev) ECHK(hipStreamWaitEvent(s_, wait_ev, 0));   // the inputs have arrived
-    if (multi && in.solid) {
-        // plain CG where a mask cuts the fluid into parts.  The host waits for
-        // the count (20 us): set up first and found out by the kernels, such a
-        // problem was set up twice and ran idle steps (31x156x109, FP64: 16.5
-        // ms instead of 16.0)
-        const Geo g = make_geo(gr.nx, gr.ny, gr.nz, gr.ccx0 == 0, gr.ccy0 == 0);
-        int *lab = static_cast<int *>(sl.block), *count = lab + g.n, *h = reinterpret_cast<int *>(h_final_ + si);
-        launch_mg_parts(g, in.solid, lab, count, s_);
-        ECHK(hipMemcpyAsync(h, count, sizeof(int), hipMemcpyDeviceToHost, s_));
-        ECHK(hipStreamSynchronize(s_));
-        multi = *h <= 1;
-    }
     // the multigrid kernels have a tiling of their own: the replacement's
     // kernels, which walk one cell per lane, take the default shape
     sl.mg = false;
@@ -1080,7 +1107,7 @@ int Engine::pump(bool timing, std::vector<int> &finished)
         if (sl.mg && h[i].giveup) {
             // the multigrid iteration broke down: the whole solve again by
             // plain CG (its inputs and prd1 still stand)
-            if ((rc = setup_slot(i, false, nullptr))) return rc;
+            if ((rc = setup_slot(i, false))) return rc;
             continue;
         }
         done.push_back(i);

@@ -931,7 +931,7 @@ int suli_ps_graddin_batch_dev(suli_ps_ctx *ctx, suli_ps_problem *probs, int32_t 
     std::vector<int> slots(count, -1);
     int first = 0, replays = 0;   // problems first .. i - 1 are resident
     auto solve = [&](int end) {
-        if ((rc = ctx->eng.run_all(false))) return fail(ctx, rc, "%s", ctx->eng.error().c_str());
+        if ((rc = ctx->eng.set_up_counted()) || (rc = ctx->eng.run_all(false))) return fail(ctx, rc, "%s", ctx->eng.error().c_str());
         for (int i = first; i < end; ++i) fill_stats(ctx->eng.slot(slots[i]), &probs[i].stats);
         replays += ctx->eng.graph_replays();
         first = end;
@@ -941,12 +941,13 @@ int suli_ps_graddin_batch_dev(suli_ps_ctx *ctx, suli_ps_problem *probs, int32_t 
         const suli_ps_problem &p = probs[i];
         const SetupIn in = make_setup(&p.grid, p.u, p.v, p.w, p.rho, p.prd1, p.obs_lsx, p.obs_lsy, p.obs_lsz, p.dz,
                                       p.dzz, p.solid);
-        rc = ctx->eng.admit(p.grid, in, p.prd1, so, i, &slots[i]);
+        auto admit = [&] { return ctx->eng.admit(p.grid, in, p.prd1, so, i, &slots[i], nullptr, 0, nullptr, true); };
+        rc = admit();
         if (rc == SULI_PS_ENOMEM && i > first) {
             // no room beside the resident ones: they are solved first
             if ((rc = solve(i))) return rc;
             release_last(ctx);
-            rc = ctx->eng.admit(p.grid, in, p.prd1, so, i, &slots[i]);
+            rc = admit();
         }
         if (rc) {
             release_last(ctx);

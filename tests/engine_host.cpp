@@ -311,6 +311,32 @@ void chunk()
     CHECK(launches[1] <= launches[0] && launches[2] == launches[0]);
 }
 
+// The masked problems of a batch share one wait for the counts of their fluid parts.
+void masks()
+{
+    static uint8_t solid[kN * kN * kN];
+    int waits[2], k = 0;
+    for (int count : {1, 8}) {
+        suli_ps_opts o{};
+        o.precision = SULI_PS_MIXED;
+        o.stop_rule = SULI_PS_STOP_RELATIVE;
+        o.tol = 1e-8;
+        suli_ps_ctx *ctx = suli_ps_create(&o);
+        suli_ps_problem p[8] = {};
+        for (auto &q : p) {
+            q.grid = grid();
+            q.u = q.v = q.w = q.rho = q.prd1 = field;
+            q.solid = solid;
+        }
+        for (int i = 1; i < count; i += 2) p[i].solid = nullptr;
+        const int before = dev.waits;
+        CHECK(suli_ps_graddin_batch_dev(ctx, p, count) == 0);
+        waits[k++] = dev.waits - before;
+        suli_ps_destroy(ctx);
+    }
+    CHECK(waits[1] == waits[0]);
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -318,6 +344,7 @@ int main(int argc, char **argv)
     const std::map<std::string, void (*)()> scenarios = {
         {"fallback", fallback},         {"cached", cached}, {"failed_setup", failed_setup},
         {"beside", beside},             {"batch", batch},   {"chunk", chunk},
+        {"masks", masks},
     };
     const auto it = scenarios.find(argc > 1 ? argv[1] : "");
     if (it == scenarios.end()) return 2;

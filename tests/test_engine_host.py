@@ -23,7 +23,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["fallback", "cached", "failed_setup", "beside", "batch", "chunk"])
+@pytest.mark.parametrize("scenario", ["fallback", "cached", "failed_setup", "beside", "batch", "chunk", "masks"])
 def test_scenario(program, scenario):
     r = subprocess.run([program, scenario], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)
