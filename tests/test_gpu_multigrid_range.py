@@ -95,3 +95,49 @@ def test_breakdown_is_solved_again_by_plain_cg(solver, precision, tol):
             st = srv.wait(t)
             assert st.status == 0 and st.iters == alone[i][1].iters, i
             np.testing.assert_array_equal(f.prd1, alone[i][0])
+
+
+def test_stalled_replacements_end_by_plain_cg(solver):
+    """A tolerance below what FP64 resolves: after three replacements that do not
+    halve the residual the solve is plain CG's, which runs to its cap."""
+    c = cases.random_case(36, 30, 22, 97)
+    print("multigrid stalls", flush=True)
+    solver.configure(precision="mixed", stop_rule="relative", tol=1e-19, max_iter=300, verbose=False)
+    p, st = solve(solver, c, c.fields)
+    assert st.status == 1 and st.iters == 300, st.as_dict()
+    solver.configure(precision="fp64", stop_rule="relative", tol=1e-12, verbose=False)
+    p64, st64 = solve(solver, c, c.fields)
+    assert st64.status == 0
+    # 300 plain iterations: a residual of about 1e-8
+    assert st.rel_true < 1e-6 and helpers.rel_diff(p, p64, helpers.face_mask(p.shape)) < 1e-4
+
+
+def flat(shape, ax, ay, seed):
+    c = cases.random_case(*shape, seed)
+    c.grid.dx *= ax
+    c.grid.dy *= ay
+    return c
+
+
+# (grid, dx / dz, dy / dz, most iterations to 1e-12).  On cells of unequal sides the
+# point smoother and the 2x2x2 coarsening take more: 40x32x24 took 24, 73, 143 and 212
+# for 2, 4, 8 and 16 (plain CG 560, 1024, 2184, 10000 mixed), 77, 132 and 231 for
+# 1/4, 1/8 and 1/16 (656, 1024, 2584).
+FLAT = [((40, 32, 24), a, a, most) for a, most in
+        ((1, 20), (2, 35), (4, 100), (8, 190), (16, 300), (1 / 4, 110), (1 / 8, 180), (1 / 16, 320))]
+FLAT += [((64, 48, 40), 4, 4, 150), ((64, 48, 40), 1 / 4, 1 / 4, 150)]      # marched tiles
+# thin grids of cubes
+FLAT += [((160, 160, 2), 1, 1, 40), ((200, 2, 130), 1, 1, 40), ((3, 130, 128), 1, 1, 40)]
+
+
+@pytest.mark.parametrize("shape,ax,ay,most", FLAT)
+def test_iterations_on_flat_and_thin_cells(solver, shape, ax, ay, most):
+    c = flat(shape, ax, ay, 98)
+    for precision, tol in (("fp64", 1e-12), ("mixed", 1e-11)):
+        print(f"multigrid flat {shape} {ax} {ay} {precision}", flush=True)
+        solver.configure(precision=precision, stop_rule="relative", tol=tol, verbose=False)
+        _, st = solve(solver, c, c.fields)
+        assert st.status == 0 and st.iters <= most, (precision, st.as_dict())
+        solver.configure(precision=precision, stop_rule="relative", tol=tol, verbose=False, keep_null=True)
+        _, plain = solve(solver, c, c.fields)
+        assert st.iters < 0.5 * plain.iters, (st.iters, plain.iters)
