@@ -224,6 +224,7 @@ private:
     int pend_[2] = {0, 0};             // status slots of chunks not yet read (FIFO)
     int pend_head_ = 0, npend_ = 0;
     int max_slots_ = 0;
+    int counting_ = 0;                 // problems admitted since set_up_counted() that wait for it (or were released)
     int step_ = 0;                     // global step of the last enqueued iteration
     int mstep_ = 0;                    // multigrid problems' own step count
     int status_seen_ = 0;              // its value when the last state read was queued

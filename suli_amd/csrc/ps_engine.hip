@@ -434,8 +434,10 @@ int Engine::admit(const suli_ps_grid &gr, const SetupIn &in, double *prd1_out, c
     sl.o.vx = vx;
     sl.own_block = block == nullptr;
     sl.block = block ? block : pool_.get(sl.bytes, err_);
-    const bool beside = std::any_of(slots_.begin(), slots_.end(), [](const Slot &t) { return t.used && t.own_block; });
-    if (!sl.block && sl.bytes > plain && !no_alloc_active() && !beside) {
+    auto beside = [&] {
+        return std::any_of(slots_.begin(), slots_.end(), [](const Slot &t) { return t.used && t.own_block; });
+    };
+    if (!sl.block && sl.bytes > plain && !no_alloc_active() && !beside()) {
         // plain CG where the V-cycle's arrays do not fit the device at all.  (Beside
         // other problems the caller waits for their memory: which iteration a
         // problem takes does not depend on what it is solved with.)
@@ -480,16 +482,17 @@ int Engine::count_parts(int si)
     launch_mg_parts(g, sl.in.solid, lab, count, s_);
     ECHK(hipMemcpyAsync(h_final_ + si, count, sizeof(int), hipMemcpyDeviceToHost, s_));
     sl.counting = true;
+    ++counting_;
     return 0;
 }
 
 int Engine::set_up_counted()
 {
-    const auto counting = [](const Slot &sl) { return sl.used && sl.counting; };
-    if (std::none_of(slots_.begin(), slots_.end(), counting)) return 0;
+    if (!counting_) return 0;
+    counting_ = 0;
     int rc = hipStreamSynchronize(s_) == hipSuccess ? 0 : fail(SULI_PS_EHIP, "hipStreamSynchronize failed");
     for (int i = 0; i < max_slots_; ++i) {
-        if (!counting(slots_[i])) continue;
+        if (!slots_[i].used || !slots_[i].counting) continue;
         slots_[i].counting = false;
         if (!rc) rc = setup_slot(i, *reinterpret_cast<const int *>(h_final_ + i) <= 1);
         if (rc) {
