@@ -29,7 +29,10 @@ coarse correction's residual (3), z (5), the direction step (6); faces, which
 regular rows take from small tables, and the coarse levels, about a seventh of
 the cells, are not counted.  The time is the step's mean over windows of 2
 consecutive steps between HIP events on the solver's stream during two
-solves, all of its launches and the gaps between them included.
+solves, all of its launches and the gaps between them included.  `traffic` is
+the step's HBM bytes from rocprofv3's FETCH_SIZE and WRITE_SIZE counters
+(profiles/hbm_traffic.json), coarse levels included, and `traffic_achieved`
+those bytes in the same time.
 `copy_kernel` and `read_kernel` give what a plain 256 MiB copy and a plain
 read reach on the same GPU in the same run: the HBM rates a kernel that
 mixes reads and writes can be held against.
@@ -578,11 +581,15 @@ def main():
     launch_ms = mixed["step_ms"]
     alg = MG_WORDS * 4 * n
     achieved = alg / (launch_ms * 1e-3) / 1e9
+    traffic = load_traffic(f"multigrid iteration {g.nx}x{g.ny}x{g.nz}")
     spmv_gbs = SPMV_WORDS * 4 * n / (mixed["spmv_only_ms"] * 1e-3) / 1e9
     fp64_step = fp64["step_ms"]
     roofline = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": achieved / HBM_PEAK_GBS,
-                "traffic": load_traffic(f"multigrid iteration {g.nx}x{g.ny}x{g.nz}"),
+                "traffic": traffic,
+                # the bytes the step moves (profiled HBM traffic) at its rate
+                "traffic_achieved": traffic / (launch_ms * 1e-3) / 1e9 if traffic else None,
+                "traffic_frac": traffic / (launch_ms * 1e-3) / 1e9 / HBM_PEAK_GBS if traffic else None,
                 "kernel": "multigrid iteration (k_mg_fine, k_mg_level, k_mg_bottom)", "launch_ms": launch_ms,
                 "algorithmic_bytes_per_launch": alg,
                 "algorithmic_basis": "one FP32 iteration's passes over the fine grid, 22 words/cell",
