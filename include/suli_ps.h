@@ -37,9 +37,10 @@ enum suli_ps_precision {
     SULI_PS_MIXED = 1   /* FP32 CG, preconditioned likewise, inside FP64
                            residual replacement */
     /* The plain CG iteration instead: FP64 by the reference rule, keep_null,
-     * stored_residual, 0 < max_iter < 256, grids of fewer than 4096 cells, a
-     * tile shape fixed with suli_ps_set_tiles (and autotune), and masks that
-     * cut the fluid into parts. */
+     * stored_residual, 0 < max_iter < 256, grids of fewer than 4096 cells or
+     * more than some 40 million, a tile shape fixed with suli_ps_set_tiles
+     * (and autotune), masks that cut the fluid into parts, and FP64 problems
+     * whose larger state the device (the server: its budget) does not hold. */
 };
 
 enum suli_ps_stop_rule {

@@ -183,7 +183,8 @@ public:
     // Fixes the tile shape of a size (as if tuned).
     void set_tiles(int nx, int ny, int nz, bool mixed, int kz, int vx);
     // Fixed chunk length (steps between host polls; rounded up to the
-    // refresh grain), or automatic when <= 0.
+    // refresh grain; multigrid problems alone: at most kMgChunk), or automatic
+    // when <= 0.
     void set_chunk(int steps) { chunk_ = steps; }
     bool graphs() const { return graphs_; }
     int graph_captures() const { return captures_; }

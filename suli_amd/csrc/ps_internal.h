@@ -44,7 +44,11 @@ static_assert((kFold & (kFold - 1)) == 0, "kFold is a power of two");
 //
 // kMgMinCells: below, the hierarchy does not fit the memory it shares.  Plain
 // CG against this from prd1 = 0 to 1e-12 relative, mixed: 4096 cells 2.20 and
-// 0.96 ms, 15360 cells 3.25 and 1.00, 46080 cells 4.51 and 1.20.
+// 0.96 ms, 15360 cells 3.25 and 1.00, 46080 cells 4.51 and 1.20; 4096 cells eight
+// times as wide as high 6.0 and 3.5, eight times as high as wide 7.8 and 3.6; 4096
+// cells to 1e-2 only 0.90 and 0.35.  Above some 40 million cells the partial sums
+// of the fine tiles do not fit the space that mixed solves keep for them
+// (mg_entries), and plain CG stays.
 constexpr long long kMgMinCells = 4096;
 // A cap below this keeps plain CG: a capped solve returns CG's iterate.
 constexpr int kMgMinCap = 256;

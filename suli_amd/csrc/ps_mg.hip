@@ -4,7 +4,16 @@
 // that grows with the square of the grid's longest side, so plain CG takes
 // about a thousand iterations on a 256x128x96 two-phase tank.  Here one
 // iteration applies a V-cycle M to the residual first (z = M r, p = z + beta
-// p, beta and alpha from r.z) and takes 10 to 25 on any grid.
+// p, beta and alpha from r.z) and takes 10 to 25 on cells of about equal sides.
+//
+// The smoother works on points and the coarsening joins 2x2x2 cells whatever
+// their sides are, so flat and tall cells take more: 40x32x24, mixed from
+// prd1 = 0 to 1e-12, with dx = dy = 1/16, 1/8, 1/4, 1, 2, 4, 8, 16 dz: 231,
+// 132, 77, 14, 24, 73, 143, 212 iterations and 9.9, 5.8, 3.4, 0.82, 1.25, 3.2,
+// 6.2, 9.1 ms (plain CG 2584, 1024, 656, 416, 560, 1024, 2184, 10000 and 21.6,
+// 8.9, 5.9, 4.0, 5.1, 8.9, 18.4, 82.6 ms; at 256x128x96 185 to 72 ms at 1/16,
+// 218 to 61 at 16).  No grid tried, from 4096 cells to 3 million and from 1/32 to
+// 32, was faster by plain CG (FP64 at 4096 cells and 1/32: 7.4 and 5.9 ms).
 //
 // Mixed solves: everything is FP32 inside FP64 residual replacement, as the CG
 // step: dot products, alpha and beta are FP64 and convergence is judged on
@@ -266,7 +275,8 @@ __device__ __forceinline__ double mg_tile(const ProbDev &pd, int tile, const Fin
         return v_of(ld1(a_ + kk * plane, o), kTwo ? ld1(b_ + kk * plane, o) : 0.f);
     };
 
-    // the rows' table bits for the tile's planes (planes past 32 read the arrays)
+    // the rows' table bits for the tile's planes (planes past 32, which mg_plan's
+    // tiles of at most 8 do not have, would read the arrays)
     unsigned bita = 0, bitb = 0;
     if (pd.rowreg) {
         const gptr<const unsigned> rr = glob((const unsigned *)pd.rowreg);
