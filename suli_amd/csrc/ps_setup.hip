@@ -623,6 +623,24 @@ constexpr int kPressThreads = 512, kPressWaves = kPressThreads / 64, kPressChunk
 constexpr int kPressPer = kPressChunk / kPressWaves;
 constexpr int kWThreads = 256, kWWaves = kWThreads / 64, kWChunk = 16, kWPer = kWChunk / kWWaves;
 
+// Where columns are many or short, a lane per column is the faster one
+// (k_pressh_columns, k_posdin_hydro_w_columns: kColumnAhead planes' loads together,
+// the recurrence in registers): there is no LDS to wait for, and no wave without a
+// plane.  Kernel times in us, columns x planes, chunks and lanes:
+//   pressh          16384 x 4 3.4 3.1    x 8 3.5 3.7    x 16 4.1 5.2   x 128 12.4 26.2
+//                   32768 x 8 4.3 3.8    x 16 5.4 5.6   x 64 10.6 15.3  x 128 19.1 27.9
+//                   73728 x 8 6.0 4.5    x 32 10.4 10.8 x 64 16.8 18.5  x 128 30.3 32.8
+//                   98304 x 32 12.4 11.7 x 64 21.6 20.0 x 128 41.1 35.7
+//                   262144 x 2 9.8 3.6   x 32 25.6 22.6 x 64 61 50      x 128 138 115
+//                   1048576 x 2 30 6.3   x 16 73 49     x 64 292 262
+//   posdin_hydro_w  16384 x 2 4.1 4.2    x 8 4.3 5.0    x 64 13.3 20.4
+//                   65536 x 2 6.4 5.3    x 12 8.2 10.9  x 64 32 35
+//                   262144 x 4 14.6 10.3 x 8 15.8 14.4  x 12 18.7 22.2  x 64 110 119
+//                   1048576 x 8 74 55    x 17 154 135   x 32 224 236    x 64 458 475
+constexpr int kColumnAhead = 8;
+bool pressh_in_chunks(long long ncol, int nz) { return nz >= 8 && ncol <= 5 << 14 && 2048LL * nz >= ncol; }
+bool hydro_w_in_chunks(long long ncol, int nz) { return ncol <= 16384 || (nz > 8 && 32768LL * nz >= ncol); }
+
 // pressh, the hydrostatic pressure of t_press = 0 (SuLi-IC/9_grad.f90:
 // 667-702; dz(k) weights: SuLi-ICdz/9_grad.f90:665-700).  Each (i, j) column
 // goes from the top: the top cell takes dz g rho, the one below the trapezoid of
@@ -698,6 +716,60 @@ __global__ __launch_bounds__(kPressThreads) void k_pressh(Geo g, const double *_
         for (int q = 0; q < kPressPer; ++q) {
             const int m = wave + q * kPressWaves, K = K0 - m;
             if (K >= 1 && act) pc[(long long)K * pbb] = t[m][lane];
+        }
+    }
+}
+
+// The same with a lane per column, lanes of a wave consecutive i.
+__global__ __launch_bounds__(kThreads) void k_pressh_columns(Geo g, const double *__restrict__ rho, const double *dz, double dzu,
+                                                     double gz, double *__restrict__ prd1)
+{
+    const int nx = g.nx, ny = g.ny, nz = g.nz;
+    const long long col = (long long)blockIdx.x * kThreads + threadIdx.x;
+    if (col >= (long long)nx * ny) return;
+    const int i = (int)(col % nx), j = (int)(col / nx);
+    const long long plane = (long long)nx * ny;
+    const long long pbb = (long long)(nx + 2) * (ny + 2);
+    const double *rc = rho + col;
+    double *pc = prd1 + (i + 1) + (long long)(nx + 2) * (j + 1);
+    double p1 = 0.0, p2 = 0.0;  // prd1 at k+1, k+2
+    double r1 = 0.0, r2 = 0.0;  // rho at k+1, k+2
+    // rho of kColumnAhead planes loaded together, then the recurrence over
+    // them: one round trip per block of planes instead of one per plane
+    for (int K0 = nz; K0 >= 1; K0 -= kColumnAhead) {
+        double rb[kColumnAhead];
+#pragma unroll
+        for (int m = 0; m < kColumnAhead; ++m) rb[m] = K0 - m >= 1 ? rc[(long long)(K0 - m - 1) * plane] : 0.0;
+#pragma unroll
+        for (int m = 0; m < kColumnAhead; ++m) {
+            const int K = K0 - m;
+            if (K < 1) break;
+            const double r0 = rb[m];
+            double p;
+            if (dz) {
+                if (K == nz) {
+                    p = dz[K] * gz * r0;
+                } else if (K == nz - 1) {
+                    p = gz * (r0 * dz[K] + r1 * dz[K + 1]) * 0.5 + p1;
+                } else {
+                    const double intz = (r0 * dz[K] + 4. * r1 * dz[K + 1] + r2 * dz[K + 2]) / 3.;
+                    p = gz * intz + p2;
+                }
+            } else {
+                if (K == nz) {
+                    p = dzu * gz * r0;
+                } else if (K == nz - 1) {
+                    p = dzu * gz * (r0 + r1) * 0.5 + p1;
+                } else {
+                    const double intz = dzu * (r0 + 4. * r1 + r2) / 3.;
+                    p = gz * intz + p2;
+                }
+            }
+            pc[(long long)K * pbb] = p;
+            p2 = p1;
+            p1 = p;
+            r2 = r1;
+            r1 = r0;
         }
     }
 }
@@ -783,6 +855,60 @@ __global__ __launch_bounds__(kWThreads) void k_posdin_hydro_w(Geo g, const doubl
         for (int q = 0; q < kWPer; ++q) {
             const int m = wave + q * kWWaves, K = K0 + m;
             if (K <= nz && act) wc[(long long)(K + 1) * wbb] = (dry >> q & 1u) ? 0. : ta[m][lane];
+        }
+    }
+}
+
+// The same with a lane per column.
+template <bool DZ>
+__global__ __launch_bounds__(kThreads) void k_posdin_hydro_w_columns(Geo g, const double *u, const double *v,
+                                                             const double *hs, const double *dz, double dzu,
+                                                             double dx, double dy, double *w)
+{
+    const int nx = g.nx, ny = g.ny, nz = g.nz;
+    const long long t = (long long)blockIdx.x * kThreads + threadIdx.x;
+    if (t >= (long long)(nx + 2) * (ny + 2)) return;
+    const int I = (int)(t % (nx + 2)), J = (int)(t / (nx + 2));
+    const long long wbb = (long long)(nx + 2) * (ny + 2);
+    double *wc = w + t;
+    wc[wbb] = 0.;  // w(:,:,1) = 0
+    if (I < 1 || I > nx || J < 1 || J > ny) return;
+    const long long ubb = (long long)(nx + 3) * (ny + 2), vbb = (long long)(nx + 2) * (ny + 3);
+    const double *uc = u + I + (long long)(nx + 3) * J;
+    const double *vc = v + I + (long long)(nx + 2) * J;
+    double wk = 0.;
+    if (face_z(g, hs, dz, I - 1, J - 1, 0) < 0.0001) wc[wbb] = 0.;
+    // u, v and the two hs cells of the z face of kColumnAhead planes loaded
+    // together (no branch between the loads), then the chain over them
+    // (DZ: the stretched grid's dz(K) and the face weights too)
+    const long long plane = (long long)nx * ny;
+    const double *hc = hs + (long long)(J - 1) * nx + (I - 1);
+    for (int K0 = 1; K0 <= nz; K0 += kColumnAhead) {
+        double u0[kColumnAhead], u1[kColumnAhead], v0[kColumnAhead], v1[kColumnAhead];
+        double h1[kColumnAhead], h0[kColumnAhead], dk[kColumnAhead], d1[kColumnAhead], d0[kColumnAhead];
+#pragma unroll
+        for (int m = 0; m < kColumnAhead; ++m) {
+            const int K = K0 + m <= nz ? K0 + m : nz;
+            const int a = face_z_upper(g, K);
+            u1[m] = uc[(long long)K * ubb + 1];
+            u0[m] = uc[(long long)K * ubb];
+            v1[m] = vc[(long long)K * vbb + (nx + 2)];
+            v0[m] = vc[(long long)K * vbb];
+            h1[m] = hc[a * plane];
+            h0[m] = hc[(a - 1) * plane];
+            dk[m] = DZ ? dz[K] : dzu;
+            d1[m] = DZ ? dz[a + 1] : 0.0;
+            d0[m] = DZ ? dz[a] : 0.0;
+        }
+#pragma unroll
+        for (int m = 0; m < kColumnAhead; ++m) {
+            const int K = K0 + m;
+            if (K > nz) break;
+            const double dzk = dk[m];
+            const double du = u1[m] - u0[m], dv = v1[m] - v0[m];
+            wk = wk - du * dzk / dx - dv * dzk / dy;
+            const double hf = DZ ? face_z_weighted(h1[m], h0[m], d1[m], d0[m]) : (h1[m] + h0[m]) * 0.5;
+            wc[(long long)(K + 1) * wbb] = hf < 0.0001 ? 0. : wk;
         }
     }
 }
@@ -1370,8 +1496,12 @@ void launch_pressh(const Geo &g, const double *rho, const double *dz, double dzu
                    hipStream_t s)
 {
     const long long ncol = (long long)g.nx * g.ny;
-    hipLaunchKernelGGL(k_pressh, dim3((unsigned)((ncol + 63) / 64)), dim3(kPressThreads), 0, s, g, rho,
-                       dz, dzu, gz, prd1);
+    if (pressh_in_chunks(ncol, g.nz))
+        hipLaunchKernelGGL(k_pressh, dim3((unsigned)((ncol + 63) / 64)), dim3(kPressThreads), 0, s, g, rho, dz, dzu, gz,
+                           prd1);
+    else
+        hipLaunchKernelGGL(k_pressh_columns, dim3((unsigned)((ncol + kThreads - 1) / kThreads)), dim3(kThreads), 0, s,
+                           g, rho, dz, dzu, gz, prd1);
 }
 
 void launch_posdin_hydro(const Geo &g, const SetupIn &in, const double *hs, double *u, double *v, double *w,
@@ -1379,13 +1509,12 @@ void launch_posdin_hydro(const Geo &g, const SetupIn &in, const double *hs, doub
 {
     hipLaunchKernelGGL(k_posdin, cell_grid(g), dim3(kThreads), 0, s, g, in, u, v, w, false);
     const long long nplane = (long long)(g.nx + 2) * (g.ny + 2);
-    const dim3 grid((unsigned)((nplane + 63) / 64));
-    if (in.dz)
-        hipLaunchKernelGGL(k_posdin_hydro_w<true>, grid, dim3(kWThreads), 0, s, g, u, v, hs, in.dz, in.dzu, in.dx, in.dy,
-                           w);
-    else
-        hipLaunchKernelGGL(k_posdin_hydro_w<false>, grid, dim3(kWThreads), 0, s, g, u, v, hs, in.dz, in.dzu, in.dx,
-                           in.dy, w);
+    const bool chunks = hydro_w_in_chunks((long long)g.nx * g.ny, g.nz);
+    const int threads = chunks ? kWThreads : kThreads, per = chunks ? 64 : kThreads;   // columns a workgroup
+    auto *const sweep = chunks ? (in.dz ? k_posdin_hydro_w<true> : k_posdin_hydro_w<false>)
+                               : (in.dz ? k_posdin_hydro_w_columns<true> : k_posdin_hydro_w_columns<false>);
+    hipLaunchKernelGGL(sweep, dim3((unsigned)((nplane + per - 1) / per)), dim3(threads), 0, s, g, u, v, hs, in.dz,
+                       in.dzu, in.dx, in.dy, w);
     const int uv_tiles = (g.nx + 63) / 64 * ((g.ny + 3) / 4) * ((g.nz + kUvPlanes - 1) / kUvPlanes);
     hipLaunchKernelGGL(k_posdin_hydro_uv, dim3(uv_tiles), dim3(kThreads), 0, s, g, hs, u, v);
 }
